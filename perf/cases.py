@@ -368,3 +368,85 @@ def tolerance(case):
     if case["precision"] == "bf16":
         return {"rel": 5e-3, "max": 3e-2}                # a value stored as bf16 may round the other way
     return {"rel": 3e-6, "max": 3e-5}
+
+
+# --------------------------------------------------------------------------- the same in 64 bits, by torch alone
+def _double(array):
+    return _view(array).double()
+
+
+def _exact_layer(layer, x, p, training):
+    if isinstance(layer, Module):
+        return _exact_net(layer, x, p, training)
+    if isinstance(layer, Conv2D):
+        w = p(layer._parameters[0])
+        x = torch.nn.functional.conv2d(x, w, p(layer._parameters[1]).reshape(-1), layer.stride, layer.pad_size)
+        return x.relu() if layer.activation is not None else x
+    if isinstance(layer, BatchNormalization):
+        gamma, beta = (p(q).reshape(1, -1, 1, 1) for q in layer._parameters)
+        if training:
+            mean, var = x.mean((0, 2, 3), keepdim=True), x.var((0, 2, 3), unbiased=False, keepdim=True)
+        else:
+            mean, var = (_double(q.eval).reshape(1, -1, 1, 1) for q in (layer.moving_mean, layer.moving_variance))
+        return (x - mean) / torch.sqrt(var + layer.epsilon) * gamma + beta
+    if isinstance(layer, ReLU):
+        return x.relu()
+    if isinstance(layer, MaxPooling2D):
+        k, pad = layer.kernel_size, layer.padding
+        k = k if isinstance(k, int) else k[0]
+        x = torch.nn.functional.pad(x, (pad,) * 4)           # border cells compete with their zeros
+        return torch.nn.functional.max_pool2d(x, k, layer.stride)
+    if isinstance(layer, AvgPooling2D):
+        return x.mean((2, 3), keepdim=True)                  # the window is the whole map
+    if isinstance(layer, Flatten):
+        return x.flatten(1)
+    return x @ p(layer._parameters[0]) + p(layer._parameters[1])
+
+
+def _exact_seq(seq, x, p, training):
+    for layer in seq._graph or []:
+        x = _exact_layer(layer, x, p, training)
+    return x
+
+
+def _exact_net(net, x, p, training):
+    if isinstance(net, _Block):
+        return (_exact_seq(net.body, x, p, training) + _exact_seq(net.shortcut, x, p, training)).relu()
+    if isinstance(net, _ResNet18):
+        x = _exact_layer(net.pool, _exact_seq(net.stem, x, p, training), p, training)
+        return _exact_seq(net.tail, _exact_seq(net.stages, x, p, training), p, training)
+    return _exact_seq(net, x, p, training)
+
+
+def exact(case, seed):
+    """What ``run`` returns for these inputs, computed by torch in 64 bits."""
+    state = prepare(case, seed)
+    kind = case["kind"]
+    with torch.backends.cudnn.flags(enabled=False):          # torch's own convolution takes 64 bits
+        if kind == "conv":
+            x, w, b = (_double(state[q].eval).requires_grad_() for q in ("x", "w", "b"))
+            y = torch.nn.functional.conv2d(x, w, b.reshape(-1), (case["stride"],) * 2, case["pad"])
+            y = y.relu() if case["relu"] else y
+            grads = torch.autograd.grad(y, (x, w, b), _double(state["dy"].eval))
+            return [*grads, y.detach()]
+        if kind == "pool":
+            x = _double(state["x"].eval).requires_grad_()
+            y = torch.nn.functional.max_pool2d(torch.nn.functional.pad(x, (case["pad"],) * 4), case["k"], case["stride"])
+            return [torch.autograd.grad(y, x, _double(state["dy"].eval))[0], y.detach()]
+        held = {}
+
+        def p(parameter):
+            if id(parameter) not in held:
+                held[id(parameter)] = _double(parameter.eval).requires_grad_(kind != "infer")
+            return held[id(parameter)]
+
+        x = _double(state["x"].eval)
+        if kind == "infer":
+            with torch.no_grad():
+                parts = 4 if case["n"] >= 64 else 1          # the unfolded images of a whole batch are many
+                return [torch.cat([_exact_net(state["net"], part, p, False) for part in x.chunk(parts)])]
+        logits = _exact_net(state["net"], x, p, True)
+        loss = torch.nn.functional.cross_entropy(logits, _view(state["y"].eval).reshape(-1))
+        params = [p(q) for q in state["params"]]
+        grads = torch.autograd.grad(loss, params)
+        return [(q - 0.01 * g).detach() for q, g in zip(params, grads)] + [loss.detach().reshape(1), logits.detach()]
