@@ -1,0 +1,103 @@
+"""The fp32 convolution on bf16 matrix pipes (three-way split operands): every geometry it serves against the oracle,
+at the edges of its tiles, channel groups, phases and grids.
+
+Bound: the split drops products below 2^-25 of each term and adds in float32; the worst of the sizes here, 4608 terms,
+was 1.7e-7 in relative L2 norm, so 1e-6 is far above rounding and far below any misplaced term."""
+import contextlib
+
+import numpy as np
+import pytest
+
+import oracle
+from util import he_normal, rel_l2
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-6
+
+
+@contextlib.contextmanager
+def split_everywhere(gpu):
+    old = gpu.set_option("conv_split", 2)
+    try:
+        yield
+    finally:
+        gpu.set_option("conv_split", old)
+
+
+def _data(n, c, h, w, k, r, s, sh, sw, pad, gpu):
+    rng = np.random.default_rng(n + 3 * c + 7 * k + h)
+    oh, ow = gpu.kernels.conv_out_hw(h, w, r, s, (sh, sw), pad)
+    return (rng.standard_normal((n, c, h, w)).astype(np.float32), he_normal(rng, (k, c, r, s)),
+            rng.standard_normal((k,)).astype(np.float32), rng.standard_normal((n, k, oh, ow)).astype(np.float32),
+            rng.standard_normal((n, c, h, w)).astype(np.float32))
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad", [
+    (1, 16, 1, 255, 64, 1, 3, 1, 1, 1),      # one row tile, one pixel short of two 128-pixel tiles
+    (1, 17, 16, 16, 65, 3, 3, 1, 1, 1),      # 256 pixels; a channel and a row past their tiles
+    (1, 31, 11, 93, 63, 3, 3, 1, 1, 1),      # 1023 pixels: the last of the narrow tiles
+    (1, 33, 32, 32, 1, 3, 3, 1, 1, 1),       # 1024: the first of the wide ones; one row
+    (5, 1, 25, 41, 3, 2, 2, 1, 1, 0),        # one channel, even filter, no padding
+    (3, 32, 9, 3, 64, 3, 3, 1, 1, 1),        # rows of three pixels: many row and image ends in a tile
+    (2, 24, 45, 61, 40, 5, 5, 1, 1, 2),      # an image does not hold all rows' taps: one filter row per phase
+    (3, 20, 19, 23, 70, 7, 7, 2, 2, 3),      # strided, one filter row per phase: 14 phases
+    (2, 48, 14, 15, 20, 3, 3, 2, 2, 1),      # four phases forward, four classes backward
+    (2, 20, 17, 13, 70, 3, 5, 2, 1, 1),      # strides and filter sides that differ
+    (2, 40, 15, 17, 24, 1, 1, 1, 1, 0),      # 1 x 1: one step per channel group
+    (2, 18, 12, 12, 24, 3, 3, 3, 3, 0),      # stride 3: nine phases of one tap
+    (1, 512, 7, 7, 512, 3, 3, 1, 1, 1),      # every tile shared by many workgroups
+    (20, 32, 56, 56, 64, 3, 3, 1, 1, 1),     # more tiles than workgroups
+])
+def test_split_convolution_against_the_oracle(gpu, n, c, h, w, k, r, s, sh, sw, pad):
+    K = gpu.kernels
+    x, wt, b, dy, dx0 = _data(n, c, h, w, k, r, s, sh, sw, pad, gpu)
+    y_ref, col = oracle.conv2d_fwd(x, wt, b, (sh, sw), pad)
+    dx_ref, _, _ = oracle.conv2d_bwd(dy, x.shape, wt, col, (sh, sw), pad, dx0.copy(), np.zeros_like(wt), np.zeros_like(b))
+    dx_, dw_, db_, ddy = (gpu.to_device(a) for a in (x, wt, b, dy))
+    with split_everywhere(gpu):
+        y = K.conv2d_fwd(dx_, dw_, db_, (sh, sw), pad).numpy()
+        assert rel_l2(y, y_ref) <= TOL
+        mask = gpu.empty(y.shape, np.uint8)
+        act = K.conv2d_fwd(dx_, dw_, db_, (sh, sw), pad, relu=True, neg_mask=mask).numpy()
+        np.testing.assert_array_equal(act, np.maximum(y, 0.0))
+        np.testing.assert_array_equal(mask.numpy(), (y < 0).astype(np.uint8))
+        gx = gpu.to_device(dx0)
+        K.conv2d_bwd_data(ddy, dw_, x.shape, (sh, sw), pad, dx=gx, accumulate=True)
+        assert rel_l2(gx.numpy(), dx_ref) <= TOL
+
+
+def test_values_that_do_not_split_are_multiplied_one_by_one(gpu):
+    """Infinities, NaN and floats that round to a bf16 infinity: the outputs they touch are the float32 ones, signs and
+    NaNs included, and no other output is disturbed."""
+    K = gpu.kernels
+    x, wt, b, _, _ = _data(2, 20, 12, 13, 70, 3, 3, 1, 1, 1, gpu)
+    clean, _ = oracle.conv2d_fwd(x, wt, b, (1, 1), 1)
+    x[0, 3, 2, 2], x[0, 5, 8, 9], x[1, 19, 6, 6], x[1, 0, 0, 12] = np.inf, -np.inf, np.nan, np.float32(3.4e38)
+    with np.errstate(all="ignore"):
+        ref, _ = oracle.conv2d_fwd(x, wt, b, (1, 1), 1)
+    with split_everywhere(gpu):
+        y = K.conv2d_fwd(gpu.to_device(x), gpu.to_device(wt), gpu.to_device(b), (1, 1), 1).numpy()
+    for test in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(test(y), test(ref))
+    calm = np.isfinite(ref) & (ref == clean)
+    assert calm.sum() > 0.7 * calm.size and rel_l2(y[calm], ref[calm]) <= TOL
+    large = np.isfinite(ref) & ~calm                       # 3.4e38 times a weight: one term decides
+    assert large.any() and np.abs(y[large] / ref[large] - 1).max() <= 1e-6
+
+
+def test_a_partial_tile_that_never_comes_is_reported(gpu):
+    K = gpu.kernels
+    x, wt, b, _, _ = _data(1, 512, 7, 7, 512, 3, 3, 1, 1, 1, gpu)
+    ref, _ = oracle.conv2d_fwd(x, wt, b, (1, 1), 1)
+    args = [gpu.to_device(a) for a in (x, wt, b)]
+    out = gpu.empty(ref.shape)
+    gpu.synchronize()
+    old = gpu.set_option("sk_spin_limit", 0)
+    try:
+        K.conv2d_fwd(*args, (1, 1), 1, out=out)
+        with pytest.raises(gpu.XsmiError, match="gave up waiting"):
+            gpu.synchronize()
+    finally:
+        gpu.set_option("sk_spin_limit", old)
+    for _ in range(2):
+        assert rel_l2(K.conv2d_fwd(*args, (1, 1), 1, out=out).numpy(), ref) <= TOL

@@ -327,8 +327,8 @@ size_t conv_bwd_data_ws_bytes(int C, int K, int R, int S, int sh, int sw) {
 
 // Which forward / backward-data kernel family serves a geometry with the given flags and workspace size: one place,
 // so that xsmi_conv2d_pack lays a filter out for exactly the kernel that the later call will pick.
-enum class FwdPath { ChannelsLast, FirstLayer, EvenSplit, Tap, Generic };
-enum class BwdDataPath { EvenSplit, Tap, Generic };
+enum class FwdPath { ChannelsLast, FirstLayer, Split, EvenSplit, Tap, Generic };
+enum class BwdDataPath { Split, EvenSplit, Tap, Generic };
 
 static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW, unsigned flags,
                         size_t workspace_bytes) {
@@ -338,6 +338,10 @@ static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh,
     if (!bf16 && xsmi::stem_fwd_ok(N, C, H, W, K, R, S, sh, sw, pad) &&
         workspace_bytes >= xsmi::stem_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad))
         return FwdPath::FirstLayer;
+    if (!bf16 && !(flags & XSMI_CONV_WS_ONLY) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
+        const size_t need = xsmi::split_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
+        if (need && workspace_bytes >= need) return FwdPath::Split;
+    }
     if (!bf16 && !(flags & XSMI_CONV_WS_ONLY) && xsmi::sk_path_ok(C, K) && xsmi::sk_fwd_pays(N * OH * OW, K, R, S, sh, sw) &&
         workspace_bytes >= xsmi::sk_fwd_ws_bytes(C, K, R, S))
         return FwdPath::EvenSplit;
@@ -345,8 +349,12 @@ static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh,
     return FwdPath::Generic;
 }
 
-static BwdDataPath bwd_data_path(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, unsigned flags,
-                                 size_t workspace_bytes) {
+static BwdDataPath bwd_data_path(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW,
+                                 unsigned flags, size_t workspace_bytes) {
+    if (!(flags & XSMI_CONV_BF16) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
+        const size_t need = xsmi::split_bwd_data_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
+        if (need && workspace_bytes >= need) return BwdDataPath::Split;
+    }
     if (!(flags & XSMI_CONV_BF16) && xsmi::sk_bwd_data_ok(C, K, R, S, sh, sw) && xsmi::sk_bwd_data_pays(N * H * W, C, R, S, sh, sw) &&
         workspace_bytes >= xsmi::sk_bwd_data_ws_bytes(C, K, R, S, sh, sw))
         return BwdDataPath::EvenSplit;
@@ -378,6 +386,8 @@ int xsmi_conv2d_fwd(const float *x, const float *w, const float *bias, float *y,
                                    relu, opts, workspace);
     case FwdPath::FirstLayer:
         return xsmi::stem_conv_fwd(x, w, bias, y, neg_mask, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, relu, opts, workspace);
+    case FwdPath::Split:
+        return xsmi::split_conv_fwd(x, w, bias, y, neg_mask, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, relu, opts, workspace);
     case FwdPath::EvenSplit:
         return xsmi::sk_conv_fwd(x, w, bias, y, neg_mask, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, relu, opts, workspace);
     case FwdPath::Tap:
@@ -467,7 +477,9 @@ int xsmi_conv2d_bwd_data(const float *dy, const float *w, float *dx, int N, int 
     XSMI_CHECK_ARG(workspace && workspace_bytes >= need, "xsmi_conv2d_bwd_data: workspace of %zu bytes needed, %zu given",
                    need, workspace_bytes);
     const int opts = ((flags & XSMI_CONV_WS_PACKED) ? 2 : 0) | ((flags & XSMI_CONV_PACK_ONLY) ? 4 : 0);
-    switch (bwd_data_path(N, C, H, W, K, R, S, sh, sw, flags, workspace_bytes)) {
+    switch (bwd_data_path(N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, flags, workspace_bytes)) {
+    case BwdDataPath::Split:
+        return xsmi::split_conv_bwd_data(dy, w, dx, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, beta == 1.f ? 1 : 0, opts, workspace);
     case BwdDataPath::EvenSplit:
         return xsmi::sk_conv_bwd_data(dy, w, dx, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, beta == 1.f ? 1 : 0, opts, workspace);
     case BwdDataPath::Tap:
@@ -560,8 +572,8 @@ int xsmi_conv2d_pack(int count, xsmi_pack_job_t *jobs) {
         // rebuild a small table per call: nothing to do ahead of time for either
         if (j.pass == 0) {
             const FwdPath path = fwd_path(j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw, j.pad, g.OH, g.OW, 0, j.workspace_bytes);
-            if (path != FwdPath::EvenSplit && path != FwdPath::Tap) continue;
-        } else if (bwd_data_path(j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw, 0, j.workspace_bytes) == BwdDataPath::Generic) {
+            if (path != FwdPath::Split && path != FwdPath::EvenSplit && path != FwdPath::Tap) continue;
+        } else if (bwd_data_path(j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw, j.pad, g.OH, g.OW, 0, j.workspace_bytes) == BwdDataPath::Generic) {
             continue;
         }
         if (!forked) {

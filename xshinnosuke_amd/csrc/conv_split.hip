@@ -1,0 +1,780 @@
+// fp32 convolution forward and backward-data on the bf16 matrix pipes, without giving up float32 precision.
+//
+// A float32 value is the sum of three bf16 values EXACTLY: 24 significant bits are 8 + 8 + 8, and each remainder
+// a - bf16(a) is representable (rounding to nearest even leaves a signed remainder of at most 15, then 7 bits).  So
+//     a b = a0 b0 + (a0 b1 + a1 b0) + (a1 b1 + a0 b2 + a2 b0) + [a1 b2 + a2 b1 + a2 b2]
+// where the bracket is below 2^-25 |a b|, half a float32 ulp's half, and is left out: six bf16 MFMAs, whose products are
+// exact and whose sums are float32, stand for one float32 product.  The bf16 pipe does sixteen times the work of the
+// fp32 pipe per cycle, so the matrix-bound floor falls to 6/16.  The large products (a0 b0) and the five small ones
+// have accumulators of their own: the chain that carries the rounding of the full sum then has one addition per 16
+// channels and tap, against one per product pair on the fp32 pipe.
+//
+// What the split does not carry: infinities (inf - inf in a remainder) and values within a bf16 rounding of the largest
+// float.  Such a value makes the outputs that it touches non-finite; every non-finite output is therefore computed
+// again, one product at a time in float32, before it is stored (recompute_nonfinite).
+//
+// Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (128 per tile), 2 x 2 waves
+// of 32 rows x 64 pixels.  The reduction is a list of steps (phase, 16 input channels, tap).  A PHASE is a set of taps
+// that read one sub-lattice of the input (stride 1: all taps; stride 2: the taps of one row and column parity; or one
+// filter row's taps, where the input rows of all taps together would not fit the LDS).  In the phase's own coordinates
+// the walk has stride 1, so a tile needs one run of positions ("slots") of a grid of pitch Wp = OX + taps across - 1, and
+// a tap is nothing but an offset into the run.  The run is staged once per 16 channels for all taps of the phase: float32
+// values are fetched through registers (lanes = slots, eight channels per lane), split there, and written to the LDS as
+// [piece][octet][slot][8 channels], so a fragment read is 32 consecutive 16-byte slots whatever the tap is.  The LDS
+// image serves up to nine taps, which is what pays for the conversion (11 vector instructions per two values).
+// The filter is laid out split already, one 6 KB block per step ([piece][octet][row][8]); each wave fetches its fragments
+// straight into registers one step ahead (the waves of a workgroup read the same block at about the same time: L1), so
+// the loop has no barrier except around the image of a channel group.
+//
+// Scheduling is the even split of conv_tap_sk.hip: the steps of all tiles in a row are dealt over the resident
+// workgroups; a workgroup whose range starts inside a tile hands its accumulators to the one that holds the tile's
+// first step, which adds them in ascending order (bounded wait, deterministic sums).  Row tiles vary slowest, so
+// that an XCD's workgroups read few filter blocks.
+#include "conv_store.h"
+
+#include <string.h>
+#include <type_traits>
+
+namespace {
+
+using xsmi::floatx16;
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int SP_ROWS = 64;
+constexpr int sp_slots_of(int wc) { return wc == 4 ? 512 : 384; }     // slots of an LDS image
+constexpr int SP_BLOCK = 3 * 2 * SP_ROWS * 16;       // bytes of a step's filter block
+constexpr int SP_MAX_CLASSES = 4, SP_MAX_PHASES = 16;
+constexpr int sp_max_grid(int wc) { return wc == 4 ? 256 : 512; }
+static_assert((size_t)sp_max_grid(2) * 4 <= xsmi::SK_SCRATCH_FLAG_BYTES, "one flag per workgroup");
+static_assert((size_t)512 * 64 * 128 * 4 <= xsmi::SK_SCRATCH_PART_BYTES, "one partial tile per workgroup");
+
+struct SpPhase {
+    int iy0, ix0;          // input place of slot (row v, column u): (v * sy + iy0, u * sx + ix0)
+    int Tx, T;             // taps across, taps in all
+    int tap0, step0;       // first tap of the class, first step of the tile
+    int r0, rs, s0, ss;    // filter place of tap (a, b): (r0 + rs a, s0 + ss b)
+};
+struct SpClass {
+    int M, rows, OY, OX, os_y, os_x;
+    long long os_n, os_k, o_base;
+    xsmi::FastDiv dOX, dOY, dWp, dHp, dIT, dTM;      // dIT: steps per tile, dTM: pixel tiles
+    int Wp, Hp, sy, sx;
+    int phase0, nphase, taps, span;                  // span: slots past the last pixel's own that its taps reach
+    uint32_t iters, first_unit, end_unit, apk_off;
+};
+struct SpTapPlace { uint32_t off, iters, step, T; };  // block of (row tile, group): off + rt iters + step + group T
+struct SpParams {
+    const float *in, *w, *bias;
+    const char *apk;
+    float *out;
+    uint8_t *mask;
+    float *part;
+    uint32_t *flags, *err;
+    uint32_t in_bytes, out_bytes, apk_bytes, spin_limit;
+    uint32_t units, upg, urem;                       // steps in all; per workgroup, remainder
+    int N, CH, groups, IH, IW, in_n, plane;          // input channels, their groups of 16, floats per image / plane
+    int w_row, w_ch, FS;                             // floats between rows / channels of the filter, filter width
+    int ncls, relu, accumulate, wc;
+    SpClass cls[SP_MAX_CLASSES];
+    SpPhase ph[SP_MAX_PHASES];
+    SpTapPlace tap[9];     // of a 3 x 3 filter's taps
+};
+
+template <int N>
+using IC = std::integral_constant<int, N>;
+
+constexpr int AGENT = 16;                            // sc1: past the caches that are not coherent across XCDs
+
+// two floats -> bf16 pair (nearest even); the pair's values taken off the floats
+// (v_dot2_f32_bf16 with (-1, 0) and (0, -1): one instruction for a subtraction and the widening in front of it; the
+// difference is representable, so it is exact)
+__device__ __forceinline__ uint32_t split_pair(float &a, float &b) {
+    const bf16x2 p = {(__bf16)a, (__bf16)b}, hi = {(__bf16)0.f, (__bf16)-1.f};
+    uint32_t lo_bits = 0x0000bf80u;                      // (-1, 0), kept from the compiler: as an inline constant -1.0 it
+    asm("" : "+s"(lo_bits));                             // comes out as (0, -1)
+    const bf16x2 lo = __builtin_bit_cast(bf16x2, lo_bits);
+    a = __builtin_amdgcn_fdot2_f32_bf16(p, lo, a, false);
+    b = __builtin_amdgcn_fdot2_f32_bf16(p, hi, b, false);
+    return __builtin_bit_cast(uint32_t, p);
+}
+
+// eight floats -> three vectors of eight bf16
+__device__ __forceinline__ void split8(const float (&v)[8], uint32x4 &p0, uint32x4 &p1, uint32x4 &p2) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = v[2 * i], b = v[2 * i + 1];
+        p0[i] = split_pair(a, b);
+        p1[i] = split_pair(a, b);
+        const bf16x2 l = {(__bf16)a, (__bf16)b};
+        p2[i] = __builtin_bit_cast(uint32_t, l);
+    }
+}
+
+__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_inff(); }
+
+// Outputs that came out non-finite are computed again one float32 product at a time (taps outside, channels inside, as
+// the fp32 kernels add them); a tap outside the input multiplies a zero, as the reference's padding does.
+__device__ __forceinline__ void recompute_nonfinite(floatx16 &r, const SpParams &p, const SpClass &c, int tile_row0, int row0, int m0,
+                                                    int lane) {
+    uint32_t bad = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) bad |= finite(r[v]) ? 0u : 1u << v;
+    if (__builtin_amdgcn_ballot_w64(bad != 0) == 0) return;
+    const int m = m0 + (lane & 31);
+    if (m >= c.M) return;
+    const int q = (int)xsmi::fdiv((uint32_t)m, c.dOX), ox = m - q * c.OX;
+    const int n = (int)xsmi::fdiv((uint32_t)q, c.dOY), oy = q - n * c.OY;
+#pragma unroll 1
+    for (int v = 0; v < 16; ++v) {
+        const int row = tile_row0 + row0 + 4 * (lane >> 5) + 8 * (v >> 2) + (v & 3);
+        if (!((bad >> v) & 1u) || row >= c.rows) continue;
+        float sum = 0.f;
+        const float *wrow = p.w + (size_t)row * p.w_row;
+#pragma unroll 1
+        for (int f = c.phase0; f < c.phase0 + c.nphase; ++f) {
+            const SpPhase &ph = p.ph[f];
+#pragma unroll 1
+            for (int t = 0; t < ph.T; ++t) {
+                const int a = t / ph.Tx, b = t - a * ph.Tx;
+                const int iy = (oy + a) * c.sy + ph.iy0, ix = (ox + b) * c.sx + ph.ix0;
+                const bool in = iy >= 0 && iy < p.IH && ix >= 0 && ix < p.IW;
+                const float *wt = wrow + (ph.r0 + ph.rs * a) * p.FS + ph.s0 + ph.ss * b;
+                const float *src = p.in + (size_t)n * p.in_n + (size_t)(in ? iy * p.IW + ix : 0);
+#pragma unroll 1
+                for (int ch = 0; ch < p.CH; ++ch)
+                    sum = __builtin_fmaf(wt[(size_t)ch * p.w_ch], in ? src[(size_t)ch * p.plane] : 0.f, sum);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) r[i] = i == v ? sum : r[i];
+    }
+}
+
+// WC waves across the tile's pixels (2: 128 pixels and 256 threads, two workgroups per CU; 4: 256 and 512, one)
+template <int WC>
+__global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
+    constexpr int SP_PIX = 64 * WC, THREADS = 128 * WC, NJ = sp_slots_of(WC) / 64 / WC;
+    constexpr int SP_PLANE = sp_slots_of(WC) * 16;       // bytes of one (piece, octet) plane
+    constexpr int SP_IMAGE = 6 * SP_PLANE;
+    constexpr uint32_t PART_BYTES = 32 * THREADS * 4;    // a workgroup's partial tile
+    __shared__ __attribute__((aligned(16))) unsigned char s_img[2 * SP_IMAGE];
+    __shared__ __attribute__((aligned(16))) float s_bias[2][SP_ROWS];
+    __shared__ uint32_t s_fail;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wr = wave / WC, wc = wave % WC, h = lane >> 5, l31 = lane & 31;
+    const uint32_t G = gridDim.x, g = xsmi::xcd_contiguous_id(blockIdx.x, G);
+    auto range_start = [&](uint32_t j) { return j * p.upg + (j < p.urem ? j : p.urem); };
+    const uint32_t u1 = range_start(g + 1);
+    uint32_t u = range_start(g);
+    if (t == 0) s_fail = 0;
+
+    const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc((void *)p.in, 0, (int)p.in_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rapk = __builtin_amdgcn_make_buffer_rsrc((void *)p.apk, 0, (int)p.apk_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rpart =
+        __builtin_amdgcn_make_buffer_rsrc((void *)p.part, 0, (int)(sp_max_grid(WC) * PART_BYTES), 0x00020000);
+    const int a_voff = (h * SP_ROWS + wr * 32 + l31) * 16;
+    const int octet = wave & 1, chunk0 = wave >> 1;    // this wave stages slots 64 (chunk0 + WC j) .. + 63 of one octet
+    const uint32_t plane4 = (uint32_t)p.plane * 4u;
+
+    // A segment: steps [s_first, s_first + n) of one tile, beginning with tap `tap` of channel group `grp` of phase f.
+    struct Segment {
+        int ci, s_first, n, rt, m0, slot0, nslots, f, grp, tap;
+    };
+    auto slot_of = [&](const SpClass &c, int m) {
+        const int q = (int)xsmi::fdiv((uint32_t)m, c.dOX), n_ = (int)xsmi::fdiv((uint32_t)q, c.dOY);
+        return (n_ * c.Hp + (q - n_ * c.OY)) * c.Wp + (m - q * c.OX);
+    };
+    auto segment_at = [&](uint32_t v) {
+        Segment sg;
+        sg.ci = 0;
+        while (sg.ci + 1 < p.ncls && v >= p.cls[sg.ci].end_unit) ++sg.ci;
+        const SpClass &c = p.cls[sg.ci];
+        const uint32_t ul = v - c.first_unit, tile = xsmi::fdiv(ul, c.dIT);
+        sg.s_first = (int)(ul - tile * c.iters);
+        sg.n = (int)c.iters - sg.s_first;
+        if (sg.n > (int)(u1 - v)) sg.n = (int)(u1 - v);
+        const uint32_t rt = xsmi::fdiv(tile, c.dTM);
+        sg.rt = (int)rt;
+        sg.m0 = (int)(tile - rt * c.dTM.d) * SP_PIX;
+        sg.slot0 = slot_of(c, sg.m0);
+        const int m_last = sg.m0 + SP_PIX - 1 < c.M ? sg.m0 + SP_PIX - 1 : c.M - 1;
+        sg.nslots = slot_of(c, m_last) - sg.slot0 + 1 + c.span;
+        sg.f = c.phase0;
+        while (sg.f + 1 < c.phase0 + c.nphase && sg.s_first >= p.ph[sg.f + 1].step0) ++sg.f;
+        const int k = sg.s_first - p.ph[sg.f].step0, T = p.ph[sg.f].T;
+        sg.grp = k / T;
+        sg.tap = k - sg.grp * T;
+        return sg;
+    };
+    auto block_of = [&](uint32_t v) {                  // byte offset of unit v's filter block (any place past the range)
+        if (v >= u1) return 0u;
+        int ci = 0;
+        while (ci + 1 < p.ncls && v >= p.cls[ci].end_unit) ++ci;
+        const SpClass &c = p.cls[ci];
+        const uint32_t ul = v - c.first_unit, tile = xsmi::fdiv(ul, c.dIT);
+        return c.apk_off + (xsmi::fdiv(tile, c.dTM) * c.iters + (ul - tile * c.iters)) * (uint32_t)SP_BLOCK;
+    };
+    uint32_t voff[NJ];
+    auto place = [&](const Segment &sg, int f) {       // byte offsets of this lane's slots in channel 0
+        const SpClass &c = p.cls[sg.ci];
+        const SpPhase &ph = p.ph[f];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int sl = 64 * (chunk0 + WC * j) + lane;
+            const uint32_t P = (uint32_t)(sg.slot0 + sl);
+            const int q = (int)xsmi::fdiv(P, c.dWp), n_ = (int)xsmi::fdiv((uint32_t)q, c.dHp);
+            const int iy = (q - n_ * c.Hp) * c.sy + ph.iy0, ix = ((int)P - q * c.Wp) * c.sx + ph.ix0;
+            const bool ok = sl < sg.nslots && n_ < p.N && iy >= 0 && iy < p.IH && ix >= 0 && ix < p.IW;
+            voff[j] = ok ? (uint32_t)(n_ * p.in_n + iy * p.IW + ix) * 4u : 0x80000000u;
+        }
+    };
+            float pre[NJ][8];
+            // always the same number of loads (slots past the run fetch out of range): the waits below count them
+            auto load_image = [&](int grp_) {
+                const int ch0 = grp_ * 16 + octet * 8;
+                if (ch0 + 8 <= p.CH) {
+    #pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+    #pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                            rin, (int)voff[j], (int)((uint32_t)(ch0 + e) * plane4), 0));
+                } else {
+    #pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+    #pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            const bool there = ch0 + e < p.CH;
+                            pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                            rin, (int)(there ? voff[j] : 0x80000000u), (int)(there ? (uint32_t)(ch0 + e) * plane4 : 0u), 0));
+                        }
+                }
+            };
+            // the fetched values into an LDS image: a pair of channels at a time, then the three 16-byte pieces
+            uint32x4 piece[3];
+            auto split_one = [&](auto jt, auto it) {
+                constexpr int j = decltype(jt)::value, i = decltype(it)::value;
+                float a = pre[j][2 * i], b = pre[j][2 * i + 1];
+                piece[0][i] = split_pair(a, b);
+                piece[1][i] = split_pair(a, b);
+                const bf16x2 l = {(__bf16)a, (__bf16)b};
+                piece[2][i] = __builtin_bit_cast(uint32_t, l);
+            };
+            auto put = [&](auto j, int to) {
+                unsigned char *dst = s_img + to + octet * SP_PLANE + (64 * (chunk0 + WC * j) + lane) * 16;
+    #pragma unroll
+                for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32x4 *>(dst + 2 * q * SP_PLANE) = piece[q];
+            };
+            auto stage = [&](auto j, int to) {
+                split_one(j, IC<0>{}); split_one(j, IC<1>{}); split_one(j, IC<2>{}); split_one(j, IC<3>{});
+                put(j, to);
+            };
+    uint32_t a_off = 0;
+    int b_rd[2];                                       // this lane's two pixels in an image
+            // two steps of filter fragments and two of pixel fragments in registers: a step's filter loads are issued while
+            // the step two before it multiplies, its LDS reads while the one before it does
+            bf16x8 fa[2][3], fb[2][2][3];                  // [step parity][piece], [step parity][pixel block][piece]
+            auto load_a = [&](auto par, auto q) {
+                fa[par][q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                                 rapk, a_voff + (int)q * 2 * SP_ROWS * 16, (int)a_off, 0));
+            };
+            auto read_b = [&](auto par, auto q, int off) {
+    #pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    fb[par][j][q] = *reinterpret_cast<const bf16x8 *>(s_img + b_rd[j] + off + (int)q * 2 * SP_PLANE);
+            };
+    int t_left = 0, tb = 0, off = 0, Tx = 1, row_end = 0;
+    auto next_off = [&]() {                            // past the last tap: back to a place inside the image
+        off += ++tb == Tx ? row_end : 16;
+        tb = tb == Tx ? 0 : tb;
+        off = --t_left == 0 ? 0 : off;
+    };
+    floatx16 hi[2], lo[2];
+            auto mm = [&](auto par, floatx16 (&acc)[2], int qa, int qb) {
+    #pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[par][qa], fb[par][j][qb], acc[j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+    // One step.  The next tap's fragments are read from the same image (past a group's last tap: places that are not
+    // used); the filter block two steps ahead takes each piece's registers after the piece's last product.  J >= 0: a
+    // part of the next image is split and written to the other half of the LDS, a few instructions behind each pair of
+    // MFMAs.
+    int image = 0;                                     // byte offset of the image that is multiplied
+    int a_left = 0;                                    // steps of the segment whose block ahead has not been requested
+    uint32_t a_next0 = 0, a_next1 = 0;                 // blocks of the two steps after the segment
+    auto step = [&](auto par, auto jt) {
+        constexpr int P = decltype(par)::value, J = decltype(jt)::value;
+        const auto nx = IC<1 - P>{};
+        next_off();
+        a_off = a_left > 2 ? a_off + (uint32_t)SP_BLOCK : a_left == 2 ? a_next0 : a_next1;
+        --a_left;
+        mm(par, lo, 2, 0);
+        load_a(par, IC<2>{});
+        read_b(nx, IC<0>{}, image + off);
+        if constexpr (J >= 0) split_one(jt, IC<0>{});
+        __builtin_amdgcn_sched_barrier(0);
+        mm(par, lo, 1, 0);
+        read_b(nx, IC<1>{}, image + off);
+        if constexpr (J >= 0) split_one(jt, IC<1>{});
+        __builtin_amdgcn_sched_barrier(0);
+        mm(par, lo, 1, 1);
+        load_a(par, IC<1>{});
+        read_b(nx, IC<2>{}, image + off);
+        if constexpr (J >= 0) split_one(jt, IC<2>{});
+        __builtin_amdgcn_sched_barrier(0);
+        mm(par, hi, 0, 0);
+        if constexpr (J >= 0) split_one(jt, IC<3>{});
+        __builtin_amdgcn_sched_barrier(0);
+        mm(par, lo, 0, 1);
+        if constexpr (J >= 0) put(jt, SP_IMAGE - image);
+        __builtin_amdgcn_sched_barrier(0);
+        mm(par, lo, 0, 2);
+        load_a(par, IC<0>{});
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // The taps of one image.  Written out up to nine: the waits of each step and the places where the next image is
+    // staged are then compile-time facts.
+    const auto none = IC<-1>{};
+    auto run = [&](int taps) {
+        read_b(IC<0>{}, IC<0>{}, image + off); read_b(IC<0>{}, IC<1>{}, image + off); read_b(IC<0>{}, IC<2>{}, image + off);
+        int staged = 0;
+        const auto third = IC<NJ == 3 ? 2 : -1>{};
+        do {
+            step(IC<0>{}, none);
+            if (taps == 1) break;
+            step(IC<1>{}, none);
+            if (taps == 2) break;
+            step(IC<0>{}, none);
+            if (taps == 3) break;
+            step(IC<1>{}, IC<0>{});
+            staged = 1;
+            if (taps == 4) break;
+            step(IC<0>{}, none);
+            if (taps == 5) break;
+            step(IC<1>{}, IC<1>{});
+            staged = 2;
+            if (taps == 6) break;
+            step(IC<0>{}, none);
+            if (taps == 7) break;
+            step(IC<1>{}, third);
+            staged = 3;
+            for (int i = 8; i < taps; i += 2) {
+                step(IC<0>{}, none);
+                if (i + 1 < taps) step(IC<1>{}, none);
+            }
+        } while (false);
+        if (staged < 1) stage(IC<0>{}, SP_IMAGE - image);
+        if (staged < 2) stage(IC<1>{}, SP_IMAGE - image);
+        if constexpr (NJ == 3)
+            if (staged < 3) stage(third, SP_IMAGE - image);
+    };
+
+
+    // The workgroup's steps are one stream: a segment's first image and filter blocks are requested while the segment before
+    // it is multiplied, and its output stores drain behind the next one's MFMAs.
+    Segment sg = segment_at(u), nx = sg;
+    place(sg, sg.f);
+    load_image(sg.grp);
+    a_off = block_of(u);
+    load_a(IC<0>{}, IC<2>{}); load_a(IC<0>{}, IC<1>{}); load_a(IC<0>{}, IC<0>{});
+    a_off = block_of(u + 1);
+    load_a(IC<1>{}, IC<2>{}); load_a(IC<1>{}, IC<1>{}); load_a(IC<1>{}, IC<0>{});
+    stage(IC<0>{}, 0); stage(IC<1>{}, 0);
+    if constexpr (NJ == 3) stage(IC<2>{}, 0);
+    bool odd = false;
+    int bias_buf = 0;
+    while (true) {
+        const SpClass &c = p.cls[sg.ci];
+        const bool head = sg.s_first == 0, complete = sg.s_first + sg.n == (int)c.iters;
+        const uint32_t tile_end = u + (c.iters - (uint32_t)sg.s_first), u_next = u + (uint32_t)sg.n;
+        const int m0 = sg.m0, rt = sg.rt, Wp = c.Wp;
+        const bool more = u_next < u1;
+        if (more) nx = segment_at(u_next);
+        a_next0 = block_of(u_next); a_next1 = block_of(u_next + 1);
+        a_left = sg.n;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int m = m0 + wc * 64 + 32 * j + l31;
+            b_rd[j] = h * SP_PLANE + (slot_of(c, m < c.M ? m : c.M - 1) - sg.slot0) * 16;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) { hi[j][v] = 0.f; lo[j][v] = 0.f; }
+        }
+        bias_buf ^= 1;                                 // the other waves may still be reading the one before
+        if (p.bias && head && t < SP_ROWS) s_bias[bias_buf][t] = rt * SP_ROWS + t < c.rows ? p.bias[rt * SP_ROWS + t] : 0.f;
+        int left = sg.n, f = sg.f, grp = sg.grp, tap = sg.tap;
+        while (left > 0) {
+            if (odd) {                                 // the next step's filter block is in the other set
+#pragma unroll
+                for (int q = 0; q < 3; ++q) { const bf16x8 x = fa[0][q]; fa[0][q] = fa[1][q]; fa[1][q] = x; }
+            }
+            const int T = p.ph[f].T;
+            const int taps = left < T - tap ? left : T - tap;
+            left -= taps;
+            Tx = p.ph[f].Tx;
+            t_left = T - tap;
+            tb = tap % Tx;
+            off = (tap / Tx * Wp + tb) * 16;
+            row_end = (Wp - Tx + 1) * 16;
+            tap = 0;
+            // the next image, requested while this one is multiplied
+            if (left > 0) {
+                if (++grp == p.groups) { grp = 0; ++f; place(sg, f); }
+            } else if (more) {
+                grp = nx.grp;
+                place(nx, nx.f);
+            } else {
+                grp = p.groups;                        // none: channels past the last read zeros
+            }
+            load_image(grp);
+            xsmi::wait_lgkmcnt0();
+            xsmi::block_barrier();                     // this image is complete, and nobody reads the other one any more
+            run(taps);
+            odd = taps & 1;
+            image = SP_IMAGE - image;
+        }
+        u = u_next;
+        // ---- end of the segment ----
+        floatx16 acc[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = hi[j] + lo[j];
+        if (!head) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                uint32x4 q;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { const float val = acc[i >> 2][4 * (i & 3) + e]; q[e] = __builtin_bit_cast(uint32_t, val); }
+                __builtin_amdgcn_raw_buffer_store_b128(q, rpart, t * 16, (int)(g * PART_BYTES + (uint32_t)i * (THREADS * 16u)), AGENT);
+            }
+            xsmi::wait_vmcnt<0>();                     // written through, this thread's ...
+            __syncthreads();                           // ... and everybody else's
+            if (t == 0) __hip_atomic_store(p.flags + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (head && !complete) {
+            // the rest of the tile was multiplied by the workgroups that follow: a lane waits for each of them, then their
+            // parts are added in ascending order, the next one's loads in flight
+            for (uint32_t j = g + 1; j < G && range_start(j) < tile_end;) {
+                uint32_t np = 1;
+                while (np < 64 && j + np < G && range_start(j + np) < tile_end) ++np;
+                if ((uint32_t)t < np) {
+                    uint32_t spins = 0;
+                    bool there = false;
+                    while (p.spin_limit != 0u &&
+                           !(there = __hip_atomic_load(p.flags + j + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) &&
+                           ++spins < p.spin_limit)
+                        __builtin_amdgcn_s_sleep(1);
+                    if (!there) {                      // give up: the host reports the launch as failed; nothing is stored
+                        s_fail = 1u;
+                        __hip_atomic_store(p.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+                }
+                __syncthreads();
+                if (s_fail) return;
+                uint32x4 part[2][8];
+                auto fetch = [&](auto buf, uint32_t i) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k)
+                        part[buf][k] = __builtin_amdgcn_raw_buffer_load_b128(rpart, t * 16, (int)((j + i) * PART_BYTES + (uint32_t)k * (THREADS * 16u)), AGENT);
+                };
+                auto add = [&](auto buf) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const uint32_t bits = part[buf][k][e];
+                            acc[k >> 2][4 * (k & 3) + e] += __builtin_bit_cast(float, bits);
+                        }
+                };
+                fetch(IC<0>{}, 0);
+                for (uint32_t i = 0; i < np; i += 2) {
+                    if (i + 1 < np) fetch(IC<1>{}, i + 1);
+                    add(IC<0>{});
+                    if (i + 1 < np) {
+                        if (i + 2 < np) fetch(IC<0>{}, i + 2);
+                        add(IC<1>{});
+                    }
+                }
+                __syncthreads();                       // everybody has read the parts before their flags are cleared
+                if ((uint32_t)t < np) __hip_atomic_store(p.flags + j + (uint32_t)t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                j += np;
+            }
+        }
+        if (head) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                recompute_nonfinite(acc[j], p, c, rt * SP_ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
+                xsmi::store_block_32x32(acc[j], c, p.out, p.out_bytes, p.mask, p.bias ? s_bias[bias_buf] : nullptr, p.relu, p.accumulate,
+                                        rt * SP_ROWS, SP_ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
+            }
+        }
+        if (!more) break;
+        sg = nx;
+    }
+}
+
+// The filter in its steps' blocks.  A thread owns a row and an octet of channels; lanes are consecutive rows, so a
+// wavefront writes whole kilobytes.
+// 3 x 3: all nine taps of the octet in registers (each filter line is fetched once; 512 -> 512: 16 -> 6 us against a
+// thread per tap, whose 16-byte writes were scattered); every place a tap goes to is in the table `tap`.
+__global__ void __launch_bounds__(64) split_pack9_kernel(SpParams p, char *apk, int rows) {
+    const uint32_t padded = (uint32_t)((rows + SP_ROWS - 1) / SP_ROWS * SP_ROWS);
+    const uint32_t o = blockIdx.x / (padded / SP_ROWS), rt = blockIdx.x - o * (padded / SP_ROWS), row = rt * SP_ROWS + threadIdx.x;
+    float v[9][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int ch = (int)o * 8 + e;
+        const bool there = (int)row < rows && ch < p.CH;
+        const float *src = p.w + (there ? (size_t)row * p.w_row + (size_t)ch * p.w_ch : 0);
+#pragma unroll
+        for (int t = 0; t < 9; ++t) v[t][e] = there ? src[t] : 0.f;
+    }
+#pragma unroll
+    for (int t = 0; t < 9; ++t) {
+        uint32x4 q0, q1, q2;
+        split8(v[t], q0, q1, q2);
+        const SpTapPlace &w = p.tap[t];
+        const uint32_t step = rt * w.iters + w.step + (o >> 1) * w.T;
+        char *dst = apk + w.off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + threadIdx.x) * 16;
+        *reinterpret_cast<uint32x4 *>(dst) = q0;
+        *reinterpret_cast<uint32x4 *>(dst + 2 * SP_ROWS * 16) = q1;
+        *reinterpret_cast<uint32x4 *>(dst + 4 * SP_ROWS * 16) = q2;
+    }
+}
+__global__ void __launch_bounds__(256) split_pack_kernel(SpParams p, char *apk) {
+    for (int ci = 0; ci < p.ncls; ++ci) {
+        const SpClass &c = p.cls[ci];
+        const uint32_t rows = (uint32_t)((c.rows + SP_ROWS - 1) / SP_ROWS * SP_ROWS), octets = 2u * (uint32_t)p.groups;
+        const uint32_t total = rows * octets * (uint32_t)c.taps;
+        for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+            const uint32_t row = i % rows, rest = i / rows, o = rest / (uint32_t)c.taps;
+            const int tap = (int)(rest - o * (uint32_t)c.taps);
+            int f = c.phase0;
+            while (f + 1 < c.phase0 + c.nphase && tap >= p.ph[f + 1].tap0) ++f;
+            const SpPhase &ph = p.ph[f];
+            const int tl = tap - ph.tap0, a = tl / ph.Tx, b = tl - a * ph.Tx;
+            const float *src = p.w + (ph.r0 + ph.rs * a) * p.FS + ph.s0 + ph.ss * b;
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int ch = (int)o * 8 + e;
+                v[e] = (int)row < c.rows && ch < p.CH ? src[(size_t)row * p.w_row + (size_t)ch * p.w_ch] : 0.f;
+            }
+            uint32x4 q0, q1, q2;
+            split8(v, q0, q1, q2);
+            const uint32_t step = (row / SP_ROWS) * c.iters + (uint32_t)ph.step0 + (o >> 1) * (uint32_t)ph.T + (uint32_t)tl;
+            char *dst = apk + c.apk_off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + row % SP_ROWS) * 16;
+            *reinterpret_cast<uint32x4 *>(dst) = q0;
+            *reinterpret_cast<uint32x4 *>(dst + 2 * SP_ROWS * 16) = q1;
+            *reinterpret_cast<uint32x4 *>(dst + 4 * SP_ROWS * 16) = q2;
+        }
+    }
+}
+
+// slots that the tiles of a class need at most
+long sp_slots(int pix, int OY, int OX, int ty, int tx) {
+    const long wp = OX + tx - 1, hp = OY + ty - 1;
+    const long row_ends = (pix - 1 + OX - 1) / OX, image_ends = ((long)pix - 1 + (long)OX * OY - 1) / ((long)OX * OY);
+    return pix + row_ends * (wp - OX) + image_ends * (hp - OY) * wp + (ty - 1) * wp + tx - 1;
+}
+
+// Adds a class whose taps are r = r0 + rs a (a < R), s = s0 + ss b (b < S), reading input place (y sy + iy(r), ...), split
+// into phases of sub-lattice taps; false if the tables or the LDS image do not hold it.
+struct SpTaps { int R, S, r0, rs, s0, ss, iy0, ix0, dy, dx; };   // tap (a, b) reads (y sy + iy0 + dy a, x sx + ix0 + dx b)
+bool sp_add_class(SpParams &p, int &nph, uint32_t &steps_bytes, const SpTaps &k, int M, int rows, int OY, int OX, int sy, int sx) {
+    if (p.ncls == SP_MAX_CLASSES || k.R < 1 || k.S < 1) return false;
+    SpClass &c = p.cls[p.ncls];
+    const int ny = (sy < k.R && k.dy == 1) ? sy : k.dy == 1 ? k.R : 1, nx = (sx < k.S && k.dx == 1) ? sx : k.dx == 1 ? k.S : 1;
+    // all rows of a sub-lattice in one image when it fits, otherwise one filter row at a time
+    const int ty_max = (k.R + ny - 1) / ny, tx_max = (k.S + nx - 1) / nx;
+    const int pix = 64 * p.wc;
+    const bool by_row = sp_slots(pix, OY, OX, ty_max, tx_max) > sp_slots_of(p.wc);
+    const int ty = by_row ? 1 : ty_max;
+    if (sp_slots(pix, OY, OX, ty, tx_max) > sp_slots_of(p.wc)) return false;
+    const int rows_n = by_row ? k.R : ny;
+    if (nph + rows_n * nx > SP_MAX_PHASES) return false;
+    c.phase0 = nph; c.nphase = rows_n * nx; c.taps = k.R * k.S;
+    c.M = M; c.rows = rows; c.OY = OY; c.OX = OX; c.sy = sy; c.sx = sx;
+    c.Wp = OX + tx_max - 1; c.Hp = OY + ty - 1;
+    c.span = (ty - 1) * c.Wp + tx_max - 1;
+    int step = 0, tap = 0;
+    for (int i = 0; i < rows_n; ++i)
+        for (int j = 0; j < nx; ++j) {
+            SpPhase &f = p.ph[nph++];
+            const int na = by_row ? 1 : (k.R - i + ny - 1) / ny, nb = (k.S - j + nx - 1) / nx;
+            f.iy0 = k.iy0 + k.dy * i; f.ix0 = k.ix0 + k.dx * j;
+            f.Tx = nb; f.T = na * nb;
+            f.tap0 = tap; f.step0 = step;
+            f.r0 = k.r0 + k.rs * i; f.rs = k.rs * ny; f.s0 = k.s0 + k.ss * j; f.ss = k.ss * nx;
+            tap += f.T; step += f.T * p.groups;
+        }
+    c.iters = (uint32_t)step;
+    const int tiles_m = xsmi::ceil_div(M, pix), tiles_r = xsmi::ceil_div(rows, SP_ROWS);
+    c.dOX = xsmi::make_fastdiv(OX); c.dOY = xsmi::make_fastdiv(OY); c.dWp = xsmi::make_fastdiv(c.Wp); c.dHp = xsmi::make_fastdiv(c.Hp);
+    c.dIT = xsmi::make_fastdiv(c.iters); c.dTM = xsmi::make_fastdiv(tiles_m);
+    c.apk_off = steps_bytes;
+    const double bytes = (double)steps_bytes + (double)tiles_r * c.iters * SP_BLOCK, units = (double)p.units + (double)tiles_m * tiles_r * c.iters;
+    if (bytes >= 2e9 || units >= 1e9 || (double)c.Wp * c.Hp * p.N >= 1e9) return false;
+    steps_bytes += (uint32_t)tiles_r * c.iters * (uint32_t)SP_BLOCK;
+    c.first_unit = p.units;
+    p.units += (uint32_t)tiles_m * (uint32_t)tiles_r * c.iters;
+    c.end_unit = p.units;
+    ++p.ncls;
+    return true;
+}
+
+// 256-pixel tiles stage 2.0 values for each pixel of a 3 x 3 layer's tile where 128-pixel tiles stage 3.0; small passes keep
+// the smaller tile, whose last one is emptier by less
+int sp_wide(long m) { return m >= 1024 ? 4 : 2; }
+
+bool sp_plan_fwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
+    memset(&p, 0, sizeof(p));
+    p.wc = sp_wide((long)N * OH * OW);
+    p.N = N; p.CH = C; p.groups = xsmi::ceil_div(C, 16); p.IH = H; p.IW = W; p.in_n = C * H * W; p.plane = H * W;
+    p.w_row = C * R * S; p.w_ch = R * S; p.FS = S;
+    int nph = 0;
+    const SpTaps k = {R, S, 0, 1, 0, 1, -pad, -pad, 1, 1};
+    if (!sp_add_class(p, nph, p.apk_bytes, k, N * OH * OW, K, OH, OW, sh, sw)) return false;
+    SpClass &c = p.cls[0];
+    c.os_n = (long long)K * OH * OW; c.os_k = (long long)OH * OW; c.o_base = 0; c.os_y = OW; c.os_x = 1;
+    p.in_bytes = (uint32_t)((size_t)N * C * H * W * 4); p.out_bytes = (uint32_t)((size_t)N * K * OH * OW * 4);
+    return true;
+}
+
+// backward-data: a class per residue (h mod sh, w mod sw); taps in ascending order of the dy row they read
+bool sp_plan_bwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
+    memset(&p, 0, sizeof(p));
+    p.wc = sp_wide((long)N * H * W / (sh * sw));
+    p.N = N; p.CH = K; p.groups = xsmi::ceil_div(K, 16); p.IH = OH; p.IW = OW; p.in_n = K * OH * OW; p.plane = OH * OW;
+    p.w_row = R * S; p.w_ch = C * R * S; p.FS = S;
+    int nph = 0;
+    for (int ph = 0; ph < sh && ph < H; ++ph) {
+        const int r0 = (ph + pad) % sh, T = r0 < R ? xsmi::ceil_div(R - r0, sh) : 0, cy = (ph + pad - r0) / sh;
+        for (int pw = 0; pw < sw && pw < W; ++pw) {
+            const int s0 = (pw + pad) % sw, U = s0 < S ? xsmi::ceil_div(S - s0, sw) : 0, cx = (pw + pad - s0) / sw;
+            const int OYc = xsmi::ceil_div(H - ph, sh), OXc = xsmi::ceil_div(W - pw, sw);
+            const SpTaps k = {T, U, r0 + sh * (T - 1), -sh, s0 + sw * (U - 1), -sw, cy - (T - 1), cx - (U - 1), 1, 1};
+            if (!sp_add_class(p, nph, p.apk_bytes, k, N * OYc * OXc, C, OYc, OXc, 1, 1)) return false;
+            SpClass &c = p.cls[p.ncls - 1];
+            c.os_n = (long long)C * H * W; c.os_k = (long long)H * W; c.o_base = (long long)ph * W + pw;
+            c.os_y = sh * W; c.os_x = sw;
+        }
+    }
+    p.in_bytes = (uint32_t)((size_t)N * K * OH * OW * 4); p.out_bytes = (uint32_t)((size_t)N * C * H * W * 4);
+    return true;
+}
+
+int sp_run(SpParams &p, int opts, void *workspace) {
+    hipStream_t st = xsmi::stream();
+    p.apk = (const char *)workspace;
+    if (!(opts & 2)) {
+        int taps = 0;
+        for (int i = 0; i < p.ncls; ++i) taps += p.cls[i].taps;
+        const uint32_t row_tiles = (uint32_t)xsmi::ceil_div(p.cls[0].rows, SP_ROWS), octets = 2u * (uint32_t)p.groups;
+        if (taps == 9 && p.FS == 3) {
+            for (int i = 0; i < p.ncls; ++i)
+                for (int f = p.cls[i].phase0; f < p.cls[i].phase0 + p.cls[i].nphase; ++f)
+                    for (int t = 0; t < p.ph[f].T; ++t) {
+                        const SpPhase &ph = p.ph[f];
+                        const int r = ph.r0 + ph.rs * (t / ph.Tx), q = ph.s0 + ph.ss * (t % ph.Tx);
+                        p.tap[3 * r + q] = SpTapPlace{p.cls[i].apk_off, p.cls[i].iters, (uint32_t)(ph.step0 + t), (uint32_t)ph.T};
+                    }
+            hipLaunchKernelGGL(split_pack9_kernel, dim3(row_tiles * octets), dim3(64), 0, st, p, (char *)workspace, p.cls[0].rows);
+        } else {
+            uint32_t blocks = row_tiles * octets * (uint32_t)p.cls[0].taps / 4 + 1;
+            if (blocks > 4096) blocks = 4096;
+            hipLaunchKernelGGL(split_pack_kernel, dim3(blocks), dim3(256), 0, st, p, (char *)workspace);
+        }
+        XSMI_LAUNCH_CHECK("split_pack_kernel");
+    }
+    if (opts & 4) return XSMI_OK;
+    static int resident[2] = {0, 0};
+    int &res = resident[p.wc == 4];
+    if (res == 0) {
+        int per_cu = 0;
+        const hipError_t e = p.wc == 4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, split_conv_kernel<4>, 512, 0)
+                                       : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, split_conv_kernel<2>, 256, 0);
+        if (e != hipSuccess || per_cu < 1) per_cu = 1;
+        const int all = per_cu * xsmi::cu_count(), cap = sp_max_grid(p.wc);
+        res = (all > cap ? cap : all < 8 ? 8 : all) & ~7;
+    }
+    uint32_t grid = (uint32_t)res;
+    // A launch that does not fill the chip: n steps for each workgroup cost 0.45 us n, and the workgroup that adds a tile of
+    // I steps together about 0.9 us for each of the I / n - 1 others; the sum is smallest at n = sqrt(2 I).
+    uint32_t steps = 0;
+    for (int i = 0; i < p.ncls; ++i) steps = p.cls[i].iters > steps ? p.cls[i].iters : steps;
+    uint32_t least = 4;
+    while (least * least < 2 * steps) ++least;
+    if (grid > p.units / least) grid = p.units / least;
+    if (grid == 0) grid = 1;
+    p.upg = p.units / grid; p.urem = p.units % grid;
+    const int rc = xsmi::check_device_error("split convolution");
+    if (rc) return rc;
+    const xsmi::SkScratch scr = xsmi::sk_scratch();
+    p.part = scr.part; p.flags = scr.flags; p.err = xsmi::device_error_word();
+    const long spin = xsmi::option(xsmi::OPT_SK_SPIN_LIMIT);
+    p.spin_limit = spin < 0 ? 0u : spin > 0x7fffffffL ? 0x7fffffffu : (uint32_t)spin;
+    xsmi::prof_begin();
+    if (p.wc == 4) hipLaunchKernelGGL(split_conv_kernel<4>, dim3(grid), dim3(512), 0, st, p);
+    else hipLaunchKernelGGL(split_conv_kernel<2>, dim3(grid), dim3(256), 0, st, p);
+    xsmi::prof_end();
+    XSMI_LAUNCH_CHECK("split_conv_kernel");
+    return XSMI_OK;
+}
+
+}  // namespace
+
+namespace xsmi {
+
+// Where the split pays, in kernel plus layout time on random layers of 1 to 512 channels and on ResNet-18's at N = 1 to 32
+// (`pixels`: outputs of the pass, of one residue class of a strided backward-data).
+//   1 x 1 to 3 taps: no.  An image then serves one tap, and its staging costs more than the fp32 kernels' loads (64 -> 128
+//     at 28 x 28, N=32: 13.5 -> 18.6 us).
+//   fewer than 16 channels: no.  A step multiplies 16, the rest zeros (4 -> 120, 3 x 3 at 102 x 102, N=53: 112 -> 234 us).
+//   strided with whole chunks of 32 channels: only where one pixel tile holds all pixels.  The phases of a 3 x 3 / 2
+//     filter have 1, 2, 2 and 4 taps (128 -> 256 at 28 x 28, N=32: 44 -> 52 us); with one image the fp32 kernels have a few
+//     workgroups with a long chain each (256 -> 512 at 14 x 14, N=1: 61 -> 38 us).
+//   everything else: yes (64 -> 64 at 56 x 56, N=32: 69 -> 52 us; 369 -> 37, 5 x 5 at 76 x 76, N=2, which had only the
+//     table-driven kernel: 801 -> 82 us; equal at the smallest sizes, 64 -> 64 at 56 x 56, N=1: 21.4 -> 21.8 us).
+static bool split_pays(int CH, int R, int S, int sh, int sw, long pixels) {
+    if (option(OPT_CONV_SPLIT) >= 2) return true;        // wherever it applies, for tests and measurements
+    if (R * S < 4 || CH < 16) return false;
+    return (sh == 1 && sw == 1) || CH % 32 != 0 || pixels <= 256;
+}
+
+// Workspace bytes of the split form, 0 where it does not serve the geometry or does not pay.
+size_t split_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
+    SpParams p;
+    if (option(OPT_CONV_SPLIT) == 0 || !split_pays(C, R, S, sh, sw, (long)N * OH * OW)) return 0;
+    if (!sp_plan_fwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW)) return 0;
+    return align_up(p.apk_bytes, 256);
+}
+size_t split_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
+    SpParams p;
+    if (option(OPT_CONV_SPLIT) == 0 || sh > R || sw > S) return 0;
+    if (!split_pays(K, R, S, sh, sw, (long)N * ceil_div(H, sh) * ceil_div(W, sw))) return 0;
+    if (!sp_plan_bwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW)) return 0;
+    return align_up(p.apk_bytes, 256);
+}
+
+int split_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
+                   int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace) {
+    SpParams p;
+    if (!sp_plan_fwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW))
+        return set_error("split convolution: geometry not served"), XSMI_ERR_INVALID;
+    p.in = x; p.w = w; p.bias = bias; p.out = y; p.mask = relu ? mask : nullptr; p.relu = relu;
+    return sp_run(p, opts, workspace);
+}
+
+int split_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, int H, int W, int K, int R, int S, int sh,
+                        int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace) {
+    SpParams p;
+    if (!sp_plan_bwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW))
+        return set_error("split convolution: geometry not served"), XSMI_ERR_INVALID;
+    p.in = dy; p.w = w; p.out = dx; p.accumulate = accumulate;
+    return sp_run(p, opts, workspace);
+}
+
+}  // namespace xsmi

@@ -40,6 +40,7 @@ OptionRow g_options[xsmi::OPT_COUNT] = {
     {"sk_wide", "XSMI_SK_WIDE", 2, false},
     {"pool_bwd", "XSMI_POOL_BWD", 2, false},
     {"pack_lanes", "XSMI_PACK_LANES", 2, false},
+    {"conv_split", "XSMI_CONV_SPLIT", 1, false},
 };
 
 // Streams beside the second one for runs of short independent launches (filter layouts), see side_lane().

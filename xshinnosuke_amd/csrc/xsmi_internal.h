@@ -30,12 +30,12 @@ bool capturing();            // a step graph is being recorded: nothing runs, no
 bool ready();
 int cu_count();
 // Tuning switches (xsmi_set_option / environment variable / default); the order is that of the table in runtime.hip.
-enum Option { OPT_TAP_SK, OPT_SK_SPIN_LIMIT, OPT_TAP_STAGES, OPT_TAP_PERSIST, OPT_CL_HALO, OPT_CL_STEM, OPT_SK_WIDE, OPT_POOL_BWD, OPT_PACK_LANES, OPT_COUNT };
+enum Option { OPT_TAP_SK, OPT_SK_SPIN_LIMIT, OPT_TAP_STAGES, OPT_TAP_PERSIST, OPT_CL_HALO, OPT_CL_STEM, OPT_SK_WIDE, OPT_POOL_BWD, OPT_PACK_LANES, OPT_CONV_SPLIT, OPT_COUNT };
 long option(Option o);
 // Partial tiles and flags of the even-split convolution kernels for the stream that stream() hands out; allocated
 // by xsmi_init, the flags are zero between launches.
 constexpr size_t SK_SCRATCH_FLAG_BYTES = 4096;                          // 1024 workgroups
-constexpr size_t SK_SCRATCH_PART_BYTES = (size_t)1024 * 16 * 256 * 4;   // 1024 workgroups x one 64 x 64 tile of floats
+constexpr size_t SK_SCRATCH_PART_BYTES = (size_t)768 * 32 * 256 * 4;    // 768 workgroups x one 64 x 128 tile of floats
 struct SkScratch {
     uint32_t *flags;
     float *part;
@@ -146,6 +146,15 @@ int sk_conv_fwd(const float *x, const float *w, const float *bias, float *y, uin
                 int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace);
 int sk_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, int H, int W, int K, int R, int S, int sh,
                      int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace);
+
+// fp32 forward / backward-data on the bf16 matrix pipes, operands split into three bf16 values (conv_split.hip); the
+// workspace queries return 0 for geometries the kernel does not serve
+size_t split_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW);
+size_t split_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW);
+int split_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
+                   int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace);
+int split_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, int H, int W, int K, int R, int S, int sh,
+                        int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace);
 
 // forward for very few input channels (conv_stem.hip): 1 or 3 channels, square filter of 3, 5 or 7, horizontal stride 2;
 // the workspace holds the packed filter followed by a zero-bordered copy of the input
