@@ -66,6 +66,46 @@ def test_split_convolution_against_the_oracle(gpu, n, c, h, w, k, r, s, sh, sw, 
         assert rel_l2(gx.numpy(), dx_ref) <= TOL
 
 
+@pytest.mark.parametrize("n,c,h,w,k,pad", [
+    (1, 3, 3, 3, 2, 0),                      # one output pixel
+    (2, 65, 7, 8, 63, 1),                    # rows of one octet; a channel past its tile, a filter short of it
+    (3, 16, 5, 9, 64, 1),                    # the first width of two octets; odd rows
+    (2, 64, 6, 7, 64, 0),                    # no padding: the columns of dy begin two early
+    (3, 20, 11, 17, 70, 0),                  # two column blocks, the second with one column
+    (9, 64, 14, 14, 128, 1),                 # uneven splits
+    (2, 130, 56, 56, 64, 1),                 # many splits: a wave for every eighth
+    (40, 96, 14, 15, 200, 1),                # eight to thirty-one splits
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_split_weight_gradient_against_the_oracle(gpu, n, c, h, w, k, pad, accumulate):
+    K = gpu.kernels
+    x, wt, b, dy, _ = _data(n, c, h, w, k, 3, 3, 1, 1, pad, gpu)
+    dw0, db0 = (wt, b) if accumulate else (np.zeros_like(wt), np.zeros_like(b))
+    _, col = oracle.conv2d_fwd(x, wt, b, (1, 1), pad)
+    _, dw_ref, db_ref = oracle.conv2d_bwd(dy, x.shape, wt, col, (1, 1), pad, np.zeros_like(x), dw0.copy(), db0.copy())
+    gw, gb = gpu.to_device(dw0), gpu.to_device(db0)
+    with split_everywhere(gpu):
+        K.conv2d_bwd_weight(gpu.to_device(dy), gpu.to_device(x), wt.shape, (1, 1), pad, dw=gw, db=gb, accumulate=accumulate)
+    assert rel_l2(gw.numpy(), dw_ref) <= TOL and rel_l2(gb.numpy(), db_ref) <= TOL
+
+
+def test_weight_gradient_of_values_that_do_not_split(gpu):
+    K = gpu.kernels
+    x, wt, b, dy, _ = _data(2, 20, 12, 13, 70, 3, 3, 1, 1, 1, gpu)
+    x[0, 3, 2, 2], x[0, 5, 8, 9], x[1, 19, 6, 6] = np.inf, np.nan, np.float32(3.4e38)
+    dy[1, 4, 5, 5] = -np.inf
+    _, col = oracle.conv2d_fwd(x, wt, b, (1, 1), 1)
+    with np.errstate(all="ignore"):
+        _, ref, _ = oracle.conv2d_bwd(dy, x.shape, wt, col, (1, 1), 1, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+    with split_everywhere(gpu):
+        gw, _ = K.conv2d_bwd_weight(gpu.to_device(dy), gpu.to_device(x), wt.shape, (1, 1), 1, want_db=True)
+    got = gw.numpy()
+    for test in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(test(got), test(ref))
+    calm = np.isfinite(ref) & (np.abs(ref) < 1e30)
+    assert calm.any() and rel_l2(got[calm], ref[calm]) <= TOL
+
+
 def test_values_that_do_not_split_are_multiplied_one_by_one(gpu):
     """Infinities, NaN and floats that round to a bf16 infinity: the outputs they touch are the float32 ones, signs and
     NaNs included, and no other output is disturbed."""

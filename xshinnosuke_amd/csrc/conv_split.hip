@@ -31,16 +31,17 @@
 // first step, which adds them in ascending order (bounded wait, deterministic sums).  Row tiles vary slowest, so
 // that an XCD's workgroups read few filter blocks.
 #include "conv_store.h"
+#include "split3.h"
 
 #include <string.h>
-#include <type_traits>
 
 namespace {
 
 using xsmi::floatx16;
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
+using xsmi::bf16x8;
+using xsmi::uint32x4;
+using xsmi::IC;
+using xsmi::finite;
 
 constexpr int SP_ROWS = 64;
 constexpr int sp_slots_of(int wc) { return wc == 4 ? 512 : 384; }     // slots of an LDS image
@@ -82,37 +83,17 @@ struct SpParams {
     SpTapPlace tap[9];     // of a 3 x 3 filter's taps
 };
 
-template <int N>
-using IC = std::integral_constant<int, N>;
-
 constexpr int AGENT = 16;                            // sc1: past the caches that are not coherent across XCDs
-
-// two floats -> bf16 pair (nearest even); the pair's values taken off the floats
-// (v_dot2_f32_bf16 with (-1, 0) and (0, -1): one instruction for a subtraction and the widening in front of it; the
-// difference is representable, so it is exact)
-__device__ __forceinline__ uint32_t split_pair(float &a, float &b) {
-    const bf16x2 p = {(__bf16)a, (__bf16)b}, hi = {(__bf16)0.f, (__bf16)-1.f};
-    uint32_t lo_bits = 0x0000bf80u;                      // (-1, 0), kept from the compiler: as an inline constant -1.0 it
-    asm("" : "+s"(lo_bits));                             // comes out as (0, -1)
-    const bf16x2 lo = __builtin_bit_cast(bf16x2, lo_bits);
-    a = __builtin_amdgcn_fdot2_f32_bf16(p, lo, a, false);
-    b = __builtin_amdgcn_fdot2_f32_bf16(p, hi, b, false);
-    return __builtin_bit_cast(uint32_t, p);
-}
 
 // eight floats -> three vectors of eight bf16
 __device__ __forceinline__ void split8(const float (&v)[8], uint32x4 &p0, uint32x4 &p1, uint32x4 &p2) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        float a = v[2 * i], b = v[2 * i + 1];
-        p0[i] = split_pair(a, b);
-        p1[i] = split_pair(a, b);
-        const bf16x2 l = {(__bf16)a, (__bf16)b};
-        p2[i] = __builtin_bit_cast(uint32_t, l);
+        uint32_t a, b, c;
+        xsmi::split_pair3(v[2 * i], v[2 * i + 1], a, b, c);
+        p0[i] = a; p1[i] = b; p2[i] = c;
     }
 }
-
-__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_inff(); }
 
 // Outputs that came out non-finite are computed again one float32 product at a time (taps outside, channels inside, as
 // the fp32 kernels add them); a tap outside the input multiplies a zero, as the reference's padding does.
@@ -232,60 +213,58 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         }
     };
             float pre[NJ][8];
-            // always the same number of loads (slots past the run fetch out of range): the waits below count them
-            auto load_image = [&](int grp_) {
-                const int ch0 = grp_ * 16 + octet * 8;
-                if (ch0 + 8 <= p.CH) {
-    #pragma unroll
-                    for (int j = 0; j < NJ; ++j)
-    #pragma unroll
-                        for (int e = 0; e < 8; ++e)
-                            pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                            rin, (int)voff[j], (int)((uint32_t)(ch0 + e) * plane4), 0));
-                } else {
-    #pragma unroll
-                    for (int j = 0; j < NJ; ++j)
-    #pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const bool there = ch0 + e < p.CH;
-                            pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                            rin, (int)(there ? voff[j] : 0x80000000u), (int)(there ? (uint32_t)(ch0 + e) * plane4 : 0u), 0));
-                        }
+    // always the same number of loads (slots past the run fetch out of range): the waits below count them
+    auto load_image = [&](int grp_) {
+        const int ch0 = grp_ * 16 + octet * 8;
+        if (ch0 + 8 <= p.CH) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                    rin, (int)voff[j], (int)((uint32_t)(ch0 + e) * plane4), 0));
+        } else {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const bool there = ch0 + e < p.CH;
+                    pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                    rin, (int)(there ? voff[j] : 0x80000000u), (int)(there ? (uint32_t)(ch0 + e) * plane4 : 0u), 0));
                 }
-            };
-            // the fetched values into an LDS image: a pair of channels at a time, then the three 16-byte pieces
-            uint32x4 piece[3];
-            auto split_one = [&](auto jt, auto it) {
-                constexpr int j = decltype(jt)::value, i = decltype(it)::value;
-                float a = pre[j][2 * i], b = pre[j][2 * i + 1];
-                piece[0][i] = split_pair(a, b);
-                piece[1][i] = split_pair(a, b);
-                const bf16x2 l = {(__bf16)a, (__bf16)b};
-                piece[2][i] = __builtin_bit_cast(uint32_t, l);
-            };
-            auto put = [&](auto j, int to) {
-                unsigned char *dst = s_img + to + octet * SP_PLANE + (64 * (chunk0 + WC * j) + lane) * 16;
-    #pragma unroll
-                for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32x4 *>(dst + 2 * q * SP_PLANE) = piece[q];
-            };
-            auto stage = [&](auto j, int to) {
-                split_one(j, IC<0>{}); split_one(j, IC<1>{}); split_one(j, IC<2>{}); split_one(j, IC<3>{});
-                put(j, to);
-            };
+        }
+    };
+    // the fetched values into an LDS image: a pair of channels at a time, then the three 16-byte pieces
+    uint32x4 piece[3];
+    auto split_one = [&](auto jt, auto it) {
+        constexpr int j = decltype(jt)::value, i = decltype(it)::value;
+        uint32_t a, b, c;
+        xsmi::split_pair3(pre[j][2 * i], pre[j][2 * i + 1], a, b, c);
+        piece[0][i] = a; piece[1][i] = b; piece[2][i] = c;
+    };
+    auto put = [&](auto j, int to) {
+        unsigned char *dst = s_img + to + octet * SP_PLANE + (64 * (chunk0 + WC * j) + lane) * 16;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32x4 *>(dst + 2 * q * SP_PLANE) = piece[q];
+    };
+    auto stage = [&](auto j, int to) {
+        split_one(j, IC<0>{}); split_one(j, IC<1>{}); split_one(j, IC<2>{}); split_one(j, IC<3>{});
+        put(j, to);
+    };
     uint32_t a_off = 0;
     int b_rd[2];                                       // this lane's two pixels in an image
-            // two steps of filter fragments and two of pixel fragments in registers: a step's filter loads are issued while
-            // the step two before it multiplies, its LDS reads while the one before it does
-            bf16x8 fa[2][3], fb[2][2][3];                  // [step parity][piece], [step parity][pixel block][piece]
-            auto load_a = [&](auto par, auto q) {
-                fa[par][q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
-                                 rapk, a_voff + (int)q * 2 * SP_ROWS * 16, (int)a_off, 0));
-            };
-            auto read_b = [&](auto par, auto q, int off) {
-    #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    fb[par][j][q] = *reinterpret_cast<const bf16x8 *>(s_img + b_rd[j] + off + (int)q * 2 * SP_PLANE);
-            };
+    // two steps of filter fragments and two of pixel fragments in registers: a step's filter loads are issued while
+    // the step two before it multiplies, its LDS reads while the one before it does
+    bf16x8 fa[2][3], fb[2][2][3];                  // [step parity][piece], [step parity][pixel block][piece]
+    auto load_a = [&](auto par, auto q) {
+        fa[par][q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                         rapk, a_voff + (int)q * 2 * SP_ROWS * 16, (int)a_off, 0));
+    };
+    auto read_b = [&](auto par, auto q, int off) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            fb[par][j][q] = *reinterpret_cast<const bf16x8 *>(s_img + b_rd[j] + off + (int)q * 2 * SP_PLANE);
+    };
     int t_left = 0, tb = 0, off = 0, Tx = 1, row_end = 0;
     auto next_off = [&]() {                            // past the last tap: back to a place inside the image
         off += ++tb == Tx ? row_end : 16;
@@ -293,12 +272,12 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         off = --t_left == 0 ? 0 : off;
     };
     floatx16 hi[2], lo[2];
-            auto mm = [&](auto par, floatx16 (&acc)[2], int qa, int qb) {
-    #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[par][qa], fb[par][j][qb], acc[j], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-            };
+    auto mm = [&](auto par, floatx16 (&acc)[2], int qa, int qb) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[par][qa], fb[par][j][qb], acc[j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
     // One step.  The next tap's fragments are read from the same image (past a group's last tap: places that are not
     // used); the filter block two steps ahead takes each piece's registers after the piece's last product.  J >= 0: a
     // part of the next image is split and written to the other half of the LDS, a few instructions behind each pair of
@@ -372,7 +351,6 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         if constexpr (NJ == 3)
             if (staged < 3) stage(third, SP_IMAGE - image);
     };
-
 
     // The workgroup's steps are one stream: a segment's first image and filter blocks are requested while the segment before
     // it is multiplied, and its output stores drain behind the next one's MFMAs.

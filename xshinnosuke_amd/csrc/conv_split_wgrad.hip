@@ -1,0 +1,431 @@
+// fp32 weight gradient of 3 x 3, stride-1 layers on the bf16 matrix pipes, operands split into three bf16 values as in
+// conv_split.hip (six products, exact up to 2^-25 of each term).
+//
+//     dw[k][c][r][s] = sum over (n, y, x) of dy[n][k][y][x] * in[n][c][y + r - pad][x + s - pad]
+//
+// rows = 64 filters, columns = 64 channels, reduction = pixels.  An MFMA lane wants eight consecutive reduction values of
+// a row in 16 bytes: eight neighbouring pixels of an image row (an octet).  The sum runs over output rows y and INPUT
+// columns j, dw[r][s] = sum dy[y][j + pad - s] in[y + r - pad][j]: a filter row then moves the input by whole rows, and a
+// filter column moves dy, of which there are three fragments instead of nine, by one value.  A STAGE is four octets, two
+// rows of two or, for rows of at most eight pixels, four rows of one; with the rows around them it takes 8 (6) octets of
+// input and 6 (8) of dy for each channel and filter, which 512 threads fetch (32 bytes contiguous each), split and write
+// to the LDS as [piece][channel][octet].  All nine taps read that image.  The columns of dy in the LDS begin at pad - 2, so
+// that a tap's values are the five dwords from a lane's octet on, taken 0, 1 or 2 half dwords further (v_alignbit for 1).
+// Odd pitches keep reads (lanes = channels) and writes (lanes = octets) free of bank conflicts.
+//
+// Eight waves: 2 x 2 of 32 filters x 32 channels, twice; the second four take the stage's other two octets, so each wave
+// multiplies one k-step of 16 pixels and nine taps (54 MFMAs) between two barriers, while its share of the next stage is
+// split behind the MFMAs and the one after it is in flight.  The two halves are added through the LDS at the end.
+// Workgroups take equal runs of stages; each writes its nine 64 x 64 partial products, and one launch adds them in
+// ascending order in float64.
+#include "split3.h"
+
+#include <string.h>
+
+namespace {
+
+using xsmi::bf16x8;
+using xsmi::IC;
+using xsmi::uint32x4;
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+constexpr int T64 = 64;
+constexpr int XP = 9, YP = 9;                         // octets per channel / filter in the LDS: 8 at most, made odd
+constexpr int X_PLANE = T64 * XP * 16, Y_PLANE = T64 * YP * 16;
+constexpr int STAGE = 3 * (X_PLANE + Y_PLANE);
+constexpr int TILE = 9 * T64 * T64;                   // floats of a workgroup's partial result
+static_assert(2 * STAGE <= 9 * 16 * 256 * 4, "the stages fit where the halves are added");
+
+struct WgParams {
+    const float *dy, *x;
+    float *part, *dbpart;                             // [split][k tile][c tile][tap][64][64], [split][K]
+    uint32_t x_bytes, dy_bytes;
+    int N, C, H, W, K, OH, OW, pad, CB, RB;           // CB octets across and RB output rows of a stage
+    int kt, ct, splits, stages, per, rem;             // stages of the pass, per split
+    int row_blocks, col_blocks;
+};
+
+__global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
+    __shared__ __attribute__((aligned(16))) unsigned char s_mem[9 * 16 * 256 * 4];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int half = wave >> 2, wr = (wave >> 1) & 1, wc = wave & 1, h = lane >> 5, l31 = lane & 31;
+    const int tiles = p.kt * p.ct;
+    const int id = (int)xsmi::xcd_contiguous_id(blockIdx.x, gridDim.x);
+    const int split = id / tiles, tile = id - split * tiles, k0 = tile / p.ct * T64, c0 = tile % p.ct * T64;
+    const int s0 = split * p.per + (split < p.rem ? split : p.rem), s1 = s0 + p.per + (split < p.rem ? 1 : 0);
+
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, (int)p.x_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)p.dy, 0, (int)p.dy_bytes, 0x00020000);
+
+    // ---- staging: of the stage's octets, input first, this thread takes number t and number t + 512 ----
+    const int nx = (p.RB + 2) * p.CB, ny = p.RB * (p.CB + 1);          // per channel and per filter
+    struct Mine { int ch, row, col, lds; bool live; };
+    const bool y_side[2] = {wave * 64 >= nx * T64, 512 + wave * 64 >= nx * T64};      // nx 64 is a multiple of a wave's 64
+    auto mine = [&](int o, bool y) {
+        Mine m;
+        const int per = y ? ny : nx, across = y ? p.CB + 1 : p.CB;
+        if (y) o -= nx * T64;
+        const int c = o / per, sl = o - c * per;
+        m.row = sl / across; m.col = (sl - m.row * across) * 8;
+        m.live = c < T64 && (y ? k0 + c < p.K : c0 + c < p.C);
+        m.ch = y ? (k0 + c) * p.OH * p.OW : (c0 + c) * p.H * p.W;
+        m.lds = c >= T64 ? -1 : y ? 3 * X_PLANE + (c * YP + sl) * 16 : (c * XP + sl) * 16;
+        return m;
+    };
+    const Mine m0 = mine(t, y_side[0]), m1 = mine(t + 512, y_side[1]);
+    struct Place { int n, y, x; };                    // image, first output row, first input column of a stage
+    auto place = [&](int s) {
+        Place q;
+        const int cb = s % p.col_blocks, r = s / p.col_blocks;
+        q.x = cb * p.CB * 8; q.y = r % p.row_blocks * p.RB; q.n = r / p.row_blocks;
+        return q;
+    };
+    auto next = [&](Place &q) {
+        q.x += p.CB * 8;
+        if (q.x >= p.col_blocks * p.CB * 8) {
+            q.x = 0; q.y += p.RB;
+            if (q.y >= p.row_blocks * p.RB) { q.y = 0; ++q.n; }
+        }
+    };
+    float pre[2][8];
+    int cut[2], early[2];                             // values from this one on are past the row; the octet begins that much early
+    bool ends[2];                                     // uniform: some octet of the stage crosses an end of its row
+    auto fetch = [&](auto jt, const Place &q) {
+        constexpr int j = decltype(jt)::value;
+        const Mine &m = j == 0 ? m0 : m1;
+        const bool y = y_side[j];
+        const int rows = y ? p.OH : p.H, cols = y ? p.OW : p.W;
+        const int row = q.y + m.row - (y ? 0 : p.pad), first = q.x + (y ? p.pad - 2 : 0), col = first + m.col;
+        early[j] = col < 0 ? -col : 0;                // fetched from column 0 and moved up
+        cut[j] = cols - col;
+        ends[j] = first < 0 || first + (p.CB + (y ? 1 : 0)) * 8 > cols;
+        const int from = col < 0 ? 0 : col;
+        const bool ok = m.live && row >= 0 && row < rows && from < cols;
+        const uint32_t image = (uint32_t)(y ? p.K * p.OH * p.OW : p.C * p.H * p.W);
+        const uint32_t off = ok ? (uint32_t)q.n * image + (uint32_t)(m.ch + row * cols + from) : 0x20000000u;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32x4 v = __builtin_amdgcn_raw_buffer_load_b128(y ? ry : rx, (int)(off * 4u) + 16 * i, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { const uint32_t b = v[e]; pre[j][4 * i + e] = __builtin_bit_cast(float, b); }
+        }
+    };
+    // db: the dy octets of a stage overlap by two columns on either side; the values of columns [8 i, 8 i + 8) are the ones
+    // 2 - pad and further of octet i and the first of octet i + 1, so an octet adds all of its values up to a stage's end
+    // and the last one the first 2 - pad only
+    double db_sum = 0.0;
+    const bool want_db = p.dbpart != nullptr && c0 == 0;
+    uint32x4 piece[3];
+    auto trim = [&](auto jt, const Place &q) {        // zeros outside the row
+        constexpr int j = decltype(jt)::value;
+        float *v = pre[j];
+        if (ends[j]) {
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+                if (early[j] > n) {
+#pragma unroll
+                    for (int i = 7; i > 0; --i) v[i] = v[i - 1];
+                    v[0] = 0.f;
+                }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = i < cut[j] ? v[i] : 0.f;
+        }
+        if (y_side[j] && want_db) {
+            const Mine &m = j == 0 ? m0 : m1;
+            const bool first = q.x == 0 || m.col > 0, last = m.col == p.CB * 8 && q.x + p.CB * 8 < p.col_blocks * p.CB * 8;
+            float all = ((v[2] + v[3]) + (v[4] + v[5])) + (v[6] + v[7]);
+            float head = v[0] + (p.pad == 0 ? v[1] : 0.f);
+            all += p.pad == 0 ? 0.f : v[1];
+            db_sum += (double)((first ? head : 0.f) + (last ? 0.f : all));
+        }
+    };
+    auto split_two = [&](auto jt, auto it) {          // pairs 2 it and 2 it + 1
+        constexpr int j = decltype(jt)::value, i0 = 2 * decltype(it)::value;
+#pragma unroll
+        for (int i = i0; i < i0 + 2; ++i) {
+            uint32_t a, b, c;
+            xsmi::split_pair3(pre[j][2 * i], pre[j][2 * i + 1], a, b, c);
+            piece[0][i] = a; piece[1][i] = b; piece[2][i] = c;
+        }
+    };
+    auto put = [&](auto jt, int to) {
+        constexpr int j = decltype(jt)::value;
+        const Mine &m = j == 0 ? m0 : m1;
+        if (m.lds < 0) return;
+        const int plane = y_side[j] ? Y_PLANE : X_PLANE;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32x4 *>(s_mem + to + m.lds + q * plane) = piece[q];
+    };
+
+    // ---- multiply side: this lane's octet e of the stage, its filter and its channel ----
+    const int e = 2 * half + h, e_row = e / p.CB, e_col = e - e_row * p.CB;
+    const int a_base = 3 * X_PLANE + ((wr * 32 + l31) * YP + e_row * (p.CB + 1) + e_col) * 16;
+    const int b_base = ((wc * 32 + l31) * XP + e) * 16, r_step = p.CB * 16;
+    floatx16 acc[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
+    bf16x8 fa[3][3], fb[2][3];                        // [filter column][piece], [row parity][piece]
+    typedef uint32_t uint32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+    auto read_a = [&](int from) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const unsigned char *src = s_mem + from + a_base + q * Y_PLANE;
+            const uint32x4 d = *reinterpret_cast<const uint32x4 *>(src);
+            const uint32x4 d1 = *reinterpret_cast<const uint32x4_a4 *>(src + 4);
+            uint32x4 m;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m[i] = __builtin_amdgcn_alignbit(d1[i], d[i], 16);
+            fa[2][q] = __builtin_bit_cast(bf16x8, d);
+            fa[1][q] = __builtin_bit_cast(bf16x8, m);
+            fa[0][q] = __builtin_bit_cast(bf16x8, d1);
+        }
+    };
+    auto read_b = [&](auto rt, int from) {
+        constexpr int r = decltype(rt)::value;
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            fb[r & 1][q] = *reinterpret_cast<const bf16x8 *>(s_mem + from + b_base + q * X_PLANE + r * r_step);
+    };
+    auto multiply = [&](auto rt, int qa, int qb) {
+        constexpr int r = decltype(rt)::value;
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+            acc[3 * r + s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s][qa], fb[r & 1][qb], acc[3 * r + s], 0, 0, 0);
+    };
+
+    Place at = place(s0), at1 = at;                   // of the values in flight, and of the next ones
+    fetch(IC<0>{}, at); fetch(IC<1>{}, at);
+    trim(IC<0>{}, at); split_two(IC<0>{}, IC<0>{}); split_two(IC<0>{}, IC<1>{}); put(IC<0>{}, 0);
+    trim(IC<1>{}, at); split_two(IC<1>{}, IC<0>{}); split_two(IC<1>{}, IC<1>{}); put(IC<1>{}, 0);
+    next(at);
+    fetch(IC<0>{}, at); fetch(IC<1>{}, at);           // past the last image: out of range
+    at1 = at;
+    int cur = 0;
+    for (int s = s0; s < s1; ++s) {
+        xsmi::wait_lgkmcnt0();
+        xsmi::block_barrier();                        // this stage is complete, and nobody reads the other one any more
+        const int to = STAGE - cur;
+        const bool more = s + 1 < s1;
+        next(at1);
+        read_b(IC<0>{}, cur);
+        read_a(cur);
+        read_b(IC<1>{}, cur);
+        __builtin_amdgcn_sched_barrier(0);
+        auto row = [&](auto rt) {
+            constexpr int r = decltype(rt)::value;
+            multiply(rt, 2, 0);
+            if constexpr (r > 0) { if (more) trim(IC<r - 1>{}, at); }
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(rt, 1, 0);
+            if constexpr (r > 0) split_two(IC<r - 1>{}, IC<0>{});
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(rt, 0, 0);
+            if constexpr (r > 0) split_two(IC<r - 1>{}, IC<1>{});
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(rt, 1, 1);
+            if constexpr (r > 0) { if (more) put(IC<r - 1>{}, to); }
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(rt, 0, 1);
+            if constexpr (r > 0) fetch(IC<r - 1>{}, at1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(rt, 0, 2);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (r == 0) read_b(IC<2>{}, cur);
+        };
+        row(IC<0>{});
+        row(IC<1>{});
+        row(IC<2>{});
+        at = at1;
+        cur = to;
+    }
+
+    // the two halves of the waves, then the partial result: register v of lane l is filter 8 (v / 4) + 4 (l / 32) + v % 4,
+    // channel l % 32 of the wave's block
+    xsmi::wait_lgkmcnt0();
+    __syncthreads();
+    float *s_acc = reinterpret_cast<float *>(s_mem);
+    if (half == 1) {
+#pragma unroll
+        for (int i = 0; i < 9; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s_acc[(i * 16 + v) * 256 + (t & 255)] = acc[i][v];
+    }
+    __syncthreads();
+    if (half == 0) {
+        float *dst = p.part + ((size_t)split * tiles + tile) * TILE + (wr * 32 + 4 * h) * T64 + wc * 32 + l31;
+#pragma unroll
+        for (int i = 0; i < 9; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                dst[i * T64 * T64 + (8 * (v >> 2) + (v & 3)) * T64] = acc[i][v] + s_acc[(i * 16 + v) * 256 + t];
+    }
+    if (want_db) {                                    // a filter's octets are in up to ny threads: added in their order
+        double *s_db = reinterpret_cast<double *>(s_mem);
+        __syncthreads();
+        if (y_side[1] && m1.lds >= 0) s_db[t + 512 - nx * T64] = db_sum;
+        if (y_side[0]) s_db[t - nx * T64] = db_sum;
+        __syncthreads();
+        if (t < T64 && k0 + t < p.K) {
+            double sum = 0.0;
+            for (int i = 0; i < ny; ++i) sum += s_db[t * ny + i];
+            p.dbpart[(size_t)split * p.K + k0 + t] = (float)sum;
+        }
+    }
+}
+
+// dw (+)= the partial results in ascending order, in float64.  A workgroup owns 8 / GW filters and 64 channels, TAPS taps
+// of them; GW waves share the splits of a filter.  Many splits (64 -> 64 channels: 256): GW = 8 and one tap, so that 576
+// workgroups read the 38 MB (12.7 us; 192 of three taps: 23 us); few (512 -> 512: 4): GW = 1 and all nine taps (12.6 us; GW = 8: 20 us).  Results that are not finite (an operand was not, or
+// rounds to a bf16 infinity) are formed again from the products themselves.  The workgroups behind them add db.
+template <int GW, int TAPS>
+__global__ void __launch_bounds__(512) split_wgrad_reduce_kernel(WgParams p, float *dw, float *db, int accumulate, int dw_blocks) {
+    constexpr int KB = 8 / GW, ROW = T64 * TAPS, FLIGHT = GW == 1 ? 2 : GW == 2 ? 4 : 8;
+    __shared__ double s_sum[8][ROW];
+    __shared__ double s_part[512];
+    __shared__ uint32_t s_bad;
+    const int t = threadIdx.x, c = t & 63, w = t >> 6;
+    if ((int)blockIdx.x >= dw_blocks) {
+        const int k = ((int)blockIdx.x - dw_blocks) * 64 + c;
+        double sum = 0.0;
+        if (k < p.K) {
+#pragma unroll 4
+            for (int s = w; s < p.splits; s += 8) sum += (double)p.dbpart[(size_t)s * p.K + k];
+        }
+        s_part[t] = sum;
+        __syncthreads();
+        if (t >= 64 || k >= p.K) return;
+        sum = accumulate ? (double)db[k] : 0.0;
+        for (int j = 0; j < 8; ++j) sum += s_part[j * 64 + t];
+        db[k] = (float)sum;
+        return;
+    }
+    const int r0 = (int)blockIdx.x % (9 / TAPS) * TAPS, kc = (int)blockIdx.x / (9 / TAPS), kb = kc / p.ct * KB, ctile = kc % p.ct, c0 = ctile * T64;
+    const int k = kb + w / GW, tiles = p.kt * p.ct, tile = k / T64 * p.ct + ctile;
+    double sum[TAPS];
+#pragma unroll
+    for (int i = 0; i < TAPS; ++i) sum[i] = 0.0;
+    if (k < p.K) {
+        const float *src = p.part + (size_t)tile * TILE + (r0 * T64 + k % T64) * T64 + c;
+        const size_t step = (size_t)tiles * TILE;
+        for (int s = w % GW; s < p.splits; s += GW * FLIGHT) {
+            float v[FLIGHT][TAPS];
+#pragma unroll
+            for (int j = 0; j < FLIGHT; ++j)
+#pragma unroll
+                for (int i = 0; i < TAPS; ++i) v[j][i] = s + GW * j < p.splits ? src[(size_t)(s + GW * j) * step + i * T64 * T64] : 0.f;
+#pragma unroll
+            for (int j = 0; j < FLIGHT; ++j)
+#pragma unroll
+                for (int i = 0; i < TAPS; ++i) sum[i] += (double)v[j][i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TAPS; ++i) s_sum[w][c * TAPS + i] = sum[i];
+    if (t == 0) s_bad = 0;
+    __syncthreads();
+    const int live = (p.C - c0 < T64 ? p.C - c0 : T64) * TAPS;
+    auto out = [&](int kk, int i) { return dw + ((size_t)(kb + kk) * p.C + c0 + i / TAPS) * 9 + r0 + i % TAPS; };
+    for (int o = t; o < KB * ROW; o += 512) {
+        const int kk = o / ROW, i = o - kk * ROW;
+        double all = 0.0;
+#pragma unroll
+        for (int j = 0; j < GW; ++j) all += s_sum[kk * GW + j][i];
+        const bool mine = i < live && kb + kk < p.K, good = xsmi::finite((float)all);
+        s_sum[kk * GW][i] = mine && !good ? 1.0 : 0.0;
+        if (mine && good) {
+            float *q = out(kk, i);
+            *q = (float)(accumulate ? all + (double)*q : all);
+        } else if (mine) {
+            atomicOr(&s_bad, 1u);
+        }
+    }
+    __syncthreads();
+    if (s_bad == 0) return;
+    for (int o = 0; o < KB * ROW; ++o) {
+        const int kk = o / ROW, i = o - kk * ROW;
+        if (s_sum[kk * GW][i] == 0.0) continue;       // uniform
+        const int cc = c0 + i / TAPS, tap = r0 + i % TAPS, total = p.N * p.OH * p.OW;
+        double part = 0.0;
+        for (int m = t; m < total; m += 512) {
+            const int q = m / p.OW, ox = m - q * p.OW, n = q / p.OH, oy = q - n * p.OH;
+            const int iy = oy + tap / 3 - p.pad, ix = ox + tap % 3 - p.pad;
+            const float a = p.dy[((size_t)n * p.K + kb + kk) * p.OH * p.OW + (size_t)oy * p.OW + ox];
+            const float b = iy >= 0 && iy < p.H && ix >= 0 && ix < p.W ? p.x[((size_t)n * p.C + cc) * p.H * p.W + (size_t)iy * p.W + ix] : 0.f;
+            part += (double)a * (double)b;
+        }
+        __syncthreads();
+        s_part[t] = part;
+        __syncthreads();
+        if (t == 0) {
+            double all = 0.0;
+            for (int j = 0; j < 512; ++j) all += s_part[j];
+            float *q = out(kk, i);
+            *q = (float)(accumulate ? all + (double)*q : all);
+        }
+    }
+}
+
+void wg_plan(WgParams &p, int N, int C, int H, int W, int K, int pad, int OH, int OW) {
+    memset(&p, 0, sizeof(p));
+    p.N = N; p.C = C; p.H = H; p.W = W; p.K = K; p.OH = OH; p.OW = OW; p.pad = pad;
+    p.CB = W <= 8 ? 1 : 2; p.RB = 4 / p.CB;
+    p.kt = xsmi::ceil_div(K, T64); p.ct = xsmi::ceil_div(C, T64);
+    p.row_blocks = xsmi::ceil_div(OH, p.RB); p.col_blocks = xsmi::ceil_div(W, 8 * p.CB);
+    p.stages = N * p.row_blocks * p.col_blocks;
+    // splits: a stage takes about 2 us in each round of workgroups over the 256 compute units (a constant: a workspace may
+    // be sized before a device is open), and a partial result 0.06 us to write and read again
+    const int tiles = p.kt * p.ct;
+    long best = -1;
+    for (int s = 1; s <= 256 && s <= p.stages; ++s) {
+        const long cost = (long)xsmi::ceil_div(tiles * s, 256) * xsmi::ceil_div(p.stages, s) * 200 + (long)tiles * s * 6;
+        if (best < 0 || cost < best) { best = cost; p.splits = s; }
+    }
+    p.per = p.stages / p.splits; p.rem = p.stages % p.splits;
+    p.x_bytes = (uint32_t)((size_t)N * C * H * W * 4); p.dy_bytes = (uint32_t)((size_t)N * K * OH * OW * 4);
+}
+
+}  // namespace
+
+namespace xsmi {
+
+size_t split_wgrad_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad) {
+    const long opt = option(OPT_CONV_SPLIT);
+    if (opt == 0 || R != 3 || S != 3 || sh != 1 || sw != 1 || pad > 1) return 0;
+    const int OH = H + 2 * pad - 2, OW = W + 2 * pad - 2;
+    WgParams p;
+    wg_plan(p, N, C, H, W, K, pad, OH, OW);
+    // Below about seven stages for each compute unit the fp32 kernels' smaller partial results win (128 -> 128 at 28 x 28:
+    // N=8 33 -> 37 us, N=16 46 -> 45, N=32 72 -> 61), with a few channels the columns that multiply zeros (2 -> 480 at
+    // 93 x 93, N=6: 62 -> 140 us).
+    if (opt < 2 && (C < 16 || (long)p.stages * p.kt * p.ct < 1750)) return 0;
+    return align_up((size_t)p.splits * p.kt * p.ct * TILE * sizeof(float), 256) + align_up((size_t)p.splits * K * sizeof(float), 256);
+}
+
+int split_conv_bwd_weight(const float *dy, const float *x, float *dw, float *db, int N, int C, int H, int W, int K, int pad, int OH,
+                          int OW, int accumulate, void *workspace) {
+    WgParams p;
+    wg_plan(p, N, C, H, W, K, pad, OH, OW);
+    p.dy = dy; p.x = x;
+    p.part = (float *)workspace;
+    if (db) p.dbpart = (float *)((char *)workspace + align_up((size_t)p.splits * p.kt * p.ct * TILE * sizeof(float), 256));
+    hipStream_t st = stream();
+    prof_begin();
+    hipLaunchKernelGGL(split_wgrad_kernel, dim3(p.splits * p.kt * p.ct), dim3(512), 0, st, p);
+    prof_end();
+    XSMI_LAUNCH_CHECK("split_wgrad_kernel");
+    const int db_blocks = db ? ceil_div(K, 64) : 0;
+    auto reduce = [&](auto kernel, int per_filters, int parts) {
+        const int dw_blocks = ceil_div(K, per_filters) * p.ct * parts;
+        hipLaunchKernelGGL(kernel, dim3(dw_blocks + db_blocks), dim3(512), 0, st, p, dw, db, accumulate, dw_blocks);
+    };
+    if (p.splits >= 32) reduce(split_wgrad_reduce_kernel<8, 1>, 1, 9);
+    else if (p.splits >= 8) reduce(split_wgrad_reduce_kernel<2, 3>, 4, 3);
+    else reduce(split_wgrad_reduce_kernel<1, 9>, 8, 1);
+    XSMI_LAUNCH_CHECK("split_wgrad_reduce_kernel");
+    return XSMI_OK;
+}
+
+}  // namespace xsmi

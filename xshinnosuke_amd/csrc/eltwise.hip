@@ -90,6 +90,7 @@ size_t xsmi_conv2d_pass_workspace_bytes(int N, int C, int H, int W, int K, int R
         m = xsmi::conv_bwd_weight_ws_bytes(N, C, K, R, S, OH, OW);
         if (!bf16 && xsmi::stem_wgrad_ok(N, C, H, W, K, R, S, sh, sw, pad))
             m = larger(m, xsmi::stem_wgrad_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad));
+        m = larger(m, xsmi::split_wgrad_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad));
     }
     return m;
 }
