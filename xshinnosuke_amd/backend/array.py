@@ -5,10 +5,11 @@ import weakref
 
 import numpy as np
 
-from .capi import lib, ensure_init, XsmiError, flush_deferred
+from .capi import lib, ensure_init, XsmiError, flush_deferred, _deferred
 
 
-_DTYPE_CLASS = np.dtype(np.float32).__class__
+_F32 = np.dtype(np.float32)
+_DTYPE_CLASS = _F32.__class__
 
 _POOL = {}            # rounded size -> list of free device pointers
 _CL_POOL = {}         # (n, c, h, w, border) -> ChannelsLast forms of released arrays (their borders are zero)
@@ -46,7 +47,6 @@ class _Block:
     __slots__ = ("ptr", "nbytes", "logical", "lazy_zero", "version", "cl", "owner", "unwritten", "__weakref__")
 
     def __init__(self, nbytes):
-        ensure_init()
         self.logical = int(nbytes)
         self.lazy_zero = False
         self.unwritten = None                # why the contents were never produced (a message), see never_written()
@@ -67,6 +67,7 @@ class _Block:
             self.ptr = free.pop()
             _POOL_BYTES[0] -= size
         else:
+            ensure_init()                    # (a pooled block has been through here)
             p = ctypes.c_void_p()
             try:
                 lib.call("xsmi_malloc", ctypes.byref(p), size)
@@ -143,12 +144,16 @@ class DeviceArray:
 
     def __init__(self, shape, dtype=np.float32, _block=None, _offset=0):
         self.shape = shape = tuple(map(int, shape))
-        self.dtype = dtype if dtype.__class__ is _DTYPE_CLASS else np.dtype(dtype)
-        self.size = math.prod(shape)
-        self.nbytes = self.size * self.dtype.itemsize
+        if dtype is np.float32:
+            dtype = _F32
+        elif dtype.__class__ is not _DTYPE_CLASS:
+            dtype = np.dtype(dtype)
+        self.dtype = dtype
+        self.size = size = math.prod(shape)
+        self.nbytes = nbytes = size * dtype.itemsize
         if _block is None:
-            _block = _Block(max(self.nbytes, 16))
-            _block.logical = self.nbytes
+            _block = _Block(nbytes if nbytes > 16 else 16)
+            _block.logical = nbytes
         self._block = _block
         self._offset = int(_offset)
 
@@ -313,7 +318,8 @@ class DeviceArray:
         """Clear the array.  ``lazy=True`` only marks a whole allocation as zero: the memset happens on
         the first ordinary use, and not at all if the first use overwrites everything (take_fresh)."""
         blk = self._block
-        flush_deferred(blk)                   # a held-back operation that uses this allocation comes first
+        if _deferred:
+            flush_deferred(blk)               # a held-back operation that uses this allocation comes first
         self._overwritten()
         if lazy and self._offset == 0 and self.nbytes >= blk.logical:
             blk.lazy_zero = True
@@ -326,6 +332,8 @@ class DeviceArray:
     def reshape(self, *shape):
         if len(shape) == 1 and isinstance(shape[0], (tuple, list)):
             shape = tuple(shape[0])
+        if shape == (-1,):
+            shape = (self.size,)
         shape = list(shape)
         if -1 in shape:
             known = math.prod(s for s in shape if s != -1)

@@ -161,7 +161,7 @@ class _Lib:
             _flush_deferred()
         if _side_hold and name not in _SIDE_SAFE:
             join_side()
-        dll = self._open()
+        dll = self._dll or self._open()
         rc = getattr(dll, name)(*args)
         if rc != 0:
             msg = dll.xsmi_last_error().decode("utf-8", "replace")

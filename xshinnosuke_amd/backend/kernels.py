@@ -30,10 +30,10 @@ def _dims(x_shape, w_shape, stride, pad):
     k, c2, r, s = w_shape
     if c2 != c:
         raise ValueError("conv2d: input has %d channels, weight expects %d" % (c, c2))
-    return [int(v) for v in (n, c, h, w, k, r, s, stride[0], stride[1], pad)]
+    return tuple(map(int, (n, c, h, w, k, r, s, stride[0], stride[1], pad)))
 
 
-_NEED = {}                  # geometry -> xsmi_conv2d_workspace_bytes (a pure function of the ten numbers)
+_NEED = {}                  # geometry -> xsmi_conv2d_workspace_bytes (a pure function of the ten numbers); channels -> batch norm's
 
 
 def _need(dims):
@@ -50,6 +50,13 @@ def _need_pass(dims, pass_):
     need = _NEED.get(key)
     if need is None:
         need = _NEED[key] = lib.raw("xsmi_conv2d_pass_workspace_bytes")(*dims, pass_, 0)
+    return need
+
+
+def _need_bn(channels):
+    need = _NEED.get(channels)
+    if need is None:
+        need = _NEED[channels] = lib.raw("xsmi_bn_workspace_bytes")(channels)
     return need
 
 
@@ -171,8 +178,11 @@ def refresh_layouts(arrays):
         capi.layouts_enqueued(*held)
 
 
+_F32 = np.dtype(np.float32)
+
+
 def _f32(a, what):
-    if not isinstance(a, DeviceArray) or a.dtype != np.float32:
+    if not isinstance(a, DeviceArray) or (a.dtype is not _F32 and a.dtype != _F32):
         raise TypeError("%s must be a float32 DeviceArray" % what)
     return a
 
@@ -216,19 +226,19 @@ def conv2d_fwd(x, w, bias=None, stride=(1, 1), pad=0, relu=False, out=None, neg_
     if channels_last and bf16 and neg_mask is None:
         xcl = x.channels_last()
         if xcl is not None and not (c % 32 == 0 and xcl.border >= pad):
-            xcl = None                                # read through the float32 form (x.cptr converts)
+            xcl = None                                # read through the float32 form (x.ptr converts)
         if xcl is not None or c % 32 == 0 or c <= 8:
             ycl = out.channels_last_out(1) if k % 8 == 0 else None
-            lib.call("xsmi_conv2d_fwd_cl", None if xcl is not None else x.cptr, xcl.buf.cptr if xcl is not None else None,
-                     xcl.border if xcl is not None else 0, w.cptr, bias.cptr if bias is not None else None,
-                     None if ycl is not None else out.cptr, ycl.buf.cptr if ycl is not None else None, 1, *dims,
+            lib.call("xsmi_conv2d_fwd_cl", None if xcl is not None else x.ptr, xcl.buf.ptr if xcl is not None else None,
+                     xcl.border if xcl is not None else 0, w.ptr, bias.ptr if bias is not None else None,
+                     None if ycl is not None else out.ptr, ycl.buf.ptr if ycl is not None else None, 1, *dims,
                      flags & ~CONV_BF16, ws, ws_bytes)
             return out
     out._overwritten()
     # a filter whose layout is in place is not read: its address goes along without counting as handed out
-    wptr = ctypes.c_void_p(w.address()) if layout is not None and packed else w.cptr
-    lib.call("xsmi_conv2d_fwd", x.cptr, wptr, bias.cptr if bias is not None else None, out.cptr,
-             neg_mask.cptr if neg_mask is not None else None, *dims, flags, ws, ws_bytes)
+    wptr = ctypes.c_void_p(w.address()) if layout is not None and packed else w.ptr
+    lib.call("xsmi_conv2d_fwd", x.ptr, wptr, bias.ptr if bias is not None else None, out.ptr,
+             neg_mask.ptr if neg_mask is not None else None, *dims, flags, ws, ws_bytes)
     if layout is not None and not packed:
         layout.key = _filter_key(w)               # the call has laid the present filter out in this workspace
     return out
@@ -264,8 +274,8 @@ def conv2d_bwd_data(dy, w, x_shape, stride=(1, 1), pad=0, dx=None, accumulate=Fa
         layout, packed = _layout_for(w, 1, dims)
     ws, ws_bytes = _workspace(dims) if layout is None else layout.ws.get(_need_pass(dims, 1))
     beta = _beta(accumulate, dx)
-    wptr = ctypes.c_void_p(w.address()) if layout is not None and packed else w.cptr
-    lib.call("xsmi_conv2d_bwd_data", dy.cptr, wptr, dx.cptr, *dims, beta,
+    wptr = ctypes.c_void_p(w.address()) if layout is not None and packed else w.ptr
+    lib.call("xsmi_conv2d_bwd_data", dy.ptr, wptr, dx.ptr, *dims, beta,
              (CONV_BF16 if bf16 else 0) | (CONV_WS_PACKED if packed else 0), ws, ws_bytes)
     if layout is not None and not packed:
         layout.key = _filter_key(w)
@@ -291,7 +301,7 @@ def conv2d_bwd_weight(dy, x, w_shape, stride=(1, 1), pad=0, dw=None, db=None, ac
         raise ValueError("conv2d backward: db has %d elements for %d filters" % (db.size, k))
     ws, ws_bytes = _workspace(dims)
     beta = _beta(accumulate, dw, db)
-    lib.call("xsmi_conv2d_bwd_weight", dy.cptr, x.cptr, dw.cptr, db.cptr if db is not None else None, *dims,
+    lib.call("xsmi_conv2d_bwd_weight", dy.ptr, x.ptr, dw.ptr, db.ptr if db is not None else None, *dims,
              beta, CONV_BF16 if bf16 else 0, ws, ws_bytes)
     return dw, db
 
@@ -323,8 +333,8 @@ def conv2d_bwd(dy, x, w, dx, dw, db=None, stride=(1, 1), pad=0, accumulate=False
     beta_dw = _beta(accumulate, dw, db)
     beta_dx = _beta(accumulate, dx)
     flags = (CONV_BF16 if bf16 else 0) | (CONV_DW_ASYNC if async_dw else 0) | (CONV_WS_PACKED if packed else 0)
-    wptr = ctypes.c_void_p(w.address()) if layout is not None and packed else w.cptr
-    lib.call("xsmi_conv2d_bwd", dy.cptr, x.cptr, wptr, dx.cptr, dw.cptr, db.cptr if db is not None else None, *dims,
+    wptr = ctypes.c_void_p(w.address()) if layout is not None and packed else w.ptr
+    lib.call("xsmi_conv2d_bwd", dy.ptr, x.ptr, wptr, dx.ptr, dw.ptr, db.ptr if db is not None else None, *dims,
              beta_dx, beta_dw, flags, ws, ws_bytes, ws_dw, ws_dw_bytes)
     if layout is not None and not packed:
         layout.key = _filter_key(w)
@@ -371,10 +381,10 @@ def maxpool2d_fwd(x, k, stride, pad=0, out=None, idx=None, want_idx=True):
     if xcl is not None and xcl.border >= pad:         # no argmax wanted and the input lives in channels-last form
         ycl = out.channels_last_out(1)
         if ycl is not None:
-            lib.call("xsmi_cl_maxpool2d", xcl.buf.cptr, xcl.border, ycl.buf.cptr, ycl.border, n, c, h, w, int(k),
+            lib.call("xsmi_cl_maxpool2d", xcl.buf.ptr, xcl.border, ycl.buf.ptr, ycl.border, n, c, h, w, int(k),
                      int(stride[0]), int(stride[1]), int(pad))
             return out, None
-    lib.call("xsmi_maxpool2d_fwd", x.cptr, out.cptr, idx.cptr if idx is not None else None,
+    lib.call("xsmi_maxpool2d_fwd", x.ptr, out.ptr, idx.ptr if idx is not None else None,
              n, c, h, w, int(k), int(stride[0]), int(stride[1]), int(pad))
     return out, idx
 
@@ -400,7 +410,7 @@ def maxpool2d_bwd(dy, idx, x_shape, k, stride, pad=0, dx=None, accumulate=False)
         dy.ptr; idx.ptr                               # pending clears are settled now
         capi.defer_pool_bwd(e)
         return dx
-    lib.call("xsmi_maxpool2d_bwd", dy.cptr, idx.cptr, dx.cptr, n, c, h, w, int(k), int(stride[0]), int(stride[1]),
+    lib.call("xsmi_maxpool2d_bwd", dy.ptr, idx.ptr, dx.ptr, n, c, h, w, int(k), int(stride[0]), int(stride[1]),
              int(pad), beta)
     return dx
 
@@ -416,7 +426,7 @@ class PoolBwdEntry:
 
     def launch(self):
         n, c, h, w = self.dims
-        lib.call("xsmi_maxpool2d_bwd", self.dy.cptr, self.idx.cptr, self.dx.cptr, n, c, h, w, 3, 2, 2, 1, 0.0)
+        lib.call("xsmi_maxpool2d_bwd", self.dy.ptr, self.idx.ptr, self.dx.ptr, n, c, h, w, 3, 2, 2, 1, 0.0)
 
 
 def relu_mask_bwd(dy, neg_mask, dx=None, accumulate=False):
@@ -425,7 +435,7 @@ def relu_mask_bwd(dy, neg_mask, dx=None, accumulate=False):
         dx = empty(dy.shape)
         accumulate = False
     beta = 0.0 if dx is dy else _beta(accumulate, dx)
-    lib.call("xsmi_relu_mask_bwd", dy.cptr, neg_mask.cptr, dx.cptr, dy.size, beta)
+    lib.call("xsmi_relu_mask_bwd", dy.ptr, neg_mask.ptr, dx.ptr, dy.size, beta)
     return dx
 
 
@@ -435,12 +445,12 @@ def relu_mask_bwd2(dy, neg_mask, dx1, dx2, accumulate=True):
     if dx1.size != dy.size or dx2.size != dy.size or dx1 is dx2:
         raise ValueError("relu_mask_bwd2: needs two different outputs of dy's size")
     b1, b2 = _beta(accumulate, dx1), _beta(accumulate, dx2)
-    lib.call("xsmi_relu_mask_bwd2", dy.cptr, neg_mask.cptr, dx1.cptr, b1, dx2.cptr, b2, dy.size)
+    lib.call("xsmi_relu_mask_bwd2", dy.ptr, neg_mask.ptr, dx1.ptr, b1, dx2.ptr, b2, dy.size)
     return dx1, dx2
 
 
 def copy_kernel(dst, src):
-    lib.call("xsmi_copy_kernel", dst.cptr, src.cptr, src.nbytes)
+    lib.call("xsmi_copy_kernel", dst.ptr, src.ptr, src.nbytes)
 
 
 # ---- neighbours of conv / pool (device-resident element-wise, normalisation, reduction ops) ----
@@ -460,9 +470,9 @@ def axpy(y, x, a):
     if y.take_fresh():                        # y is a pending all-zero buffer: y = a * x, no clear, no read of y
         if float(a) == 1.0:
             return y.copy_from(x)
-        lib.call("xsmi_scale_shift", x.cptr, y.cptr, float(a), 0.0, y.size)
+        lib.call("xsmi_scale_shift", x.ptr, y.ptr, float(a), 0.0, y.size)
         return y
-    lib.call("xsmi_axpy", y.cptr, x.cptr, float(a), y.size)
+    lib.call("xsmi_axpy", y.ptr, x.ptr, float(a), y.size)
     return y
 
 
@@ -507,14 +517,14 @@ def add(a, b, out=None, defer=False):
         capi.defer_add(a, b, out)
         return out
     out = _like(a, out)
-    lib.call("xsmi_add", a.cptr, b.cptr, out.cptr, a.size)
+    lib.call("xsmi_add", a.ptr, b.ptr, out.ptr, a.size)
     return out
 
 
 def scale(a, s, t=0.0, out=None):
     _f32(a, "a")
     out = _like(a, out)
-    lib.call("xsmi_scale_shift", a.cptr, out.cptr, float(s), float(t), a.size)
+    lib.call("xsmi_scale_shift", a.ptr, out.ptr, float(s), float(t), a.size)
     return out
 
 
@@ -531,12 +541,12 @@ def relu_fwd(x, out=None):
             if acl is not None and bcl is not None and acl.same_layout(bcl):
                 xcl = x.channels_last_out(acl.border)     # both operands live in channels-last form: so does the sum
                 if xcl is not None:
-                    lib.call("xsmi_cl_add", acl.buf.cptr, bcl.buf.cptr, xcl.buf.cptr, xcl.buf.size, 1)
+                    lib.call("xsmi_cl_add", acl.buf.ptr, bcl.buf.ptr, xcl.buf.ptr, xcl.buf.size, 1)
                     return x
-            lib.call("xsmi_add_relu", ops[0].cptr, ops[1].cptr, x.cptr, None, x.size)
+            lib.call("xsmi_add_relu", ops[0].ptr, ops[1].ptr, x.ptr, None, x.size)
             return x
     out = _like(x, out)
-    lib.call("xsmi_relu_fwd", x.cptr, out.cptr, x.size)
+    lib.call("xsmi_relu_fwd", x.ptr, out.ptr, x.size)
     return out
 
 
@@ -551,18 +561,18 @@ def relu_fwd_mask(x, out=None):
                 entry = ops[2]
                 entry.launch(residual=ops[1] if entry.y is ops[0] else ops[0], out=x, neg_mask=mask)
                 return x, mask
-            lib.call("xsmi_add_relu", ops[0].cptr, ops[1].cptr, x.cptr, mask.cptr, x.size)
+            lib.call("xsmi_add_relu", ops[0].ptr, ops[1].ptr, x.ptr, mask.ptr, x.size)
             return x, mask
     out = _like(x, out)
     mask = empty(x.shape, np.uint8)
-    lib.call("xsmi_relu_fwd_mask", x.cptr, out.cptr, mask.cptr, x.size)
+    lib.call("xsmi_relu_fwd_mask", x.ptr, out.ptr, mask.ptr, x.size)
     return out, mask
 
 
 def relu_bwd(dy, pre, dx=None):
     _f32(dy, "dy"); _f32(pre, "pre")
     dx = _like(dy, dx)
-    lib.call("xsmi_relu_bwd", dy.cptr, pre.cptr, dx.cptr, dy.size)
+    lib.call("xsmi_relu_bwd", dy.ptr, pre.ptr, dx.ptr, dy.size)
     return dx
 
 
@@ -573,7 +583,7 @@ def act_fwd(x, kind, out=None):
     """sigmoid or tanh of x (``out`` may be x)."""
     _f32(x, "x")
     out = _like(x, out)
-    lib.call("xsmi_act_fwd", x.cptr, out.cptr, x.size, ACT_KINDS[kind])
+    lib.call("xsmi_act_fwd", x.ptr, out.ptr, x.size, ACT_KINDS[kind])
     return out
 
 
@@ -583,13 +593,13 @@ def act_bwd(dy, y, kind, dx=None):
     if y.size != dy.size:
         raise ValueError("act_bwd: %s vs %s" % (dy.shape, y.shape))
     dx = _like(dy, dx)
-    lib.call("xsmi_act_bwd", dy.cptr, y.cptr, dx.cptr, dy.size, ACT_KINDS[kind])
+    lib.call("xsmi_act_bwd", dy.ptr, y.ptr, dx.ptr, dy.size, ACT_KINDS[kind])
     return dx
 
 
 def lerp_(m, cur, momentum):
     """m = momentum*m + (1-momentum)*cur"""
-    lib.call("xsmi_lerp", m.cptr, cur.cptr, float(momentum), m.size)
+    lib.call("xsmi_lerp", m.ptr, cur.ptr, float(momentum), m.size)
     return m
 
 
@@ -621,24 +631,24 @@ class BnEntry:
         n, c, hw = self.dims
         ws, ws_bytes = self.ws
         mm, mv = self.mm, self.mv
-        stats = (self.sqrtvar.cptr, self.mean.cptr, self.var.cptr, mm.cptr if mm is not None else None,
-                 mv.cptr if mv is not None else None, float(self.momentum))
+        stats = (self.sqrtvar.ptr, self.mean.ptr, self.var.ptr, mm.ptr if mm is not None else None,
+                 mv.ptr if mv is not None else None, float(self.momentum))
         if pooled is not None:
             _, _, h, w = self.x.shape
             self.y.never_written("this batch normalisation's result was consumed by the max-pool that followed it, in one "
                                  "pass, and was not stored (XSMI_FUSE_BN_ADD_RELU=0 keeps the passes apart)")
-            lib.call("xsmi_bn_relu_maxpool_fwd", self.x.cptr, self.gamma.cptr, self.beta.cptr, pooled.cptr,
-                     idx.cptr if idx is not None else None, self.relu_mask.cptr, *stats, n, c, h, w, float(self.eps),
+            lib.call("xsmi_bn_relu_maxpool_fwd", self.x.ptr, self.gamma.ptr, self.beta.ptr, pooled.ptr,
+                     idx.ptr if idx is not None else None, self.relu_mask.ptr, *stats, n, c, h, w, float(self.eps),
                      ws, ws_bytes)
             return
         if residual is None:
-            lib.call("xsmi_bn_fwd", self.x.cptr, self.gamma.cptr, self.beta.cptr, self.y.cptr, None, *stats,
-                     self.relu_mask.cptr if self.relu_mask is not None else None, n, c, hw, float(self.eps), ws, ws_bytes)
+            lib.call("xsmi_bn_fwd", self.x.ptr, self.gamma.ptr, self.beta.ptr, self.y.ptr, None, *stats,
+                     self.relu_mask.ptr if self.relu_mask is not None else None, n, c, hw, float(self.eps), ws, ws_bytes)
             return
         self.y.never_written("this batch normalisation's result was consumed by the add and ReLU that followed it, in "
                              "one pass, and was not stored (XSMI_FUSE_BN_ADD_RELU=0 keeps the three passes apart)")
-        lib.call("xsmi_bn_add_relu_fwd", self.x.cptr, self.gamma.cptr, self.beta.cptr, residual.cptr, out.cptr, *stats,
-                 neg_mask.cptr, n, c, hw, float(self.eps), ws, ws_bytes)
+        lib.call("xsmi_bn_add_relu_fwd", self.x.ptr, self.gamma.ptr, self.beta.ptr, residual.ptr, out.ptr, *stats,
+                 neg_mask.ptr, n, c, hw, float(self.eps), ws, ws_bytes)
 
 
 def bn_fwd(x, gamma, beta, eps, y=None, moving=None, momentum=0.0, neg_mask=None, want_xhat=True, defer=False):
@@ -657,7 +667,7 @@ def bn_fwd(x, gamma, beta, eps, y=None, moving=None, momentum=0.0, neg_mask=None
     mm, mv = moving if moving is not None else (None, None)
     if mm is not None and (mm.size != c or mv.size != c):
         raise ValueError("bn_fwd: moving statistics must have %d elements" % c)
-    ws, ws_bytes = _ws.get(lib.raw("xsmi_bn_workspace_bytes")(c))
+    ws, ws_bytes = _ws.get(_need_bn(c))
     if defer and FUSE_BN_ADD_RELU and not want_xhat and y.is_whole():
         e = BnEntry()
         e.relu_mask = neg_mask
@@ -668,10 +678,10 @@ def bn_fwd(x, gamma, beta, eps, y=None, moving=None, momentum=0.0, neg_mask=None
             a.ptr                                     # pending clears and channels-last forms are settled now
         capi.defer_bn(e)
         return y, None, sqrtvar, mean, var
-    lib.call("xsmi_bn_fwd", x.cptr, gamma.cptr, beta.cptr, y.cptr, xhat.cptr if want_xhat else None, sqrtvar.cptr,
-             mean.cptr, var.cptr,
-             mm.cptr if mm is not None else None, mv.cptr if mv is not None else None, float(momentum),
-             neg_mask.cptr if neg_mask is not None else None, n, c, hw, float(eps), ws, ws_bytes)
+    lib.call("xsmi_bn_fwd", x.ptr, gamma.ptr, beta.ptr, y.ptr, xhat.ptr if want_xhat else None, sqrtvar.ptr,
+             mean.ptr, var.ptr,
+             mm.ptr if mm is not None else None, mv.ptr if mv is not None else None, float(momentum),
+             neg_mask.ptr if neg_mask is not None else None, n, c, hw, float(eps), ws, ws_bytes)
     return y, xhat, sqrtvar, mean, var
 
 
@@ -679,7 +689,7 @@ def bn_infer(x, gamma, beta, mean, var, eps, y=None, relu=False):
     n, c, hw = _nchw3(x.shape)
     y = _like(x, y)
     y.take_fresh()
-    lib.call("xsmi_bn_infer", x.cptr, gamma.cptr, beta.cptr, mean.cptr, var.cptr, y.cptr, n, c, hw, float(eps),
+    lib.call("xsmi_bn_infer", x.ptr, gamma.ptr, beta.ptr, mean.ptr, var.ptr, y.ptr, n, c, hw, float(eps),
              1 if relu else 0)
     return y
 
@@ -694,8 +704,8 @@ def bn_fold(w, bias, gamma, beta, mean, var, eps):
     if bias is not None and bias.size != k:
         raise ValueError("bn_fold: bias has %d elements for %d filters" % (bias.size, k))
     w_out, b_out = empty(w.shape), empty((k,))
-    lib.call("xsmi_bn_fold", w.cptr, bias.cptr if bias is not None else None, gamma.cptr, beta.cptr, mean.cptr, var.cptr,
-             w_out.cptr, b_out.cptr, k, w.size // k, float(eps))
+    lib.call("xsmi_bn_fold", w.ptr, bias.ptr if bias is not None else None, gamma.ptr, beta.ptr, mean.ptr, var.ptr,
+             w_out.ptr, b_out.ptr, k, w.size // k, float(eps))
     return w_out, b_out
 
 
@@ -717,7 +727,7 @@ def bn_bwd(dy, xhat, sqrtvar, gamma, dx=None, dgamma=None, dbeta=None, neg_mask=
             raise ValueError("bn_bwd: output buffers do not match %s" % (dy.shape,))
         for o in (dx, dgamma, dbeta):
             o.take_fresh()
-        ws, ws_bytes = _ws.get(lib.raw("xsmi_bn_workspace_bytes")(c))
+        ws, ws_bytes = _ws.get(_need_bn(c))
     except Exception:
         if pool is not None:
             pool.launch()                             # what was asked for before this call still happens
@@ -728,13 +738,13 @@ def bn_bwd(dy, xhat, sqrtvar, gamma, dx=None, dgamma=None, dbeta=None, neg_mask=
             pn, pc, ph, pw = pool.dims
             dy.never_written("this max-pool gradient was consumed by the batch-norm backward that followed it and was not "
                              "stored (XSMI_FUSE_BN_ADD_RELU=0 keeps the passes apart)")
-            lib.call("xsmi_bn_bwd_maxpool", pool.dy.cptr, pool.idx.cptr, xhat.cptr, mean.cptr, sqrtvar.cptr, gamma.cptr,
-                     neg_mask.cptr if neg_mask is not None else None, dx.cptr, dgamma.cptr, dbeta.cptr, pn, pc, ph, pw,
+            lib.call("xsmi_bn_bwd_maxpool", pool.dy.ptr, pool.idx.ptr, xhat.ptr, mean.ptr, sqrtvar.ptr, gamma.ptr,
+                     neg_mask.ptr if neg_mask is not None else None, dx.ptr, dgamma.ptr, dbeta.ptr, pn, pc, ph, pw,
                      ws, ws_bytes)
             return dx, dgamma, dbeta
         pool.launch()
-    lib.call("xsmi_bn_bwd", dy.cptr, xhat.cptr, mean.cptr if mean is not None else None, sqrtvar.cptr, gamma.cptr,
-             neg_mask.cptr if neg_mask is not None else None, dx.cptr, dgamma.cptr, dbeta.cptr, n, c, hw, ws, ws_bytes)
+    lib.call("xsmi_bn_bwd", dy.ptr, xhat.ptr, mean.ptr if mean is not None else None, sqrtvar.ptr, gamma.ptr,
+             neg_mask.ptr if neg_mask is not None else None, dx.ptr, dgamma.ptr, dbeta.ptr, n, c, hw, ws, ws_bytes)
     return dx, dgamma, dbeta
 
 
@@ -744,7 +754,7 @@ def avgpool_fwd(x, k, stride=None):
     if k > h or k > w or sh < 1 or sw < 1:
         raise ValueError("avg_pool2d: window %d does not fit the input %dx%d" % (k, h, w))
     y = empty((n, c, (h - k) // sh + 1, (w - k) // sw + 1))
-    lib.call("xsmi_avgpool_fwd", x.cptr, y.cptr, n, c, h, w, int(k), sh, sw)
+    lib.call("xsmi_avgpool_fwd", x.ptr, y.ptr, n, c, h, w, int(k), sh, sw)
     return y
 
 
@@ -754,7 +764,7 @@ def avgpool_bwd(dy, x_shape, k, stride=None):
     if dy.shape != (n, c, (h - k) // sh + 1, (w - k) // sw + 1):
         raise ValueError("avg_pool2d backward: dy %s does not match the pooled shape of %s" % (dy.shape, tuple(x_shape)))
     dx = empty(x_shape)
-    lib.call("xsmi_avgpool_bwd", dy.cptr, dx.cptr, n, c, h, w, int(k), sh, sw)
+    lib.call("xsmi_avgpool_bwd", dy.ptr, dx.ptr, n, c, h, w, int(k), sh, sw)
     return dx
 
 
@@ -771,7 +781,7 @@ def gemm(a, b, bias=None, trans_a=False, trans_b=False, out=None):
         raise ValueError("gemm: output has shape %s, expected %s" % (out.shape, (m, n)))
     # room for a split of K over the chip when the output is small (the dense layer's batch of rows)
     ws, ws_bytes = _ws.get(min(64 * m * n * 4, 1 << 24))
-    lib.call("xsmi_gemm", a.cptr, b.cptr, bias.cptr if bias is not None else None, out.cptr, int(m), int(n), int(k),
+    lib.call("xsmi_gemm", a.ptr, b.ptr, bias.ptr if bias is not None else None, out.ptr, int(m), int(n), int(k),
              1 if trans_a else 0, 1 if trans_b else 0, ws, ws_bytes)
     return out
 
@@ -783,13 +793,13 @@ def dense_fwd(x, w, b=None, out=None):
 def colsum(a):
     m, n = a.shape
     out = empty((n,))
-    lib.call("xsmi_colsum", a.cptr, out.cptr, int(m), int(n))
+    lib.call("xsmi_colsum", a.ptr, out.ptr, int(m), int(n))
     return out
 
 
 def sum_all(a):
     out = empty((1,))
-    lib.call("xsmi_sum_all", a.cptr, out.cptr, a.size)
+    lib.call("xsmi_sum_all", a.ptr, out.ptr, a.size)
     return out
 
 
@@ -805,7 +815,7 @@ def softmax_ce_fwd(logits, labels, reduction):
     labels = _labels(labels)
     sm = empty(logits.shape)
     buf = empty((1 + m,))
-    lib.call("xsmi_softmax_ce_fwd", logits.cptr, labels.cptr, sm.cptr, buf.cptr, int(m), int(n),
+    lib.call("xsmi_softmax_ce_fwd", logits.ptr, labels.ptr, sm.ptr, buf.ptr, int(m), int(n),
              1 if reduction == 'mean' else 0)
     return buf.leading(0, 1), sm
 
@@ -821,12 +831,12 @@ def softmax_ce_bwd(sm, labels, reduction, upstream):
     up = 1.0 if up_dev is not None else float(np.asarray(upstream).reshape(-1)[0])
     scale_ = up / m if reduction == 'mean' else up
     dz = empty(sm.shape)
-    lib.call("xsmi_softmax_ce_bwd", sm.cptr, labels.cptr, up_dev.cptr if up_dev is not None else None, dz.cptr,
+    lib.call("xsmi_softmax_ce_bwd", sm.ptr, labels.ptr, up_dev.ptr if up_dev is not None else None, dz.ptr,
              int(m), int(n), scale_)
     return dz
 
 
 def full(shape, value):
     out = empty(shape)
-    lib.call("xsmi_fill", out.cptr, float(value), out.size)
+    lib.call("xsmi_fill", out.ptr, float(value), out.size)
     return out

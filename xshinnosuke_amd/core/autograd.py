@@ -33,14 +33,11 @@ def _sweep(graph, retain_graph):
             node.grad_fn(node)
         for layer in node.next_layers:
             layer.data = None
-        keep = retain_graph or node.is_leaf or node.retain_grad()
-        kwargs = dict(requires_grad=node.requires_grad, name=node.name, slices=node.slices(),
-                      static_graph_tensor=node.is_static)
-        if keep:
-            node.reset_(retain_grad=node.retain_grad(), grad=node._grad, **kwargs)
+        if retain_graph or node.is_leaf or node._retain:
+            node.reset_(None, node.requires_grad, node.name, None, node._grad, node._slices, node._static, node._retain)
         else:
             node.free_memory()
-            node.reset_(**kwargs)
+            node.reset_(None, node.requires_grad, node.name, None, None, node._slices, node._static)
 
 
 def backward(outputs, inputs, retain_graph=False):

@@ -34,22 +34,23 @@ class Tensor(object):
         self._data = None
         self.reset_(data, requires_grad, name, dtype, **kwargs)
 
-    def reset_(self, data=None, requires_grad=False, name=None, dtype=None, **kwargs):
+    def reset_(self, data=None, requires_grad=False, name=None, dtype=None, grad=None, slices=_FULL, static_graph_tensor=False,
+               retain_grad=False, **kwargs):
         if data is not None:
-            if is_device(data):
+            if isinstance(data, DeviceArray):
                 self._data = data
             else:
                 self._data = np.asarray(data, dtype=dtype)
-        self._grad = kwargs.pop('grad', None)
+        self._grad = grad
         self._in_bounds = []
         self._out_bounds = []
         self.name = name
         self.grad_fn = None
         self.requires_grad = requires_grad
-        self._slices = kwargs.pop('slices', _FULL)
-        self._static = kwargs.pop('static_graph_tensor', False)
+        self._slices = slices
+        self._static = static_graph_tensor
         self._cache = {}
-        self._retain = kwargs.pop('retain_grad', False)
+        self._retain = retain_grad
         self._is_leaf = None
         self.next_layers = []
 
@@ -63,9 +64,10 @@ class Tensor(object):
         d = self._data
         if d is None:
             return None
-        if d.size == 1 or self._slices == _FULL:
+        s = self._slices
+        if s is _FULL or d.size == 1 or s == _FULL:
             return d
-        return d[self._slices]
+        return d[s]
 
     @eval.setter
     def eval(self, v):
@@ -131,9 +133,10 @@ class Tensor(object):
 
     @property
     def grad(self):
-        if self._grad is not None:
-            self._grad.slices(self._slices)
-        return self._grad
+        g = self._grad
+        if g is not None:
+            g._slices = self._slices
+        return g
 
     @grad.setter
     def grad(self, g):

@@ -77,7 +77,7 @@ def conv2d(inputs, weight, bias=None, stride=(1, 1), padding=0, out=None, activa
     on_device = is_device(x)
     x_dev = _f32_device(x)
     w_dev = _f32_device(weight.eval)
-    b_dev = None if bias is None else _f32_device(bias.eval).reshape(-1)
+    b_dev = None if bias is None else _f32_device(bias.eval)
     n, c, h, w = x.shape
     k, _, r, s = weight.shape
     oh, ow = K.conv_out_hw(h, w, r, s, stride, padding)
@@ -475,7 +475,7 @@ def batch_norm(inputs, gamma, beta, moving_mean, moving_variance, axis=1, traini
         # the shortcut and then the in-place ReLU, behind the first convolution of a ResNet the 3x3/2 max-pool, and
         # either runs inside the normalisation's second pass (backend/kernels.bn_fwd); anything else sees the plain result.
         y, xhat, sqrtvar, mean_, var_ = A.batch_norm_train(x, gamma.eval, beta.eval, epsilon, dst,
-                                                           (mm.reshape(-1), mv.reshape(-1)) if fused else None, momentum,
+                                                           (mm, mv) if fused else None, momentum,
                                                            neg_mask, want_xhat=False,
                                                            defer=fused and track)
         if not track:

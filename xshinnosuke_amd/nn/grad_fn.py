@@ -18,7 +18,7 @@ from . import array_ops as A
 def initialize_ops_grad(*ops):
     """Give every input that needs a gradient a zero buffer (reference xs/utils/common.py:29-32)."""
     for op in ops:
-        if op is not None and op.grad is None and op.requires_grad:
+        if op is not None and op._grad is None and op.requires_grad:
             op.zero_grad()
 
 
@@ -81,7 +81,7 @@ def Conv2DBackward(outputs):
         if is_device(dw_buf) and is_device(dx_buf) and (not want_db or is_device(db_buf)):
             # all gradients live on the device: one call; the weight gradient keeps running on the second
             # stream beside the rest of the sweep (the backend joins it before anything else can touch it)
-            K.conv2d_bwd(dy, x_dev, w_dev, dx_buf, dw_buf, db_buf.reshape(-1) if want_db else None, stride, pad,
+            K.conv2d_bwd(dy, x_dev, w_dev, dx_buf, dw_buf, db_buf, stride, pad,
                          accumulate=True, bf16=bf16, async_dw=True, keep_layout=w_dev is weight.eval)
             return
     if want_dw or want_db:
@@ -89,7 +89,7 @@ def Conv2DBackward(outputs):
         db_buf = bias.grad.eval if want_db else None
         if want_dw and is_device(dw_buf) and (not want_db or is_device(db_buf)):
             K.conv2d_bwd_weight(dy, x_dev, weight.shape, stride, pad, dw=dw_buf,
-                                db=db_buf.reshape(-1) if want_db else None, accumulate=True)
+                                db=db_buf, accumulate=True)
         else:
             dw, db = K.conv2d_bwd_weight(dy, x_dev, weight.shape, stride, pad, want_db=want_db)
             if want_dw:
@@ -303,8 +303,7 @@ def BatchNormBackward(outputs):
         if xhat is None:                             # not stored by the forward: x and the batch mean stand in
             xhat = inputs.eval
         dx, dgamma, dbeta = K.bn_bwd(dy, xhat, outputs.cache['sqrtvar'], gam,
-                                     dx=out_dx, dgamma=None if out_dg is None else out_dg.reshape(-1),
-                                     dbeta=None if out_db is None else out_db.reshape(-1),
+                                     dx=out_dx, dgamma=out_dg, dbeta=out_db,
                                      neg_mask=outputs.cache.get('neg_mask'),       # fused ReLU: strict mask on dy
                                      mean=mean if outputs.cache['normalized_x'] is None else None)
     else:
