@@ -253,17 +253,18 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
     };
     uint32_t a_off = 0;
     int b_rd[2];                                       // this lane's two pixels in an image
-    // two steps of filter fragments and two of pixel fragments in registers: a step's filter loads are issued while
-    // the step two before it multiplies, its LDS reads while the one before it does
-    bf16x8 fa[2][3], fb[2][2][3];                  // [step parity][piece], [step parity][pixel block][piece]
+    // Three steps of filter fragments and one of pixel fragments in registers.  A step's filter loads are issued while the
+    // step three before it multiplies: vector loads return in order, so they also wait for the image's loads in front of
+    // them, which come from memory.
+    bf16x8 fa[3][3], fb[2][3];                         // [step % 3][piece], [pixel block][piece]
     auto load_a = [&](auto par, auto q) {
         fa[par][q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
                          rapk, a_voff + (int)q * 2 * SP_ROWS * 16, (int)a_off, 0));
     };
-    auto read_b = [&](auto par, auto q, int off) {
+    auto read_b = [&](auto q, int off) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            fb[par][j][q] = *reinterpret_cast<const bf16x8 *>(s_img + b_rd[j] + off + (int)q * 2 * SP_PLANE);
+            fb[j][q] = *reinterpret_cast<const bf16x8 *>(s_img + b_rd[j] + off + (int)q * 2 * SP_PLANE);
     };
     int t_left = 0, tb = 0, off = 0, Tx = 1, row_end = 0;
     auto next_off = [&]() {                            // past the last tap: back to a place inside the image
@@ -275,51 +276,49 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
     auto mm = [&](auto par, floatx16 (&acc)[2], int qa, int qb) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[par][qa], fb[par][j][qb], acc[j], 0, 0, 0);
+            acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[par][qa], fb[j][qb], acc[j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
-    // One step.  The next tap's fragments are read from the same image (past a group's last tap: places that are not
-    // used); the filter block two steps ahead takes each piece's registers after the piece's last product.  J >= 0: a
-    // part of the next image is split and written to the other half of the LDS, a few instructions behind each pair of
-    // MFMAs.
+    // One step.  A piece's registers take the next tap's fragments (past a group's last tap: places that are not used), or
+    // the filter block three steps ahead, after the piece's last product.  J >= 0: a part of the next image is split and
+    // written to the other half of the LDS, a few instructions behind each pair of MFMAs.
     int image = 0;                                     // byte offset of the image that is multiplied
     int a_left = 0;                                    // steps of the segment whose block ahead has not been requested
-    uint32_t a_next0 = 0, a_next1 = 0;                 // blocks of the two steps after the segment
+    uint32_t a_next[3] = {0, 0, 0};                    // blocks of the three steps after the segment
     auto step = [&](auto par, auto jt) {
-        constexpr int P = decltype(par)::value, J = decltype(jt)::value;
-        const auto nx = IC<1 - P>{};
+        constexpr int J = decltype(jt)::value;
         next_off();
-        a_off = a_left > 2 ? a_off + (uint32_t)SP_BLOCK : a_left == 2 ? a_next0 : a_next1;
+        a_off = a_left > 3 ? a_off + (uint32_t)SP_BLOCK : a_left == 3 ? a_next[0] : a_left == 2 ? a_next[1] : a_next[2];
         --a_left;
         mm(par, lo, 2, 0);
         load_a(par, IC<2>{});
-        read_b(nx, IC<0>{}, image + off);
         if constexpr (J >= 0) split_one(jt, IC<0>{});
         __builtin_amdgcn_sched_barrier(0);
         mm(par, lo, 1, 0);
-        read_b(nx, IC<1>{}, image + off);
         if constexpr (J >= 0) split_one(jt, IC<1>{});
+        __builtin_amdgcn_sched_barrier(0);
+        mm(par, hi, 0, 0);
+        read_b(IC<0>{}, image + off);
+        if constexpr (J >= 0) split_one(jt, IC<2>{});
         __builtin_amdgcn_sched_barrier(0);
         mm(par, lo, 1, 1);
         load_a(par, IC<1>{});
-        read_b(nx, IC<2>{}, image + off);
-        if constexpr (J >= 0) split_one(jt, IC<2>{});
-        __builtin_amdgcn_sched_barrier(0);
-        mm(par, hi, 0, 0);
         if constexpr (J >= 0) split_one(jt, IC<3>{});
         __builtin_amdgcn_sched_barrier(0);
         mm(par, lo, 0, 1);
+        read_b(IC<1>{}, image + off);
         if constexpr (J >= 0) put(jt, SP_IMAGE - image);
         __builtin_amdgcn_sched_barrier(0);
         mm(par, lo, 0, 2);
         load_a(par, IC<0>{});
+        read_b(IC<2>{}, image + off);
         __builtin_amdgcn_sched_barrier(0);
     };
     // The taps of one image.  Written out up to nine: the waits of each step and the places where the next image is
     // staged are then compile-time facts.
     const auto none = IC<-1>{};
     auto run = [&](int taps) {
-        read_b(IC<0>{}, IC<0>{}, image + off); read_b(IC<0>{}, IC<1>{}, image + off); read_b(IC<0>{}, IC<2>{}, image + off);
+        read_b(IC<0>{}, image + off); read_b(IC<1>{}, image + off); read_b(IC<2>{}, image + off);
         int staged = 0;
         const auto third = IC<NJ == 3 ? 2 : -1>{};
         do {
@@ -327,23 +326,26 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
             if (taps == 1) break;
             step(IC<1>{}, none);
             if (taps == 2) break;
-            step(IC<0>{}, none);
+            step(IC<2>{}, none);
             if (taps == 3) break;
-            step(IC<1>{}, IC<0>{});
+            step(IC<0>{}, IC<0>{});
             staged = 1;
             if (taps == 4) break;
-            step(IC<0>{}, none);
+            step(IC<1>{}, none);
             if (taps == 5) break;
-            step(IC<1>{}, IC<1>{});
+            step(IC<2>{}, IC<1>{});
             staged = 2;
             if (taps == 6) break;
             step(IC<0>{}, none);
             if (taps == 7) break;
             step(IC<1>{}, third);
             staged = 3;
-            for (int i = 8; i < taps; i += 2) {
+            if (taps == 8) break;
+            step(IC<2>{}, none);
+            for (int i = 9; i < taps; i += 3) {
                 step(IC<0>{}, none);
                 if (i + 1 < taps) step(IC<1>{}, none);
+                if (i + 2 < taps) step(IC<2>{}, none);
             }
         } while (false);
         if (staged < 1) stage(IC<0>{}, SP_IMAGE - image);
@@ -359,11 +361,13 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
     load_image(sg.grp);
     a_off = block_of(u);
     load_a(IC<0>{}, IC<2>{}); load_a(IC<0>{}, IC<1>{}); load_a(IC<0>{}, IC<0>{});
-    a_off = block_of(u + 1);
+    a_off = sg.n > 1 ? a_off + (uint32_t)SP_BLOCK : block_of(u + 1);
     load_a(IC<1>{}, IC<2>{}); load_a(IC<1>{}, IC<1>{}); load_a(IC<1>{}, IC<0>{});
+    a_off = sg.n > 2 ? a_off + (uint32_t)SP_BLOCK : block_of(u + 2);
+    load_a(IC<2>{}, IC<2>{}); load_a(IC<2>{}, IC<1>{}); load_a(IC<2>{}, IC<0>{});
     stage(IC<0>{}, 0); stage(IC<1>{}, 0);
     if constexpr (NJ == 3) stage(IC<2>{}, 0);
-    bool odd = false;
+    int turn = 0;                                      // the set that the next step's filter block is in
     int bias_buf = 0;
     while (true) {
         const SpClass &c = p.cls[sg.ci];
@@ -372,7 +376,9 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         const int m0 = sg.m0, rt = sg.rt, Wp = c.Wp;
         const bool more = u_next < u1;
         if (more) nx = segment_at(u_next);
-        a_next0 = block_of(u_next); a_next1 = block_of(u_next + 1);
+        a_next[0] = block_of(u_next);
+#pragma unroll
+        for (int i = 1; i < 3; ++i) a_next[i] = more && nx.n > i ? a_next[0] + (uint32_t)(i * SP_BLOCK) : block_of(u_next + i);
         a_left = sg.n;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -385,9 +391,14 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         if (p.bias && head && t < SP_ROWS) s_bias[bias_buf][t] = rt * SP_ROWS + t < c.rows ? p.bias[rt * SP_ROWS + t] : 0.f;
         int left = sg.n, f = sg.f, grp = sg.grp, tap = sg.tap;
         while (left > 0) {
-            if (odd) {                                 // the next step's filter block is in the other set
+            if (turn) {
 #pragma unroll
-                for (int q = 0; q < 3; ++q) { const bf16x8 x = fa[0][q]; fa[0][q] = fa[1][q]; fa[1][q] = x; }
+                for (int q = 0; q < 3; ++q) {
+                    const bf16x8 x = fa[0][q], y = fa[1][q], z = fa[2][q];
+                    fa[0][q] = turn == 1 ? y : z;
+                    fa[1][q] = turn == 1 ? z : x;
+                    fa[2][q] = turn == 1 ? x : y;
+                }
             }
             const int T = p.ph[f].T;
             const int taps = left < T - tap ? left : T - tap;
@@ -411,7 +422,7 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
             xsmi::wait_lgkmcnt0();
             xsmi::block_barrier();                     // this image is complete, and nobody reads the other one any more
             run(taps);
-            odd = taps & 1;
+            turn = taps % 3;
             image = SP_IMAGE - image;
         }
         u = u_next;
