@@ -174,44 +174,63 @@ __global__ void __launch_bounds__(256) wgrad_f32_kernel(WgradParams p) {
 }
 
 // dw[k][j] = beta*dw + sum over splits of part[split][k][j]; blocks past the last dw block do the same for
-// db[k] from dbpart[split][k].  256 threads = 64 consecutive columns x 4 interleaved split groups with two
-// running sums each; the groups are combined in a fixed order, all in float64 (deterministic, no atomics).
-__global__ void __launch_bounds__(256) wgrad_reduce_kernel(const float *__restrict__ part, float *__restrict__ dw,
-                                                            const float *__restrict__ dbpart, float *__restrict__ db,
-                                                            int K, int J, int Kp, int Jp, int splits, int dw_blocks,
-                                                            int accumulate) {
-    __shared__ double sm[4][64];
-    const int cl = threadIdx.x & 63, g = threadIdx.x >> 6;
-    const int jt = (J + 63) / 64;
+// db[k] from dbpart[split][k].  The threads of a result are combined in a fixed order, all in float64 (deterministic, no
+// atomics).
+// CL results for a workgroup, every (THREADS / CL)-th split for a thread, eight loads in flight.
+template <int CL, int THREADS>
+__global__ void __launch_bounds__(THREADS) wgrad_reduce_kernel(const float *__restrict__ part, float *__restrict__ dw,
+                                                               const float *__restrict__ dbpart, float *__restrict__ db,
+                                                               int K, int J, int Kp, int Jp, int splits, int dw_blocks,
+                                                               int accumulate) {
+    constexpr int G = THREADS / CL;
+    __shared__ double sm[G][CL];
+    const int cl = threadIdx.x % CL, g = threadIdx.x / CL;
+    const int jt = (J + CL - 1) / CL;
     const bool bias_block = (int)blockIdx.x >= dw_blocks;      // uniform per block
     const float *src = nullptr;
     float *dst = nullptr;
     size_t stride = 0;
     if (bias_block) {
-        const int k = ((int)blockIdx.x - dw_blocks) * 64 + cl;
+        const int k = ((int)blockIdx.x - dw_blocks) * CL + cl;
         if (k < K) { src = dbpart + k; dst = db + k; }
         stride = (size_t)Kp;
     } else {
-        const int k = (int)blockIdx.x / jt, j = ((int)blockIdx.x - k * jt) * 64 + cl;
+        const int k = (int)blockIdx.x / jt, j = ((int)blockIdx.x - k * jt) * CL + cl;
         if (j < J) { src = part + (size_t)k * Jp + j; dst = dw + (size_t)k * J + j; }
         stride = (size_t)Kp * Jp;
     }
-    double s0 = 0.0, s1 = 0.0;
+    double s = 0.0;
     if (src) {
-        int sp = g;
-        for (; sp + 4 < splits; sp += 8) {
-            s0 += (double)src[(size_t)sp * stride];
-            s1 += (double)src[(size_t)(sp + 4) * stride];
+        for (int sp = g; sp < splits; sp += 8 * G) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = sp + e * G < splits ? src[(size_t)(sp + e * G) * stride] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s += (double)v[e];
         }
-        if (sp < splits) s0 += (double)src[(size_t)sp * stride];
     }
-    sm[g][cl] = s0 + s1;
+    sm[g][cl] = s;
     __syncthreads();
     if (g == 0 && dst) {
-        double s = ((sm[0][cl] + sm[1][cl]) + sm[2][cl]) + sm[3][cl];
-        if (accumulate) s += (double)*dst;
+        s = accumulate ? (double)*dst : 0.0;
+        for (int i = 0; i < G; ++i) s += sm[i][cl];
         *dst = (float)s;
     }
+}
+
+// Many splits of few results (the first layer of the README network: 8 x 4 results, 972 splits) are a chain of loads: 64
+// threads for a result instead of 4, 33 -> 6 us.  Few splits keep 64 neighbouring results for a workgroup.
+void launch_wgrad_reduce(const float *part, float *dw, const float *dbpart, float *db, int K, int J, int Kp, int Jp, int splits,
+                         int accumulate) {
+    hipStream_t st = xsmi::stream();
+    const int cl = splits >= 128 ? 16 : 64;
+    const int dw_blocks = K * xsmi::ceil_div(J, cl), blocks = dw_blocks + (db ? xsmi::ceil_div(K, cl) : 0);
+    if (cl == 16)
+        hipLaunchKernelGGL((wgrad_reduce_kernel<16, 1024>), dim3(blocks), dim3(1024), 0, st, part, dw, dbpart, db, K, J, Kp, Jp, splits,
+                           dw_blocks, accumulate);
+    else
+        hipLaunchKernelGGL((wgrad_reduce_kernel<64, 256>), dim3(blocks), dim3(256), 0, st, part, dw, dbpart, db, K, J, Kp, Jp, splits,
+                           dw_blocks, accumulate);
 }
 
 void plan_splits(int M, int K, int J, int *splits, int *chunks_per_split) {
@@ -243,9 +262,7 @@ size_t conv_bwd_weight_ws_bytes(int N, int C, int K, int R, int S, int OH, int O
 
 int wgrad_reduce_partials(const float *part, float *dw, const float *dbpart, float *db, int K, int J, int Kp, int Jp, int splits,
                           int accumulate) {
-    const int dw_blocks = K * ceil_div(J, 64);
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(dw_blocks + (db ? ceil_div(K, 64) : 0)), dim3(256), 0, stream(), part, dw, dbpart,
-                       db, K, J, Kp, Jp, splits, dw_blocks, accumulate);
+    launch_wgrad_reduce(part, dw, dbpart, db, K, J, Kp, Jp, splits, accumulate);
     XSMI_LAUNCH_CHECK("wgrad_reduce_kernel");
     return XSMI_OK;
 }
@@ -312,9 +329,7 @@ int xsmi_conv2d_bwd_weight(const float *dy, const float *x, float *dw, float *db
     xsmi::prof_end();
     XSMI_LAUNCH_CHECK("wgrad_f32_kernel");
     const int acc = beta == 1.f ? 1 : 0;
-    const int dw_blocks = K * xsmi::ceil_div(p.J, 64);
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(dw_blocks + (db ? xsmi::ceil_div(K, 64) : 0)), dim3(256), 0, st, p.part, dw,
-                       dbpart, db, K, p.J, p.Kp, p.Jp, splits, dw_blocks, acc);
+    launch_wgrad_reduce(p.part, dw, dbpart, db, K, p.J, p.Kp, p.Jp, splits, acc);
     XSMI_LAUNCH_CHECK("wgrad_reduce_kernel");
     return XSMI_OK;
 }

