@@ -125,6 +125,25 @@ def test_values_that_do_not_split_are_multiplied_one_by_one(gpu):
     assert large.any() and np.abs(y[large] / ref[large] - 1).max() <= 1e-6
 
 
+@pytest.mark.parametrize("scale", [2.0 ** -104, 2.0 ** -116, 2.0 ** -122])
+def test_small_values_keep_their_last_bits(gpu, scale):
+    """Below 2^-110 a value's third piece is lost: the results are formed from the products instead.  Powers of two are exact,
+    so the bound is that of ordinary values."""
+    K = gpu.kernels
+    x, wt, b, dy, _ = _data(2, 20, 12, 13, 70, 3, 3, 1, 1, 1, gpu)
+    y_ref, col = oracle.conv2d_fwd(x, wt, 0 * b, (1, 1), 1)
+    dx_ref, dw_ref, _ = oracle.conv2d_bwd(dy, x.shape, wt, col, (1, 1), 1, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+    up = 1.0 / scale
+    small = lambda a: gpu.to_device(a * np.float32(scale))  # noqa: E731
+    dx_, dw_ = gpu.to_device(x), gpu.to_device(wt)
+    with split_everywhere(gpu):
+        y = K.conv2d_fwd(small(x), dw_, None, (1, 1), 1).numpy()
+        gx = K.conv2d_bwd_data(small(dy), dw_, x.shape, (1, 1), 1).numpy()
+        gw, _ = K.conv2d_bwd_weight(small(dy), dx_, wt.shape, (1, 1), 1, want_db=True)
+    for got, ref in ((y, y_ref), (gx, dx_ref), (gw.numpy(), dw_ref)):
+        assert rel_l2(got.astype(np.float64) * up, ref) <= TOL
+
+
 def test_a_partial_tile_that_never_comes_is_reported(gpu):
     K = gpu.kernels
     x, wt, b, _, _ = _data(1, 512, 7, 7, 512, 3, 3, 1, 1, 1, gpu)

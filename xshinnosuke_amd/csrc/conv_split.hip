@@ -9,9 +9,10 @@
 // have accumulators of their own: the chain that carries the rounding of the full sum then has one addition per 16
 // channels and tap, against one per product pair on the fp32 pipe.
 //
-// What the split does not carry: infinities (inf - inf in a remainder) and values within a bf16 rounding of the largest
-// float.  Such a value makes the outputs that it touches non-finite; every non-finite output is therefore computed
-// again, one product at a time in float32, before it is stored (recompute_nonfinite).
+// What the split does not carry: infinities (inf - inf in a remainder), values within a bf16 rounding of the largest
+// float, and the last bits of values below 2^-110.  The first two make the outputs that they touch non-finite, the third
+// are found by outputs below 2^-100 (split3.h); such outputs are computed again, one product at a time in float64, before
+// they are stored (recompute).
 //
 // Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (128 per tile), 2 x 2 waves
 // of 32 rows x 64 pixels.  The reduction is a list of steps (phase, 16 input channels, tap).  A PHASE is a set of taps
@@ -23,7 +24,7 @@
 // [piece][octet][slot][8 channels], so a fragment read is 32 consecutive 16-byte slots whatever the tap is.  The LDS
 // image serves up to nine taps, which is what pays for the conversion (11 vector instructions per two values).
 // The filter is laid out split already, one 6 KB block per step ([piece][octet][row][8]); each wave fetches its fragments
-// straight into registers one step ahead (the waves of a workgroup read the same block at about the same time: L1), so
+// straight into registers three steps ahead (the waves of a workgroup read the same block at about the same time: L1), so
 // the loop has no barrier except around the image of a channel group.
 //
 // Scheduling is the even split of conv_tap_sk.hip: the steps of all tiles in a row are dealt over the resident
@@ -41,7 +42,7 @@ using xsmi::floatx16;
 using xsmi::bf16x8;
 using xsmi::uint32x4;
 using xsmi::IC;
-using xsmi::finite;
+using xsmi::carried;
 
 constexpr int SP_ROWS = 64;
 constexpr int sp_slots_of(int wc) { return wc == 4 ? 512 : 384; }     // slots of an LDS image
@@ -95,13 +96,12 @@ __device__ __forceinline__ void split8(const float (&v)[8], uint32x4 &p0, uint32
     }
 }
 
-// Outputs that came out non-finite are computed again one float32 product at a time (taps outside, channels inside, as
-// the fp32 kernels add them); a tap outside the input multiplies a zero, as the reference's padding does.
-__device__ __forceinline__ void recompute_nonfinite(floatx16 &r, const SpParams &p, const SpClass &c, int tile_row0, int row0, int m0,
-                                                    int lane) {
+// Outputs that the split does not carry are computed again one product at a time, in float64 (taps outside, channels
+// inside); a tap outside the input multiplies a zero, as the reference's padding does.
+__device__ __forceinline__ void recompute(floatx16 &r, const SpParams &p, const SpClass &c, int tile_row0, int row0, int m0, int lane) {
     uint32_t bad = 0;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) bad |= finite(r[v]) ? 0u : 1u << v;
+    for (int v = 0; v < 16; ++v) bad |= carried(r[v]) ? 0u : 1u << v;
     if (__builtin_amdgcn_ballot_w64(bad != 0) == 0) return;
     const int m = m0 + (lane & 31);
     if (m >= c.M) return;
@@ -111,7 +111,7 @@ __device__ __forceinline__ void recompute_nonfinite(floatx16 &r, const SpParams 
     for (int v = 0; v < 16; ++v) {
         const int row = tile_row0 + row0 + 4 * (lane >> 5) + 8 * (v >> 2) + (v & 3);
         if (!((bad >> v) & 1u) || row >= c.rows) continue;
-        float sum = 0.f;
+        double sum = 0.0;
         const float *wrow = p.w + (size_t)row * p.w_row;
 #pragma unroll 1
         for (int f = c.phase0; f < c.phase0 + c.nphase; ++f) {
@@ -125,11 +125,11 @@ __device__ __forceinline__ void recompute_nonfinite(floatx16 &r, const SpParams 
                 const float *src = p.in + (size_t)n * p.in_n + (size_t)(in ? iy * p.IW + ix : 0);
 #pragma unroll 1
                 for (int ch = 0; ch < p.CH; ++ch)
-                    sum = __builtin_fmaf(wt[(size_t)ch * p.w_ch], in ? src[(size_t)ch * p.plane] : 0.f, sum);
+                    sum += (double)wt[(size_t)ch * p.w_ch] * (double)(in ? src[(size_t)ch * p.plane] : 0.f);
             }
         }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) r[i] = i == v ? sum : r[i];
+        for (int i = 0; i < 16; ++i) r[i] = i == v ? (float)sum : r[i];
     }
 }
 
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
             voff[j] = ok ? (uint32_t)(n_ * p.in_n + iy * p.IW + ix) * 4u : 0x80000000u;
         }
     };
-            float pre[NJ][8];
+    float pre[NJ][8];
     // always the same number of loads (slots past the run fetch out of range): the waits below count them
     auto load_image = [&](int grp_) {
         const int ch0 = grp_ * 16 + octet * 8;
@@ -494,7 +494,7 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         if (head) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                recompute_nonfinite(acc[j], p, c, rt * SP_ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
+                recompute(acc[j], p, c, rt * SP_ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
                 xsmi::store_block_32x32(acc[j], c, p.out, p.out_bytes, p.mask, p.bias ? s_bias[bias_buf] : nullptr, p.relu, p.accumulate,
                                         rt * SP_ROWS, SP_ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
             }

@@ -278,8 +278,8 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
 
 // dw (+)= the partial results in ascending order, in float64.  A workgroup owns 8 / GW filters and 64 channels, TAPS taps
 // of them; GW waves share the splits of a filter.  Many splits (64 -> 64 channels: 256): GW = 8 and one tap, so that 576
-// workgroups read the 38 MB (12.7 us; 192 of three taps: 23 us); few (512 -> 512: 4): GW = 1 and all nine taps (12.6 us; GW = 8: 20 us).  Results that are not finite (an operand was not, or
-// rounds to a bf16 infinity) are formed again from the products themselves.  The workgroups behind them add db.
+// workgroups read the 38 MB (12.7 us; 192 of three taps: 23 us); few (512 -> 512: 4): GW = 1 and all nine taps (12.6 us; GW = 8: 20 us).  Results that the split does not carry (split3.h)
+// are formed again from the products themselves.  The workgroups behind them add db.
 template <int GW, int TAPS>
 __global__ void __launch_bounds__(512) split_wgrad_reduce_kernel(WgParams p, float *dw, float *db, int accumulate, int dw_blocks) {
     constexpr int KB = 8 / GW, ROW = T64 * TAPS, FLIGHT = GW == 1 ? 2 : GW == 2 ? 4 : 8;
@@ -333,7 +333,7 @@ __global__ void __launch_bounds__(512) split_wgrad_reduce_kernel(WgParams p, flo
         double all = 0.0;
 #pragma unroll
         for (int j = 0; j < GW; ++j) all += s_sum[kk * GW + j][i];
-        const bool mine = i < live && kb + kk < p.K, good = xsmi::finite((float)all);
+        const bool mine = i < live && kb + kk < p.K, good = xsmi::carried((float)all);
         s_sum[kk * GW][i] = mine && !good ? 1.0 : 0.0;
         if (mine && good) {
             float *q = out(kk, i);

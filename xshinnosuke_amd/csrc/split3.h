@@ -34,6 +34,13 @@ __device__ __forceinline__ void split_pair3(float a, float b, uint32_t &p0, uint
     p2 = __builtin_bit_cast(uint32_t, l);
 }
 
-__device__ __forceinline__ bool finite(float v) { return __builtin_fabsf(v) < __builtin_inff(); }
+// Whether a sum of split products is the float32 one.  It is not if an operand had no split (the sum is then non-finite), and
+// may not be if an operand was below 2^-110, whose third piece is below the smallest normal number and is lost (3 x 3,
+// 64 channels, values of 2^-112: 1.6e-7 against 64 bits, of 2^-124: 5.7e-4; fp32 pipe 1.2e-7).  2^-100 is reached by such
+// operands only against a row of the other operand with a norm above 2^10.
+__device__ __forceinline__ bool carried(float v) {
+    const float a = __builtin_fabsf(v);
+    return a < __builtin_inff() && (a >= 0x1p-100f || a == 0.f);
+}
 
 }  // namespace xsmi

@@ -35,7 +35,7 @@ long option(Option o);
 // Partial tiles and flags of the even-split convolution kernels for the stream that stream() hands out; allocated
 // by xsmi_init, the flags are zero between launches.
 constexpr size_t SK_SCRATCH_FLAG_BYTES = 4096;                          // 1024 workgroups
-constexpr size_t SK_SCRATCH_PART_BYTES = (size_t)768 * 32 * 256 * 4;    // 768 workgroups x one 64 x 128 tile of floats
+constexpr size_t SK_SCRATCH_PART_BYTES = (size_t)1024 * 16 * 256 * 4;   // 1024 workgroups x one 64 x 64 tile of floats
 struct SkScratch {
     uint32_t *flags;
     float *part;
