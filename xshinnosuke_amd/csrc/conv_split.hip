@@ -99,6 +99,13 @@ __device__ __forceinline__ void split8(const float (&v)[8], uint32x4 &p0, uint32
 // Outputs that the split does not carry are computed again one product at a time, in float64 (taps outside, channels
 // inside); a tap outside the input multiplies a zero, as the reference's padding does.
 __device__ __forceinline__ void recompute(floatx16 &r, const SpParams &p, const SpClass &c, int tile_row0, int row0, int m0, int lane) {
+    float smallest = __builtin_fabsf(r[0]), zero = 0.f;  // two instructions a value where nothing is the matter
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        smallest = __builtin_fminf(smallest, __builtin_fabsf(r[v]));
+        zero = __builtin_fmaf(r[v], 0.f, zero);        // NaN from an infinity or a NaN on
+    }
+    if (__builtin_amdgcn_ballot_w64(!(zero == 0.f) || !carried(smallest) || smallest == 0.f) == 0) return;
     uint32_t bad = 0;
 #pragma unroll
     for (int v = 0; v < 16; ++v) bad |= carried(r[v]) ? 0u : 1u << v;
