@@ -106,6 +106,27 @@ def test_weight_gradient_of_values_that_do_not_split(gpu):
     assert calm.any() and rel_l2(got[calm], ref[calm]) <= TOL
 
 
+@pytest.mark.parametrize("w,pad", [(13, 1), (16, 1), (7, 1), (32, 1), (16, 0)])      # the last block of columns ragged or full
+@pytest.mark.parametrize("column", [0, -1])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_weight_gradient_of_a_border_column_that_is_not_finite(gpu, w, pad, column, value):
+    """Under some taps a border column of dy meets only padding: zero times such a value is NaN, as in the reference's
+    product over the padded matrix."""
+    x, wt, b, dy, _ = _data(2, 70, 9, w, 66, 3, 3, 1, 1, pad, gpu)
+    dy[1, 65, 4, column] = value
+    dy[0, 3, 0, column] = -value
+    _, col = oracle.conv2d_fwd(x, wt, b, (1, 1), pad)
+    with np.errstate(all="ignore"):
+        _, ref, db_ref = oracle.conv2d_bwd(dy, x.shape, wt, col, (1, 1), pad, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+    with split_everywhere(gpu):
+        gw, gb = gpu.kernels.conv2d_bwd_weight(gpu.to_device(dy), gpu.to_device(x), wt.shape, (1, 1), pad, want_db=True)
+    for got, want in ((gw.numpy(), ref), (gb.numpy(), db_ref)):
+        for test in (np.isnan, np.isposinf, np.isneginf):
+            np.testing.assert_array_equal(test(got), test(want))
+        calm = np.isfinite(want)
+        assert calm.any() and rel_l2(got[calm], want[calm]) <= TOL
+
+
 def test_values_that_do_not_split_are_multiplied_one_by_one(gpu):
     """Infinities, NaN and floats that round to a bf16 infinity: the outputs they touch are the float32 ones, signs and
     NaNs included, and no other output is disturbed."""

@@ -17,7 +17,7 @@
 // multiplies one k-step of 16 pixels and nine taps (54 MFMAs) between two barriers, while its share of the next stage is
 // split behind the MFMAs and the one after it is in flight.  The two halves are added through the LDS at the end.
 // Workgroups take equal runs of stages; each writes its nine 64 x 64 partial products, and one launch adds them in
-// ascending order in float64.
+// ascending order in float64.  A workgroup whose sums the split does not carry (split3.h) forms them again in float64.
 #include "split3.h"
 
 #include <string.h>
@@ -28,6 +28,7 @@ using xsmi::bf16x8;
 using xsmi::IC;
 using xsmi::uint32x4;
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 constexpr int T64 = 64;
 constexpr int XP = 9, YP = 9;                         // octets per channel / filter in the LDS: 8 at most, made odd
@@ -45,8 +46,82 @@ struct WgParams {
     int row_blocks, col_blocks;
 };
 
+struct Place { int n, y, x; };                        // image, first output row, first input column of a stage
+__device__ __forceinline__ void next_stage(const WgParams &p, Place &q) {
+    q.x += p.CB * 8;
+    if (q.x >= p.col_blocks * p.CB * 8) {
+        q.x = 0; q.y += p.RB;
+        if (q.y >= p.row_blocks * p.RB) { q.y = 0; ++q.n; }
+    }
+}
+
+// The partial result of `stages` stages from `q` on, formed from the products themselves in float64: an output pixel times the
+// input under each tap, a zero where that is outside, as the fp32 kernels and the reference's padding have it (a border column
+// of dy that is not finite then reaches the taps that the walk over input columns has no place for).  Bound by the fp64
+// matrix pipe: a tap at a time, 16 x 16 blocks (D: register v of lane l is row l / 16 + 4 v, column l % 16), a lane's quarter
+// of the half's 16 pixels four deep.  All of 64 -> 64 at 56 x 56, N=8, not finite: 187 us (a product at a time behind the
+// partial results: 2850).
+__device__ __forceinline__ void form_again(const WgParams &p, float *part, double *s_half, Place q0, int stages, int k0, int c0,
+                                        int half, int wr, int wc, int lane) {
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, (int)p.x_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)p.dy, 0, (int)p.dy_bytes, 0x00020000);
+    const int l15 = lane & 15, quarter = lane >> 4, octet = 2 * half + (quarter >> 1);
+    const int o_row = octet / p.CB, o_col = (octet - o_row * p.CB) * 8 + (quarter & 1) * 4;
+    const int row0 = wr * 32 + l15, col0 = wc * 32 + l15;
+    auto at = [](__amdgpu_buffer_rsrc_t r, bool there, int index) {    // a value, zero where there is none
+        const int b = __builtin_amdgcn_raw_buffer_load_b32(r, there ? (int)((uint32_t)index * 4u) : (int)0x80000000u, 0, 0);
+        return (double)__builtin_bit_cast(float, b);
+    };
+#pragma unroll 1
+    for (int tap = 0; tap < 9; ++tap) {
+        const int r = tap / 3 - p.pad, s = tap % 3 - p.pad;
+        doublex4 d[2][2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[i >> 1][i & 1] = doublex4{0.0, 0.0, 0.0, 0.0};
+        Place q = q0;
+#pragma unroll 1
+        for (int st = 0; st < stages; ++st) {
+            const int y = q.y + o_row, iy = y + r;
+            double a[4][2], b[4][2];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int x = q.x + o_col + i, ix = x + s;
+                const bool there = y < p.OH && x < p.OW, in = there && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int k = k0 + row0 + 16 * j, c = c0 + col0 + 16 * j;
+                    a[i][j] = at(ry, there && k < p.K, ((q.n * p.K + k) * p.OH + y) * p.OW + x);
+                    b[i][j] = at(rx, in && c < p.C, ((q.n * p.C + c) * p.H + iy) * p.W + ix);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    d[j >> 1][j & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][j >> 1], b[i][j & 1], d[j >> 1][j & 1], 0, 0, 0);
+            next_stage(p, q);
+        }
+        auto place = [&](int j, int v) { return (wr * 32 + 16 * (j >> 1) + quarter + 4 * v) * T64 + col0 + 16 * (j & 1); };
+        if (half == 1) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) s_half[place(j, v)] = d[j >> 1][j & 1][v];
+        }
+        __syncthreads();
+        if (half == 0) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) part[tap * T64 * T64 + place(j, v)] = (float)(d[j >> 1][j & 1][v] + s_half[place(j, v)]);
+        }
+        __syncthreads();
+    }
+}
+
 __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
     __shared__ __attribute__((aligned(16))) unsigned char s_mem[9 * 16 * 256 * 4];
+    __shared__ uint32_t s_again;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int half = wave >> 2, wr = (wave >> 1) & 1, wc = wave & 1, h = lane >> 5, l31 = lane & 31;
@@ -74,20 +149,13 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
         return m;
     };
     const Mine m0 = mine(t, y_side[0]), m1 = mine(t + 512, y_side[1]);
-    struct Place { int n, y, x; };                    // image, first output row, first input column of a stage
     auto place = [&](int s) {
         Place q;
         const int cb = s % p.col_blocks, r = s / p.col_blocks;
         q.x = cb * p.CB * 8; q.y = r % p.row_blocks * p.RB; q.n = r / p.row_blocks;
         return q;
     };
-    auto next = [&](Place &q) {
-        q.x += p.CB * 8;
-        if (q.x >= p.col_blocks * p.CB * 8) {
-            q.x = 0; q.y += p.RB;
-            if (q.y >= p.row_blocks * p.RB) { q.y = 0; ++q.n; }
-        }
-    };
+    auto next = [&](Place &q) { next_stage(p, q); };
     float pre[2][8];
     int cut[2], early[2];                             // values from this one on are past the row; the octet begins that much early
     bool ends[2];                                     // uniform: some octet of the stage crosses an end of its row
@@ -242,8 +310,8 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
         cur = to;
     }
 
-    // the two halves of the waves, then the partial result: register v of lane l is filter 8 (v / 4) + 4 (l / 32) + v % 4,
-    // channel l % 32 of the wave's block
+    // the two halves of the waves are added: register v of lane l is filter 8 (v / 4) + 4 (l / 32) + v % 4, channel l % 32
+    // of the wave's block
     xsmi::wait_lgkmcnt0();
     __syncthreads();
     float *s_acc = reinterpret_cast<float *>(s_mem);
@@ -253,14 +321,27 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) s_acc[(i * 16 + v) * 256 + (t & 255)] = acc[i][v];
     }
+    if (t == 0) s_again = 0;
     __syncthreads();
+    float *part = p.part + ((size_t)split * tiles + tile) * TILE;
     if (half == 0) {
-        float *dst = p.part + ((size_t)split * tiles + tile) * TILE + (wr * 32 + 4 * h) * T64 + wc * 32 + l31;
+        float *dst = part + (wr * 32 + 4 * h) * T64 + wc * 32 + l31;
+        xsmi::CarriedTest test;
 #pragma unroll
         for (int i = 0; i < 9; ++i)
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
-                dst[i * T64 * T64 + (8 * (v >> 2) + (v & 3)) * T64] = acc[i][v] + s_acc[(i * 16 + v) * 256 + t];
+            for (int v = 0; v < 16; ++v) {
+                const float sum = acc[i][v] + s_acc[(i * 16 + v) * 256 + t];
+                test.add(sum);
+                dst[i * T64 * T64 + (8 * (v >> 2) + (v & 3)) * T64] = sum;
+            }
+        if (!test.all()) s_again = 1;
+    }
+    __syncthreads();
+    if (s_again) {
+        xsmi::wait_vmcnt<0>();                        // what is overwritten now has been written
+        __syncthreads();
+        form_again(p, part, reinterpret_cast<double *>(s_mem), place(s0), s1 - s0, k0, c0, half, wr, wc, lane);
     }
     if (want_db) {                                    // a filter's octets are in up to ny threads: added in their order
         double *s_db = reinterpret_cast<double *>(s_mem);
@@ -278,14 +359,13 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
 
 // dw (+)= the partial results in ascending order, in float64.  A workgroup owns 8 / GW filters and 64 channels, TAPS taps
 // of them; GW waves share the splits of a filter.  Many splits (64 -> 64 channels: 256): GW = 8 and one tap, so that 576
-// workgroups read the 38 MB (12.7 us; 192 of three taps: 23 us); few (512 -> 512: 4): GW = 1 and all nine taps (12.6 us; GW = 8: 20 us).  Results that the split does not carry (split3.h)
-// are formed again from the products themselves.  The workgroups behind them add db.
+// workgroups read the 38 MB (12.7 us; 192 of three taps: 23 us); few (512 -> 512: 4): GW = 1 and all nine taps (12.6 us;
+// GW = 8: 20 us).  The workgroups behind them add db.
 template <int GW, int TAPS>
 __global__ void __launch_bounds__(512) split_wgrad_reduce_kernel(WgParams p, float *dw, float *db, int accumulate, int dw_blocks) {
     constexpr int KB = 8 / GW, ROW = T64 * TAPS, FLIGHT = GW == 1 ? 2 : GW == 2 ? 4 : 8;
     __shared__ double s_sum[8][ROW];
     __shared__ double s_part[512];
-    __shared__ uint32_t s_bad;
     const int t = threadIdx.x, c = t & 63, w = t >> 6;
     if ((int)blockIdx.x >= dw_blocks) {
         const int k = ((int)blockIdx.x - dw_blocks) * 64 + c;
@@ -324,47 +404,16 @@ __global__ void __launch_bounds__(512) split_wgrad_reduce_kernel(WgParams p, flo
     }
 #pragma unroll
     for (int i = 0; i < TAPS; ++i) s_sum[w][c * TAPS + i] = sum[i];
-    if (t == 0) s_bad = 0;
     __syncthreads();
     const int live = (p.C - c0 < T64 ? p.C - c0 : T64) * TAPS;
-    auto out = [&](int kk, int i) { return dw + ((size_t)(kb + kk) * p.C + c0 + i / TAPS) * 9 + r0 + i % TAPS; };
     for (int o = t; o < KB * ROW; o += 512) {
         const int kk = o / ROW, i = o - kk * ROW;
+        if (i >= live || kb + kk >= p.K) continue;
+        float *q = dw + ((size_t)(kb + kk) * p.C + c0 + i / TAPS) * 9 + r0 + i % TAPS;
         double all = 0.0;
 #pragma unroll
         for (int j = 0; j < GW; ++j) all += s_sum[kk * GW + j][i];
-        const bool mine = i < live && kb + kk < p.K, good = xsmi::carried((float)all);
-        s_sum[kk * GW][i] = mine && !good ? 1.0 : 0.0;
-        if (mine && good) {
-            float *q = out(kk, i);
-            *q = (float)(accumulate ? all + (double)*q : all);
-        } else if (mine) {
-            atomicOr(&s_bad, 1u);
-        }
-    }
-    __syncthreads();
-    if (s_bad == 0) return;
-    for (int o = 0; o < KB * ROW; ++o) {
-        const int kk = o / ROW, i = o - kk * ROW;
-        if (s_sum[kk * GW][i] == 0.0) continue;       // uniform
-        const int cc = c0 + i / TAPS, tap = r0 + i % TAPS, total = p.N * p.OH * p.OW;
-        double part = 0.0;
-        for (int m = t; m < total; m += 512) {
-            const int q = m / p.OW, ox = m - q * p.OW, n = q / p.OH, oy = q - n * p.OH;
-            const int iy = oy + tap / 3 - p.pad, ix = ox + tap % 3 - p.pad;
-            const float a = p.dy[((size_t)n * p.K + kb + kk) * p.OH * p.OW + (size_t)oy * p.OW + ox];
-            const float b = iy >= 0 && iy < p.H && ix >= 0 && ix < p.W ? p.x[((size_t)n * p.C + cc) * p.H * p.W + (size_t)iy * p.W + ix] : 0.f;
-            part += (double)a * (double)b;
-        }
-        __syncthreads();
-        s_part[t] = part;
-        __syncthreads();
-        if (t == 0) {
-            double all = 0.0;
-            for (int j = 0; j < 512; ++j) all += s_part[j];
-            float *q = out(kk, i);
-            *q = (float)(accumulate ? all + (double)*q : all);
-        }
+        *q = (float)(accumulate ? all + (double)*q : all);
     }
 }
 
