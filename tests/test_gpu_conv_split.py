@@ -89,6 +89,74 @@ def test_split_weight_gradient_against_the_oracle(gpu, n, c, h, w, k, pad, accum
     assert rel_l2(gw.numpy(), dw_ref) <= TOL and rel_l2(gb.numpy(), db_ref) <= TOL
 
 
+FORMED_AGAIN = [   # what the kernel that forms sums again walks differently
+    (1, 17, 16, 16, 65, 3, 3, 1, 1, 1),      # a channel and a row past their tiles
+    (5, 1, 25, 41, 3, 2, 2, 1, 1, 0),        # one channel, even filter
+    (2, 24, 45, 61, 40, 5, 5, 1, 1, 2),      # one filter row per phase
+    (3, 20, 19, 23, 70, 7, 7, 2, 2, 3),      # strided: 14 phases
+    (2, 48, 14, 15, 20, 3, 3, 2, 2, 1),      # four phases forward, four classes backward
+    (2, 20, 17, 13, 70, 3, 5, 2, 1, 1),      # strides and filter sides that differ
+    (1, 512, 7, 7, 512, 3, 3, 1, 1, 1),      # segments that begin and end anywhere in a tile
+]
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad", FORMED_AGAIN)
+def test_sums_that_are_formed_again(gpu, n, c, h, w, k, r, s, sh, sw, pad):
+    """Every sum is below 2^-100, so every one is formed a second time; powers of two are exact: the bound is that of
+    ordinary values."""
+    K = gpu.kernels
+    x, wt, b, dy, _ = _data(n, c, h, w, k, r, s, sh, sw, pad, gpu)
+    y_ref, col = oracle.conv2d_fwd(x, wt, 0 * b, (sh, sw), pad)
+    dx_ref, _, _ = oracle.conv2d_bwd(dy, x.shape, wt, col, (sh, sw), pad, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+    small = lambda a: gpu.to_device(a * np.float32(2.0 ** -107))  # noqa: E731
+    with split_everywhere(gpu):
+        y = K.conv2d_fwd(small(x), gpu.to_device(wt), None, (sh, sw), pad).numpy()
+        gx = K.conv2d_bwd_data(small(dy), gpu.to_device(wt), x.shape, (sh, sw), pad).numpy()
+    assert rel_l2(y.astype(np.float64) * 2.0 ** 107, y_ref) <= TOL and rel_l2(gx.astype(np.float64) * 2.0 ** 107, dx_ref) <= TOL
+
+
+@pytest.mark.parametrize("pass_", [0, 1])
+def test_a_filter_whose_layout_is_in_place_is_not_read(gpu, pass_):
+    """What is passed as the filter is another one by then; a value that does not split, on either side, takes the sums that
+    are formed again, and those take the filter from its layout too."""
+    import ctypes
+    from xshinnosuke_amd.backend import capi
+    dims = (2, 40, 12, 13, 40, 3, 3, 1, 1, 1)
+    x, wt, _, _, _ = _data(*dims, gpu)
+    x[:, [2, 33]] *= np.float32(0.1)                     # products with 3.4e38 stay finite in 32 bits as well
+    x[0, 3, 2, 2], x[1, 19, 6, 6], x[1, 20, 11, 12] = np.inf, np.nan, np.float32(3.4e38)
+    wt[5, 3, 0, 2], wt[7, 30, 1, 1], wt[33, 2, 2, 0] = -np.inf, np.nan, np.float32(-3.4e38)
+    K = gpu.kernels
+    run = lambda: (K.conv2d_bwd_data(dx, dw, x.shape, (1, 1), 1) if pass_ else K.conv2d_fwd(dx, dw, None, (1, 1), 1)).numpy()  # noqa: E731
+    dx, dw, other = gpu.to_device(x), gpu.to_device(wt), gpu.to_device(np.ones_like(wt))
+    with split_everywhere(gpu):
+        ref = run()
+        size = capi.lib.raw("xsmi_conv2d_pass_workspace_bytes")(*dims, pass_, 0)
+        ws, y = gpu.empty(((size + 3) // 4,)), gpu.empty(ref.shape)
+        job = (capi.PackJob * 1)()
+        job[0].w, job[0].workspace, job[0].workspace_bytes = dw.ptr, ws.ptr, size
+        for field, v in zip(("N", "C", "H", "W", "K", "R", "S", "sh", "sw", "pad", "pass_"), dims + (pass_,)):
+            setattr(job[0], field, v)
+        capi.lib.call("xsmi_conv2d_pack", 1, ctypes.cast(job, ctypes.c_void_p))
+        capi.lib.call("xsmi_conv2d_bwd_join")
+        assert job[0].packed == 1
+        if pass_ == 0:
+            capi.lib.call("xsmi_conv2d_fwd", dx.ptr, other.ptr, None, y.ptr, None, *dims, capi.CONV_WS_PACKED, ws.ptr, size)
+        else:
+            capi.lib.call("xsmi_conv2d_bwd_data", dx.ptr, other.ptr, y.ptr, *dims, 0.0, capi.CONV_WS_PACKED, ws.ptr, size)
+    got = y.numpy()
+    assert got.tobytes() == ref.tobytes()
+    old = gpu.set_option("conv_split", 0)
+    try:
+        plain = run()
+    finally:
+        gpu.set_option("conv_split", old)
+    for test in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(test(got), test(plain))
+    calm = np.isfinite(plain)
+    assert calm.any() and rel_l2(got[calm], plain[calm]) <= TOL
+
+
 def test_weight_gradient_of_values_that_do_not_split(gpu):
     K = gpu.kernels
     x, wt, b, dy, _ = _data(2, 20, 12, 13, 70, 3, 3, 1, 1, 1, gpu)

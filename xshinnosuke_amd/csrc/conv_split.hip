@@ -10,9 +10,8 @@
 // channels and tap, against one per product pair on the fp32 pipe.
 //
 // What the split does not carry: infinities (inf - inf in a remainder), values within a bf16 rounding of the largest
-// float, and the last bits of values below 2^-110.  The first two make the outputs that they touch non-finite, the third
-// are found by outputs below 2^-100 (split3.h); such outputs are computed again, one product at a time in float64, before
-// they are stored (recompute).
+// float, and the last bits of values below 2^-110.  The first two make the sums that they touch non-finite, the third
+// are found by sums below 2^-100 (split3.h); such sums are formed again in float64 (form_again).
 //
 // Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (128 per tile), 2 x 2 waves
 // of 32 rows x 64 pixels.  The reduction is a list of steps (phase, 16 input channels, tap).  A PHASE is a set of taps
@@ -43,6 +42,8 @@ using xsmi::bf16x8;
 using xsmi::uint32x4;
 using xsmi::IC;
 using xsmi::carried;
+typedef uint32_t uint32x2 __attribute__((ext_vector_type(2)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 constexpr int SP_ROWS = 64;
 constexpr int sp_slots_of(int wc) { return wc == 4 ? 512 : 384; }     // slots of an LDS image
@@ -77,7 +78,7 @@ struct SpParams {
     uint32_t in_bytes, out_bytes, apk_bytes, spin_limit;
     uint32_t units, upg, urem;                       // steps in all; per workgroup, remainder
     int N, CH, groups, IH, IW, in_n, plane;          // input channels, their groups of 16, floats per image / plane
-    int w_row, w_ch, FS;                             // floats between rows / channels of the filter, filter width
+    int w_row, w_ch, FS;                             // of the layout launches: floats between rows / channels of the filter, filter width
     int ncls, relu, accumulate, wc;
     SpClass cls[SP_MAX_CLASSES];
     SpPhase ph[SP_MAX_PHASES];
@@ -86,57 +87,90 @@ struct SpParams {
 
 constexpr int AGENT = 16;                            // sc1: past the caches that are not coherent across XCDs
 
-// eight floats -> three vectors of eight bf16
-__device__ __forceinline__ void split8(const float (&v)[8], uint32x4 &p0, uint32x4 &p1, uint32x4 &p2) {
+// Eight filter values -> three vectors of eight bf16.  A value that does not split is left as it is in the second and third
+// piece, behind a first one that makes every sum it enters a NaN.
+__device__ __forceinline__ void split_filter8(const float (&v)[8], uint32x4 &p0, uint32x4 &p1, uint32x4 &p2) {
+    constexpr uint32_t NAN16 = 0x7fc0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+        const bool there_l = xsmi::splits(v[2 * i]), there_h = xsmi::splits(v[2 * i + 1]);
+        const uint32_t l = __builtin_bit_cast(uint32_t, v[2 * i]), h = __builtin_bit_cast(uint32_t, v[2 * i + 1]);
         uint32_t a, b, c;
-        xsmi::split_pair3(v[2 * i], v[2 * i + 1], a, b, c);
+        xsmi::split_pair3(there_l ? v[2 * i] : 0.f, there_h ? v[2 * i + 1] : 0.f, a, b, c);
+        if (!there_l) { a |= NAN16; b |= l >> 16; c |= l & 0xffffu; }
+        if (!there_h) { a |= NAN16 << 16; b |= h & 0xffff0000u; c |= h << 16; }
         p0[i] = a; p1[i] = b; p2[i] = c;
     }
 }
+// The value again, from the low halves of its three pieces.
+__device__ __forceinline__ double unsplit(uint32_t p0, uint32_t p1, uint32_t p2) {
+    auto wide = [](uint32_t bits) { return (double)__builtin_bit_cast(float, bits); };
+    return (p0 & 0x7fffu) > 0x7f80u ? wide(p1 << 16 | (p2 & 0xffffu)) : wide(p0 << 16) + wide(p1 << 16) + wide(p2 << 16);
+}
 
-// Outputs that the split does not carry are computed again one product at a time, in float64 (taps outside, channels
-// inside); a tap outside the input multiplies a zero, as the reference's padding does.
-__device__ __forceinline__ void recompute(floatx16 &r, const SpParams &p, const SpClass &c, int tile_row0, int row0, int m0, int lane) {
-    float smallest = __builtin_fabsf(r[0]), zero = 0.f;  // two instructions a value where nothing is the matter
+// The sums of a segment that the split does not carry (split3.h) are formed again in float64, 16 x 16 blocks on the fp64 matrix
+// instructions (D: register v of lane l is row l / 16 + 4 v, column l % 16): a step's 16 channels are four products deep,
+// a lane has channels 4 (l / 16) .. + 3 of a row and of a pixel.  The filter comes out of its layout, whose pieces are the
+// value (split_filter8), so the filter itself is not read here either; a tap outside the input multiplies a zero, as the
+// reference's padding does.  Every workgroup does this for its own steps.  All of 64 -> 64 at 56 x 56, N=8, not finite:
+// 93 us (one product at a time, by the workgroups that store the outputs: 2490), 256 -> 256 at 14 x 14: 110 (10100).
+struct SpSteps { int rt, s_first, n, f, grp, tap; };
+__device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const SpClass &c, const SpSteps &sg, int row0, int m0, int lane,
+                                           __amdgpu_buffer_rsrc_t rin, __amdgpu_buffer_rsrc_t rapk) {
+    const int l15 = lane & 15, quarter = lane >> 4;
+    int oy[2], ox[2], image[2];
+    bool there[2];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        smallest = __builtin_fminf(smallest, __builtin_fabsf(r[v]));
-        zero = __builtin_fmaf(r[v], 0.f, zero);        // NaN from an infinity or a NaN on
+    for (int j = 0; j < 2; ++j) {
+        const int m = m0 + 16 * j + l15, q = (int)xsmi::fdiv((uint32_t)m, c.dOX), n = (int)xsmi::fdiv((uint32_t)q, c.dOY);
+        there[j] = m < c.M;
+        ox[j] = m - q * c.OX; oy[j] = q - n * c.OY; image[j] = n * p.in_n;
     }
-    if (__builtin_amdgcn_ballot_w64(!(zero == 0.f) || !carried(smallest) || smallest == 0.f) == 0) return;
-    uint32_t bad = 0;
+    doublex4 d[2][2];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) bad |= carried(r[v]) ? 0u : 1u << v;
-    if (__builtin_amdgcn_ballot_w64(bad != 0) == 0) return;
-    const int m = m0 + (lane & 31);
-    if (m >= c.M) return;
-    const int q = (int)xsmi::fdiv((uint32_t)m, c.dOX), ox = m - q * c.OX;
-    const int n = (int)xsmi::fdiv((uint32_t)q, c.dOY), oy = q - n * c.OY;
+    for (int j = 0; j < 4; ++j) d[j >> 1][j & 1] = doublex4{0.0, 0.0, 0.0, 0.0};
+    const int a_lane = ((quarter >> 1) * SP_ROWS + row0 + l15) * 16 + (quarter & 1) * 8;
+    uint32_t block = c.apk_off + ((uint32_t)sg.rt * c.iters + (uint32_t)sg.s_first) * (uint32_t)SP_BLOCK;
+    int f = sg.f, grp = sg.grp, tap = sg.tap;
 #pragma unroll 1
-    for (int v = 0; v < 16; ++v) {
-        const int row = tile_row0 + row0 + 4 * (lane >> 5) + 8 * (v >> 2) + (v & 3);
-        if (!((bad >> v) & 1u) || row >= c.rows) continue;
-        double sum = 0.0;
-        const float *wrow = p.w + (size_t)row * p.w_row;
-#pragma unroll 1
-        for (int f = c.phase0; f < c.phase0 + c.nphase; ++f) {
-            const SpPhase &ph = p.ph[f];
-#pragma unroll 1
-            for (int t = 0; t < ph.T; ++t) {
-                const int a = t / ph.Tx, b = t - a * ph.Tx;
-                const int iy = (oy + a) * c.sy + ph.iy0, ix = (ox + b) * c.sx + ph.ix0;
-                const bool in = iy >= 0 && iy < p.IH && ix >= 0 && ix < p.IW;
-                const float *wt = wrow + (ph.r0 + ph.rs * a) * p.FS + ph.s0 + ph.ss * b;
-                const float *src = p.in + (size_t)n * p.in_n + (size_t)(in ? iy * p.IW + ix : 0);
-#pragma unroll 1
-                for (int ch = 0; ch < p.CH; ++ch)
-                    sum += (double)wt[(size_t)ch * p.w_ch] * (double)(in ? src[(size_t)ch * p.plane] : 0.f);
+    for (int s = 0; s < sg.n; ++s, block += SP_BLOCK) {
+        const SpPhase &ph = p.ph[f];
+        const int ta = tap / ph.Tx, tb = tap - ta * ph.Tx, ch0 = grp * 16 + 4 * quarter;
+        double a[2][4], b[2][4];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            uint32x2 piece[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                piece[q] = __builtin_amdgcn_raw_buffer_load_b64(rapk, a_lane + j * 256 + q * 2 * SP_ROWS * 16, (int)block, 0);
+            const int iy = (oy[j] + ta) * c.sy + ph.iy0, ix = (ox[j] + tb) * c.sx + ph.ix0;
+            const bool in = there[j] && iy >= 0 && iy < p.IH && ix >= 0 && ix < p.IW;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t place = ((uint32_t)image[j] + (uint32_t)(ch0 + i) * (uint32_t)p.plane + (uint32_t)(iy * p.IW + ix)) * 4u;
+                const int bits = __builtin_amdgcn_raw_buffer_load_b32(rin, in && ch0 + i < p.CH ? (int)place : (int)0x80000000u, 0, 0);
+                b[j][i] = (double)__builtin_bit_cast(float, bits);
+                const int sh = 16 * (i & 1);
+                a[j][i] = unsplit(piece[0][i >> 1] >> sh, piece[1][i >> 1] >> sh, piece[2][i >> 1] >> sh);
             }
         }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) r[i] = i == v ? (float)sum : r[i];
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                d[j >> 1][j & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j >> 1][i], b[j & 1][i], d[j >> 1][j & 1], 0, 0, 0);
+        if (++tap == ph.T) { tap = 0; if (++grp == p.groups) { grp = 0; ++f; } }
+    }
+    // to the 32 x 32 block's order: register v of lane l is row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        float from[2][2];                              // [right half of the columns][upper half of the lanes]
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            from[k >> 1][k & 1] = __shfl((float)d[v >> 3][k >> 1][2 * ((v >> 2) & 1) + (k & 1)], 16 * (v & 3) + l15);
+        const float low = (lane & 16) ? from[1][0] : from[0][0], high = (lane & 16) ? from[1][1] : from[0][1];
+        const float again = (lane & 32) ? high : low;
+        r[v] = carried(r[v]) ? r[v] : again;
     }
 }
 
@@ -436,7 +470,14 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         // ---- end of the segment ----
         floatx16 acc[2];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[j] = hi[j] + lo[j];
+        for (int j = 0; j < 2; ++j) {
+            acc[j] = hi[j] + lo[j];
+            xsmi::CarriedTest test;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) test.add(acc[j][v]);
+            if (__builtin_amdgcn_ballot_w64(!test.all()) != 0)
+                form_again(acc[j], p, c, SpSteps{rt, sg.s_first, sg.n, sg.f, sg.grp, sg.tap}, wr * 32, m0 + wc * 64 + 32 * j, lane, rin, rapk);
+        }
         if (!head) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -501,7 +542,6 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         if (head) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                recompute(acc[j], p, c, rt * SP_ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
                 xsmi::store_block_32x32(acc[j], c, p.out, p.out_bytes, p.mask, p.bias ? s_bias[bias_buf] : nullptr, p.relu, p.accumulate,
                                         rt * SP_ROWS, SP_ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
             }
@@ -530,7 +570,7 @@ __global__ void __launch_bounds__(64) split_pack9_kernel(SpParams p, char *apk, 
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
         uint32x4 q0, q1, q2;
-        split8(v[t], q0, q1, q2);
+        split_filter8(v[t], q0, q1, q2);
         const SpTapPlace &w = p.tap[t];
         const uint32_t step = rt * w.iters + w.step + (o >> 1) * w.T;
         char *dst = apk + w.off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + threadIdx.x) * 16;
@@ -559,7 +599,7 @@ __global__ void __launch_bounds__(256) split_pack_kernel(SpParams p, char *apk) 
                 v[e] = (int)row < c.rows && ch < p.CH ? src[(size_t)row * p.w_row + (size_t)ch * p.w_ch] : 0.f;
             }
             uint32x4 q0, q1, q2;
-            split8(v, q0, q1, q2);
+            split_filter8(v, q0, q1, q2);
             const uint32_t step = (row / SP_ROWS) * c.iters + (uint32_t)ph.step0 + (o >> 1) * (uint32_t)ph.T + (uint32_t)tl;
             char *dst = apk + c.apk_off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + row % SP_ROWS) * 16;
             *reinterpret_cast<uint32x4 *>(dst) = q0;

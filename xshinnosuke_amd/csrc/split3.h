@@ -34,6 +34,9 @@ __device__ __forceinline__ void split_pair3(float a, float b, uint32_t &p0, uint
     p2 = __builtin_bit_cast(uint32_t, l);
 }
 
+// Whether a value has a split: finite, and not so large that its first piece would be an infinity.
+__device__ __forceinline__ bool splits(float v) { return __builtin_fabsf(v) < __builtin_bit_cast(float, 0x7f7f8000u); }
+
 // Whether a sum of split products is the float32 one.  It is not if an operand had no split (the sum is then non-finite), and
 // may not be if an operand was below 2^-110, whose third piece is below the smallest normal number and is lost (3 x 3,
 // 64 channels, values of 2^-112: 1.6e-7 against 64 bits, of 2^-124: 5.7e-4; fp32 pipe 1.2e-7).  2^-100 is reached by such
