@@ -195,6 +195,24 @@ def test_weight_gradient_of_a_border_column_that_is_not_finite(gpu, w, pad, colu
         assert calm.any() and rel_l2(got[calm], want[calm]) <= TOL
 
 
+@pytest.mark.parametrize("w,column", [(w, c) for w in (16, 17, 18, 32, 40) for c in (0, 15, 16, -1) if c < w])
+def test_weight_gradient_formed_again_by_some_workgroups_only(gpu, w, column):
+    """One value that is not finite: the workgroups that meet it form all their sums again, the others do not, and together
+    they have every product once."""
+    x, wt, b, dy, _ = _data(6, 40, 9, w, 66, 3, 3, 1, 1, 1, gpu)
+    x[0, 31, 5, column] = np.nan
+    dy[3, 60, 4, column] = np.inf
+    _, col = oracle.conv2d_fwd(x, wt, b, (1, 1), 1)
+    with np.errstate(all="ignore"):
+        _, ref, _ = oracle.conv2d_bwd(dy, x.shape, wt, col, (1, 1), 1, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+    with split_everywhere(gpu):
+        got = gpu.kernels.conv2d_bwd_weight(gpu.to_device(dy), gpu.to_device(x), wt.shape, (1, 1), 1)[0].numpy()
+    for test in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(test(got), test(ref))
+    calm = np.isfinite(ref)
+    assert calm.any() and rel_l2(got[calm], ref[calm]) <= TOL
+
+
 def test_values_that_do_not_split_are_multiplied_one_by_one(gpu):
     """Infinities, NaN and floats that round to a bf16 infinity: the outputs they touch are the float32 ones, signs and
     NaNs included, and no other output is disturbed."""

@@ -55,10 +55,10 @@ __device__ __forceinline__ void next_stage(const WgParams &p, Place &q) {
     }
 }
 
-// The partial result of `stages` stages from `q` on, formed from the products themselves in float64: an output pixel times the
-// input under each tap, a zero where that is outside, as the fp32 kernels and the reference's padding have it (a border column
-// of dy that is not finite then reaches the taps that the walk over input columns has no place for).  Bound by the fp64
-// matrix pipe: a tap at a time, 16 x 16 blocks (D: register v of lane l is row l / 16 + 4 v, column l % 16), a lane's quarter
+// The partial result of `stages` stages from `q` on, formed from the products themselves in float64.  A workgroup decides this
+// for itself, so its share is the one that it has among workgroups that do not: the stages' output rows and input columns.
+// A border column of dy has no input column under some taps: it meets a zero there, as in the fp32 kernels and in the
+// reference's product over the padded matrix, so that it shows if it is not finite.  Bound by the fp64 matrix pipe: a tap at a time, 16 x 16 blocks (D: register v of lane l is row l / 16 + 4 v, column l % 16), a lane's quarter
 // of the half's 16 pixels four deep.  All of 64 -> 64 at 56 x 56, N=8, not finite: 187 us (a product at a time behind the
 // partial results: 2850).
 __device__ __forceinline__ void form_again(const WgParams &p, float *part, double *s_half, Place q0, int stages, int k0, int c0,
@@ -85,13 +85,24 @@ __device__ __forceinline__ void form_again(const WgParams &p, float *part, doubl
             double a[4][2], b[4][2];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int x = q.x + o_col + i, ix = x + s;
-                const bool there = y < p.OH && x < p.OW, in = there && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W;
+                const int ix = q.x + o_col + i, x = ix - s;
+                const bool there = y < p.OH && x >= 0 && x < p.OW, in = there && iy >= 0 && iy < p.H && ix < p.W;
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     const int k = k0 + row0 + 16 * j, c = c0 + col0 + 16 * j;
                     a[i][j] = at(ry, there && k < p.K, ((q.n * p.K + k) * p.OH + y) * p.OW + x);
                     b[i][j] = at(rx, in && c < p.C, ((q.n * p.C + c) * p.H + iy) * p.W + ix);
+                }
+            }
+            // columns -1 and W of the input, where the walk has no place for them
+            const int beside = s < 0 && q.x == 0 ? 0 : s > 0 && q.x + p.CB * 8 == p.W ? p.OW - 1 : -1;
+            if (p.pad == 1 && beside >= 0) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int k = k0 + row0 + 16 * j;
+                    const double edge = at(ry, y < p.OH && o_col == 0 && k < p.K, ((q.n * p.K + k) * p.OH + y) * p.OW + beside);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) d[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(edge, 0.0, d[j][i], 0, 0, 0);
                 }
             }
 #pragma unroll
