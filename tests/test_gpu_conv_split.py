@@ -251,6 +251,63 @@ def test_small_values_keep_their_last_bits(gpu, scale):
         assert rel_l2(got.astype(np.float64) * up, ref) <= TOL
 
 
+@pytest.mark.parametrize("which", ["activations", "filter"])
+@pytest.mark.parametrize("small,large", [(-116, 40), (-124, 100), (-130, 60), (-140, 110), (-148, 120)])
+def test_small_values_against_large_ones(gpu, which, small, large):
+    """Values below 2^-110, subnormal ones among them, whose products are ordinary again: the bound is that of ordinary values,
+    of what is left of them as float32."""
+    K = gpu.kernels
+    x, wt, b, dy, _ = _data(2, 20, 12, 13, 70, 3, 3, 1, 1, 1, gpu)
+    down, up = np.float32(2.0 ** small), np.float32(2.0 ** large)
+    rest = 2.0 ** -(small + large)
+    xs_, ws_ = (x * down, wt * up) if which == "activations" else (x * up, wt * down)
+    ds = dy * (down if which == "activations" else up)
+    dw = dy * (up if which == "activations" else down)               # against the input of the weight gradient
+    wide = lambda a, e: np.ldexp(a.astype(np.float64), -e).astype(np.float32)  # noqa: E731 -- what float32 kept, scaled back
+    e1, e2 = (small, large) if which == "activations" else (large, small)
+    y_ref, col = oracle.conv2d_fwd(wide(xs_, e1), wide(ws_, e2), 0 * b, (1, 1), 1)
+    dx_ref, _, _ = oracle.conv2d_bwd(wide(ds, e1), x.shape, wide(ws_, e2), col, (1, 1), 1, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+    _, dw_ref, _ = oracle.conv2d_bwd(wide(dw, e2), x.shape, wt, col, (1, 1), 1, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+    with split_everywhere(gpu):
+        y = K.conv2d_fwd(gpu.to_device(xs_), gpu.to_device(ws_), None, (1, 1), 1).numpy()
+        gx = K.conv2d_bwd_data(gpu.to_device(ds), gpu.to_device(ws_), x.shape, (1, 1), 1).numpy()
+        gw, _ = K.conv2d_bwd_weight(gpu.to_device(dw), gpu.to_device(xs_), wt.shape, (1, 1), 1, want_db=True)
+    for got, ref in ((y, y_ref), (gx, dx_ref), (gw.numpy(), dw_ref)):
+        assert rel_l2(got.astype(np.float64) * rest, ref) <= TOL
+
+
+@pytest.mark.parametrize("value", [2.0 ** -111, 2.0 ** -149])
+def test_one_small_value_is_found_wherever_it_lies(gpu, value):
+    """One value below 2^-110 and zeros around it, so that the results are its products alone: at the first and last places
+    of octets, slots, rows and tiles."""
+    K = gpu.kernels
+    n, c, h, w, k = 2, 40, 9, 18, 66
+    _, wt, _, _, _ = _data(n, c, h, w, k, 3, 3, 1, 1, 1, gpu)
+    wt *= np.float32(2.0 ** 60)
+    places = [(0, 0, 0, 0), (0, 7, 0, 17), (1, 8, 8, 0), (1, 39, 8, 17), (0, 15, 4, 7), (1, 16, 3, 8), (0, 31, 5, 15), (1, 32, 2, 16)]
+    rest = np.float64(1.0 / value) * 2.0 ** -60
+    with split_everywhere(gpu):
+        for i, q in enumerate(places):
+            x, dy = np.zeros((n, c, h, w), np.float32), np.zeros((n, k, h, w), np.float32)
+            x[q] = value
+            xr = np.zeros_like(x); xr[q] = 1
+            y_ref, col = oracle.conv2d_fwd(xr, (wt * np.float32(2.0 ** -60)), None, (1, 1), 1)
+            y = K.conv2d_fwd(gpu.to_device(x), gpu.to_device(wt), None, (1, 1), 1).numpy()
+            assert rel_l2(y.astype(np.float64) * rest, y_ref) <= TOL, q
+            # the weight gradient, once with the small value in the input and once in dy
+            big = np.random.default_rng(i).standard_normal(dy.shape).astype(np.float32)
+            _, ref, _ = oracle.conv2d_bwd(big, x.shape, wt, col, (1, 1), 1, np.zeros_like(x), np.zeros_like(wt), np.zeros(k, np.float32))
+            gw = K.conv2d_bwd_weight(gpu.to_device(big * np.float32(2.0 ** 60)), gpu.to_device(x), wt.shape, (1, 1), 1)[0].numpy()
+            assert rel_l2(gw.astype(np.float64) * rest, ref) <= TOL, q
+            dy[(q[0], q[1] + 26) + q[2:]] = value
+            dr = (dy / np.float32(value)).astype(np.float32) if value > 2.0 ** -120 else (dy > 0).astype(np.float32)
+            big = np.random.default_rng(i).standard_normal(x.shape).astype(np.float32)
+            _, col = oracle.conv2d_fwd(big, wt, None, (1, 1), 1)
+            _, ref, _ = oracle.conv2d_bwd(dr, x.shape, wt, col, (1, 1), 1, np.zeros_like(x), np.zeros_like(wt), np.zeros(k, np.float32))
+            gw = K.conv2d_bwd_weight(gpu.to_device(dy), gpu.to_device(big * np.float32(2.0 ** 60)), wt.shape, (1, 1), 1)[0].numpy()
+            assert rel_l2(gw.astype(np.float64) * rest, ref) <= TOL, q
+
+
 def test_a_partial_tile_that_never_comes_is_reported(gpu):
     K = gpu.kernels
     x, wt, b, _, _ = _data(1, 512, 7, 7, 512, 3, 3, 1, 1, 1, gpu)

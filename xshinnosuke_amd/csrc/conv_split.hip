@@ -10,8 +10,8 @@
 // channels and tap, against one per product pair on the fp32 pipe.
 //
 // What the split does not carry: infinities (inf - inf in a remainder), values within a bf16 rounding of the largest
-// float, and the last bits of values below 2^-110.  The first two make the sums that they touch non-finite, the third
-// are found by sums below 2^-100 (split3.h); such sums are formed again in float64 (form_again).
+// float, and the last bits of values below 2^-110.  The first two make the sums that they touch non-finite, the third are
+// looked for and given a NaN (split3.h); such sums are formed again in float64 (form_again).
 //
 // Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (128 per tile), 2 x 2 waves
 // of 32 rows x 64 pixels.  The reduction is a list of steps (phase, 16 input channels, tap).  A PHASE is a set of taps
@@ -87,10 +87,19 @@ struct SpParams {
 
 constexpr int AGENT = 16;                            // sc1: past the caches that are not coherent across XCDs
 
-// Eight filter values -> three vectors of eight bf16.  A value that does not split is left as it is in the second and third
-// piece, behind a first one that makes every sum it enters a NaN.
-__device__ __forceinline__ void split_filter8(const float (&v)[8], uint32x4 &p0, uint32x4 &p1, uint32x4 &p2) {
-    constexpr uint32_t NAN16 = 0x7fc0;
+// Eight filter values -> three vectors of eight bf16.
+__device__ __forceinline__ void split8(const float (&v)[8], uint32x4 &p0, uint32x4 &p1, uint32x4 &p2) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t a, b, c;
+        xsmi::split_pair3(v[2 * i], v[2 * i + 1], a, b, c);
+        p0[i] = a; p1[i] = b; p2[i] = c;
+    }
+}
+// The same where some value of the wavefront does not split: it is left as it is in the second and third piece, behind a first
+// one that makes every sum it enters a NaN.
+__device__ __forceinline__ void split8_any(const float (&v)[8], uint32x4 &p0, uint32x4 &p1, uint32x4 &p2) {
+    constexpr uint32_t NAN16 = xsmi::NAN_PAIR & 0xffffu;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const bool there_l = xsmi::splits(v[2 * i]), there_h = xsmi::splits(v[2 * i + 1]);
@@ -111,7 +120,7 @@ __device__ __forceinline__ double unsplit(uint32_t p0, uint32_t p1, uint32_t p2)
 // The sums of a segment that the split does not carry (split3.h) are formed again in float64, 16 x 16 blocks on the fp64 matrix
 // instructions (D: register v of lane l is row l / 16 + 4 v, column l % 16): a step's 16 channels are four products deep,
 // a lane has channels 4 (l / 16) .. + 3 of a row and of a pixel.  The filter comes out of its layout, whose pieces are the
-// value (split_filter8), so the filter itself is not read here either; a tap outside the input multiplies a zero, as the
+// value (split8_any), so the filter itself is not read here either; a tap outside the input multiplies a zero, as the
 // reference's padding does.  Every workgroup does this for its own steps.  All of 64 -> 64 at 56 x 56, N=8, not finite:
 // 93 us (one product at a time, by the workgroups that store the outputs: 2490), 256 -> 256 at 14 x 14: 110 (10100).
 struct SpSteps { int rt, s_first, n, f, grp, tap; };
@@ -277,14 +286,18 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
     };
     // the fetched values into an LDS image: a pair of channels at a time, then the three 16-byte pieces
     uint32x4 piece[3];
+    xsmi::SmallTest small;
     auto split_one = [&](auto jt, auto it) {
         constexpr int j = decltype(jt)::value, i = decltype(it)::value;
         uint32_t a, b, c;
+        if constexpr (i == 0) small = xsmi::SmallTest{};
+        small.add(pre[j][2 * i], pre[j][2 * i + 1]);
         xsmi::split_pair3(pre[j][2 * i], pre[j][2 * i + 1], a, b, c);
         piece[0][i] = a; piece[1][i] = b; piece[2][i] = c;
     };
     auto put = [&](auto j, int to) {
         unsigned char *dst = s_img + to + octet * SP_PLANE + (64 * (chunk0 + WC * j) + lane) * 16;
+        piece[0][0] = small.found() ? xsmi::NAN_PAIR : piece[0][0];
 #pragma unroll
         for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32x4 *>(dst + 2 * q * SP_PLANE) = piece[q];
     };
@@ -559,24 +572,41 @@ __global__ void __launch_bounds__(64) split_pack9_kernel(SpParams p, char *apk, 
     const uint32_t padded = (uint32_t)((rows + SP_ROWS - 1) / SP_ROWS * SP_ROWS);
     const uint32_t o = blockIdx.x / (padded / SP_ROWS), rt = blockIdx.x - o * (padded / SP_ROWS), row = rt * SP_ROWS + threadIdx.x;
     float v[9][8];
+    xsmi::SplitTest test;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const int ch = (int)o * 8 + e;
         const bool there = (int)row < rows && ch < p.CH;
         const float *src = p.w + (there ? (size_t)row * p.w_row + (size_t)ch * p.w_ch : 0);
 #pragma unroll
-        for (int t = 0; t < 9; ++t) v[t][e] = there ? src[t] : 0.f;
+        for (int t = 0; t < 9; ++t) { v[t][e] = there ? src[t] : 0.f; test.add(v[t][e]); }
     }
-#pragma unroll
-    for (int t = 0; t < 9; ++t) {
-        uint32x4 q0, q1, q2;
-        split_filter8(v[t], q0, q1, q2);
+    auto put = [&](int t, const uint32x4 &q0, const uint32x4 &q1, const uint32x4 &q2) {
         const SpTapPlace &w = p.tap[t];
         const uint32_t step = rt * w.iters + w.step + (o >> 1) * w.T;
         char *dst = apk + w.off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + threadIdx.x) * 16;
         *reinterpret_cast<uint32x4 *>(dst) = q0;
         *reinterpret_cast<uint32x4 *>(dst + 2 * SP_ROWS * 16) = q1;
         *reinterpret_cast<uint32x4 *>(dst + 4 * SP_ROWS * 16) = q2;
+    };
+    uint32x4 q0, q1, q2;
+    if (__builtin_amdgcn_ballot_w64(!test.all()) == 0) {
+#pragma unroll
+        for (int t = 0; t < 9; ++t) { split8(v[t], q0, q1, q2); put(t, q0, q1, q2); }
+        return;
+    }
+    // rolled up and from memory once more: with a choice for each value in the loop above the layout of 64 -> 64 took 9.7 us
+    // instead of 6.3, most of it for instructions fetched for the first time
+#pragma unroll 1
+    for (int t = 0; t < 9; ++t) {
+        float u[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int ch = (int)o * 8 + e;
+            u[e] = (int)row < rows && ch < p.CH ? p.w[(size_t)row * p.w_row + (size_t)ch * p.w_ch + t] : 0.f;
+        }
+        split8_any(u, q0, q1, q2);
+        put(t, q0, q1, q2);
     }
 }
 __global__ void __launch_bounds__(256) split_pack_kernel(SpParams p, char *apk) {
@@ -599,7 +629,7 @@ __global__ void __launch_bounds__(256) split_pack_kernel(SpParams p, char *apk) 
                 v[e] = (int)row < c.rows && ch < p.CH ? src[(size_t)row * p.w_row + (size_t)ch * p.w_ch] : 0.f;
             }
             uint32x4 q0, q1, q2;
-            split_filter8(v, q0, q1, q2);
+            split8_any(v, q0, q1, q2);
             const uint32_t step = (row / SP_ROWS) * c.iters + (uint32_t)ph.step0 + (o >> 1) * (uint32_t)ph.T + (uint32_t)tl;
             char *dst = apk + c.apk_off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + row % SP_ROWS) * 16;
             *reinterpret_cast<uint32x4 *>(dst) = q0;

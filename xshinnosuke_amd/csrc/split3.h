@@ -34,18 +34,43 @@ __device__ __forceinline__ void split_pair3(float a, float b, uint32_t &p0, uint
     p2 = __builtin_bit_cast(uint32_t, l);
 }
 
-// Whether a value has a split: finite, and not so large that its first piece would be an infinity.
-__device__ __forceinline__ bool splits(float v) { return __builtin_fabsf(v) < __builtin_bit_cast(float, 0x7f7f8000u); }
+// Which values have a split.  Infinities, NaN and values that round to a bf16 infinity make every sum they enter a NaN by
+// themselves.  Values below 2^-110 lose bits instead: the last piece ends at 2^-133, the smallest bf16 (3 x 3, 64 channels,
+// values of 2^-112: 1.6e-7 against 64 bits, of 2^-124: 5.7e-4, of 2^-136: everything; fp32 pipe 1.1e-7), whatever the other
+// operand is.  The kernels look for them while they split and put a NaN in the first piece.
+constexpr uint32_t NAN_PAIR = 0x7fc07fc0u;
+struct SmallTest {                                     // one and a half instructions a value
+    uint32_t smallest = 0xffffffffu;                   // twice a value's bits without the sign, less one: zero is the largest
+    __device__ __forceinline__ void add(float a, float b) {
+        const uint32_t x = __builtin_bit_cast(uint32_t, a) * 2u - 1u, y = __builtin_bit_cast(uint32_t, b) * 2u - 1u;
+        smallest = x < smallest ? x : smallest;
+        smallest = y < smallest ? y : smallest;
+    }
+    __device__ __forceinline__ bool found() const { return smallest < 2u * 0x08800000u - 1u; }
+};
+static_assert(__builtin_bit_cast(float, 0x08800000u) == 0x1p-110f, "the bits of 2^-110");
+__device__ __forceinline__ bool splits(float v) {
+    const float a = __builtin_fabsf(v);
+    return a < __builtin_bit_cast(float, 0x7f7f8000u) && (a >= 0x1p-110f || a == 0.f);
+}
+struct SplitTest {                                     // whether many values all split, three instructions a value
+    uint32_t smallest = 0xffffffffu, largest = 0;      // of twice the bits without the sign, the smallest less one
+    __device__ __forceinline__ void add(float v) {
+        const uint32_t x = __builtin_bit_cast(uint32_t, v) * 2u, m = x - 1u;
+        smallest = m < smallest ? m : smallest;
+        largest = x > largest ? x : largest;
+    }
+    __device__ __forceinline__ bool all() const { return smallest >= 2u * 0x08800000u - 1u && largest < 2u * 0x7f7f8000u; }
+};
 
-// Whether a sum of split products is the float32 one.  It is not if an operand had no split (the sum is then non-finite), and
-// may not be if an operand was below 2^-110, whose third piece is below the smallest normal number and is lost (3 x 3,
-// 64 channels, values of 2^-112: 1.6e-7 against 64 bits, of 2^-124: 5.7e-4; fp32 pipe 1.2e-7).  2^-100 is reached by such
-// operands only against a row of the other operand with a norm above 2^10.
+// Whether a sum of split products is as good as the float32 one.  It is not if an operand had no split (the sum is then a NaN
+// or infinite).  Sums below 2^-100 are formed again as well: their small products run out of bits, as the fp32 pipe's do
+// (2^-66 times 2^-66: 2.7e-5 against 64 bits, fp32 pipe 4.4e-5, formed again 3.8e-6).
 __device__ __forceinline__ bool carried(float v) {
     const float a = __builtin_fabsf(v);
     return a < __builtin_inff() && (a >= 0x1p-100f || a == 0.f);
 }
-// The same for many values at two and a half instructions each.
+// The same for many values, at two and a half instructions each.
 struct CarriedTest {
     float zero = 0.f;                                  // NaN from an infinity or a NaN on
     uint32_t smallest = 0xffffffffu;                   // twice a value's bits without the sign, less one: zero is the largest
