@@ -58,12 +58,6 @@ extern "C" {
 
 #define XSMI_CONV_DW_ASYNC 0x8u  /* xsmi_conv2d_bwd only: the weight gradient stays on the library's
                                     second stream when the call returns; see xsmi_conv2d_bwd_join */
-#define XSMI_CONV_FP32_PIPE 0x10u /* xsmi_conv2d_fwd only: stay on the kernels that multiply float32 on the
-                                    fp32 matrix instructions.  For forwards whose sign mask is kept: a
-                                    pre-activation within rounding of zero then falls on the side that
-                                    these kernels' sums put it on, whichever kernel is the fastest for
-                                    the geometry.  The workspace then holds that kernel's filter layout:
-                                    XSMI_CONV_WS_PACKED does not mix calls with and without this flag. */
 
 typedef struct xsmi_device_info {
     int device;
@@ -163,7 +157,7 @@ size_t xsmi_conv2d_workspace_bytes(int N, int C, int H, int W, int K, int R, int
                                    int sh, int sw, int pad);
 
 /* The same for one pass alone (0 forward, 1 backward-data, 2 backward-weight) with the
- * given flags (XSMI_CONV_BF16, XSMI_CONV_FP32_PIPE or 0): the size with which that pass's entry point picks
+ * given flags (XSMI_CONV_BF16 or 0): the size with which that pass's entry point picks
  * its fastest kernel.  For callers that keep one workspace per filter and pass (a filter
  * layout made ahead, XSMI_CONV_WS_PACKED): a ResNet-18 training step at N=32 then holds
  * tens of megabytes of layouts instead of a full-size workspace per filter and pass.
@@ -278,9 +272,8 @@ int xsmi_conv2d_bwd_join(void);
 /* Lay filters out ahead of time.  Every conv call first rewrites w into the layout its kernel reads
  * (a few microseconds of a tiny launch in front of each of the ~40 convolution passes of a ResNet-18
  * step; the reference has no counterpart, its im2col GEMM reads w as it is, xs/nn/functional.py:428).
- * This entry point runs only that step, for every job: pass 0 (xsmi_conv2d_fwd), 1
- * (xsmi_conv2d_bwd_data / the data gradient of xsmi_conv2d_bwd) or 3 (xsmi_conv2d_fwd with
- * XSMI_CONV_FP32_PIPE) of the given fp32 geometry, all on the
+ * This entry point runs only that step, for every job: pass 0 (xsmi_conv2d_fwd) or 1
+ * (xsmi_conv2d_bwd_data / the data gradient of xsmi_conv2d_bwd) of the given fp32 geometry, all on the
  * library's second stream: ordered after everything enqueued so far, beside whatever the main stream is
  * given next.  job.packed is set to 1 when the job's workspace now holds a layout that the later call
  * accepts through XSMI_CONV_WS_PACKED (same geometry, same workspace size, w unchanged in between), and

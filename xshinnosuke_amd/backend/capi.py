@@ -120,7 +120,6 @@ CONV_RELU = 0x1
 CONV_BF16 = 0x2
 CONV_WS_PACKED = 0x4
 CONV_DW_ASYNC = 0x8
-CONV_FP32_PIPE = 0x10
 NOALLOC_SCRATCH_BYTES = 16 << 20      # XSMI_NOALLOC_SCRATCH_BYTES of the header
 
 

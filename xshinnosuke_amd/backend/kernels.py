@@ -11,7 +11,7 @@ import weakref
 import numpy as np
 
 from . import capi
-from .capi import lib, CONV_RELU, CONV_BF16, CONV_WS_PACKED, CONV_DW_ASYNC, CONV_FP32_PIPE
+from .capi import lib, CONV_RELU, CONV_BF16, CONV_WS_PACKED, CONV_DW_ASYNC
 from . import array as _array
 from .array import DeviceArray, Workspace, empty
 
@@ -45,12 +45,11 @@ def _need(dims):
 
 
 def _need_pass(dims, pass_):
-    """Workspace of one fp32 pass alone (0 forward, 1 backward-data, 3 forward with ``fp32_pipe``, as in
-    xsmi_conv2d_pack): what a filter's layout workspace holds."""
+    """Workspace of one fp32 pass alone (0 forward, 1 backward-data): what a filter's layout workspace holds."""
     key = (pass_,) + tuple(dims)
     need = _NEED.get(key)
     if need is None:
-        need = _NEED[key] = lib.raw("xsmi_conv2d_pass_workspace_bytes")(*dims, pass_ % 3, CONV_FP32_PIPE if pass_ == 3 else 0)
+        need = _NEED[key] = lib.raw("xsmi_conv2d_pass_workspace_bytes")(*dims, pass_, 0)
     return need
 
 
@@ -189,7 +188,7 @@ def _f32(a, what):
 
 
 def conv2d_fwd(x, w, bias=None, stride=(1, 1), pad=0, relu=False, out=None, neg_mask=None, bf16=False, packed=False,
-               workspace=None, channels_last=False, keep_layout=False, fp32_pipe=False):
+               workspace=None, channels_last=False, keep_layout=False):
     """``keep_layout=True`` (training steps; fp32, the shared workspace): the call works in a workspace that belongs
     to this filter, pass and geometry, whose layout ``refresh_layouts`` renews after each update of the filter.
     ``packed=True`` promises that the previous conv call on this workspace was this same forward with the same
@@ -197,9 +196,7 @@ def conv2d_fwd(x, w, bias=None, stride=(1, 1), pad=0, relu=False, out=None, neg_
     ``workspace``: a ``Workspace`` of the caller's instead of the shared one (a layer that keeps its packed filter).
     ``channels_last=True`` (with ``bf16``, no mask): the result may be left in channels-last bf16 form, and an input
     that lives in that form is read as it is (``DeviceArray.channels_last``); results equal the plain bf16 path's up
-    to the bf16 rounding of the stored activations.
-    ``fp32_pipe=True`` (fp32): the kernels that multiply on the fp32 matrix instructions, whichever is the fastest
-    (XSMI_CONV_FP32_PIPE); a ``packed`` workspace is then one that such a call has left."""
+    to the bf16 rounding of the stored activations."""
     _f32(x, "x"); _f32(w, "w")
     dims = _dims(x.shape, w.shape, stride, pad)
     n, c, h, wd, k, r, s = dims[:7]
@@ -218,13 +215,12 @@ def conv2d_fwd(x, w, bias=None, stride=(1, 1), pad=0, relu=False, out=None, neg_
         raise ValueError("conv2d: neg_mask must be uint8 with one byte per output element")
     layout = None
     if keep_layout and _PREPACK and not bf16 and not packed and workspace is None:
-        layout, packed = _layout_for(w, 3 if fp32_pipe else 0, dims)
+        layout, packed = _layout_for(w, 0, dims)
         if layout is not None:
             workspace = layout.ws
-    flags = ((CONV_RELU if relu else 0) | (CONV_BF16 if bf16 else 0) | (CONV_WS_PACKED if packed else 0)
-             | (CONV_FP32_PIPE if fp32_pipe else 0))
+    flags = (CONV_RELU if relu else 0) | (CONV_BF16 if bf16 else 0) | (CONV_WS_PACKED if packed else 0)
     if layout is not None:
-        ws, ws_bytes = workspace.get(_need_pass(dims, 3 if fp32_pipe else 0))
+        ws, ws_bytes = workspace.get(_need_pass(dims, 0))
     else:
         ws, ws_bytes = _workspace(dims) if workspace is None else workspace.get(_need(dims))
     if channels_last and bf16 and neg_mask is None:
@@ -236,7 +232,7 @@ def conv2d_fwd(x, w, bias=None, stride=(1, 1), pad=0, relu=False, out=None, neg_
             lib.call("xsmi_conv2d_fwd_cl", None if xcl is not None else x.ptr, xcl.buf.ptr if xcl is not None else None,
                      xcl.border if xcl is not None else 0, w.ptr, bias.ptr if bias is not None else None,
                      None if ycl is not None else out.ptr, ycl.buf.ptr if ycl is not None else None, 1, *dims,
-                     flags & ~(CONV_BF16 | CONV_FP32_PIPE), ws, ws_bytes)
+                     flags & ~CONV_BF16, ws, ws_bytes)
             return out
     out._overwritten()
     # a filter whose layout is in place is not read: its address goes along without counting as handed out

@@ -338,7 +338,7 @@ static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh,
     if (!bf16 && xsmi::stem_fwd_ok(N, C, H, W, K, R, S, sh, sw, pad) &&
         workspace_bytes >= xsmi::stem_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad))
         return FwdPath::FirstLayer;
-    if (!bf16 && !(flags & (XSMI_CONV_WS_ONLY | XSMI_CONV_FP32_PIPE)) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
+    if (!bf16 && !(flags & XSMI_CONV_WS_ONLY) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
         const size_t need = xsmi::split_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
         if (need && workspace_bytes >= need) return FwdPath::Split;
     }
@@ -372,8 +372,7 @@ int xsmi_conv2d_fwd(const float *x, const float *w, const float *bias, float *y,
     int rc = check_conv("xsmi_conv2d_fwd", N, C, H, W, K, R, S, sh, sw, pad, &g);
     if (rc) return rc;
     XSMI_CHECK_ARG(x && w && y, "xsmi_conv2d_fwd: null tensor pointer");
-    XSMI_CHECK_ARG((flags & ~(XSMI_CONV_RELU | XSMI_CONV_BF16 | XSMI_CONV_WS_PACKED | XSMI_CONV_FP32_PIPE | XSMI_CONV_PACK_ONLY |
-                              XSMI_CONV_WS_ONLY)) == 0,
+    XSMI_CHECK_ARG((flags & ~(XSMI_CONV_RELU | XSMI_CONV_BF16 | XSMI_CONV_WS_PACKED | XSMI_CONV_PACK_ONLY | XSMI_CONV_WS_ONLY)) == 0,
                    "xsmi_conv2d_fwd: unknown flags 0x%x", flags);
     const int J = C * R * S;
     const size_t need = xsmi::conv_fwd_ws_bytes(C, K, R, S);
@@ -564,16 +563,15 @@ int xsmi_conv2d_pack(int count, xsmi_pack_job_t *jobs) {
         ConvGeom g;
         rc = check_conv("xsmi_conv2d_pack", j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw, j.pad, &g);
         if (rc) break;
-        if (!j.w || (j.pass != 0 && j.pass != 1 && j.pass != 3)) {
+        if (!j.w || (j.pass != 0 && j.pass != 1)) {
             xsmi::set_error("xsmi_conv2d_pack: job %d has a null filter or an unknown pass %d", i, j.pass);
             rc = XSMI_ERR_INVALID;
             break;
         }
         // the first-layer kernels lay their filter out inside the launch that pads the input, the generic kernels
         // rebuild a small table per call: nothing to do ahead of time for either
-        const unsigned pipe = j.pass == 3 ? XSMI_CONV_FP32_PIPE : 0u;
-        if (j.pass != 1) {
-            const FwdPath path = fwd_path(j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw, j.pad, g.OH, g.OW, pipe, j.workspace_bytes);
+        if (j.pass == 0) {
+            const FwdPath path = fwd_path(j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw, j.pad, g.OH, g.OW, 0, j.workspace_bytes);
             if (path != FwdPath::Split && path != FwdPath::EvenSplit && path != FwdPath::Tap) continue;
         } else if (bwd_data_path(j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw, j.pad, g.OH, g.OW, 0, j.workspace_bytes) == BwdDataPath::Generic) {
             continue;
@@ -590,8 +588,8 @@ int xsmi_conv2d_pack(int count, xsmi_pack_job_t *jobs) {
         rc = xsmi::side_lane(lanes++ % nlanes);
         if (rc) break;
         float *unused = const_cast<float *>(j.w);        // activations are not touched by a layout-only call
-        rc = j.pass != 1 ? xsmi_conv2d_fwd(unused, j.w, nullptr, unused, nullptr, j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw,
-                                           j.pad, XSMI_CONV_PACK_ONLY | pipe, j.workspace, j.workspace_bytes)
+        rc = j.pass == 0 ? xsmi_conv2d_fwd(unused, j.w, nullptr, unused, nullptr, j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw,
+                                           j.pad, XSMI_CONV_PACK_ONLY, j.workspace, j.workspace_bytes)
                          : xsmi_conv2d_bwd_data(unused, j.w, unused, j.N, j.C, j.H, j.W, j.K, j.R, j.S, j.sh, j.sw, j.pad, 0.f,
                                                 XSMI_CONV_PACK_ONLY, j.workspace, j.workspace_bytes);
         if (rc == XSMI_OK) j.packed = 1;

@@ -90,23 +90,17 @@ def conv2d(inputs, weight, bias=None, stride=(1, 1), padding=0, out=None, activa
     cl = bf16 and not track and on_device
     # a tracked forward on a device-resident filter is a training step's: the filter's layout is kept between calls
     keep = track and w_dev is weight.eval
-    # The sign mask decides which gradients flow.  Pre-activations within rounding of zero fall on one side or the other with the
-    # order of the sums (24 -> 40, 5 x 5 at 45 x 61, N=7: one of 769 thousand in every fifteenth pass), and each that changes
-    # sides changes a whole footprint of the gradients: the mask is that of the fp32 matrix instructions' sums, whichever
-    # kernel would be the fastest (that layer, forward with its layout launch: 34 -> 61 us).
-    pipe = neg_mask is not None and not bf16
     if out is None:
         y_dev = K.conv2d_fwd(x_dev, w_dev, b_dev, stride, padding, relu=activation == 'relu', neg_mask=neg_mask, bf16=bf16,
-                             channels_last=cl, keep_layout=keep, fp32_pipe=pipe)
+                             channels_last=cl, keep_layout=keep)
         out = Tensor(y_dev if on_device else y_dev.numpy().astype(x.dtype, copy=False))
     else:
         dst = out.eval
         if is_device(dst):
             K.conv2d_fwd(x_dev, w_dev, b_dev, stride, padding, relu=activation == 'relu', out=dst, neg_mask=neg_mask, bf16=bf16,
-                         channels_last=cl, keep_layout=keep, fp32_pipe=pipe)
+                         channels_last=cl, keep_layout=keep)
         else:
-            y_dev = K.conv2d_fwd(x_dev, w_dev, b_dev, stride, padding, relu=activation == 'relu', neg_mask=neg_mask, bf16=bf16,
-                                 fp32_pipe=pipe)
+            y_dev = K.conv2d_fwd(x_dev, w_dev, b_dev, stride, padding, relu=activation == 'relu', neg_mask=neg_mask, bf16=bf16)
             out.eval = y_dev.numpy()              # cast to the buffer's dtype on store
     out.requires_grad = requires_grad
     _wire(out, inputs, weight, bias)
