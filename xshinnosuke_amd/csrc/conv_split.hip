@@ -113,8 +113,8 @@ __device__ __forceinline__ void split8_any(const float (&v)[8], uint32x4 &p0, ui
 }
 // The value again, from the low halves of its three pieces.
 __device__ __forceinline__ double unsplit(uint32_t p0, uint32_t p1, uint32_t p2) {
-    auto wide = [](uint32_t bits) { return (double)__builtin_bit_cast(float, bits); };
-    return (p0 & 0x7fffu) > 0x7f80u ? wide(p1 << 16 | (p2 & 0xffffu)) : wide(p0 << 16) + wide(p1 << 16) + wide(p2 << 16);
+    auto wide = [](uint32_t bits) { return __builtin_bit_cast(float, bits); };   // (the sums are exact)
+    return (double)((p0 & 0x7fffu) > 0x7f80u ? wide(p1 << 16 | (p2 & 0xffffu)) : (wide(p0 << 16) + wide(p1 << 16)) + wide(p2 << 16));
 }
 
 // The sums of a segment that the split does not carry (split3.h) are formed again in float64, 16 x 16 blocks on the fp64 matrix
@@ -183,8 +183,90 @@ __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const
     }
 }
 
+// Where a sign mask is kept, the sign of a pre-activation decides which gradients flow, and one within rounding of zero falls on
+// one side or the other with the order of the sums: it moves a whole footprint of the gradients (24 -> 40, 5 x 5 at 45 x 61,
+// N=7: 2e-4 to 3e-3 of their norm; of 200 passes of that layer 2 had such a sign on the other side than 64 bits, 12 on the fp32
+// kernels).  Pre-activations within 2^-21 of the largest sum around them (the lane's 16 rows by 16 pixels; no sum of layers of
+// 64 to 12,544 terms was further than 2^-21.6 from 64 bits) are therefore formed again in float64, and taken from there where
+// that changes the sign (none of 400 passes).  About one in a million is that small; it costs its wavefront one sum over all
+// its lanes (that layer 28.6 -> 29.3 us without one, 35.6 with one; 512 -> 512 at 7 x 7, N=32: 51.0 -> 52.2, 63.7).  A block
+// that has more than four of them is left as it is: its largest sum says nothing about the others.
+constexpr int SP_DECIDED = 4;
+template <int BATCH>
+__device__ __forceinline__ void decide_signs(floatx16 &r, const floatx16 &sum, const SpParams &p, const SpClass &c, const float *bias,
+                                             int rt, int row0, int m0, int lane, __amdgpu_buffer_rsrc_t rin, __amdgpu_buffer_rsrc_t rapk) {
+    float largest = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) largest = __builtin_fmaxf(largest, __builtin_fabsf(sum[v]));
+    // ... of the lane's 16 rows, and of its row of 16 lanes (rotated by 1, 2, 4 and 8)
+    auto other = [&](auto ctrl) {
+        const int bits = __builtin_bit_cast(int, largest);
+        largest = __builtin_fmaxf(largest, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(bits, bits, decltype(ctrl)::value, 15, 15, false)));
+    };
+    other(IC<0x121>{}); other(IC<0x122>{}); other(IC<0x124>{}); other(IC<0x128>{});
+    const float bound = largest * 0x1p-21f;
+    uint32_t near = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) near |= __builtin_fabsf(r[v]) <= bound && sum[v] != 0.f ? 1u << v : 0u;
+    near = m0 + (lane & 31) < c.M ? near : 0u;
+    uint64_t lanes = __builtin_amdgcn_ballot_w64(near != 0);
+    if (lanes == 0) return;
+    int count = __builtin_popcount(near);
+#pragma unroll
+    for (int i = 1; i < 64; i *= 2) count += __shfl_xor(count, i);
+    if (count > SP_DECIDED) return;
+    const int ch16 = lane & 15, a_lane = (ch16 >> 3) * SP_ROWS * 16 + (ch16 & 7) * 2;
+    for (; lanes != 0; lanes = __builtin_amdgcn_ballot_w64(near != 0)) {
+        const int from = __builtin_ctzll(lanes);
+        const int v = __builtin_ctz(__builtin_amdgcn_readlane((int)near, from));
+        const int row = row0 + 4 * (from >> 5) + 8 * (v >> 2) + (v & 3), m = m0 + (from & 31);
+        const int q = (int)xsmi::fdiv((uint32_t)m, c.dOX), n = (int)xsmi::fdiv((uint32_t)q, c.dOY);
+        const int oy = q - n * c.OY, ox = m - q * c.OX, image = n * p.in_n;
+        // sixteen lanes for the channels of a step, four steps at a time, BATCH of those in flight
+        double total = 0.0;
+        uint32_t block = c.apk_off + (uint32_t)rt * c.iters * (uint32_t)SP_BLOCK + (uint32_t)(a_lane + row * 16);
+#pragma unroll 1
+        for (int f = c.phase0; f < c.phase0 + c.nphase; ++f) {
+            const SpPhase &ph = p.ph[f];
+            const uint32_t T = (uint32_t)ph.T, Tx = (uint32_t)ph.Tx, steps = T * (uint32_t)p.groups;
+            const uint32_t on = 4 / T, by = 4 - on * T, inv = 65536u / Tx + 1;      // x inv >> 16 = x / Tx, at most 961 taps of 31 across
+            uint32_t grp = ((uint32_t)lane >> 4) / T, tap = ((uint32_t)lane >> 4) - grp * T;
+#pragma unroll 1
+            for (uint32_t base = (uint32_t)lane >> 4; base < steps; base += 4 * BATCH) {
+                uint32_t piece[BATCH][3];
+                int bits[BATCH];
+#pragma unroll
+                for (int k = 0; k < BATCH; ++k) {
+                    const uint32_t step = base + 4u * k, ta = tap * inv >> 16, tb = tap - ta * Tx;
+                    const int ch = (int)grp * 16 + ch16, iy = (oy + (int)ta) * c.sy + ph.iy0, ix = (ox + (int)tb) * c.sx + ph.ix0;
+                    const bool in = step < steps && ch < p.CH && iy >= 0 && iy < p.IH && ix >= 0 && ix < p.IW;
+                    const uint32_t place = ((uint32_t)image + (uint32_t)ch * (uint32_t)p.plane + (uint32_t)(iy * p.IW + ix)) * 4u;
+                    bits[k] = __builtin_amdgcn_raw_buffer_load_b32(rin, in ? (int)place : (int)0x80000000u, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                        piece[k][i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
+                            rapk, (int)(step < steps ? block + step * (uint32_t)SP_BLOCK + (uint32_t)(i * 2 * SP_ROWS * 16) : 0x80000000u), 0, 0);
+                    grp += on; tap += by;
+                    if (tap >= T) { tap -= T; ++grp; }
+                }
+#pragma unroll
+                for (int k = 0; k < BATCH; ++k)
+                    total += unsplit(piece[k][0], piece[k][1], piece[k][2]) * (double)__builtin_bit_cast(float, bits[k]);
+            }
+            block += steps * (uint32_t)SP_BLOCK;
+        }
+#pragma unroll
+        for (int i = 1; i < 64; i *= 2) total += __shfl_xor(total, i);
+        const float again = (float)(total + (bias ? (double)bias[row] : 0.0));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) r[i] = i == v && lane == from && (again < 0.f) != (r[i] < 0.f) ? again : r[i];
+        if (lane == from) near &= near - 1u;
+    }
+}
+
 // WC waves across the tile's pixels (2: 128 pixels and 256 threads, two workgroups per CU; 4: 256 and 512, one)
-template <int WC>
+// SIGNS: a sign mask is kept (a kernel of its own: the others would pay for the registers of decide_signs, half a microsecond)
+template <int WC, bool SIGNS>
 __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
     constexpr int SP_PIX = 64 * WC, THREADS = 128 * WC, NJ = sp_slots_of(WC) / 64 / WC;
     constexpr int SP_PLANE = sp_slots_of(WC) * 16;       // bytes of one (piece, octet) plane
@@ -555,7 +637,16 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         if (head) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                xsmi::store_block_32x32(acc[j], c, p.out, p.out_bytes, p.mask, p.bias ? s_bias[bias_buf] : nullptr, p.relu, p.accumulate,
+                const float *bias = p.bias ? s_bias[bias_buf] : nullptr;
+                if constexpr (SIGNS) {
+                    floatx16 r = acc[j];
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) r[v] += bias ? bias[wr * 32 + 4 * h + 8 * (v >> 2) + (v & 3)] : 0.f;
+                    decide_signs<WC == 4 ? 8 : 4>(r, acc[j], p, c, bias, rt, wr * 32, m0 + wc * 64 + 32 * j, lane, rin, rapk);
+                    acc[j] = r;
+                    bias = nullptr;
+                }
+                xsmi::store_block_32x32(acc[j], c, p.out, p.out_bytes, SIGNS ? p.mask : nullptr, bias, p.relu, p.accumulate,
                                         rt * SP_ROWS, SP_ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
             }
         }
@@ -756,12 +847,14 @@ int sp_run(SpParams &p, int opts, void *workspace) {
         XSMI_LAUNCH_CHECK("split_pack_kernel");
     }
     if (opts & 4) return XSMI_OK;
-    static int resident[2] = {0, 0};
-    int &res = resident[p.wc == 4];
+    static int resident[4] = {0, 0, 0, 0};
+    const int which = (p.wc == 4 ? 1 : 0) + (p.mask ? 2 : 0), threads = 128 * p.wc;
+    void (*const kernels[4])(SpParams) = {split_conv_kernel<2, false>, split_conv_kernel<4, false>, split_conv_kernel<2, true>,
+                                          split_conv_kernel<4, true>};
+    int &res = resident[which];
     if (res == 0) {
         int per_cu = 0;
-        const hipError_t e = p.wc == 4 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, split_conv_kernel<4>, 512, 0)
-                                       : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, split_conv_kernel<2>, 256, 0);
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernels[which], threads, 0);
         if (e != hipSuccess || per_cu < 1) per_cu = 1;
         const int all = per_cu * xsmi::cu_count(), cap = sp_max_grid(p.wc);
         res = (all > cap ? cap : all < 8 ? 8 : all) & ~7;
@@ -783,8 +876,7 @@ int sp_run(SpParams &p, int opts, void *workspace) {
     const long spin = xsmi::option(xsmi::OPT_SK_SPIN_LIMIT);
     p.spin_limit = spin < 0 ? 0u : spin > 0x7fffffffL ? 0x7fffffffu : (uint32_t)spin;
     xsmi::prof_begin();
-    if (p.wc == 4) hipLaunchKernelGGL(split_conv_kernel<4>, dim3(grid), dim3(512), 0, st, p);
-    else hipLaunchKernelGGL(split_conv_kernel<2>, dim3(grid), dim3(256), 0, st, p);
+    hipLaunchKernelGGL(kernels[which], dim3(grid), dim3(threads), 0, st, p);
     xsmi::prof_end();
     XSMI_LAUNCH_CHECK("split_conv_kernel");
     return XSMI_OK;
