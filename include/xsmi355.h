@@ -162,7 +162,8 @@ size_t xsmi_conv2d_workspace_bytes(int N, int C, int H, int W, int K, int R, int
  * layout made ahead, XSMI_CONV_WS_PACKED): a ResNet-18 training step at N=32 then holds
  * tens of megabytes of layouts instead of a full-size workspace per filter and pass.
  * No counterpart in the reference (its conv2d allocates the im2col matrix per call,
- * xs/utils/common.py:35-46).  Returns 0 for a bad geometry or pass. */
+ * xs/utils/common.py:35-46).  Returns 0 for a bad geometry or pass and for tensors of 2^29
+ * elements or more, which every pass refuses. */
 size_t xsmi_conv2d_pass_workspace_bytes(int N, int C, int H, int W, int K, int R, int S,
                                         int sh, int sw, int pad, int pass, unsigned flags);
 

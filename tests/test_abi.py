@@ -43,6 +43,18 @@ def test_workspace_query_needs_no_device():
     assert f(1, 1, 2, 2, 1, 5, 5, 1, 1, 0) == 0           # filter larger than the input -> 0
 
 
+def test_workspace_queries_of_tensors_that_are_too_large_give_zero():
+    """Tensors of 2^29 elements or more are refused by every pass; their counts of pixels and stages do not fit 32 bits."""
+    whole = libmod.lib.raw("xsmi_conv2d_workspace_bytes")
+    one = libmod.lib.raw("xsmi_conv2d_pass_workspace_bytes")
+    for dims in ((65536, 16, 256, 256, 16, 3, 3, 1, 1, 1),            # 2^32 output pixels
+                 (65536, 16, 256, 256, 16, 5, 5, 1, 1, 2), (1 << 20, 16, 1024, 1024, 16, 3, 3, 1, 1, 1),
+                 (1, 1 << 15, 8, 8, 1 << 15, 3, 3, 1, 1, 1),          # a filter that is too large
+                 (8192, 16, 64, 64, 16, 3, 3, 1, 1, 1)):              # 2^29 elements
+        assert whole(*dims) == 0 and all(one(*dims, p, f) == 0 for p in range(3) for f in (0, libmod.CONV_BF16)), dims
+    assert whole(8191, 16, 64, 64, 16, 3, 3, 1, 1, 1) > 0
+
+
 def test_per_pass_workspace_queries_need_no_device():
     """The size of one pass alone never exceeds the size for all passes, the maximum over passes and flags is that
     size, a pass outside 0..2 and a bad geometry give 0; what the library holds itself is a constant."""

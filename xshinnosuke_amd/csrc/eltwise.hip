@@ -70,6 +70,9 @@ size_t xsmi_conv2d_pass_workspace_bytes(int N, int C, int H, int W, int K, int R
     if (N <= 0 || C <= 0 || H <= 0 || W <= 0 || K <= 0 || R <= 0 || S <= 0 || sh <= 0 || sw <= 0 || pad < 0) return 0;
     if (H + 2 * pad < R || W + 2 * pad < S) return 0;
     const int OH = (H + 2 * pad - R) / sh + 1, OW = (W + 2 * pad - S) / sw + 1;
+    // what the passes refuse; their plans below count in 32 bits
+    const double lim = 536870912.0;
+    if ((double)N * C * H * W >= lim || (double)N * K * OH * OW >= lim || (double)K * C * R * S >= lim) return 0;
     const bool bf16 = (flags & XSMI_CONV_BF16) != 0;
     auto larger = [](size_t a, size_t b) { return a > b ? a : b; };
     size_t m = 0;
