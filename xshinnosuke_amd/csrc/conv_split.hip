@@ -739,11 +739,11 @@ long sp_slots(int pix, int OY, int OX, int ty, int tx) {
 
 // Adds a class whose taps are r = r0 + rs a (a < R), s = s0 + ss b (b < S), reading input place (y sy + iy(r), ...), split
 // into phases of sub-lattice taps; false if the tables or the LDS image do not hold it.
-struct SpTaps { int R, S, r0, rs, s0, ss, iy0, ix0, dy, dx; };   // tap (a, b) reads (y sy + iy0 + dy a, x sx + ix0 + dx b)
+struct SpTaps { int R, S, r0, rs, s0, ss, iy0, ix0; };            // tap (a, b) reads (y sy + iy0 + a, x sx + ix0 + b)
 bool sp_add_class(SpParams &p, int &nph, uint32_t &steps_bytes, const SpTaps &k, int M, int rows, int OY, int OX, int sy, int sx) {
     if (p.ncls == SP_MAX_CLASSES || k.R < 1 || k.S < 1) return false;
     SpClass &c = p.cls[p.ncls];
-    const int ny = (sy < k.R && k.dy == 1) ? sy : k.dy == 1 ? k.R : 1, nx = (sx < k.S && k.dx == 1) ? sx : k.dx == 1 ? k.S : 1;
+    const int ny = sy < k.R ? sy : k.R, nx = sx < k.S ? sx : k.S;
     // all rows of a sub-lattice in one image when it fits, otherwise one filter row at a time
     const int ty_max = (k.R + ny - 1) / ny, tx_max = (k.S + nx - 1) / nx;
     const int pix = 64 * p.wc;
@@ -761,7 +761,7 @@ bool sp_add_class(SpParams &p, int &nph, uint32_t &steps_bytes, const SpTaps &k,
         for (int j = 0; j < nx; ++j) {
             SpPhase &f = p.ph[nph++];
             const int na = by_row ? 1 : (k.R - i + ny - 1) / ny, nb = (k.S - j + nx - 1) / nx;
-            f.iy0 = k.iy0 + k.dy * i; f.ix0 = k.ix0 + k.dx * j;
+            f.iy0 = k.iy0 + i; f.ix0 = k.ix0 + j;
             f.Tx = nb; f.T = na * nb;
             f.tap0 = tap; f.step0 = step;
             f.r0 = k.r0 + k.rs * i; f.rs = k.rs * ny; f.s0 = k.s0 + k.ss * j; f.ss = k.ss * nx;
@@ -792,7 +792,7 @@ bool sp_plan_fwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, i
     p.N = N; p.CH = C; p.groups = xsmi::ceil_div(C, 16); p.IH = H; p.IW = W; p.in_n = C * H * W; p.plane = H * W;
     p.w_row = C * R * S; p.w_ch = R * S; p.FS = S;
     int nph = 0;
-    const SpTaps k = {R, S, 0, 1, 0, 1, -pad, -pad, 1, 1};
+    const SpTaps k = {R, S, 0, 1, 0, 1, -pad, -pad};
     if (!sp_add_class(p, nph, p.apk_bytes, k, N * OH * OW, K, OH, OW, sh, sw)) return false;
     SpClass &c = p.cls[0];
     c.os_n = (long long)K * OH * OW; c.os_k = (long long)OH * OW; c.o_base = 0; c.os_y = OW; c.os_x = 1;
@@ -812,7 +812,7 @@ bool sp_plan_bwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, i
         for (int pw = 0; pw < sw && pw < W; ++pw) {
             const int s0 = (pw + pad) % sw, U = s0 < S ? xsmi::ceil_div(S - s0, sw) : 0, cx = (pw + pad - s0) / sw;
             const int OYc = xsmi::ceil_div(H - ph, sh), OXc = xsmi::ceil_div(W - pw, sw);
-            const SpTaps k = {T, U, r0 + sh * (T - 1), -sh, s0 + sw * (U - 1), -sw, cy - (T - 1), cx - (U - 1), 1, 1};
+            const SpTaps k = {T, U, r0 + sh * (T - 1), -sh, s0 + sw * (U - 1), -sw, cy - (T - 1), cx - (U - 1)};
             if (!sp_add_class(p, nph, p.apk_bytes, k, N * OYc * OXc, C, OYc, OXc, 1, 1)) return false;
             SpClass &c = p.cls[p.ncls - 1];
             c.os_n = (long long)C * H * W; c.os_k = (long long)H * W; c.o_base = (long long)ph * W + pw;
