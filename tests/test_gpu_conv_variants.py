@@ -120,3 +120,29 @@ def test_a_wait_that_runs_out_is_reported_and_the_library_recovers(gpu):
 def test_unknown_option_is_refused(gpu):
     with pytest.raises(ValueError, match="no option named"):
         gpu.set_option("no_such_switch", 1)
+
+
+@pytest.mark.parametrize("geom", GEOMETRIES)
+def test_fp32_kernels_by_their_own_rule(gpu, geom):
+    """Without the split-operand kernels: the even split where it pays, the form of its loads where that pays, and the
+    weight gradient's own forms.  A workspace too small for a split kernel's filter layout selects the same ones."""
+    from xshinnosuke_amd.backend import capi
+    n, c, h, w, k, r, s, sh, sw, pad = geom
+    K = gpu.kernels
+    rng = np.random.default_rng(k + h)
+    x, wt = rng.standard_normal((n, c, h, w)).astype(np.float32), he_normal(rng, (k, c, r, s))
+    dy = rng.standard_normal((n, k) + tuple(K.conv_out_hw(h, w, r, s, (sh, sw), pad))).astype(np.float32)
+    dx_, dw_, ddy = gpu.to_device(x), gpu.to_device(wt), gpu.to_device(dy)
+    with options(gpu, conv_split=0, tap_sk=1, sk_wide=2):
+        _run(gpu, *geom, seed=9)
+        y = K.conv2d_fwd(dx_, dw_, None, (sh, sw), pad).numpy()
+        size = capi.lib.raw("xsmi_conv2d_pass_workspace_bytes")(*geom, 0, 0)
+        _, col = oracle.conv2d_fwd(x, wt, None, (sh, sw), pad)
+        _, dw_ref, _ = oracle.conv2d_bwd(dy, x.shape, wt, col, (sh, sw), pad, np.zeros_like(x), np.zeros_like(wt), np.zeros(k, np.float32))
+        assert rel_l2(K.conv2d_bwd_weight(ddy, dx_, wt.shape, (sh, sw), pad)[0].numpy(), dw_ref) <= TOL
+    split = capi.lib.raw("xsmi_conv2d_pass_workspace_bytes")(*geom, 0, 0)
+    assert split >= size
+    if split > size:                                     # 6 bytes a value against 4
+        ws, out = gpu.empty((size // 4,)), gpu.empty(y.shape)
+        capi.lib.call("xsmi_conv2d_fwd", dx_.ptr, dw_.ptr, None, out.ptr, None, *geom, 0, ws.ptr, size)
+        assert out.numpy().tobytes() == y.tobytes()
