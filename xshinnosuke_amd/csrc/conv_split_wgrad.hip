@@ -15,7 +15,10 @@
 //
 // Eight waves: 2 x 2 of 32 filters x 32 channels, twice; the second four take the stage's other two octets, so each wave
 // multiplies one k-step of 16 pixels and nine taps (54 MFMAs) between two barriers, while its share of the next stage is
-// split behind the MFMAs and the one after it is in flight.  The two halves are added through the LDS at the end.
+// split behind the MFMAs and the one after it is in flight.  The second half multiplies with -dy (the rows of a stage that it
+// owns are split as their negatives) and is subtracted through the LDS at the end: the bf16 MFMA drops what the small
+// products have below the accumulator's last bits, always downwards, and what one half loses by that the other then gains
+// (24 -> 32 at 112 x 112, N=32, against 64 bits: 1.0e-6, nine tenths of it one sign, -> 4.3e-7; fp32 pipe 7.1e-7).
 // Workgroups take equal runs of stages; each writes its nine 64 x 64 partial products, and one launch adds them in
 // ascending order in float64.  A workgroup whose sums the split does not carry (split3.h) forms them again in float64.
 #include "split3.h"
@@ -144,22 +147,23 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)p.x, 0, (int)p.x_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)p.dy, 0, (int)p.dy_bytes, 0x00020000);
 
-    // ---- staging: of the stage's octets, input first, this thread takes number t and number t + 512 ----
+    // ---- staging: of the stage's octets of the input this thread takes number t, and of dy, those of the first half's rows of
+    // all filters first, likewise.  A thread past the last octet (8 and 6, or 6 and 8, for each of 64) stages zeros beside them.
     const int nx = (p.RB + 2) * p.CB, ny = p.RB * (p.CB + 1);          // per channel and per filter
-    struct Mine { int ch, row, col, lds; bool live; };
-    const bool y_side[2] = {wave * 64 >= nx * T64, 512 + wave * 64 >= nx * T64};      // nx 64 is a multiple of a wave's 64
-    auto mine = [&](int o, bool y) {
+    struct Mine { int ch, row, col, lds; bool live, own; };
+    auto mine = [&](bool y) {
         Mine m;
-        const int per = y ? ny : nx, across = y ? p.CB + 1 : p.CB;
-        if (y) o -= nx * T64;
-        const int c = o / per, sl = o - c * per;
+        const int per = y ? ny / 2 : nx, part = t / (per * T64), i = t - part * per * T64, c = i / per;   // two parts of dy
+        const int across = y ? p.CB + 1 : p.CB, sl = part * per + i - c * per;
+        m.own = part < (y ? 2 : 1);
         m.row = sl / across; m.col = (sl - m.row * across) * 8;
-        m.live = c < T64 && (y ? k0 + c < p.K : c0 + c < p.C);
+        m.live = m.own && (y ? k0 + c < p.K : c0 + c < p.C);
         m.ch = y ? (k0 + c) * p.OH * p.OW : (c0 + c) * p.H * p.W;
-        m.lds = c >= T64 ? -1 : y ? 3 * X_PLANE + (c * YP + sl) * 16 : (c * XP + sl) * 16;
+        m.lds = y ? 3 * X_PLANE + (c * YP + (m.own ? sl : YP - 1)) * 16 : (c * XP + (m.own ? sl : XP - 1)) * 16;
         return m;
     };
-    const Mine m0 = mine(t, y_side[0]), m1 = mine(t + 512, y_side[1]);
+    const Mine m0 = mine(false), m1 = mine(true);
+    const bool minus = wave * 64 >= ny / 2 * T64;     // uniform: this wavefront's octets of dy are the second half's
     auto place = [&](int s) {
         Place q;
         const int cb = s % p.col_blocks, r = s / p.col_blocks;
@@ -173,7 +177,7 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
     auto fetch = [&](auto jt, const Place &q) {
         constexpr int j = decltype(jt)::value;
         const Mine &m = j == 0 ? m0 : m1;
-        const bool y = y_side[j];
+        constexpr bool y = j == 1;
         const int rows = y ? p.OH : p.H, cols = y ? p.OW : p.W;
         const int row = q.y + m.row - (y ? 0 : p.pad), first = q.x + (y ? p.pad - 2 : 0), col = first + m.col;
         early[j] = col < 0 ? -col : 0;                // fetched from column 0 and moved up
@@ -214,8 +218,8 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
         small = xsmi::SmallTest{};
 #pragma unroll
         for (int i = 0; i < 4; ++i) small.add(v[2 * i], v[2 * i + 1]);
-        if (y_side[j] && want_db) {
-            const Mine &m = j == 0 ? m0 : m1;
+        if (j == 1 && want_db) {
+            const Mine &m = m1;
             const bool first = q.x == 0 || m.col > 0, last = m.col == p.CB * 8 && q.x + p.CB * 8 < p.col_blocks * p.CB * 8;
             float all = ((v[2] + v[3]) + (v[4] + v[5])) + (v[6] + v[7]);
             float head = v[0] + (p.pad == 0 ? v[1] : 0.f);
@@ -225,18 +229,21 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
     };
     auto split_two = [&](auto jt, auto it) {          // pairs 2 it and 2 it + 1
         constexpr int j = decltype(jt)::value, i0 = 2 * decltype(it)::value;
+        auto two = [&](auto negative) {
 #pragma unroll
-        for (int i = i0; i < i0 + 2; ++i) {
-            uint32_t a, b, c;
-            xsmi::split_pair3(pre[j][2 * i], pre[j][2 * i + 1], a, b, c);
-            piece[0][i] = a; piece[1][i] = b; piece[2][i] = c;
-        }
+            for (int i = i0; i < i0 + 2; ++i) {
+                uint32_t a, b, c;
+                xsmi::split_pair3<decltype(negative)::value != 0>(pre[j][2 * i], pre[j][2 * i + 1], a, b, c);
+                piece[0][i] = a; piece[1][i] = b; piece[2][i] = c;
+            }
+        };
+        if (j == 1 && minus) two(IC<1>{});
+        else two(IC<0>{});
     };
     auto put = [&](auto jt, int to) {
         constexpr int j = decltype(jt)::value;
         const Mine &m = j == 0 ? m0 : m1;
-        if (m.lds < 0) return;
-        const int plane = y_side[j] ? Y_PLANE : X_PLANE;
+        constexpr int plane = j == 1 ? Y_PLANE : X_PLANE;
         piece[0][0] = small.found() ? xsmi::NAN_PAIR : piece[0][0];    // the first dword of an octet is read under some tap
 #pragma unroll
         for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32x4 *>(s_mem + to + m.lds + q * plane) = piece[q];
@@ -347,7 +354,7 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
         for (int i = 0; i < 9; ++i)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const float sum = acc[i][v] + s_acc[(i * 16 + v) * 256 + t];
+                const float sum = acc[i][v] - s_acc[(i * 16 + v) * 256 + t];
                 test.add(sum);
                 dst[i * T64 * T64 + (8 * (v >> 2) + (v & 3)) * T64] = sum;
             }
@@ -362,12 +369,11 @@ __global__ void __launch_bounds__(512, 2) split_wgrad_kernel(WgParams p) {
     if (want_db) {                                    // a filter's octets are in up to ny threads: added in their order
         double *s_db = reinterpret_cast<double *>(s_mem);
         __syncthreads();
-        if (y_side[1] && m1.lds >= 0) s_db[t + 512 - nx * T64] = db_sum;
-        if (y_side[0]) s_db[t - nx * T64] = db_sum;
+        if (m1.own) s_db[(m1.lds - 3 * X_PLANE) / 16] = db_sum;
         __syncthreads();
         if (t < T64 && k0 + t < p.K) {
             double sum = 0.0;
-            for (int i = 0; i < ny; ++i) sum += s_db[t * ny + i];
+            for (int i = 0; i < ny; ++i) sum += s_db[t * YP + i];
             p.dbpart[(size_t)split * p.K + k0 + t] = (float)sum;
         }
     }
