@@ -1,7 +1,7 @@
 """The fp32 convolution on bf16 matrix pipes (three-way split operands): every geometry it serves against the oracle,
 at the edges of its tiles, channel groups, phases and grids.
 
-Bound: the split drops products below 2^-25 of each term and adds in float32; the worst of the sizes here, 4608 terms,
+Bound: the split drops at most 2^-24 of each term and adds in float32; the worst of the sizes here, 4608 terms,
 was 1.7e-7 in relative L2 norm, so 1e-6 is far above rounding and far below any misplaced term."""
 import contextlib
 

@@ -3,8 +3,8 @@
 // A float32 value is the sum of three bf16 values EXACTLY: 24 significant bits are 8 + 8 + 8, and each remainder
 // a - bf16(a) is representable (rounding to nearest even leaves a signed remainder of at most 15, then 7 bits).  So
 //     a b = a0 b0 + (a0 b1 + a1 b0) + (a1 b1 + a0 b2 + a2 b0) + [a1 b2 + a2 b1 + a2 b2]
-// where the bracket is below 2^-25 |a b|, half a float32 ulp's half, and is left out: six bf16 MFMAs, whose products are
-// exact and whose sums are float32, stand for one float32 product.  The bf16 pipe does sixteen times the work of the
+// where the bracket is at most 2^-24 |a b| (|a1| is at most 2^-8 of a's binade, |a2| 2^-17), half a float32 ulp, and is left
+// out: six bf16 MFMAs, whose products are exact and whose sums are float32, stand for one float32 product.  The bf16 pipe does sixteen times the work of the
 // fp32 pipe per cycle, so the matrix-bound floor falls to 6/16.  The large products (a0 b0) and the five small ones
 // have accumulators of their own: the chain that carries the rounding of the full sum then has one addition per 16
 // channels and tap, against one per product pair on the fp32 pipe.

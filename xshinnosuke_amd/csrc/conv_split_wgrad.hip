@@ -1,5 +1,5 @@
 // fp32 weight gradient of 3 x 3, stride-1 layers on the bf16 matrix pipes, operands split into three bf16 values as in
-// conv_split.hip (six products, exact up to 2^-25 of each term).
+// conv_split.hip (six products, exact up to 2^-24 of each term).
 //
 //     dw[k][c][r][s] = sum over (n, y, x) of dy[n][k][y][x] * in[n][c][y + r - pad][x + s - pad]
 //

@@ -48,7 +48,7 @@ hipStream_t g_lanes[xsmi::SIDE_LANES] = {nullptr, nullptr, nullptr, nullptr};
 hipEvent_t g_lane_done[xsmi::SIDE_LANES] = {nullptr, nullptr, nullptr, nullptr};
 bool g_lane_used[xsmi::SIDE_LANES] = {false, false, false, false};
 
-// Partial tiles and flags of the even-split convolution kernels: one area per stream, owned by the library (a
+// Partial tiles and flags of the convolution kernels that share tiles between workgroups (even split, split operands): one area per stream, owned by the library (a
 // launch's partial tiles are dead when it ends, and launches of one stream run one after the other).
 xsmi::SkScratch g_sk_scratch[2] = {{nullptr, nullptr}, {nullptr, nullptr}};
 // A word in page-locked host memory that kernels write when a bounded wait ran out; the host reads it directly.
@@ -121,7 +121,7 @@ long option(Option o) {
 SkScratch sk_scratch() { return g_sk_scratch[g_current == g_side ? 1 : 0]; }
 uint32_t *device_error_word() { return g_dev_error_dev; }
 // Non-zero when a kernel has reported a wait that ran out.  Outside a capture the streams are drained, the flags
-// of the even-split kernels are cleared (a late producer may have left one raised) and the word is reset, so the
+// of the tile-sharing kernels are cleared (a late producer may have left one raised) and the word is reset, so the
 // library is usable again after the caller has seen the error.
 int check_device_error(const char *where) {
     if (!g_dev_error_host || *g_dev_error_host == 0) return XSMI_OK;
@@ -134,7 +134,7 @@ int check_device_error(const char *where) {
             if (g_sk_scratch[i].flags) (void)hipMemset(g_sk_scratch[i].flags, 0, SK_SCRATCH_FLAG_BYTES);
         *g_dev_error_host = 0;
     }
-    set_error("%s: an even-split convolution kernel gave up waiting for a partial tile (code %u): the output of that "
+    set_error("%s: a convolution kernel gave up waiting for a partial tile of another workgroup (code %u): the output of that "
               "launch is incomplete; results since then are not valid", where, code);
     return XSMI_ERR_RUNTIME;
 }

@@ -32,7 +32,7 @@ int cu_count();
 // Tuning switches (xsmi_set_option / environment variable / default); the order is that of the table in runtime.hip.
 enum Option { OPT_TAP_SK, OPT_SK_SPIN_LIMIT, OPT_TAP_STAGES, OPT_TAP_PERSIST, OPT_CL_HALO, OPT_CL_STEM, OPT_SK_WIDE, OPT_POOL_BWD, OPT_PACK_LANES, OPT_CONV_SPLIT, OPT_COUNT };
 long option(Option o);
-// Partial tiles and flags of the even-split convolution kernels for the stream that stream() hands out; allocated
+// Partial tiles and flags of the convolution kernels that share tiles between workgroups, for the stream that stream() hands out; allocated
 // by xsmi_init, the flags are zero between launches.
 constexpr size_t SK_SCRATCH_FLAG_BYTES = 4096;                          // 1024 workgroups
 constexpr size_t SK_SCRATCH_PART_BYTES = (size_t)1024 * 16 * 256 * 4;   // 1024 workgroups x one 64 x 64 tile of floats
