@@ -889,13 +889,13 @@ namespace xsmi {
 // Where the split pays, in kernel plus layout time on random layers of 1 to 512 channels and on ResNet-18's at N = 1 to 32
 // (`pixels`: outputs of the pass, of one residue class of a strided backward-data).
 //   1 x 1 to 3 taps: no.  An image then serves one tap, and its staging costs more than the fp32 kernels' loads (64 -> 128
-//     at 28 x 28, N=32: 13.5 -> 18.6 us).
-//   fewer than 16 channels: no.  A step multiplies 16, the rest zeros (4 -> 120, 3 x 3 at 102 x 102, N=53: 112 -> 234 us).
+//     at 28 x 28, N=32: 12.1 -> 19.2 us).
+//   fewer than 16 channels: no.  A step multiplies 16, the rest zeros (4 -> 120, 3 x 3 at 102 x 102, N=53: 109 -> 226 us).
 //   strided with whole chunks of 32 channels: only where one pixel tile holds all pixels.  The phases of a 3 x 3 / 2
-//     filter have 1, 2, 2 and 4 taps (128 -> 256 at 28 x 28, N=32: 44 -> 52 us); with one image the fp32 kernels have a few
-//     workgroups with a long chain each (256 -> 512 at 14 x 14, N=1: 61 -> 38 us).
-//   everything else: yes (64 -> 64 at 56 x 56, N=32: 69 -> 52 us; 369 -> 37, 5 x 5 at 76 x 76, N=2, which had only the
-//     table-driven kernel: 801 -> 82 us; equal at the smallest sizes, 64 -> 64 at 56 x 56, N=1: 21.4 -> 21.8 us).
+//     filter have 1, 2, 2 and 4 taps (128 -> 256 at 28 x 28, N=32: 43 -> 55 us); with one image the fp32 kernels have a few
+//     workgroups with a long chain each (256 -> 512 at 14 x 14, N=1: 59 -> 42 us).
+//   everything else: yes (64 -> 64 at 56 x 56, N=32: 67 -> 52 us; 369 -> 37, 5 x 5 at 76 x 76, N=2, which had only the
+//     table-driven kernel: 801 -> 93 us; equal at the smallest sizes, 64 -> 64 at 56 x 56, N=1: 20.2 -> 21.1 us).
 static bool split_pays(int CH, int R, int S, int sh, int sw, long pixels) {
     if (option(OPT_CONV_SPLIT) >= 2) return true;        // wherever it applies, for tests and measurements
     if (R * S < 4 || CH < 16) return false;

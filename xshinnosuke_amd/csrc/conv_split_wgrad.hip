@@ -11,7 +11,8 @@
 // input and 6 (8) of dy for each channel and filter, which 512 threads fetch (32 bytes contiguous each), split and write
 // to the LDS as [piece][channel][octet].  All nine taps read that image.  The columns of dy in the LDS begin at pad - 2, so
 // that a tap's values are the five dwords from a lane's octet on, taken 0, 1 or 2 half dwords further (v_alignbit for 1).
-// Odd pitches keep reads (lanes = channels) and writes (lanes = octets) free of bank conflicts.
+// Odd pitches spread the lanes of a 128-bit read (channels) over all banks; the reads a dword further are dword by dword and
+// meet in a quarter of the banks (9 % of a CU's cycles at 64 -> 64, 56 x 56, N=32; one dword instead of four: no faster).
 //
 // Eight waves: 2 x 2 of 32 filters x 32 channels, twice; the second four take the stage's other two octets, so each wave
 // multiplies one k-step of 16 pixels and nine taps (54 MFMAs) between two barriers, while its share of the next stage is
@@ -469,8 +470,8 @@ size_t split_wgrad_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int
     WgParams p;
     wg_plan(p, N, C, H, W, K, pad, OH, OW);
     // Below about seven stages for each compute unit the fp32 kernels' smaller partial results win (128 -> 128 at 28 x 28:
-    // N=8 33 -> 37 us, N=16 46 -> 45, N=32 72 -> 61), with a few channels the columns that multiply zeros (2 -> 480 at
-    // 93 x 93, N=6: 62 -> 140 us).
+    // N=8 32 -> 38 us, N=16 45 -> 44, N=32 72 -> 60), with a few channels the columns that multiply zeros (2 -> 480 at
+    // 93 x 93, N=6: 64 -> 147 us).
     if (opt < 2 && (C < 16 || (long)p.stages * p.kt * p.ct < 1750)) return 0;
     return align_up((size_t)p.splits * p.kt * p.ct * TILE * sizeof(float), 256) + align_up((size_t)p.splits * K * sizeof(float), 256);
 }
