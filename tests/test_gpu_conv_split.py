@@ -127,6 +127,31 @@ FORMED_AGAIN = [   # what the kernel that forms sums again walks differently
 ]
 
 
+@pytest.mark.parametrize("n,c,h,k,split", [
+    (32, 512, 7, 512, False),                # 104 tiles of the data gradient
+    (41, 256, 14, 128, False),               # 252: the most that leave a compute unit
+    (42, 256, 14, 128, True),                # 260: the data gradient fills the chip
+    (4, 64, 56, 256, True),                  # four times as many filters as channels
+    (5, 64, 56, 255, False),
+])
+def test_weight_gradient_beside_a_bf16_data_gradient(gpu, n, c, h, k, split):
+    """A bf16 data gradient that leaves compute units idle runs beside the weight gradient, whose split form would keep it
+    out of them.  One call for both gradients and one for each give the same bits."""
+    K = gpu.kernels
+    rng = np.random.default_rng(h)
+    x, w, dy = (gpu.to_device(rng.standard_normal(s).astype(np.float32)) for s in ((n, c, h, h), (k, c, 3, 3), (n, k, h, h)))
+    own = K.conv2d_bwd_weight(dy, x, w.shape, (1, 1), 1, bf16=True)[0].numpy()
+    dw = gpu.empty(w.shape)
+    K.conv2d_bwd(dy, x, w, gpu.empty(x.shape), dw, None, (1, 1), 1, bf16=True)
+    np.testing.assert_array_equal(dw.numpy(), own)
+    old = gpu.set_option("conv_split", 0)
+    try:
+        fp32 = K.conv2d_bwd_weight(dy, x, w.shape, (1, 1), 1)[0].numpy()
+    finally:
+        gpu.set_option("conv_split", old)
+    assert np.array_equal(own, fp32) is not split
+
+
 @pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad", FORMED_AGAIN)
 def test_sums_that_are_formed_again(gpu, n, c, h, w, k, r, s, sh, sw, pad):
     """Every sum is below 2^-100, so every one is formed a second time; powers of two are exact: the bound is that of

@@ -4,17 +4,17 @@
 // a - bf16(a) is representable (rounding to nearest even leaves a signed remainder of at most 15, then 7 bits).  So
 //     a b = a0 b0 + (a0 b1 + a1 b0) + (a1 b1 + a0 b2 + a2 b0) + [a1 b2 + a2 b1 + a2 b2]
 // where the bracket is at most 2^-24 |a b| (|a1| is at most 2^-8 of a's binade, |a2| 2^-17), half a float32 ulp, and is left
-// out: six bf16 MFMAs, whose products are exact and whose sums are float32, stand for one float32 product.  The bf16 pipe does sixteen times the work of the
-// fp32 pipe per cycle, so the matrix-bound floor falls to 6/16.  The large products (a0 b0) and the five small ones
-// have accumulators of their own: the chain that carries the rounding of the full sum then has one addition per 16
+// out: six bf16 MFMAs, whose products are exact and whose sums are float32, stand for one float32 product.  The bf16 pipe
+// does sixteen times the work of the fp32 pipe per cycle, so the matrix-bound floor falls to 6/16.  The large products
+// (a0 b0) and the five small ones have accumulators of their own: the chain that carries the rounding of the full sum then has one addition per 16
 // channels and tap, against one per product pair on the fp32 pipe.
 //
 // What the split does not carry: infinities (inf - inf in a remainder), values within a bf16 rounding of the largest
 // float, and the last bits of values below 2^-110.  The first two make the sums that they touch non-finite, the third are
 // looked for and given a NaN (split3.h); such sums are formed again in float64 (form_again).
 //
-// Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (128 per tile), 2 x 2 waves
-// of 32 rows x 64 pixels.  The reduction is a list of steps (phase, 16 input channels, tap).  A PHASE is a set of taps
+// Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (256 per tile, 128 in
+// small launches), 2 x 4 (2 x 2) waves of 32 rows x 64 pixels.  The reduction is a list of steps (phase, 16 input channels, tap).  A PHASE is a set of taps
 // that read one sub-lattice of the input (stride 1: all taps; stride 2: the taps of one row and column parity; or one
 // filter row's taps, where the input rows of all taps together would not fit the LDS).  In the phase's own coordinates
 // the walk has stride 1, so a tile needs one run of positions ("slots") of a grid of pitch Wp = OX + taps across - 1, and

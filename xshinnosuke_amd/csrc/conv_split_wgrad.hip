@@ -62,8 +62,8 @@ __device__ __forceinline__ void next_stage(const WgParams &p, Place &q) {
 // The partial result of `stages` stages from `q` on, formed from the products themselves in float64.  A workgroup decides this
 // for itself, so its share is the one that it has among workgroups that do not: the stages' output rows and input columns.
 // A border column of dy has no input column under some taps: it meets a zero there, as in the fp32 kernels and in the
-// reference's product over the padded matrix, so that it shows if it is not finite.  Bound by the fp64 matrix pipe: a tap at a time, 16 x 16 blocks (D: register v of lane l is row l / 16 + 4 v, column l % 16), a lane's quarter
-// of the half's 16 pixels four deep.  All of 64 -> 64 at 56 x 56, N=8, not finite: 187 us (a product at a time behind the
+// reference's product over the padded matrix, so that it shows if it is not finite.  Bound by the fp64 matrix pipe: a tap at a time, 16 x 16
+// blocks (D: register v of lane l is row l / 16 + 4 v, column l % 16), a lane's quarter of the half's 16 pixels four deep.  All of 64 -> 64 at 56 x 56, N=8, not finite: 187 us (a product at a time behind the
 // partial results: 2850).
 __device__ __forceinline__ void form_again(const WgParams &p, float *part, double *s_half, Place q0, int stages, int k0, int c0,
                                         int half, int wr, int wc, int lane) {
@@ -463,7 +463,7 @@ void wg_plan(WgParams &p, int N, int C, int H, int W, int K, int pad, int OH, in
 
 namespace xsmi {
 
-size_t split_wgrad_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad) {
+size_t split_wgrad_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, bool bf16) {
     const long opt = option(OPT_CONV_SPLIT);
     if (opt == 0 || R != 3 || S != 3 || sh != 1 || sw != 1 || pad > 1) return 0;
     const int OH = H + 2 * pad - 2, OW = W + 2 * pad - 2;
@@ -473,6 +473,14 @@ size_t split_wgrad_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int
     // N=8 32 -> 38 us, N=16 45 -> 44, N=32 72 -> 60), with a few channels the columns that multiply zeros (2 -> 480 at
     // 93 x 93, N=6: 64 -> 147 us).
     if (opt < 2 && (C < 16 || (long)p.stages * p.kt * p.ct < 1750)) return 0;
+    // A workgroup here fills a compute unit's LDS and registers.  A bf16 data gradient of few tiles, which is started beside the
+    // weight gradient (xsmi_conv2d_bwd), then waits and lands on the first units that come free, several of its workgroups on
+    // one: the fp32 kernels let it in (both gradients, 512 -> 512 at 7 x 7: N=32 235 -> 163 us, N=64 334 -> 208; 256 -> 256 at
+    // 14 x 14, N=32: 117 -> 110; slower only below 100 channels, 48 -> 80 at 61 x 61, N=8: 125 -> 131).  With four times as
+    // many filters as channels this kernel stays ahead (64 -> 512 at 56 x 56, N=4: 153 us, fp32 kernels 185), and so it does
+    // beside a float32 data gradient (512 -> 512, N=32: 146, fp32 kernels 163) or one that fills the chip by itself (N=128: 310,
+    // fp32 kernels 453).  The rule looks at the flag, so that both ways to ask for a weight gradient give the same bits.
+    if (opt < 2 && bf16 && K < 4 * C && data_gradient_tiles(N, C, H, W) <= cu_count()) return 0;
     return align_up((size_t)p.splits * p.kt * p.ct * TILE * sizeof(float), 256) + align_up((size_t)p.splits * K * sizeof(float), 256);
 }
 

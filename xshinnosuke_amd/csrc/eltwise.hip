@@ -93,7 +93,7 @@ size_t xsmi_conv2d_pass_workspace_bytes(int N, int C, int H, int W, int K, int R
         m = xsmi::conv_bwd_weight_ws_bytes(N, C, K, R, S, OH, OW);
         if (!bf16 && xsmi::stem_wgrad_ok(N, C, H, W, K, R, S, sh, sw, pad))
             m = larger(m, xsmi::stem_wgrad_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad));
-        m = larger(m, xsmi::split_wgrad_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad));
+        m = larger(m, xsmi::split_wgrad_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, bf16));
     }
     return m;
 }
@@ -137,9 +137,8 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     // data gradient's grid (128-pixel x 64-channel tiles) leaves compute units idle the weight gradient still runs
     // beside it (6-9 % less time for both at 7x7 and 14x14 feature maps) and is joined at once; grids that fill the
     // chip alone only get in each other's way (15 % more time at 56x56) and run one after the other.
-    const long long tiles = (((long long)N * H * W + 127) / 128) * xsmi::ceil_div(C, 64);
     const bool async = (flags & XSMI_CONV_DW_ASYNC) != 0;
-    const bool beside = async || tiles <= xsmi::cu_count();
+    const bool beside = async || xsmi::data_gradient_tiles(N, C, H, W) <= xsmi::cu_count();
     int rc = beside ? xsmi::side_begin() : xsmi::side_join();    // in main-stream order: after any earlier async work
     if (rc) return rc;
     rc = xsmi_conv2d_bwd_weight(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, beta_dw, kflags, workspace_dw, workspace_dw_bytes);

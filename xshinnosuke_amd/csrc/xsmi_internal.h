@@ -157,7 +157,7 @@ int split_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C
                         int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace);
 
 // weight gradient of 3 x 3, stride-1 layers with at most one pixel of padding, likewise (conv_split_wgrad.hip)
-size_t split_wgrad_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad);
+size_t split_wgrad_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, bool bf16);
 int split_conv_bwd_weight(const float *dy, const float *x, float *dw, float *db, int N, int C, int H, int W, int K, int pad, int OH,
                           int OW, int accumulate, void *workspace);
 
@@ -300,5 +300,9 @@ __device__ __forceinline__ void block_barrier() {
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+// 128-pixel x 64-channel tiles of a data gradient: up to cu_count() of them leave compute units to a weight gradient beside it
+inline long long data_gradient_tiles(int N, int C, int H, int W) {
+    return (((long long)N * H * W + 127) / 128) * ceil_div(C, 64);
+}
 
 }  // namespace xsmi
