@@ -1,35 +1,35 @@
 // fp32 convolution forward and backward-data on the bf16 matrix pipes, without giving up float32 precision.
 //
-// A float32 value is the sum of three bf16 values EXACTLY: 24 significant bits are 8 + 8 + 8, and each remainder
-// a - bf16(a) is representable (rounding to nearest even leaves a signed remainder of at most 15, then 7 bits).  So
+// A float32 value is the sum of three bf16 values EXACTLY: 24 significant bits are 8 + 8 + 8, and each remainder a - bf16(a)
+// is representable (rounding to nearest even leaves a signed remainder of at most 15, then 7 bits).  So
 //     a b = a0 b0 + (a0 b1 + a1 b0) + (a1 b1 + a0 b2 + a2 b0) + [a1 b2 + a2 b1 + a2 b2]
 // where the bracket is at most 2^-24 |a b| (|a1| is at most 2^-8 of a's binade, |a2| 2^-17), half a float32 ulp, and is left
 // out: six bf16 MFMAs, whose products are exact and whose sums are float32, stand for one float32 product.  The bf16 pipe
-// does sixteen times the work of the fp32 pipe per cycle, so the matrix-bound floor falls to 6/16.  The large products
-// (a0 b0) and the five small ones have accumulators of their own: the chain that carries the rounding of the full sum then has one addition per 16
-// channels and tap, against one per product pair on the fp32 pipe.
+// does sixteen times the work of the fp32 pipe per cycle, so the matrix-bound floor falls to 6/16.  The large products (a0
+// b0) and the five small ones have accumulators of their own: the chain that carries the rounding of the full sum then has
+// one addition per 16 channels and tap, against one per product pair on the fp32 pipe.
 //
-// What the split does not carry: infinities (inf - inf in a remainder), values within a bf16 rounding of the largest
-// float, and the last bits of values below 2^-110.  The first two make the sums that they touch non-finite, the third are
-// looked for and given a NaN (split3.h); such sums are formed again in float64 (form_again).
+// What the split does not carry: infinities (inf - inf in a remainder), values within a bf16 rounding of the largest float,
+// and the last bits of values below 2^-110.  The first two make the sums that they touch non-finite, the third are looked
+// for and given a NaN (split3.h); such sums are formed again in float64 (form_again).
 //
-// Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (256 per tile, 128 in
-// small launches), 2 x 4 (2 x 2) waves of 32 rows x 64 pixels.  The reduction is a list of steps (phase, 16 input channels, tap).  A PHASE is a set of taps
-// that read one sub-lattice of the input (stride 1: all taps; stride 2: the taps of one row and column parity; or one
-// filter row's taps, where the input rows of all taps together would not fit the LDS).  In the phase's own coordinates
-// the walk has stride 1, so a tile needs one run of positions ("slots") of a grid of pitch Wp = OX + taps across - 1, and
-// a tap is nothing but an offset into the run.  The run is staged once per 16 channels for all taps of the phase: float32
-// values are fetched through registers (lanes = slots, eight channels per lane), split there, and written to the LDS as
-// [piece][octet][slot][8 channels], so a fragment read is 32 consecutive 16-byte slots whatever the tap is.  The LDS
-// image serves up to nine taps, which is what pays for the conversion (11 vector instructions per two values).
-// The filter is laid out split already, one 6 KB block per step ([piece][octet][row][8]); each wave fetches its fragments
-// straight into registers three steps ahead (the waves of a workgroup read the same block at about the same time: L1), so
-// the loop has no barrier except around the image of a channel group.
+// Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (256 per tile, 128 in small
+// launches), 2 x 4 (2 x 2) waves of 32 rows x 64 pixels.  The reduction is a list of steps (phase, 16 input channels, tap).
+// A PHASE is a set of taps that read one sub-lattice of the input (stride 1: all taps; stride 2: the taps of one row and
+// column parity; or one filter row's taps, where the input rows of all taps together would not fit the LDS).  In the phase's
+// own coordinates the walk has stride 1, so a tile needs one run of positions ("slots") of a grid of pitch Wp = OX + taps
+// across - 1, and a tap is nothing but an offset into the run.  The run is staged once per 16 channels for all taps of the
+// phase: float32 values are fetched through registers (lanes = slots, eight channels per lane), split there, and written to
+// the LDS as [piece][octet][slot][8 channels], so a fragment read is 32 consecutive 16-byte slots whatever the tap is.  The
+// LDS image serves up to nine taps, which is what pays for the conversion (ten vector instructions per two values: seven
+// split, three look for small ones). The filter is laid out split already, one 6 KB block per step ([piece][octet][row][8]);
+// each wave fetches its fragments straight into registers three steps ahead (the waves of a workgroup read the same block at
+// about the same time: L1), so the loop has no barrier except around the image of a channel group.
 //
-// Scheduling is the even split of conv_tap_sk.hip: the steps of all tiles in a row are dealt over the resident
-// workgroups; a workgroup whose range starts inside a tile hands its accumulators to the one that holds the tile's
-// first step, which adds them in ascending order (bounded wait, deterministic sums).  Row tiles vary slowest, so
-// that an XCD's workgroups read few filter blocks.
+// Scheduling is the even split of conv_tap_sk.hip: the steps of all tiles in a row are dealt over the resident workgroups; a
+// workgroup whose range starts inside a tile hands its accumulators to the one that holds the tile's first step, which adds
+// them in ascending order (bounded wait, deterministic sums).  Row tiles vary slowest, so that an XCD's workgroups read few
+// filter blocks.
 #include "conv_store.h"
 #include "split3.h"
 
