@@ -376,3 +376,23 @@ def test_a_partial_tile_that_never_comes_is_reported(gpu):
         gpu.set_option("sk_spin_limit", old)
     for _ in range(2):
         assert rel_l2(K.conv2d_fwd(*args, (1, 1), 1, out=out).numpy(), ref) <= TOL
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,s,stride,pad", [
+    (2, 48, 14, 19, 70, 3, 3, 1, 1),         # neither channel count has a bf16 kernel
+    (1, 33, 9, 31, 90, 7, 7, 2, 3),
+    (2, 16, 20, 11, 18, 5, 5, 1, 0),         # the fewest channels that the split kernels take
+    (2, 2, 28, 37, 40, 7, 7, 2, 3),          # forward in bf16, backward-data from 40 channels
+])
+def test_bf16_calls_without_a_bf16_kernel_have_float32_precision(gpu, n, c, h, w, k, r, s, stride, pad):
+    K = gpu.kernels
+    x, wt, b, dy, _ = _data(n, c, h, w, k, r, s, stride, stride, pad, gpu)
+    y_ref, col = oracle.conv2d_fwd(x, wt, b, (stride, stride), pad)
+    dx_ref, _, _ = oracle.conv2d_bwd(dy, x.shape, wt, col, (stride, stride), pad, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+    dx_, dw_, db_, ddy = (gpu.to_device(a) for a in (x, wt, b, dy))
+    if c > 8:
+        mask = gpu.empty(y_ref.shape, np.uint8)
+        y = K.conv2d_fwd(dx_, dw_, db_, (stride, stride), pad, relu=True, neg_mask=mask, bf16=True).numpy()
+        assert rel_l2(y, np.maximum(y_ref, 0)) <= TOL
+    dx = K.conv2d_bwd_data(ddy, dw_, x.shape, (stride, stride), pad, bf16=True).numpy()
+    assert rel_l2(dx, dx_ref) <= TOL

@@ -338,7 +338,7 @@ static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh,
     if (!bf16 && xsmi::stem_fwd_ok(N, C, H, W, K, R, S, sh, sw, pad) &&
         workspace_bytes >= xsmi::stem_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad))
         return FwdPath::FirstLayer;
-    if (!bf16 && !(flags & XSMI_CONV_WS_ONLY) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
+    if (xsmi::split_may_serve(C, bf16) && !(flags & XSMI_CONV_WS_ONLY) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
         const size_t need = xsmi::split_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
         if (need && workspace_bytes >= need) return FwdPath::Split;
     }
@@ -351,7 +351,7 @@ static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh,
 
 static BwdDataPath bwd_data_path(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW,
                                  unsigned flags, size_t workspace_bytes) {
-    if (!(flags & XSMI_CONV_BF16) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
+    if (xsmi::split_may_serve(K, (flags & XSMI_CONV_BF16) != 0) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
         const size_t need = xsmi::split_bwd_data_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
         if (need && workspace_bytes >= need) return BwdDataPath::Split;
     }

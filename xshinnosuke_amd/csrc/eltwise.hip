@@ -82,13 +82,13 @@ size_t xsmi_conv2d_pass_workspace_bytes(int N, int C, int H, int W, int K, int R
             m = larger(m, xsmi::stem_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad));
         // the even-split fp32 kernels read their own filter layout (their partial tiles live in the library)
         if (!bf16 && xsmi::sk_path_ok(C, K)) m = larger(m, xsmi::sk_fwd_ws_bytes(C, K, R, S));
-        if (!bf16) m = larger(m, xsmi::split_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW));
+        if (xsmi::split_may_serve(C, bf16)) m = larger(m, xsmi::split_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW));
         // the bf16 forward takes its fastest form when the workspace also holds a channels-last copy of x
         if (bf16 && xsmi::nhwc_fwd_ok(N, C, H, W, K, R, S, pad)) m = larger(m, xsmi::nhwc_fwd_ws_bytes(N, C, H, W, K, R, S, pad));
     } else if (pass == 1) {
         m = xsmi::conv_bwd_data_ws_bytes(C, K, R, S, sh, sw);
         if (!bf16 && xsmi::sk_bwd_data_ok(C, K, R, S, sh, sw)) m = larger(m, xsmi::sk_bwd_data_ws_bytes(C, K, R, S, sh, sw));
-        if (!bf16) m = larger(m, xsmi::split_bwd_data_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW));
+        if (xsmi::split_may_serve(K, bf16)) m = larger(m, xsmi::split_bwd_data_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW));
     } else if (pass == 2) {
         m = xsmi::conv_bwd_weight_ws_bytes(N, C, K, R, S, OH, OW);
         if (!bf16 && xsmi::stem_wgrad_ok(N, C, H, W, K, R, S, sh, sw, pad))

@@ -147,6 +147,12 @@ int sk_conv_fwd(const float *x, const float *w, const float *bias, float *y, uin
 int sk_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, int H, int W, int K, int R, int S, int sh,
                      int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace);
 
+// Whether a call may take the split kernels below.  With XSMI_CONV_BF16 the bf16 kernels come first; they have none for
+// reduction channels that are no multiple of 32 (the channels-last forward takes up to 8), and what is left there is float32
+// precision by the table-driven kernel, which the split kernels beat (backward-data of 2 -> 400, 7 x 7 / 2 at 28 x 89, N=2:
+// 1712 -> 44 us; forward and backward-data of 48 -> 203, 7 x 7 at 14 x 57, N=5: 1033 -> 88; of 60 -> 48, 3 x 3 at 64 x 64, N=13: 144 -> 87).
+inline bool split_may_serve(int reduce_channels, bool bf16) { return !bf16 || !tap_path_ok(reduce_channels); }
+
 // fp32 forward / backward-data on the bf16 matrix pipes, operands split into three bf16 values (conv_split.hip); the
 // workspace queries return 0 for geometries the kernel does not serve
 size_t split_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW);
