@@ -47,6 +47,10 @@ def _data(n, c, h, w, k, r, s, sh, sw, pad, gpu):
     (2, 18, 12, 12, 24, 3, 3, 3, 3, 0),      # stride 3: nine phases of one tap
     (1, 512, 7, 7, 512, 3, 3, 1, 1, 1),      # every tile shared by many workgroups
     (20, 32, 56, 56, 64, 3, 3, 1, 1, 1),     # more tiles than workgroups
+    (20, 64, 45, 57, 32, 3, 3, 1, 1, 1),     # few rows: tiles of 32 x 512, the last one 100 pixels
+    (17, 31, 56, 56, 1, 5, 5, 1, 1, 2),      # the same with two images for five filter rows, one row
+    (11, 17, 61, 70, 33, 7, 7, 1, 1, 3),     # a row past them: 64 x 256, images of 3, 3 and 1 filter rows
+    (24, 33, 56, 57, 20, 5, 5, 2, 2, 2),     # few rows, strided: 28 x 29 outputs, backward-data of four classes
 ])
 def test_split_convolution_against_the_oracle(gpu, n, c, h, w, k, r, s, sh, sw, pad):
     K = gpu.kernels

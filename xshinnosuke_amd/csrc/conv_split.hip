@@ -14,9 +14,12 @@
 // for and given a NaN (split3.h); such sums are formed again in float64 (form_again).
 //
 // Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (256 per tile, 128 in small
-// launches), 2 x 4 (2 x 2) waves of 32 rows x 64 pixels.  The reduction is a list of steps (phase, 16 input channels, tap).
+// launches), 2 x 4 (2 x 2) waves of 32 rows x 64 pixels; passes of at most 32 rows 1 x 8 such waves (sp_plan_tiled).  Waves of
+// 64 x 64 halve the conversion and the LDS reads for a product, but their accumulators and fragments spill (128 -> 128 at 28 x
+// 28, N=256: 305 -> 342 us; the loop runs 1.22 PFLOP/s of bf16 products there, a large library product 1.30).  The reduction is a list of steps (phase, 16 input channels, tap).
 // A PHASE is a set of taps that read one sub-lattice of the input (stride 1: all taps; stride 2: the taps of one row and
-// column parity; or one filter row's taps, where the input rows of all taps together would not fit the LDS).  In the phase's
+// column parity; or, where the input rows of all taps together would not fit the LDS, those of as many filter rows as do: 216 -> 2,
+// 5 x 5 at 32 x 32, N=52, in images of 3 and 2 rows instead of five of one: 202 -> 162 us).  In the phase's
 // own coordinates the walk has stride 1, so a tile needs one run of positions ("slots") of a grid of pitch Wp = OX + taps
 // across - 1, and a tap is nothing but an offset into the run.  The run is staged once per 16 channels for all taps of the
 // phase: float32 values are fetched through registers (lanes = slots, eight channels per lane), split there, and written to
@@ -45,13 +48,23 @@ using xsmi::carried;
 typedef uint32_t uint32x2 __attribute__((ext_vector_type(2)));
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 
-constexpr int SP_ROWS = 64;
-constexpr int sp_slots_of(int wc) { return wc == 4 ? 512 : 384; }     // slots of an LDS image
+constexpr int SP_ROWS = 64;                          // rows of a filter block
+// Tilings: WR x WC waves of 32 rows x 64 pixels, slots of an LDS image, most workgroups of a launch.
+struct SpTiling {
+    int wr, wc, slots, max_grid;
+    constexpr int rows() const { return 32 * wr; }
+    constexpr int pixels() const { return 64 * wc; }
+    constexpr int threads() const { return 64 * wr * wc; }
+};
+constexpr SpTiling SP_TILINGS[] = {{2, 2, 384, 512}, {2, 4, 512, 256}, {1, 8, 768, 256}};
 constexpr int SP_BLOCK = 3 * 2 * SP_ROWS * 16;       // bytes of a step's filter block
 constexpr int SP_MAX_CLASSES = 4, SP_MAX_PHASES = 16;
-constexpr int sp_max_grid(int wc) { return wc == 4 ? 256 : 512; }
-static_assert((size_t)sp_max_grid(2) * 4 <= xsmi::SK_SCRATCH_FLAG_BYTES, "one flag per workgroup");
-static_assert((size_t)512 * 64 * 128 * 4 <= xsmi::SK_SCRATCH_PART_BYTES, "one partial tile per workgroup");
+constexpr bool sp_scratch_holds() {
+    for (const SpTiling &k : SP_TILINGS)
+        if ((size_t)k.max_grid * 4 > xsmi::SK_SCRATCH_FLAG_BYTES || (size_t)k.max_grid * k.rows() * k.pixels() * 4 > xsmi::SK_SCRATCH_PART_BYTES) return false;
+    return true;
+}
+static_assert(sp_scratch_holds(), "one flag and one partial tile per workgroup");
 
 struct SpPhase {
     int iy0, ix0;          // input place of slot (row v, column u): (v * sy + iy0, u * sx + ix0)
@@ -79,7 +92,7 @@ struct SpParams {
     uint32_t units, upg, urem;                       // steps in all; per workgroup, remainder
     int N, CH, groups, IH, IW, in_n, plane;          // input channels, their groups of 16, floats per image / plane
     int w_row, w_ch, FS;                             // of the layout launches: floats between rows / channels of the filter, filter width
-    int ncls, relu, accumulate, wc;
+    int ncls, relu, accumulate, tiling;
     SpClass cls[SP_MAX_CLASSES];
     SpPhase ph[SP_MAX_PHASES];
     SpTapPlace tap[9];     // of a 3 x 3 filter's taps
@@ -264,16 +277,17 @@ __device__ __forceinline__ void decide_signs(floatx16 &r, const floatx16 &sum, c
     }
 }
 
-// WC waves across the tile's pixels (2: 128 pixels and 256 threads, two workgroups per CU; 4: 256 and 512, one)
 // SIGNS: a sign mask is kept (a kernel of its own: the others would pay for the registers of decide_signs, half a microsecond)
-template <int WC, bool SIGNS>
-__global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
-    constexpr int SP_PIX = 64 * WC, THREADS = 128 * WC, NJ = sp_slots_of(WC) / 64 / WC;
-    constexpr int SP_PLANE = sp_slots_of(WC) * 16;       // bytes of one (piece, octet) plane
+template <int TILING, bool SIGNS>
+__global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_kernel(SpParams p) {
+    constexpr SpTiling TL = SP_TILINGS[TILING];
+    constexpr int WC = TL.wc, ROWS = TL.rows(), SP_PIX = TL.pixels(), THREADS = TL.threads();
+    constexpr int CHUNKS = THREADS / 128, NJ = TL.slots / 64 / CHUNKS;    // 64-slot chunks staged at a time, and how often
+    constexpr int SP_PLANE = TL.slots * 16;              // bytes of one (piece, octet) plane
     constexpr int SP_IMAGE = 6 * SP_PLANE;
     constexpr uint32_t PART_BYTES = 32 * THREADS * 4;    // a workgroup's partial tile
     __shared__ __attribute__((aligned(16))) unsigned char s_img[2 * SP_IMAGE];
-    __shared__ __attribute__((aligned(16))) float s_bias[2][SP_ROWS];
+    __shared__ __attribute__((aligned(16))) float s_bias[2][ROWS];
     __shared__ uint32_t s_fail;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -287,9 +301,9 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
     const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc((void *)p.in, 0, (int)p.in_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rapk = __builtin_amdgcn_make_buffer_rsrc((void *)p.apk, 0, (int)p.apk_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rpart =
-        __builtin_amdgcn_make_buffer_rsrc((void *)p.part, 0, (int)(sp_max_grid(WC) * PART_BYTES), 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc((void *)p.part, 0, (int)(TL.max_grid * PART_BYTES), 0x00020000);
     const int a_voff = (h * SP_ROWS + wr * 32 + l31) * 16;
-    const int octet = wave & 1, chunk0 = wave >> 1;    // this wave stages slots 64 (chunk0 + WC j) .. + 63 of one octet
+    const int octet = wave & 1, chunk0 = wave >> 1;    // this wave stages slots 64 (chunk0 + CHUNKS j) .. + 63 of one octet
     const uint32_t plane4 = (uint32_t)p.plane * 4u;
 
     // A segment: steps [s_first, s_first + n) of one tile, beginning with tap `tap` of channel group `grp` of phase f.
@@ -336,7 +350,7 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         const SpPhase &ph = p.ph[f];
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            const int sl = 64 * (chunk0 + WC * j) + lane;
+            const int sl = 64 * (chunk0 + CHUNKS * j) + lane;
             const uint32_t P = (uint32_t)(sg.slot0 + sl);
             const int q = (int)xsmi::fdiv(P, c.dWp), n_ = (int)xsmi::fdiv((uint32_t)q, c.dHp);
             const int iy = (q - n_ * c.Hp) * c.sy + ph.iy0, ix = ((int)P - q * c.Wp) * c.sx + ph.ix0;
@@ -378,7 +392,7 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
         piece[0][i] = a; piece[1][i] = b; piece[2][i] = c;
     };
     auto put = [&](auto j, int to) {
-        unsigned char *dst = s_img + to + octet * SP_PLANE + (64 * (chunk0 + WC * j) + lane) * 16;
+        unsigned char *dst = s_img + to + octet * SP_PLANE + (64 * (chunk0 + CHUNKS * j) + lane) * 16;
         piece[0][0] = small.found() ? xsmi::NAN_PAIR : piece[0][0];
 #pragma unroll
         for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32x4 *>(dst + 2 * q * SP_PLANE) = piece[q];
@@ -524,7 +538,7 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
             for (int v = 0; v < 16; ++v) { hi[j][v] = 0.f; lo[j][v] = 0.f; }
         }
         bias_buf ^= 1;                                 // the other waves may still be reading the one before
-        if (p.bias && head && t < SP_ROWS) s_bias[bias_buf][t] = rt * SP_ROWS + t < c.rows ? p.bias[rt * SP_ROWS + t] : 0.f;
+        if (p.bias && head && t < ROWS) s_bias[bias_buf][t] = rt * ROWS + t < c.rows ? p.bias[rt * ROWS + t] : 0.f;
         int left = sg.n, f = sg.f, grp = sg.grp, tap = sg.tap;
         while (left > 0) {
             if (turn) {
@@ -642,12 +656,12 @@ __global__ void __launch_bounds__(128 * WC, 2) split_conv_kernel(SpParams p) {
                     floatx16 r = acc[j];
 #pragma unroll
                     for (int v = 0; v < 16; ++v) r[v] += bias ? bias[wr * 32 + 4 * h + 8 * (v >> 2) + (v & 3)] : 0.f;
-                    decide_signs<WC == 4 ? 8 : 4>(r, acc[j], p, c, bias, rt, wr * 32, m0 + wc * 64 + 32 * j, lane, rin, rapk);
+                    decide_signs<TILING != 0 ? 8 : 4>(r, acc[j], p, c, bias, rt, wr * 32, m0 + wc * 64 + 32 * j, lane, rin, rapk);
                     acc[j] = r;
                     bias = nullptr;
                 }
                 xsmi::store_block_32x32(acc[j], c, p.out, p.out_bytes, SIGNS ? p.mask : nullptr, bias, p.relu, p.accumulate,
-                                        rt * SP_ROWS, SP_ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
+                                        rt * ROWS, ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
             }
         }
         if (!more) break;
@@ -744,37 +758,45 @@ bool sp_add_class(SpParams &p, int &nph, uint32_t &steps_bytes, const SpTaps &k,
     if (p.ncls == SP_MAX_CLASSES || k.R < 1 || k.S < 1) return false;
     SpClass &c = p.cls[p.ncls];
     const int ny = sy < k.R ? sy : k.R, nx = sx < k.S ? sx : k.S;
-    // all rows of a sub-lattice in one image when it fits, otherwise one filter row at a time
+    // all rows of a sub-lattice in one image when it fits, otherwise as many at a time as do
     const int ty_max = (k.R + ny - 1) / ny, tx_max = (k.S + nx - 1) / nx;
-    const int pix = 64 * p.wc;
-    const bool by_row = sp_slots(pix, OY, OX, ty_max, tx_max) > sp_slots_of(p.wc);
-    const int ty = by_row ? 1 : ty_max;
-    if (sp_slots(pix, OY, OX, ty, tx_max) > sp_slots_of(p.wc)) return false;
-    const int rows_n = by_row ? k.R : ny;
-    if (nph + rows_n * nx > SP_MAX_PHASES) return false;
-    c.phase0 = nph; c.nphase = rows_n * nx; c.taps = k.R * k.S;
+    const SpTiling &tl = SP_TILINGS[p.tiling];
+    if (tl.rows() < SP_ROWS && rows > tl.rows()) return false;
+    const int pix = tl.pixels();
+    int ty = ty_max;
+    while (ty > 1 && sp_slots(pix, OY, OX, ty, tx_max) > tl.slots) --ty;
+    if (sp_slots(pix, OY, OX, ty, tx_max) > tl.slots) return false;
+    // no more rows than the images need: seven in threes are 3 + 3 + 1, in images of 3 + 2 + 2 no fewer, but shorter ones
+    const int images = (ty_max + ty - 1) / ty;
+    ty = (ty_max + images - 1) / images;
+    int nphase = 0;
+    for (int i = 0; i < ny; ++i) nphase += ((k.R - i + ny - 1) / ny + ty - 1) / ty;
+    nphase *= nx;
+    if (nph + nphase > SP_MAX_PHASES) return false;
+    c.phase0 = nph; c.nphase = nphase; c.taps = k.R * k.S;
     c.M = M; c.rows = rows; c.OY = OY; c.OX = OX; c.sy = sy; c.sx = sx;
     c.Wp = OX + tx_max - 1; c.Hp = OY + ty - 1;
     c.span = (ty - 1) * c.Wp + tx_max - 1;
     int step = 0, tap = 0;
-    for (int i = 0; i < rows_n; ++i)
-        for (int j = 0; j < nx; ++j) {
-            SpPhase &f = p.ph[nph++];
-            const int na = by_row ? 1 : (k.R - i + ny - 1) / ny, nb = (k.S - j + nx - 1) / nx;
-            f.iy0 = k.iy0 + i; f.ix0 = k.ix0 + j;
-            f.Tx = nb; f.T = na * nb;
-            f.tap0 = tap; f.step0 = step;
-            f.r0 = k.r0 + k.rs * i; f.rs = k.rs * ny; f.s0 = k.s0 + k.ss * j; f.ss = k.ss * nx;
-            tap += f.T; step += f.T * p.groups;
-        }
+    for (int i = 0; i < ny; ++i)
+        for (int first = i; first < k.R; first += ny * ty)        // filter rows first, first + ny, ...: at most ty
+            for (int j = 0; j < nx; ++j) {
+                SpPhase &f = p.ph[nph++];
+                const int left = (k.R - first + ny - 1) / ny, na = left < ty ? left : ty, nb = (k.S - j + nx - 1) / nx;
+                f.iy0 = k.iy0 + first; f.ix0 = k.ix0 + j;
+                f.Tx = nb; f.T = na * nb;
+                f.tap0 = tap; f.step0 = step;
+                f.r0 = k.r0 + k.rs * first; f.rs = k.rs * ny; f.s0 = k.s0 + k.ss * j; f.ss = k.ss * nx;
+                tap += f.T; step += f.T * p.groups;
+            }
     c.iters = (uint32_t)step;
-    const int tiles_m = xsmi::ceil_div(M, pix), tiles_r = xsmi::ceil_div(rows, SP_ROWS);
+    const int tiles_m = xsmi::ceil_div(M, pix), tiles_r = xsmi::ceil_div(rows, tl.rows()), blocks_r = xsmi::ceil_div(rows, SP_ROWS);
     c.dOX = xsmi::make_fastdiv(OX); c.dOY = xsmi::make_fastdiv(OY); c.dWp = xsmi::make_fastdiv(c.Wp); c.dHp = xsmi::make_fastdiv(c.Hp);
     c.dIT = xsmi::make_fastdiv(c.iters); c.dTM = xsmi::make_fastdiv(tiles_m);
     c.apk_off = steps_bytes;
-    const double bytes = (double)steps_bytes + (double)tiles_r * c.iters * SP_BLOCK, units = (double)p.units + (double)tiles_m * tiles_r * c.iters;
+    const double bytes = (double)steps_bytes + (double)blocks_r * c.iters * SP_BLOCK, units = (double)p.units + (double)tiles_m * tiles_r * c.iters;
     if (bytes >= 2e9 || units >= 1e9 || (double)c.Wp * c.Hp * p.N >= 1e9) return false;
-    steps_bytes += (uint32_t)tiles_r * c.iters * (uint32_t)SP_BLOCK;
+    steps_bytes += (uint32_t)blocks_r * c.iters * (uint32_t)SP_BLOCK;
     c.first_unit = p.units;
     p.units += (uint32_t)tiles_m * (uint32_t)tiles_r * c.iters;
     c.end_unit = p.units;
@@ -782,45 +804,70 @@ bool sp_add_class(SpParams &p, int &nph, uint32_t &steps_bytes, const SpTaps &k,
     return true;
 }
 
-// 256-pixel tiles stage 2.0 values for each pixel of a 3 x 3 layer's tile where 128-pixel tiles stage 3.0; small passes keep
-// the smaller tile, whose last one is emptier by less
-int sp_wide(long m) { return m >= 1024 ? 4 : 2; }
+// Steps that a workgroup of a launch has at least.  In a launch that does not fill the chip n steps for each workgroup cost
+// 0.45 us n, and the workgroup that adds a tile of I steps together about 0.9 us for each of the I / n - 1 others; the sum is
+// smallest at n = sqrt(2 I).
+uint32_t sp_least(const SpParams &p) {
+    uint32_t steps = 0, least = 4;
+    for (int i = 0; i < p.ncls; ++i) steps = p.cls[i].iters > steps ? p.cls[i].iters : steps;
+    while (least * least < 2 * steps) ++least;
+    return least;
+}
+
+// The tiling of a pass of m pixels (of its largest class), and its plan.
+//   256-pixel tiles stage 2.0 values for each pixel of a 3 x 3 layer's tile where 128-pixel tiles stage 3.0; passes below 1024
+//   pixels keep the smaller tile, whose last one is emptier by less.
+//   At most 32 rows leave half of a 64-row tile's matrix work to zeros: tiles of 32 x 512 instead, where 64 x 256 would fill the
+//   chip (44 x 64 -> 16, 83 x 83: 139 -> 87 us; 10 x 448 -> 5, 5 x 5 at 66 x 66: 278 -> 161).  Below that the number of
+//   workgroups bounds the launch, of which there are then half as many (8 x 160 -> 17 at 12 x 59: 25.7 us, 29.5 in wide tiles).
+template <typename Plan>
+bool sp_plan_tiled(SpParams &p, long m, int rows, const Plan &plan) {
+    auto as = [&](int tiling) {
+        memset(&p, 0, sizeof(p));
+        p.tiling = tiling;
+        return plan(p);
+    };
+    if (m < 1024) return as(0);
+    if (!as(1)) return false;
+    if (rows > SP_TILINGS[2].rows() || p.units < 256u * sp_least(p)) return true;
+    return as(2) || as(1);
+}
 
 bool sp_plan_fwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
-    memset(&p, 0, sizeof(p));
-    p.wc = sp_wide((long)N * OH * OW);
-    p.N = N; p.CH = C; p.groups = xsmi::ceil_div(C, 16); p.IH = H; p.IW = W; p.in_n = C * H * W; p.plane = H * W;
-    p.w_row = C * R * S; p.w_ch = R * S; p.FS = S;
-    int nph = 0;
-    const SpTaps k = {R, S, 0, 1, 0, 1, -pad, -pad};
-    if (!sp_add_class(p, nph, p.apk_bytes, k, N * OH * OW, K, OH, OW, sh, sw)) return false;
-    SpClass &c = p.cls[0];
-    c.os_n = (long long)K * OH * OW; c.os_k = (long long)OH * OW; c.o_base = 0; c.os_y = OW; c.os_x = 1;
-    p.in_bytes = (uint32_t)((size_t)N * C * H * W * 4); p.out_bytes = (uint32_t)((size_t)N * K * OH * OW * 4);
-    return true;
+    return sp_plan_tiled(p, (long)N * OH * OW, K, [&](SpParams &p) {
+        p.N = N; p.CH = C; p.groups = xsmi::ceil_div(C, 16); p.IH = H; p.IW = W; p.in_n = C * H * W; p.plane = H * W;
+        p.w_row = C * R * S; p.w_ch = R * S; p.FS = S;
+        int nph = 0;
+        const SpTaps k = {R, S, 0, 1, 0, 1, -pad, -pad};
+        if (!sp_add_class(p, nph, p.apk_bytes, k, N * OH * OW, K, OH, OW, sh, sw)) return false;
+        SpClass &c = p.cls[0];
+        c.os_n = (long long)K * OH * OW; c.os_k = (long long)OH * OW; c.o_base = 0; c.os_y = OW; c.os_x = 1;
+        p.in_bytes = (uint32_t)((size_t)N * C * H * W * 4); p.out_bytes = (uint32_t)((size_t)N * K * OH * OW * 4);
+        return true;
+    });
 }
 
 // backward-data: a class per residue (h mod sh, w mod sw); taps in ascending order of the dy row they read
 bool sp_plan_bwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
-    memset(&p, 0, sizeof(p));
-    p.wc = sp_wide((long)N * H * W / (sh * sw));
-    p.N = N; p.CH = K; p.groups = xsmi::ceil_div(K, 16); p.IH = OH; p.IW = OW; p.in_n = K * OH * OW; p.plane = OH * OW;
-    p.w_row = R * S; p.w_ch = C * R * S; p.FS = S;
-    int nph = 0;
-    for (int ph = 0; ph < sh && ph < H; ++ph) {
-        const int r0 = (ph + pad) % sh, T = r0 < R ? xsmi::ceil_div(R - r0, sh) : 0, cy = (ph + pad - r0) / sh;
-        for (int pw = 0; pw < sw && pw < W; ++pw) {
-            const int s0 = (pw + pad) % sw, U = s0 < S ? xsmi::ceil_div(S - s0, sw) : 0, cx = (pw + pad - s0) / sw;
-            const int OYc = xsmi::ceil_div(H - ph, sh), OXc = xsmi::ceil_div(W - pw, sw);
-            const SpTaps k = {T, U, r0 + sh * (T - 1), -sh, s0 + sw * (U - 1), -sw, cy - (T - 1), cx - (U - 1)};
-            if (!sp_add_class(p, nph, p.apk_bytes, k, N * OYc * OXc, C, OYc, OXc, 1, 1)) return false;
-            SpClass &c = p.cls[p.ncls - 1];
-            c.os_n = (long long)C * H * W; c.os_k = (long long)H * W; c.o_base = (long long)ph * W + pw;
-            c.os_y = sh * W; c.os_x = sw;
+    return sp_plan_tiled(p, (long)N * H * W / (sh * sw), C, [&](SpParams &p) {
+        p.N = N; p.CH = K; p.groups = xsmi::ceil_div(K, 16); p.IH = OH; p.IW = OW; p.in_n = K * OH * OW; p.plane = OH * OW;
+        p.w_row = R * S; p.w_ch = C * R * S; p.FS = S;
+        int nph = 0;
+        for (int ph = 0; ph < sh && ph < H; ++ph) {
+            const int r0 = (ph + pad) % sh, T = r0 < R ? xsmi::ceil_div(R - r0, sh) : 0, cy = (ph + pad - r0) / sh;
+            for (int pw = 0; pw < sw && pw < W; ++pw) {
+                const int s0 = (pw + pad) % sw, U = s0 < S ? xsmi::ceil_div(S - s0, sw) : 0, cx = (pw + pad - s0) / sw;
+                const int OYc = xsmi::ceil_div(H - ph, sh), OXc = xsmi::ceil_div(W - pw, sw);
+                const SpTaps k = {T, U, r0 + sh * (T - 1), -sh, s0 + sw * (U - 1), -sw, cy - (T - 1), cx - (U - 1)};
+                if (!sp_add_class(p, nph, p.apk_bytes, k, N * OYc * OXc, C, OYc, OXc, 1, 1)) return false;
+                SpClass &c = p.cls[p.ncls - 1];
+                c.os_n = (long long)C * H * W; c.os_k = (long long)H * W; c.o_base = (long long)ph * W + pw;
+                c.os_y = sh * W; c.os_x = sw;
+            }
         }
-    }
-    p.in_bytes = (uint32_t)((size_t)N * K * OH * OW * 4); p.out_bytes = (uint32_t)((size_t)N * C * H * W * 4);
-    return true;
+        p.in_bytes = (uint32_t)((size_t)N * K * OH * OW * 4); p.out_bytes = (uint32_t)((size_t)N * C * H * W * 4);
+        return true;
+    });
 }
 
 int sp_run(SpParams &p, int opts, void *workspace) {
@@ -847,25 +894,22 @@ int sp_run(SpParams &p, int opts, void *workspace) {
         XSMI_LAUNCH_CHECK("split_pack_kernel");
     }
     if (opts & 4) return XSMI_OK;
-    static int resident[4] = {0, 0, 0, 0};
-    const int which = (p.wc == 4 ? 1 : 0) + (p.mask ? 2 : 0), threads = 128 * p.wc;
-    void (*const kernels[4])(SpParams) = {split_conv_kernel<2, false>, split_conv_kernel<4, false>, split_conv_kernel<2, true>,
-                                          split_conv_kernel<4, true>};
+    constexpr int TILINGS = sizeof(SP_TILINGS) / sizeof(SP_TILINGS[0]);
+    static int resident[2 * TILINGS] = {};
+    const SpTiling &tl = SP_TILINGS[p.tiling];
+    const int which = p.mask ? TILINGS + p.tiling : p.tiling, threads = tl.threads();
+    void (*const kernels[2 * TILINGS])(SpParams) = {split_conv_kernel<0, false>, split_conv_kernel<1, false>, split_conv_kernel<2, false>,
+                                                    split_conv_kernel<0, true>, split_conv_kernel<1, true>, split_conv_kernel<2, true>};
     int &res = resident[which];
     if (res == 0) {
         int per_cu = 0;
         const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernels[which], threads, 0);
         if (e != hipSuccess || per_cu < 1) per_cu = 1;
-        const int all = per_cu * xsmi::cu_count(), cap = sp_max_grid(p.wc);
+        const int all = per_cu * xsmi::cu_count(), cap = tl.max_grid;
         res = (all > cap ? cap : all < 8 ? 8 : all) & ~7;
     }
     uint32_t grid = (uint32_t)res;
-    // A launch that does not fill the chip: n steps for each workgroup cost 0.45 us n, and the workgroup that adds a tile of
-    // I steps together about 0.9 us for each of the I / n - 1 others; the sum is smallest at n = sqrt(2 I).
-    uint32_t steps = 0;
-    for (int i = 0; i < p.ncls; ++i) steps = p.cls[i].iters > steps ? p.cls[i].iters : steps;
-    uint32_t least = 4;
-    while (least * least < 2 * steps) ++least;
+    const uint32_t least = sp_least(p);
     if (grid > p.units / least) grid = p.units / least;
     if (grid == 0) grid = 1;
     p.upg = p.units / grid; p.urem = p.units % grid;
