@@ -93,6 +93,44 @@ def test_split_weight_gradient_against_the_oracle(gpu, n, c, h, w, k, pad, accum
     assert rel_l2(gw.numpy(), dw_ref) <= TOL and rel_l2(gb.numpy(), db_ref) <= TOL
 
 
+@pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad", [
+    (1, 3, 3, 3, 2, 3, 3, 1, 1, 0),          # one output pixel; an octet of three channels
+    (2, 65, 7, 8, 63, 3, 3, 1, 1, 1),        # a channel past an octet, a filter short of a tile
+    (3, 20, 19, 23, 70, 7, 7, 2, 2, 3),      # strided, few filters past a tile of 64
+    (2, 20, 17, 13, 33, 3, 5, 2, 1, 1),      # strides and filter sides that differ
+    (2, 40, 15, 17, 24, 1, 1, 2, 2, 0),      # one tap across: slots are the columns that are read
+    (2, 18, 12, 12, 24, 2, 2, 3, 3, 0),      # columns between the taps
+    (1, 8, 20, 40, 130, 15, 16, 1, 1, 7),    # the widest filter that is served but one
+    (7, 5, 9, 1, 40, 3, 1, 2, 1, 1),         # one input column: rows of three slots
+    (4, 24, 5, 4, 40, 5, 5, 1, 1, 2),        # rows of four pixels, many row and image ends in a stage
+    (2, 24, 1, 70, 16, 1, 7, 1, 1, 3),       # one row, padding above and below it only
+    (3, 96, 9, 9, 8, 3, 3, 1, 1, 2),         # more padding than the filter needs
+    (9, 64, 14, 14, 128, 3, 3, 1, 1, 1),     # uneven splits
+    (40, 96, 14, 15, 200, 3, 3, 2, 2, 1),    # eight to thirty-one splits
+    (2, 12, 60, 60, 24, 5, 5, 1, 1, 2),      # many splits
+    (1, 8, 3, 2700, 8, 1, 3, 1, 1, 0),       # rows that 24-bit division does not hold: the fp32 kernels
+])
+def test_split_weight_gradient_of_any_filter(gpu, n, c, h, w, k, r, s, sh, sw, pad):
+    """Against the oracle, with ordinary values, and with values that are not finite in both operands: the workgroups that meet
+    them form their sums again."""
+    K = gpu.kernels
+    x, wt, b, dy, _ = _data(n, c, h, w, k, r, s, sh, sw, pad, gpu)
+    for finite in (True, False):
+        if not finite:
+            x[-1, c // 2, h // 2, w // 2] = np.nan
+            dy[0, k // 2, dy.shape[2] // 2, -1] = np.inf
+        _, col = oracle.conv2d_fwd(x, wt, b, (sh, sw), pad)
+        with np.errstate(all="ignore"):
+            _, ref, db_ref = oracle.conv2d_bwd(dy, x.shape, wt, col, (sh, sw), pad, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+        with split_everywhere(gpu):
+            gw, gb = K.conv2d_bwd_weight(gpu.to_device(dy), gpu.to_device(x), wt.shape, (sh, sw), pad, want_db=True)
+        for got, want in ((gw.numpy(), ref), (gb.numpy(), db_ref)):
+            for test in (np.isnan, np.isposinf, np.isneginf):
+                np.testing.assert_array_equal(test(got), test(want))
+            calm = np.isfinite(want)
+            assert not calm.any() or rel_l2(got[calm], want[calm]) <= TOL
+
+
 @pytest.mark.parametrize("w,pad", [(56, 1), (7, 1)])       # stages of two rows and of four
 @pytest.mark.parametrize("relu", [False, True])
 def test_weight_gradient_rounds_to_both_sides(gpu, w, pad, relu):

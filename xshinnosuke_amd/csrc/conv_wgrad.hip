@@ -299,9 +299,10 @@ int xsmi_conv2d_bwd_weight(const float *dy, const float *x, float *dw, float *db
     if (xsmi::stem_wgrad_ok(N, C, H, W, K, R, S, sh, sw, pad) && ((uintptr_t)dy & 15) == 0 &&
         workspace_bytes >= xsmi::stem_wgrad_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad))
         return xsmi::stem_conv_bwd_weight(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, OH, OW, beta == 1.f ? 1 : 0, workspace);
-    const size_t split_need = xsmi::split_wgrad_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, (flags & XSMI_CONV_BF16) != 0);
-    if (split_need && workspace_bytes >= split_need)
-        return xsmi::split_conv_bwd_weight(dy, x, dw, db, N, C, H, W, K, pad, OH, OW, beta == 1.f ? 1 : 0, workspace);
+    bool served;
+    const int rs = xsmi::split_conv_bwd_weight(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, (flags & XSMI_CONV_BF16) != 0,
+                                               beta == 1.f ? 1 : 0, workspace, workspace_bytes, served);
+    if (served) return rs;
     if (xsmi::wgrad_tap_ok(dy, x, C, K, OH, OW))
         return xsmi::wgrad_tap(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, OH, OW, beta == 1.f ? 1 : 0, workspace);
 

@@ -13,13 +13,11 @@ typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
 template <int N>
 using IC = std::integral_constant<int, N>;
 
-// two floats, or with NEGATIVE their negatives, -> bf16 pair (nearest even); the pair's values taken off the floats
-// (v_dot2_f32_bf16 with (-1, 0) and (0, -1): one instruction for a subtraction and the widening in front of it; the
-// difference is representable, so it is exact.  The negative is a modifier of the conversion and other constants.)
-template <bool NEGATIVE = false>
+// two floats -> bf16 pair (nearest even); the pair's values taken off the floats (v_dot2_f32_bf16 with (-1, 0) and (0, -1): one
+// instruction for a subtraction and the widening in front of it; the difference is representable, so it is exact)
 __device__ __forceinline__ uint32_t split_pair(float &a, float &b) {
-    const bf16x2 p = {(__bf16)(NEGATIVE ? -a : a), (__bf16)(NEGATIVE ? -b : b)}, hi = {(__bf16)0.f, (__bf16)(NEGATIVE ? 1.f : -1.f)};
-    uint32_t lo_bits = NEGATIVE ? 0x00003f80u : 0x0000bf80u;   // (-1, 0), kept from the compiler: as an inline constant -1.0
+    const bf16x2 p = {(__bf16)a, (__bf16)b}, hi = {(__bf16)0.f, (__bf16)-1.f};
+    uint32_t lo_bits = 0x0000bf80u;                            // (-1, 0), kept from the compiler: as an inline constant -1.0
     asm("" : "+s"(lo_bits));                                   // it comes out as (0, -1)
     const bf16x2 lo = __builtin_bit_cast(bf16x2, lo_bits);
     a = __builtin_amdgcn_fdot2_f32_bf16(p, lo, a, false);
@@ -27,12 +25,11 @@ __device__ __forceinline__ uint32_t split_pair(float &a, float &b) {
     return __builtin_bit_cast(uint32_t, p);
 }
 
-// two floats, or their negatives, -> the three bf16 pairs of their split
-template <bool NEGATIVE = false>
+// two floats -> the three bf16 pairs of their split
 __device__ __forceinline__ void split_pair3(float a, float b, uint32_t &p0, uint32_t &p1, uint32_t &p2) {
-    p0 = split_pair<NEGATIVE>(a, b);
-    p1 = split_pair<NEGATIVE>(a, b);
-    const bf16x2 l = {(__bf16)(NEGATIVE ? -a : a), (__bf16)(NEGATIVE ? -b : b)};
+    p0 = split_pair(a, b);
+    p1 = split_pair(a, b);
+    const bf16x2 l = {(__bf16)a, (__bf16)b};
     p2 = __builtin_bit_cast(uint32_t, l);
 }
 

@@ -162,10 +162,11 @@ int split_conv_fwd(const float *x, const float *w, const float *bias, float *y, 
 int split_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, int H, int W, int K, int R, int S, int sh,
                         int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace);
 
-// weight gradient of 3 x 3, stride-1 layers with at most one pixel of padding, likewise (conv_split_wgrad.hip)
+// weight gradient, likewise (conv_split_wgrad.hip): filters up to 16 x 16, any stride; `served` is false, and nothing done, for a
+// geometry or a workspace that it does not serve
 size_t split_wgrad_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, bool bf16);
-int split_conv_bwd_weight(const float *dy, const float *x, float *dw, float *db, int N, int C, int H, int W, int K, int pad, int OH,
-                          int OW, int accumulate, void *workspace);
+int split_conv_bwd_weight(const float *dy, const float *x, float *dw, float *db, int N, int C, int H, int W, int K, int R, int S, int sh,
+                          int sw, int pad, bool bf16, int accumulate, void *workspace, size_t workspace_bytes, bool &served);
 
 // forward for very few input channels (conv_stem.hip): 1 or 3 channels, square filter of 3, 5 or 7, horizontal stride 2;
 // the workspace holds the packed filter followed by a zero-bordered copy of the input
