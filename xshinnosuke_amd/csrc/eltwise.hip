@@ -130,15 +130,21 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
                        (char *)workspace_dw + workspace_dw_bytes <= (char *)workspace,
                    "xsmi_conv2d_bwd: the two workspaces overlap");
     const unsigned kflags = flags & XSMI_CONV_BF16;
-    // The two kernels share only their inputs.  XSMI_CONV_DW_ASYNC: the weight gradient goes to the second stream
-    // and stays there; the main stream runs on (data gradient, then whatever the caller enqueues next: the
-    // memory-bound passes between two convolutions of a backward sweep fit beside a matrix-bound kernel) until
-    // xsmi_conv2d_bwd_join.  Without the flag the call is complete in main-stream order when it returns: where the
-    // data gradient's grid (128-pixel x 64-channel tiles) leaves compute units idle the weight gradient still runs
-    // beside it (6-9 % less time for both at 7x7 and 14x14 feature maps) and is joined at once; grids that fill the
-    // chip alone only get in each other's way (15 % more time at 56x56) and run one after the other.
+    // The two kernels share only their inputs.  On the second stream (XSMI_CONV_DW_ASYNC: until xsmi_conv2d_bwd_join, otherwise
+    // joined at once) the weight gradient runs beside what follows, but the fork and the join cost the host 18 us each, and the
+    // split-operand kernels fill the chip alone.  In order on the main stream therefore, but for
+    //   a bf16 data gradient whose grid (128-pixel x 64-channel tiles) leaves compute units idle, from 4e8 products on (both
+    //     gradients, beside -> in order: 512 -> 512 at 7 x 7, N=32: 168 -> 212 us; 256 -> 224 at 14 x 14, N=8: 78 -> 90; below, 48 -> 64
+    //     at 28 x 28, N=16: 56 -> 51);
+    //   layers of 2e9 products or more of a sweep that goes on, in float32 too: the passes between the convolutions find room
+    //     (ResNet-18 steps: 224 x 224, N=32, 3.7e9 products a layer: 3.72 -> 4.01 ms; 192 x 192, 2.7e9: 3.13 -> 3.45; 224 x 224, N=16,
+    //     1.85e9: 3.00 -> 2.76; 56 x 56, N=32: 3.01 -> 2.56).  A layer by itself is faster in order (64 -> 64 at 56 x 56, N=32, 3.7e9,
+    //     forward and backward: 183 -> 164; 64 -> 64 at 17 x 8, N=8: 98 -> 56).
+    // Behind a weight gradient that is still on the second stream an asynchronous one goes there too, whatever its size.
     const bool async = (flags & XSMI_CONV_DW_ASYNC) != 0;
-    const bool beside = async || xsmi::data_gradient_tiles(N, C, H, W) <= xsmi::cu_count();
+    const double products = (double)N * OH * OW * C * K * R * S;
+    const bool idle_units = kflags && xsmi::data_gradient_tiles(N, C, H, W) <= xsmi::cu_count();
+    const bool beside = (idle_units && products >= 4e8) || (async && (products >= 2e9 || xsmi::side_pending()));
     int rc = beside ? xsmi::side_begin() : xsmi::side_join();    // in main-stream order: after any earlier async work
     if (rc) return rc;
     rc = xsmi_conv2d_bwd_weight(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, beta_dw, kflags, workspace_dw, workspace_dw_bytes);
