@@ -271,6 +271,10 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w,
 /* The main stream waits for everything on the second stream (weight gradients that xsmi_conv2d_bwd
  * left there, filter layouts of xsmi_conv2d_pack); a no-op when there is nothing. */
 int xsmi_conv2d_bwd_join(void);
+/* 1 while the second stream holds work that the main stream does not wait for yet, else 0.  Right after
+ * xsmi_conv2d_bwd with XSMI_CONV_DW_ASYNC: whether that weight gradient is there (otherwise it was enqueued
+ * in order, behind a join of whatever was there before, and there is nothing to keep or to wait for). */
+int xsmi_conv2d_bwd_pending(void);
 
 /* Lay filters out ahead of time.  Every conv call first rewrites w into the layout its kernel reads
  * (a few microseconds of a tiny launch in front of each of the ~40 convolution passes of a ResNet-18

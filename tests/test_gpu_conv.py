@@ -202,15 +202,24 @@ def test_conv_bf16_forward_channels_last(gpu, n, c, h, w, k, r, s, sh, sw, pad):
     assert rel_l2(y0 + b.reshape(1, -1, 1, 1), pre_ref) <= TOL
 
 
-@pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad", [CASES[2], CASES[4], CASES[6], CASES[9], CASES[11]])
+BESIDE = (32, 64, 56, 56, 64, 3, 3, 1, 1, 1)    # 3.7e9 products: asked to, the library leaves the weight gradient on its second stream
+
+
+def _left_beside():
+    from xshinnosuke_amd.backend import capi
+    pending = bool(capi.lib.raw("xsmi_conv2d_bwd_pending")())
+    assert capi.side_pending() == pending            # the operands are kept exactly as long as the library's stream is not joined
+    return pending
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad", [CASES[2], CASES[4], CASES[6], CASES[9], CASES[11], BESIDE])
 @pytest.mark.parametrize("accumulate", [False, True])
 @pytest.mark.parametrize("async_dw", [False, True])
 def test_conv_both_gradients_in_one_call(gpu, n, c, h, w, k, r, s, sh, sw, pad, accumulate, async_dw):
     """xsmi_conv2d_bwd runs the two backward kernels on two streams: same bits as the two calls one after the
     other, also when adding into gradients that are already there, and twice in a row (the second call's kernels
-    must wait for the first call's).  With async_dw the weight gradient is still on the second stream when the call
-    returns; reading it back joins first."""
-    from xshinnosuke_amd.backend import capi
+    must wait for the first call's).  With async_dw the weight gradient of a large layer is still on the second stream
+    when the call returns, that of a small one has been enqueued in order; reading it back joins first."""
     K = gpu.kernels
     rng = np.random.default_rng(77 + c + k)
     x = gpu.to_device(rng.standard_normal((n, c, h, w)).astype(np.float32))
@@ -225,20 +234,19 @@ def test_conv_both_gradients_in_one_call(gpu, n, c, h, w, k, r, s, sh, sw, pad, 
         K.conv2d_bwd_data(dy, wt, x.shape, (sh, sw), pad, dx=a[0], accumulate=accumulate)
     for dy in dys:
         K.conv2d_bwd(dy, x, wt, b[0], b[1], b[2], (sh, sw), pad, accumulate=accumulate, async_dw=async_dw)
-        assert capi.side_pending() == async_dw
+        assert _left_beside() == (async_dw and (n, c, h, w, k, r, s, sh, sw, pad) == BESIDE)
     for u, v in zip(a, b):
         assert np.array_equal(u.numpy(), v.numpy())
-    assert not capi.side_pending()
+    assert not _left_beside()
 
 
 def test_conv_async_weight_gradient_is_joined_before_use(gpu):
     """Whatever touches the weight gradient after an asynchronous xsmi_conv2d_bwd (an optimizer update, the plain
     weight-gradient entry point adding into the same buffer) sees it complete; the passes of a backward sweep that
     cannot touch it do not wait."""
-    from xshinnosuke_amd.backend import capi
     K = gpu.kernels
     rng = np.random.default_rng(5)
-    n, c, h, k = 8, 64, 28, 64
+    n, c, h, _, k = BESIDE[:5]
     x = gpu.to_device(rng.standard_normal((n, c, h, h)).astype(np.float32))
     wt = gpu.to_device(he_normal(rng, (k, c, 3, 3)))
     dy = gpu.to_device(rng.standard_normal((n, k, h, h)).astype(np.float32))
@@ -252,20 +260,44 @@ def test_conv_async_weight_gradient_is_joined_before_use(gpu):
         mask = gpu.to_device(np.zeros(x.shape, np.uint8))
         K.conv2d_bwd(dy, x, wt, dx, dw, None, (1, 1), 1, async_dw=True)
         K.relu_mask_bwd(dx, mask, dx=other)                  # a pass of the sweep: does not join
-        assert capi.side_pending()
+        assert _left_beside()
         if use == "axpy":
             p = gpu.to_device(np.zeros(wt.shape, np.float32))
             K.axpy(p, dw, 1.0)
-            assert not capi.side_pending()
+            assert not _left_beside()
             np.testing.assert_array_equal(p.numpy(), ref)
         elif use == "bwd_weight":
             K.conv2d_bwd_weight(dy, x, wt.shape, (1, 1), 1, dw=dw, accumulate=True)
-            assert not capi.side_pending()
+            assert not _left_beside()
             np.testing.assert_array_equal(dw.numpy(), twice.numpy())
         else:
             gpu.synchronize()
-            assert not capi.side_pending()
+            assert not _left_beside()
             np.testing.assert_array_equal(dw.numpy(), ref)
+
+
+def test_conv_async_weight_gradients_of_a_sweep_share_the_second_stream(gpu):
+    """Layers of a backward sweep, large and small, each with a gradient of its own and one workspace for all: a small layer's
+    runs in order, unless a large one's is still on the second stream, behind which it goes.  Same bits as one at a time."""
+    K = gpu.kernels
+    rng = np.random.default_rng(11)
+    small = (4, 64, 20, 20, 96, 3, 3, 1, 1, 1)
+    layers, left = [small, BESIDE, small, BESIDE, (2, 16, 9, 9, 24, 5, 5, 2, 2, 2)], []
+    data = []
+    for n, c, h, w, k, r, s, sh, sw, pad in layers:
+        oh, ow = K.conv_out_hw(h, w, r, s, (sh, sw), pad)
+        data.append([gpu.to_device(v.astype(np.float32)) for v in (rng.standard_normal((n, k, oh, ow)), rng.standard_normal((n, c, h, w)),
+                                                                   rng.standard_normal((k, c, r, s)))])
+    want = [K.conv2d_bwd_weight(dy, x, w.shape, g[7:9], g[9], want_db=True) for g, (dy, x, w) in zip(layers, data)]
+    got = [(gpu.empty(w.shape), gpu.empty((w.shape[0],))) for _, _, w in data]
+    for g, (dy, x, w), (dw, db) in zip(layers, data, got):
+        K.conv2d_bwd(dy, x, w, gpu.empty(x.shape), dw, db, g[7:9], g[9], async_dw=True)
+        left.append(_left_beside())
+    assert left == [False, True, True, True, True]
+    for a, b in zip(want, got):
+        for u, v in zip(a, b):
+            np.testing.assert_array_equal(u.numpy(), v.numpy())
+    assert not _left_beside()
 
 
 def test_conv_packed_workspace_flag(gpu):

@@ -82,22 +82,28 @@ def test_resnet18_trains_on_device():
 
 
 def test_resnet18_steps_do_not_depend_on_the_weight_gradient_overlap(monkeypatch):
-    """Conv layers leave their weight gradients running on the backend's second stream across the backward sweep.
-    Three SGD steps with that overlap and three with every weight gradient joined at once end in the same bits."""
-    from xshinnosuke_amd.backend import kernels as K
+    """The layers of a large network leave their weight gradients running on the backend's second stream across the
+    backward sweep.  Three SGD steps with that overlap and three with every weight gradient in order end in the same bits."""
+    from xshinnosuke_amd.backend import capi, kernels as K
+    left = []
 
     def run(overlap):
-        if not overlap:
-            plain = K.conv2d_bwd
-            monkeypatch.setattr(K, "conv2d_bwd", lambda *a, **kw: plain(*a, **dict(kw, async_dw=False)))
+        plain = K.conv2d_bwd
+
+        def conv2d_bwd(*a, **kw):
+            out = plain(*a, **(kw if overlap else dict(kw, async_dw=False)))
+            left.append(capi.lib.raw("xsmi_conv2d_bwd_pending")())
+            return out
+        monkeypatch.setattr(K, "conv2d_bwd", conv2d_bwd)
+        del left[:]
         np.random.seed(3)
-        X = np.random.randn(8, 3, 64, 64).astype(np.float32)
-        Y = np.random.randint(0, 10, (8,))
-        net = ResNet18(classes=10, pool=2).to('cuda')
+        X = np.random.randn(32, 3, 224, 224).astype(np.float32)     # 3.7e9 products in most layers
+        Y = np.random.randint(0, 10, (32,))
+        net = ResNet18(classes=10, pool=7).to('cuda')
         x, y = xs.tensor(X).to('cuda'), xs.tensor(Y).to('cuda')
         net(x)
         xs.GLOBAL.INPUTS = None
-        opt = SGD(net.parameters(), lr=0.05)
+        opt = SGD(net.parameters(), lr=0.01)
         crit = xs.nn.CrossEntropyLoss()
         losses = []
         for _ in range(3):
@@ -109,6 +115,7 @@ def test_resnet18_steps_do_not_depend_on_the_weight_gradient_overlap(monkeypatch
         out = [p.numpy().copy() for p in _named_params(net)]
         monkeypatch.undo()
         xs.GLOBAL.INPUTS = None
+        assert np.isfinite(losses).all() and any(left) == overlap
         return losses, out
 
     la, pa = run(True)

@@ -16,6 +16,7 @@ class _Recorder:
         self.calls = []
         self.next_address = 0x7000_0000_0000
         self.unpackable = set()          # passes whose jobs report "nothing to lay out ahead"
+        self.side_pending = 0            # what the library says of its second stream
 
     def raw(self, name):
         if name == "xsmi_is_initialized":
@@ -24,6 +25,8 @@ class _Recorder:
             return lambda *dims: 1 << 16
         if name == "xsmi_conv2d_pass_workspace_bytes":
             return lambda *dims_pass_flags: 1 << 12
+        if name == "xsmi_conv2d_bwd_pending":
+            return lambda: self.side_pending
         if name == "xsmi_last_error":
             return lambda: b""
         raise AssertionError(name)
@@ -123,6 +126,19 @@ def test_a_filter_layout_is_current_exactly_until_the_filter_address_is_handed_o
     # another geometry of the same filter is a layout of its own
     other, current = K._layout_for(w, 0, [8] + dims[1:])
     assert other is not entry and not current
+
+
+def test_operands_are_kept_only_for_a_weight_gradient_that_the_library_left_on_its_second_stream(recorder):
+    x, dy, w, dx, dw = (dev.empty(s) for s in ((2, 8, 6, 6), (2, 8, 6, 6), (8, 8, 3, 3), (2, 8, 6, 6), (8, 8, 3, 3)))
+    run = lambda **kw: K.conv2d_bwd(dy, x, w, dx, dw, None, (1, 1), 1, **kw)  # noqa: E731
+    run(async_dw=True)
+    assert not capi.side_pending()                    # ran in order: nothing to keep, nothing to wait for
+    recorder.side_pending = 1
+    run(async_dw=True); run(async_dw=True)
+    assert capi._side_hold == [(dy, x, dw, None)] * 2
+    recorder.side_pending = 0                         # a call in order joins what was there
+    run()
+    assert not capi.side_pending() and "xsmi_conv2d_bwd_join" not in recorder.calls
 
 
 def test_refresh_reuses_its_job_table_and_drops_layouts_nobody_used(recorder):

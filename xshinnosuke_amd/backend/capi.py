@@ -74,6 +74,7 @@ SIGNATURES = {
     "xsmi_conv2d_bwd_weight": (_i, [_vp, _vp, _vp, _vp] + _CONV_DIMS + [_f, _u, _vp, _sz]),
     "xsmi_conv2d_bwd": (_i, [_vp] * 6 + _CONV_DIMS + [_f, _f, _u, _vp, _sz, _vp, _sz]),
     "xsmi_conv2d_bwd_join": (_i, []),
+    "xsmi_conv2d_bwd_pending": (_i, []),
     "xsmi_conv2d_pack": (_i, [_i, _vp]),
     "xsmi_maxpool2d_fwd": (_i, [_vp, _vp, _vp] + [_i] * 8),
     "xsmi_maxpool2d_bwd": (_i, [_vp, _vp, _vp] + [_i] * 8 + [_f]),
@@ -170,7 +171,8 @@ class _Lib:
             raise XsmiError(msg)
 
 
-_QUERIES = frozenset(("xsmi_scratch_bytes", "xsmi_conv2d_workspace_bytes", "xsmi_conv2d_pass_workspace_bytes", "xsmi_bn_workspace_bytes", "xsmi_is_initialized", "xsmi_last_error"))
+_QUERIES = frozenset(("xsmi_scratch_bytes", "xsmi_conv2d_workspace_bytes", "xsmi_conv2d_pass_workspace_bytes", "xsmi_bn_workspace_bytes",
+                      "xsmi_conv2d_bwd_pending", "xsmi_is_initialized", "xsmi_last_error"))
 
 lib = _Lib()
 
@@ -183,8 +185,13 @@ _SIDE_SAFE = frozenset(("xsmi_conv2d_bwd", "xsmi_bn_bwd", "xsmi_relu_mask_bwd", 
                         "xsmi_maxpool2d_bwd", "xsmi_avgpool_bwd", "xsmi_conv2d_bwd_join"))
 
 
-def hold_side(*arrays):
-    _side_hold.append(arrays)
+def settle_side(*arrays):
+    """After xsmi_conv2d_bwd: its weight gradient's operands are kept if the library left it on the second stream;
+    otherwise that call has joined whatever was there, and nothing is kept any longer."""
+    if lib.raw("xsmi_conv2d_bwd_pending")():
+        _side_hold.append(arrays)
+    else:
+        del _side_hold[:]
 
 
 def side_pending():

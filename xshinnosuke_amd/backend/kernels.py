@@ -309,9 +309,10 @@ def conv2d_bwd_weight(dy, x, w_shape, stride=(1, 1), pad=0, dw=None, db=None, ac
 def conv2d_bwd(dy, x, w, dx, dw, db=None, stride=(1, 1), pad=0, accumulate=False, bf16=False, async_dw=False,
                keep_layout=False):
     """Both gradients of one layer in one call, into existing device buffers.  Same results as ``conv2d_bwd_weight``
-    followed by ``conv2d_bwd_data``.  ``async_dw=True`` leaves the weight gradient running on the library's second
-    stream beside whatever is enqueued next; dw and db are complete after ``capi.join_side()``, which every call into
-    the library performs by itself except the passes of a backward sweep that cannot touch them."""
+    followed by ``conv2d_bwd_data``.  With ``async_dw=True`` the library may leave the weight gradient running on its
+    second stream beside whatever is enqueued next, where that pays; dw and db are then complete after
+    ``capi.join_side()``, which every call into the library performs by itself except the passes of a backward sweep
+    that cannot touch them."""
     _f32(dy, "dy"); _f32(x, "x"); _f32(w, "w")
     dims = _dims(x.shape, w.shape, stride, pad)
     n, c, h, wd, k, r, s = dims[:7]
@@ -338,8 +339,8 @@ def conv2d_bwd(dy, x, w, dx, dw, db=None, stride=(1, 1), pad=0, accumulate=False
              beta_dx, beta_dw, flags, ws, ws_bytes, ws_dw, ws_dw_bytes)
     if layout is not None and not packed:
         layout.key = _filter_key(w)
-    if async_dw:
-        capi.hold_side(dy, x, dw, db)
+    if async_dw or capi.side_pending():
+        capi.settle_side(dy, x, dw, db)
     return dx, dw, db
 
 

@@ -349,6 +349,8 @@ int xsmi_conv2d_bwd_join(void) {
     return xsmi::check_device_error("xsmi_conv2d_bwd_join");
 }
 
+int xsmi_conv2d_bwd_pending(void) { return g_side_pending ? 1 : 0; }
+
 size_t xsmi_scratch_bytes(void) {
     return 2 * (xsmi::SK_SCRATCH_FLAG_BYTES + xsmi::SK_SCRATCH_PART_BYTES) + (size_t)XSMI_NOALLOC_SCRATCH_BYTES;
 }
