@@ -256,12 +256,14 @@ int xsmi_conv2d_bwd_weight(const float *dy, const float *x, float *dw, float *db
  * Without XSMI_CONV_DW_ASYNC the call is complete in stream order when it returns (the
  * library decides whether the two kernels run side by side or one after the other).
  * With it, dx is complete in stream order, but the weight gradient may keep running on the
- * second stream (layers below 2e9 products run in order) beside whatever is enqueued next, until xsmi_conv2d_bwd_join() (or
+ * second stream beside whatever is enqueued next, until xsmi_conv2d_bwd_join() (or
  * xsmi_sync(), xsmi_conv2d_bwd_weight() or a call of this function without the flag,
- * which join first).  Until then the caller must not free, write or hand to another
+ * which join first).  Whether it does is the library's choice, call by call and not by the
+ * size of the layer alone; a caller that passes the flag always joins, or asks
+ * xsmi_conv2d_bwd_pending().  Until then the caller must not free, write or hand to another
  * entry point: dw, db, workspace_dw (other than through further calls of this function,
- * which the second stream runs in order), and must not free or write dy and x. A
- * ResNet-18 step of 224 x 224 images at N=32 is 0.3 ms of 4.0 shorter for it. */
+ * which run in order with it), and must not free or write dy and x. A ResNet-18 step of
+ * 224 x 224 images at N=32 is 0.3 ms of 4.0 shorter for it. */
 int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w,
                     float *dx, float *dw, float *db,
                     int N, int C, int H, int W, int K, int R, int S,
