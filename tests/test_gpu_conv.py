@@ -290,8 +290,9 @@ def test_conv_async_weight_gradients_of_a_sweep_share_the_second_stream(gpu):
                                                                    rng.standard_normal((k, c, r, s)))])
     want = [K.conv2d_bwd_weight(dy, x, w.shape, g[7:9], g[9], want_db=True) for g, (dy, x, w) in zip(layers, data)]
     got = [(gpu.empty(w.shape), gpu.empty((w.shape[0],))) for _, _, w in data]
-    for g, (dy, x, w), (dw, db) in zip(layers, data, got):
-        K.conv2d_bwd(dy, x, w, gpu.empty(x.shape), dw, db, g[7:9], g[9], async_dw=True)
+    dxs = [gpu.empty(x.shape) for _, x, _ in data]        # here: an allocation that the pool does not serve joins
+    for g, (dy, x, w), dx, (dw, db) in zip(layers, data, dxs, got):
+        K.conv2d_bwd(dy, x, w, dx, dw, db, g[7:9], g[9], async_dw=True)
         left.append(_left_beside())
     assert left == [False, True, True, True, True]
     for a, b in zip(want, got):
