@@ -301,6 +301,25 @@ def test_conv_async_weight_gradients_of_a_sweep_share_the_second_stream(gpu):
     assert not _left_beside()
 
 
+@pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad,beside", [
+    (12, 64, 38, 38, 192, 3, 3, 1, 1, 1, True),      # 1.9e9 products, 136 tiles of a bf16 data gradient
+    (12, 64, 38, 38, 194, 3, 3, 1, 1, 1, False),     # no bf16 kernel for 194 filters: the data gradient fills the chip
+    (2, 64, 38, 38, 192, 3, 3, 1, 1, 1, False),      # 3.2e8 products
+])
+def test_conv_weight_gradient_beside_a_bf16_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad, beside):
+    """The second stream below 2e9 products: where there is a bf16 kernel for the data gradient, and it leaves units idle."""
+    K = gpu.kernels
+    rng = np.random.default_rng(k)
+    x, wt, dy = (gpu.to_device(rng.standard_normal(v).astype(np.float32)) for v in ((n, c, h, w), (k, c, r, s), (n, k, h, w)))
+    want_dw, _ = K.conv2d_bwd_weight(dy, x, wt.shape, (sh, sw), pad, bf16=True)
+    want_dx = K.conv2d_bwd_data(dy, wt, x.shape, (sh, sw), pad, bf16=True)
+    dx, dw = gpu.empty(x.shape), gpu.empty(wt.shape)
+    K.conv2d_bwd(dy, x, wt, dx, dw, None, (sh, sw), pad, bf16=True, async_dw=True)
+    assert _left_beside() == beside
+    np.testing.assert_array_equal(dx.numpy(), want_dx.numpy())
+    np.testing.assert_array_equal(dw.numpy(), want_dw.numpy())
+
+
 def test_conv_packed_workspace_flag(gpu):
     """XSMI_CONV_WS_PACKED: a repeated forward / backward-data call may skip laying the filter out again."""
     K = gpu.kernels

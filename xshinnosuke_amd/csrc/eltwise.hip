@@ -135,7 +135,8 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     // split-operand kernels fill the chip alone.  In order on the main stream therefore, but for
     //   a bf16 data gradient whose grid (128-pixel x 64-channel tiles) leaves compute units idle, from 4e8 products on (both
     //     gradients, beside -> in order: 512 -> 512 at 7 x 7, N=32: 168 -> 212 us; 256 -> 224 at 14 x 14, N=8: 78 -> 90; below, 48 -> 64
-    //     at 28 x 28, N=16: 56 -> 51);
+    //     at 28 x 28, N=16: 56 -> 51).  Under the flag, filters that no bf16 kernel takes have a split data gradient like float32
+    //     (96 -> 200 at 44 x 44, N=6: 107 -> 94; 160 -> 40, 5 x 5 at 51 x 51, N=3: 86 -> 74);
     //   layers of 2e9 products or more of a sweep that goes on, in float32 too: the passes between the convolutions find room
     //     (ResNet-18 steps: 224 x 224, N=32, 3.7e9 products a layer: 3.72 -> 4.01 ms; 192 x 192, 2.7e9: 3.13 -> 3.45; 224 x 224, N=16,
     //     1.85e9: 3.00 -> 2.76; 56 x 56, N=32: 3.01 -> 2.56).  A layer by itself is faster in order (64 -> 64 at 56 x 56, N=32, 3.7e9,
@@ -143,7 +144,7 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     // Behind a weight gradient that is still on the second stream an asynchronous one goes there too, whatever its size.
     const bool async = (flags & XSMI_CONV_DW_ASYNC) != 0;
     const double products = (double)N * OH * OW * C * K * R * S;
-    const bool idle_units = kflags && xsmi::data_gradient_tiles(N, C, H, W) <= xsmi::cu_count();
+    const bool idle_units = kflags && xsmi::tap_path_ok(K) && xsmi::data_gradient_tiles(N, C, H, W) <= xsmi::cu_count();
     const bool beside = (idle_units && products >= 4e8) || (async && (products >= 2e9 || xsmi::side_pending()));
     int rc = beside ? xsmi::side_begin() : xsmi::side_join();    // in main-stream order: after any earlier async work
     if (rc) return rc;
