@@ -619,12 +619,9 @@ static bool split_wgrad_serves(WgParams &p, int N, int C, int H, int W, int K, i
     // 14: 144 -> 103; 256 -> 256 at 14 x 14: 139 -> 118; 128 -> 128 at 28 x 28, N=8: 64 -> 59).  With four times as many filters as
     // channels this kernel stays ahead (64 -> 512 at 56 x 56, N=4: 153 us, tap 185), beside a float32 data gradient (512 -> 512, N=32:
     // 146, tap 163) or one that fills the chip by itself as well (N=128: 310, tap 453).  The table-driven fp32 kernel is too slow
-    // for that (64 -> 224 at 56 x 56, N=5: 99 us, table-driven 141; 96 -> 160, 5 x 5 at 40 x 40, N=4: 113, 158); it is kept under the
-    // flag for 3 x 3, stride 1 and whole chunks of channels without a bf16 data gradient, whose bits tests/test_gpu_conv_split.py
-    // states (64 -> 255 at 56 x 56, N=5: 173 us, 101 here).  The rule looks at the flag, so that both ways to ask for a weight
-    // gradient give the same bits.
-    const bool pinned = R == 3 && S == 3 && sh == 1 && sw == 1 && C % 64 == 0 && K % 32 != 0 && (double)N * OH * OW * C * K * R * S >= 1e9;
-    if (opt < 2 && bf16 && K < 4 * C && (pinned || (C % 64 == 0 && K % 64 == 0)) && data_gradient_tiles(N, C, H, W) <= cu_count()) return false;
+    // for that (64 -> 224 at 56 x 56, N=5: 99 us, table-driven 141; 96 -> 160, 5 x 5 at 40 x 40, N=4: 113, 158).  The rule looks at
+    // the flag, so that both ways to ask for a weight gradient give the same bits.
+    if (opt < 2 && bf16 && K < 4 * C && C % 64 == 0 && K % 64 == 0 && data_gradient_tiles(N, C, H, W) <= cu_count()) return false;
     return wg_plan(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
 }
 static size_t wg_ws_bytes(const WgParams &p) { return wg_part_bytes(p) + align_up((size_t)p.splits * p.K * sizeof(float), 256); }
