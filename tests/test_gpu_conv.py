@@ -301,20 +301,24 @@ def test_conv_async_weight_gradients_of_a_sweep_share_the_second_stream(gpu):
     assert not _left_beside()
 
 
-@pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad,beside", [
-    (12, 64, 38, 38, 192, 3, 3, 1, 1, 1, True),      # 1.9e9 products, 136 tiles of a bf16 data gradient
-    (12, 64, 38, 38, 194, 3, 3, 1, 1, 1, False),     # no bf16 kernel for 194 filters: the data gradient fills the chip
-    (2, 64, 38, 38, 192, 3, 3, 1, 1, 1, False),      # 3.2e8 products
+@pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad,bf16,beside", [
+    (12, 64, 38, 38, 192, 3, 3, 1, 1, 1, True, True),      # 1.9e9 products, 136 tiles of a bf16 data gradient
+    (12, 64, 38, 38, 194, 3, 3, 1, 1, 1, True, False),     # no bf16 kernel for 194 filters: the data gradient fills the chip
+    (2, 64, 38, 38, 192, 3, 3, 1, 1, 1, True, False),      # 3.2e8 products
+    (5, 64, 7, 8, 64, 15, 15, 1, 1, 7, False, True),       # a few workgroups with a long chain: 2.6e8, 3 tiles, 14400 for a sum
+    (5, 64, 7, 8, 64, 15, 15, 1, 1, 7, True, True),
+    (1, 64, 7, 8, 64, 15, 15, 1, 1, 7, False, False),      # 5e7
+    (5, 64, 7, 8, 64, 9, 9, 1, 1, 4, False, False),        # 5184 for a sum
 ])
-def test_conv_weight_gradient_beside_a_bf16_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad, beside):
-    """The second stream below 2e9 products: where there is a bf16 kernel for the data gradient, and it leaves units idle."""
+def test_conv_weight_gradient_beside_a_small_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad, bf16, beside):
+    """The second stream below 2e9 products: beside a data gradient that leaves compute units idle."""
     K = gpu.kernels
     rng = np.random.default_rng(k)
     x, wt, dy = (gpu.to_device(rng.standard_normal(v).astype(np.float32)) for v in ((n, c, h, w), (k, c, r, s), (n, k, h, w)))
-    want_dw, _ = K.conv2d_bwd_weight(dy, x, wt.shape, (sh, sw), pad, bf16=True)
-    want_dx = K.conv2d_bwd_data(dy, wt, x.shape, (sh, sw), pad, bf16=True)
+    want_dw, _ = K.conv2d_bwd_weight(dy, x, wt.shape, (sh, sw), pad, bf16=bf16)
+    want_dx = K.conv2d_bwd_data(dy, wt, x.shape, (sh, sw), pad, bf16=bf16)
     dx, dw = gpu.empty(x.shape), gpu.empty(wt.shape)
-    K.conv2d_bwd(dy, x, wt, dx, dw, None, (sh, sw), pad, bf16=True, async_dw=True)
+    K.conv2d_bwd(dy, x, wt, dx, dw, None, (sh, sw), pad, bf16=bf16, async_dw=True)
     assert _left_beside() == beside
     np.testing.assert_array_equal(dx.numpy(), want_dx.numpy())
     np.testing.assert_array_equal(dw.numpy(), want_dw.numpy())

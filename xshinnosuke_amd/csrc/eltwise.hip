@@ -137,6 +137,10 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     //     gradients, beside -> in order: 512 -> 512 at 7 x 7, N=32: 168 -> 212 us; 256 -> 224 at 14 x 14, N=8: 78 -> 90; below, 48 -> 64
     //     at 28 x 28, N=16: 56 -> 51).  Under the flag, filters that no bf16 kernel takes have a split data gradient like float32
     //     (96 -> 200 at 44 x 44, N=6: 107 -> 94; 160 -> 40, 5 x 5 at 51 x 51, N=3: 86 -> 74);
+    //   a data gradient of either precision with at most 16 such tiles and 9000 or more products for a sum, from 1e8 products on: a
+    //     few workgroups with a long chain each (float32, beside -> in order: 256 -> 64, 15 x 15 / 3 at 2 x 5, N=22: 101 -> 134; 64 ->
+    //     410, 5 x 5 at 4 x 4, N=28: 55 -> 63; 384 -> 200, 7 x 7 at 8 x 8, N=1: 75 -> 82; of 56 layers in both precisions 0.93 in the
+    //     mean and 1.02 at the worst; below 1e8 products 2 of 78 lose 12 %);
     //   layers of 2e9 products or more of a sweep that goes on, in float32 too: the passes between the convolutions find room
     //     (ResNet-18 steps: 224 x 224, N=32, 3.7e9 products a layer: 3.72 -> 4.01 ms; 192 x 192, 2.7e9: 3.13 -> 3.45; 224 x 224, N=16,
     //     1.85e9: 3.00 -> 2.76; 56 x 56, N=32: 3.01 -> 2.56).  A layer by itself is faster in order (64 -> 64 at 56 x 56, N=32, 3.7e9,
@@ -144,8 +148,10 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     // Behind a weight gradient that is still on the second stream an asynchronous one goes there too, whatever its size.
     const bool async = (flags & XSMI_CONV_DW_ASYNC) != 0;
     const double products = (double)N * OH * OW * C * K * R * S;
-    const bool idle_units = kflags && xsmi::tap_path_ok(K) && xsmi::data_gradient_tiles(N, C, H, W) <= xsmi::cu_count();
-    const bool beside = (idle_units && products >= 4e8) || (async && (products >= 2e9 || xsmi::side_pending()));
+    const long long tiles = xsmi::data_gradient_tiles(N, C, H, W);
+    const bool idle_units = kflags && xsmi::tap_path_ok(K) && tiles <= xsmi::cu_count();
+    const bool long_chain = tiles <= 16 && (double)K * R * S >= 9000;
+    const bool beside = (idle_units && products >= 4e8) || (long_chain && products >= 1e8) || (async && (products >= 2e9 || xsmi::side_pending()));
     int rc = beside ? xsmi::side_begin() : xsmi::side_join();    // in main-stream order: after any earlier async work
     if (rc) return rc;
     rc = xsmi_conv2d_bwd_weight(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, beta_dw, kflags, workspace_dw, workspace_dw_bytes);
