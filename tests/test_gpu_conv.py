@@ -309,12 +309,15 @@ def test_conv_async_weight_gradients_of_a_sweep_share_the_second_stream(gpu):
     (5, 64, 7, 8, 64, 15, 15, 1, 1, 7, True, True),
     (1, 64, 7, 8, 64, 15, 15, 1, 1, 7, False, False),      # 5e7
     (5, 64, 7, 8, 64, 9, 9, 1, 1, 4, False, False),        # 5184 for a sum
+    (29, 15, 25, 25, 160, 15, 15, 2, 2, 0, True, False),   # bf16, 142 tiles with 10240 for a sum
+    (5, 9, 55, 55, 128, 15, 15, 1, 1, 0, True, False),     # the same with 2.2e9 products
 ])
 def test_conv_weight_gradient_beside_a_small_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad, bf16, beside):
     """The second stream below 2e9 products: beside a data gradient that leaves compute units idle."""
     K = gpu.kernels
     rng = np.random.default_rng(k)
-    x, wt, dy = (gpu.to_device(rng.standard_normal(v).astype(np.float32)) for v in ((n, c, h, w), (k, c, r, s), (n, k, h, w)))
+    shapes = (n, c, h, w), (k, c, r, s), (n, k) + K.conv_out_hw(h, w, r, s, (sh, sw), pad)
+    x, wt, dy = (gpu.to_device(rng.standard_normal(v).astype(np.float32)) for v in shapes)
     want_dw, _ = K.conv2d_bwd_weight(dy, x, wt.shape, (sh, sw), pad, bf16=bf16)
     want_dx = K.conv2d_bwd_data(dy, wt, x.shape, (sh, sw), pad, bf16=bf16)
     dx, dw = gpu.empty(x.shape), gpu.empty(wt.shape)

@@ -136,7 +136,11 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     //   a bf16 data gradient whose grid (128-pixel x 64-channel tiles) leaves compute units idle, from 4e8 products on (both
     //     gradients, beside -> in order: 512 -> 512 at 7 x 7, N=32: 168 -> 212 us; 256 -> 224 at 14 x 14, N=8: 78 -> 90; below, 48 -> 64
     //     at 28 x 28, N=16: 56 -> 51).  Under the flag, filters that no bf16 kernel takes have a split data gradient like float32
-    //     (96 -> 200 at 44 x 44, N=6: 107 -> 94; 160 -> 40, 5 x 5 at 51 x 51, N=3: 86 -> 74);
+    //     (96 -> 200 at 44 x 44, N=6: 107 -> 94; 160 -> 40, 5 x 5 at 51 x 51, N=3: 86 -> 74).  Not where more
+    //     than 64 tiles have 9500 or more products for a sum of one residue class: started behind the weight gradient's workgroups,
+    //     several of them land on a unit and stay there, for a time beside which the weight gradient's is short (9 -> 128, 15 x 15 at
+    //     55 x 55, N=5: 1280 -> 883; 15 -> 160, 15 x 15 / 2 at 25 x 25, N=29: 506 -> 351).  Of 82 other bf16 layers beside costs 0.90 of in
+    //     order in the mean; five lose 10 % or more;
     //   a data gradient of either precision with at most 16 such tiles and 9000 or more products for a sum, from 1e8 products on: a
     //     few workgroups with a long chain each (float32, beside -> in order: 256 -> 64, 15 x 15 / 3 at 2 x 5, N=22: 101 -> 134; 64 ->
     //     410, 5 x 5 at 4 x 4, N=28: 55 -> 63; 384 -> 200, 7 x 7 at 8 x 8, N=1: 75 -> 82; of 56 layers in both precisions 0.93 in the
@@ -149,9 +153,11 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     const bool async = (flags & XSMI_CONV_DW_ASYNC) != 0;
     const double products = (double)N * OH * OW * C * K * R * S;
     const long long tiles = xsmi::data_gradient_tiles(N, C, H, W);
-    const bool idle_units = kflags && xsmi::tap_path_ok(K) && tiles <= xsmi::cu_count();
+    const bool few_tiles = kflags && xsmi::tap_path_ok(K) && tiles <= xsmi::cu_count();
+    const bool piles_up = few_tiles && tiles > 64 && (double)K * xsmi::ceil_div(R, sh) * xsmi::ceil_div(S, sw) >= 9500;
     const bool long_chain = tiles <= 16 && (double)K * R * S >= 9000;
-    const bool beside = (idle_units && products >= 4e8) || (long_chain && products >= 1e8) || (async && (products >= 2e9 || xsmi::side_pending()));
+    const bool pays = (few_tiles && products >= 4e8) || (long_chain && products >= 1e8) || (async && products >= 2e9);
+    const bool beside = (pays && !piles_up) || (async && xsmi::side_pending());
     int rc = beside ? xsmi::side_begin() : xsmi::side_join();    // in main-stream order: after any earlier async work
     if (rc) return rc;
     rc = xsmi_conv2d_bwd_weight(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, beta_dw, kflags, workspace_dw, workspace_dw_bytes);
