@@ -158,6 +158,32 @@ def test_weight_gradient_rounds_to_both_sides(gpu, w, pad, relu):
     assert rms[2] <= rms[0]
 
 
+@pytest.mark.parametrize("n,h,w,r,stride,pad,products", [      # at most, for an element of the gradient
+    (1, 1, 1, 3, 1, 1, 1), (1, 2, 2, 7, 2, 3, 1), (1, 7, 7, 7, 1, 0, 1), (1, 1, 2, 5, 1, 2, 2), (2, 1, 1, 3, 2, 1, 2), (1, 1, 3, 5, 1, 2, 3),
+    (1, 2, 2, 3, 1, 1, 4), (1, 3, 3, 7, 2, 3, 4),              # the last of the fp32 kernels'
+    (3, 1, 1, 3, 1, 1, 3), (2, 1, 2, 3, 1, 1, 4), (1, 3, 3, 3, 1, 1, 9), (1, 1, 8, 5, 1, 2, 8)])
+def test_weight_gradient_of_a_few_products(gpu, n, h, w, r, stride, pad, products):
+    """One product is rounded once, to nearest; a few are no further from 64 bits than the fp32 kernels' sums."""
+    c, k = 64, 96
+    rng = np.random.default_rng(n + h + w + r)
+    oh, ow = gpu.kernels.conv_out_hw(h, w, r, r, (stride, stride), pad)
+    x, dy = rng.standard_normal((n, c, h, w)).astype(np.float32), rng.standard_normal((n, k, oh, ow)).astype(np.float32)
+    xp = np.pad(x, ((0, 0), (0, 0), (pad, pad), (pad, pad))).astype(np.float64)
+    taps = [[xp[:, :, a:a + oh * stride:stride, b:b + ow * stride:stride] for b in range(r)] for a in range(r)]
+    assert max(int((t != 0).sum(axis=(0, 2, 3)).max()) for row in taps for t in row) == products
+    ref = np.stack([np.stack([np.einsum("nkhw,nchw->kc", dy.astype(np.float64), t) for t in row], 2) for row in taps], 2)
+    run = lambda: gpu.kernels.conv2d_bwd_weight(gpu.to_device(dy), gpu.to_device(x), (k, c, r, r), (stride, stride), pad)[0].numpy()  # noqa: E731
+    got = run()
+    old = gpu.set_option("conv_split", 0)
+    try:
+        fp32 = run()
+    finally:
+        gpu.set_option("conv_split", old)
+    assert rel_l2(got, ref) <= rel_l2(fp32, ref)
+    if products == 1:
+        np.testing.assert_array_equal(got, ref.astype(np.float32))
+
+
 FORMED_AGAIN = [   # what the kernel that forms sums again walks differently
     (1, 17, 16, 16, 65, 3, 3, 1, 1, 1),      # a channel and a row past their tiles
     (5, 1, 25, 41, 3, 2, 2, 1, 1, 0),        # one channel, even filter

@@ -613,6 +613,12 @@ static bool split_wgrad_serves(WgParams &p, int N, int C, int H, int W, int K, i
     const long opt = option(OPT_CONV_SPLIT);
     const int OH = (H + 2 * pad - R) / sh + 1, OW = (W + 2 * pad - S) / sw + 1;
     if (opt == 0 || (opt < 2 && !split_wgrad_pays(C, K, R, S, (double)N * OH * OW))) return false;
+    // Sums of one to a few products: what the bf16 MFMA rounds downwards has no other half to cancel against, and one fp32 product
+    // is rounded to nearest.  `most` products for an element of dw, N for a corner's: error against 64 bits, of that of the fp32
+    // kernels, 1.30 to 1.45 for one product, 1.05 to 1.27 for N = 1 and most = 2 to 4 or N = 2 and most = 2; 0.75 to 1.00 for all
+    // larger ones (11 filters, 9 maps, N = 1 to 16).
+    const double most = (double)N * (OH < ceil_div(H, sh) ? OH : ceil_div(H, sh)) * (OW < ceil_div(W, sw) ? OW : ceil_div(W, sw));
+    if (opt < 2 && N * most <= 4) return false;
     // A workgroup here fills a compute unit's LDS and registers.  A bf16 data gradient of few tiles, which is started beside the
     // weight gradient (xsmi_conv2d_bwd), then waits and lands on the first units that come free, several of its workgroups on
     // one: the fp32 tap kernel lets it in (both gradients, 512 -> 512 at 7 x 7, N=32: 241 -> 170 us; 256 -> 512, 3 x 3 / 2 at 14 x
