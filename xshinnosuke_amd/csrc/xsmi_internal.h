@@ -151,6 +151,8 @@ int sk_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, i
 // reduction channels that are no multiple of 32 (the channels-last forward takes up to 8), and what is left there is float32
 // precision by the table-driven kernel, which the split kernels beat (backward-data of 2 -> 400, 7 x 7 / 2 at 28 x 89, N=2:
 // 1712 -> 44 us; forward and backward-data of 48 -> 203, 7 x 7 at 14 x 57, N=5: 1033 -> 88; of 60 -> 48, 3 x 3 at 64 x 64, N=13: 144 -> 87).
+// The shortest sums pay for their precision: 24 -> 88, 2 x 2 at 20 x 20, N=43, 96 products: 18.9 -> 23.4 us, error 1.3e-7 -> 6e-8; equal
+// from 144 products on.
 inline bool split_may_serve(int reduce_channels, bool bf16) { return !bf16 || !tap_path_ok(reduce_channels); }
 
 // fp32 forward / backward-data on the bf16 matrix pipes, operands split into three bf16 values (conv_split.hip); the
