@@ -131,6 +131,60 @@ def test_split_weight_gradient_of_any_filter(gpu, n, c, h, w, k, r, s, sh, sw, p
             assert not calm.any() or rel_l2(got[calm], want[calm]) <= TOL
 
 
+@pytest.mark.parametrize("tile,dims", [    # filters, pixels of a stage, pairs of units, rounds of staging; a layer that fills it
+    (646422, (2, 20, 11, 13, 70, 3, 2, 1, 1, 1)), (646423, (2, 130, 11, 13, 40, 3, 1, 2, 2, 1)),
+    (646432, (2, 20, 11, 13, 40, 7, 7, 2, 2, 3)), (646433, (2, 20, 11, 13, 70, 3, 3, 2, 2, 1)),
+    (646442, (2, 20, 9, 26, 40, 5, 5, 1, 1, 2)), (646443, (2, 20, 11, 13, 40, 5, 5, 1, 1, 2)),
+    (646452, (2, 20, 9, 26, 40, 5, 5, 1, 1, 2)), (646453, (2, 20, 11, 13, 40, 7, 7, 2, 2, 3)),
+    (643222, (2, 20, 11, 13, 70, 3, 2, 3, 3, 1)), (643223, (2, 20, 11, 13, 70, 3, 2, 3, 3, 1)),
+    (643232, (2, 20, 11, 13, 70, 3, 3, 2, 2, 1)), (643233, (2, 41, 11, 13, 70, 3, 2, 3, 3, 1)),
+    (643242, (2, 41, 11, 13, 70, 3, 3, 2, 2, 1)), (643243, (2, 130, 11, 13, 40, 5, 1, 1, 1, 2)),
+    (643252, (2, 130, 11, 13, 40, 3, 2, 1, 1, 1)), (643253, (2, 90, 11, 13, 40, 3, 3, 2, 2, 1)),
+    (326422, (2, 20, 11, 13, 70, 3, 3, 1, 1, 1)), (326423, (2, 130, 11, 13, 40, 3, 2, 1, 1, 1)),
+    (326432, (2, 20, 11, 13, 40, 5, 5, 1, 1, 2)), (326433, (2, 20, 11, 13, 40, 7, 7, 2, 2, 3)),
+    (326442, (2, 20, 9, 26, 40, 7, 7, 1, 1, 3)), (326443, (2, 90, 11, 13, 40, 5, 5, 1, 1, 2)),
+    (326452, (2, 20, 9, 26, 40, 7, 7, 1, 1, 3)), (326453, (2, 130, 9, 26, 40, 5, 5, 1, 1, 2)),
+    (323222, (2, 20, 11, 13, 70, 3, 3, 2, 2, 1)), (323223, (2, 130, 11, 13, 40, 3, 2, 3, 3, 1)),
+    (323232, (2, 20, 11, 13, 40, 7, 7, 2, 2, 3)), (323233, (2, 130, 11, 13, 40, 3, 3, 2, 2, 1)),
+    (323242, (2, 20, 11, 13, 40, 7, 7, 2, 2, 3)), (323243, (2, 41, 15, 8, 40, 7, 7, 2, 2, 3)),
+    (323252, (2, 41, 9, 26, 40, 7, 7, 2, 2, 3)), (323253, (2, 41, 11, 13, 40, 7, 7, 2, 2, 3)),
+])
+def test_split_weight_gradient_of_every_tile(gpu, tile, dims):
+    """Each instantiation against the oracle: ordinary values, every sum formed again (powers of two are exact), and values that
+    are not finite in both operands."""
+    n, c, h, w, k, r, s, sh, sw, pad = dims
+    x, wt, b, dy, _ = _data(*dims, gpu)
+    run = lambda: gpu.kernels.conv2d_bwd_weight(gpu.to_device(dy), gpu.to_device(x), wt.shape, (sh, sw), pad, want_db=True)  # noqa: E731
+    old = gpu.set_option("conv_split", 0)
+    try:
+        fp32 = run()[0].numpy()
+    finally:
+        gpu.set_option("conv_split", old)
+    gpu.set_option("wgrad_tile", tile)
+    try:
+        with split_everywhere(gpu):
+            for values in ("ordinary", "small", "not finite"):
+                if values == "small":
+                    x, scale = x * np.float32(2.0 ** -107), 2.0 ** 107
+                elif values == "not finite":
+                    x, scale = x * np.float32(2.0 ** 107), 1.0
+                    x[-1, c // 2, h // 2, w // 2], dy[0, k // 2, dy.shape[2] // 2, -1] = np.nan, np.inf
+                else:
+                    scale = 1.0
+                _, col = oracle.conv2d_fwd(x * np.float32(scale), wt, b, (sh, sw), pad)
+                with np.errstate(all="ignore"):
+                    _, ref, db_ref = oracle.conv2d_bwd(dy, x.shape, wt, col, (sh, sw), pad, np.zeros_like(x), np.zeros_like(wt), np.zeros_like(b))
+                gw, gb = (a.numpy() for a in run())
+                assert values != "ordinary" or not np.array_equal(gw, fp32)      # a tile that does not fit leaves the call to them
+                for got, want in ((gw.astype(np.float64) * scale, ref), (gb, db_ref)):
+                    for test in (np.isnan, np.isposinf, np.isneginf):
+                        np.testing.assert_array_equal(test(got), test(want))
+                    calm = np.isfinite(want)
+                    assert not calm.any() or rel_l2(got[calm], want[calm]) <= TOL
+    finally:
+        gpu.set_option("wgrad_tile", 0)
+
+
 @pytest.mark.parametrize("w,pad", [(56, 1), (7, 1)])       # stages of two rows and of four
 @pytest.mark.parametrize("relu", [False, True])
 def test_weight_gradient_rounds_to_both_sides(gpu, w, pad, relu):
@@ -192,6 +246,8 @@ FORMED_AGAIN = [   # what the kernel that forms sums again walks differently
     (2, 48, 14, 15, 20, 3, 3, 2, 2, 1),      # four phases forward, four classes backward
     (2, 20, 17, 13, 70, 3, 5, 2, 1, 1),      # strides and filter sides that differ
     (1, 512, 7, 7, 512, 3, 3, 1, 1, 1),      # segments that begin and end anywhere in a tile
+    (17, 31, 56, 56, 31, 5, 5, 1, 1, 2),     # tiles of 32 x 512 in both passes, two images for five filter rows
+    (24, 33, 56, 57, 20, 5, 5, 2, 2, 2),     # 32 x 512 forward and strided
 ]
 
 

@@ -518,6 +518,7 @@ int wg_slots(const WgParams &p, int px) {
 // to 59 stages for each workgroup: 49 for each MFMA of a wave (and its neighbour on the SIMD), 264 for a round of staging, 250 for
 // the barrier; a partial result is written and read again at 0.6 ns a kilobyte.
 bool wg_plan(WgParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
+    const long only = xsmi::option(xsmi::OPT_WGRAD_TILE);      // tests run every tile
     memset(&p, 0, sizeof(p));
     if (R > MAX_TAPS || S > MAX_TAPS) return false;
     p.K = K; p.C = C; p.octets = xsmi::ceil_div(C, 8) * R; p.R = R; p.S = S; p.H = H; p.W = W; p.OH = OH; p.OW = OW; p.OHW = OH * OW;
@@ -531,6 +532,7 @@ bool wg_plan(WgParams &p, int N, int C, int H, int W, int K, int R, int S, int s
             if (ns > SMALL_PAST) continue;
             for (int NJ : {2, 3})
                 for (int P : {2, 3, 4, 5}) {
+                    if (only && only != KT * 10000 + PX * 100 + P * 10 + NJ) continue;
                     int subs = 256 * P / KT / S;       // units of a tile: 4 P by 64 rows, 8 P by 32
                     const int fit = (NJ * THREADS - y_items) / (2 * ns), all = xsmi::ceil_div(p.octets, 2);
                     if (subs > all) subs = all;

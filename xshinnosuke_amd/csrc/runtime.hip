@@ -41,6 +41,7 @@ OptionRow g_options[xsmi::OPT_COUNT] = {
     {"pool_bwd", "XSMI_POOL_BWD", 2, false},
     {"pack_lanes", "XSMI_PACK_LANES", 2, false},
     {"conv_split", "XSMI_CONV_SPLIT", 1, false},
+    {"wgrad_tile", "XSMI_WGRAD_TILE", 0, false},
 };
 
 // Streams beside the second one for runs of short independent launches (filter layouts), see side_lane().

@@ -30,7 +30,7 @@ bool capturing();            // a step graph is being recorded: nothing runs, no
 bool ready();
 int cu_count();
 // Tuning switches (xsmi_set_option / environment variable / default); the order is that of the table in runtime.hip.
-enum Option { OPT_TAP_SK, OPT_SK_SPIN_LIMIT, OPT_TAP_STAGES, OPT_TAP_PERSIST, OPT_CL_HALO, OPT_CL_STEM, OPT_SK_WIDE, OPT_POOL_BWD, OPT_PACK_LANES, OPT_CONV_SPLIT, OPT_COUNT };
+enum Option { OPT_TAP_SK, OPT_SK_SPIN_LIMIT, OPT_TAP_STAGES, OPT_TAP_PERSIST, OPT_CL_HALO, OPT_CL_STEM, OPT_SK_WIDE, OPT_POOL_BWD, OPT_PACK_LANES, OPT_CONV_SPLIT, OPT_WGRAD_TILE, OPT_COUNT };
 long option(Option o);
 // Partial tiles and flags of the convolution kernels that share tiles between workgroups, for the stream that stream() hands out; allocated
 // by xsmi_init, the flags are zero between launches.
