@@ -45,16 +45,16 @@ def _eager_noise(i):
     return out
 
 
-def _training_run(batches, graph_from=None):
+def _training_run(batches, graph_from=None, pool=2, lr=0.05):
     """Losses and final parameters of len(batches) SGD steps; from step `graph_from` on the step is a replay."""
     np.random.seed(11)
-    net = ResNet18(classes=10, pool=2).to('cuda')
+    net = ResNet18(classes=10, pool=pool).to('cuda')
     x = xs.tensor(batches[0][0]).to('cuda')
     y = xs.tensor(batches[0][1]).to('cuda')
     with xs.no_grad():
         net(x)                                    # creates the parameters
     xs.GLOBAL.INPUTS = None
-    opt = SGD(net.parameters(), lr=0.05)
+    opt = SGD(net.parameters(), lr=lr)
     crit = xs.nn.CrossEntropyLoss()
 
     def step():
@@ -88,10 +88,23 @@ def _training_run(batches, graph_from=None):
     return losses, params
 
 
-def test_replayed_training_steps_equal_eager_steps():
-    batches = _batches(6, 4, 64, 10, seed=5)
-    eager_losses, eager_params = _training_run(batches)
-    graph_losses, graph_params = _training_run(batches, graph_from=2)
+@pytest.mark.parametrize("n,size,pool,lr,beside", [
+    (4, 64, 2, 0.05, False),
+    (32, 224, 7, 0.01, True),                     # the weight gradients of most layers are on the second stream
+])
+def test_replayed_training_steps_equal_eager_steps(monkeypatch, n, size, pool, lr, beside):
+    left, plain = [], be.kernels.conv2d_bwd
+
+    def conv2d_bwd(*args, **kw):
+        out = plain(*args, **kw)
+        left.append(be.capi.lib.raw("xsmi_conv2d_bwd_pending")())
+        return out
+    monkeypatch.setattr(be.kernels, "conv2d_bwd", conv2d_bwd)
+    batches = _batches(6, n, size, 10, seed=5)
+    eager_losses, eager_params = _training_run(batches, pool=pool, lr=lr)
+    del left[:]
+    graph_losses, graph_params = _training_run(batches, graph_from=2, pool=pool, lr=lr)
+    assert any(left) == beside and np.isfinite(eager_losses).all()
     assert len(set(eager_losses)) == len(eager_losses)          # the steps really differ
     assert graph_losses == eager_losses
     assert len(graph_params) == len(eager_params) == 82
