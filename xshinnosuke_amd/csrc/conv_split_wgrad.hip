@@ -10,7 +10,8 @@
 // fragments are read transposed (ds_read_b64_tr_b16: sixteen lanes fetch four slots of sixteen entries, and each ends up with
 // the four values of its entry).  Every lane gives the place of its slot itself, so a tap, a stride and the end of a row are
 // nothing but addresses, and an MFMA's 32 columns are any two UNITS (sub-image, tap).  A slot is an input column; with one tap
-// across, only the columns that are read have slots.  No bank conflicts (counted).
+// across, only the columns that are read have slots.  Bank conflicts: none on large images, 1 to 6 % of a compute unit's cycles on rows
+// of 7 to 14 pixels and under a stride (counted).
 //
 // Workgroups of eight waves: KT filters by `subs` sub-images, a stage is PX pixels.  Waves are 2 x 2 (KT = 64) or 1 x 4 (32)
 // blocks of 32 rows by P pairs of units, twice: the second four take the second half of a stage's pixels, multiply with -dy and
@@ -19,12 +20,12 @@
 // they lie in the registers, and one launch adds them in ascending order in float64.
 //
 // Kernel and reduction, before (table-driven fp32 kernel, or one for 3 x 3, stride 1 alone that took neighbouring pixels as they lie
-// in memory) and now: 24 -> 40, 5 x 5 at 45 x 61, N=7: 39 -> 27 us; 32 -> 16, 7 x 7 at 109 x 109, N=5: 185 -> 55; 123 -> 296, 5 x 5
-// at 50 x 27, N=3: 157 -> 71; 96 -> 16, 3 x 3 at 81 x 81, N=12: 78 -> 48; 64 -> 64, 3 x 3 at 56 x 56, N=32: 69 -> 68, with a third of
-// the partial results.  What bounds it: 123 -> 296 runs 63 us at 1.9 GHz, the matrix pipes busy for 49 % of it (tiles a tenth larger
-// than the layer), the vector instructions of a SIMD's two waves as long again (splitting, 39 %, addresses, the sums), so that the
-// two hardly overlap; holding one half of the waves back or giving it priority changed nothing, a third image in the LDS with the
-// barrier in the middle of the MFMAs lost 10 % (smaller stages, more addresses).
+// in memory) and now: 24 -> 40, 5 x 5 at 45 x 61, N=7: 37 -> 26 us; 32 -> 16, 7 x 7 at 109 x 109, N=5: 179 -> 53; 123 -> 296, 5 x 5
+// at 50 x 27, N=3: 149 -> 63; 96 -> 16, 3 x 3 at 81 x 81, N=12: 75 -> 47.  3 x 3, stride 1, whole tiles: the kernel alone is 7 to 10 %
+// slower than the one before (64 -> 64 at 56 x 56, N=32: 50.1 -> 53.8), its reduction shorter (12.6 -> 6.0), the error half (2.2e-7 ->
+// 1.1e-7).  What bounds it, 123 -> 296: 55 us, the matrix pipes busy for 44 % of it, vector instructions (splitting, addresses, the
+// sums) issued for 50 %, and the two hardly overlap; holding one half of the waves back or giving it priority changed nothing, a
+// third image in the LDS with the barrier in the middle of the MFMAs lost 10 % (smaller stages, more addresses).
 #include "split3.h"
 
 #include <string.h>
@@ -515,8 +516,10 @@ int wg_slots(const WgParams &p, int px) {
 }
 
 // The tile, the stage and the split of the pixels with the least estimated time.  Nanoseconds of a stage, fitted to launches of 4
-// to 59 stages for each workgroup: 49 for each MFMA of a wave (and its neighbour on the SIMD), 264 for a round of staging, 250 for
-// the barrier; a partial result is written and read again at 0.6 ns a kilobyte.
+// to 59 stages for each workgroup: 55 for each MFMA of a wave (and its neighbour on the SIMD), 264 for a round of staging, 250 for
+// the barrier; a partial result is written and read again at 0.6 ns a kilobyte.  On 390 layers (ResNet-18's and drawn) the tile taken
+// is 3.6 % behind the fastest in the mean, 21 % at the worst.  Constants that fit better (42, 200, 700 and 0.8: 1.3 % and 16 %) prefer
+// stages of 64 pixels where two k-steps are added together, whose error is up to 1.5 times as large (5.7e-8 -> 8.2e-8).
 bool wg_plan(WgParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
     const long only = xsmi::option(xsmi::OPT_WGRAD_TILE);      // tests run every tile
     memset(&p, 0, sizeof(p));
@@ -616,8 +619,9 @@ namespace xsmi {
 //     40: 20 -> 24; 64 -> 256 at 56 x 56, N=32, on the tap kernel: 44 -> 70).
 //   channels and filters multiples of 64, on the tap kernel: from 512 pixels and 2.5e8 products on (64 -> 64 at 56 x 56, N=1: 13
 //     -> 17 us; 512 -> 512 at 3 x 3, N=32: 32 -> 34, at 7 x 7: 90 -> 65; 128 -> 256, 3 x 3 / 2 at 28 x 28: N=4 equal, N=32 52 -> 47).
-//   everything else: yes (32 -> 16, 7 x 7 at 109 x 109, N=5: 185 -> 57 us; 314 -> 32, 3 x 3 / 2 at 95 x 95, N=18: 249 -> 116; equal
-//     at the smallest sizes).
+//   everything else: yes (32 -> 16, 7 x 7 at 109 x 109, N=5: 179 -> 53 us; 314 -> 32, 3 x 3 / 2 at 95 x 95, N=18: 288 -> 86).  Below
+//     3e6 products equal in the mean (81 layers, up to a third slower: 288 -> 15, 7 x 7 / 2 at 4 x 2, N=7: 9.2 -> 12.2) at half of the
+//     fp32 kernels' error.
 static bool split_wgrad_pays(int C, int K, int R, int S, double pixels) {
     if (C < (S < 5 ? 8 : 5)) return false;
     const bool tap = C % 64 == 0 && K % 64 == 0;
