@@ -618,7 +618,8 @@ namespace xsmi {
 //   1 x 1: where the fp32 kernels have only the table-driven one, and 4096 results (96 -> 160 at 60 x 60, N=16: 59 -> 40 us; 20 ->
 //     40: 20 -> 24; 64 -> 256 at 56 x 56, N=32, on the tap kernel: 44 -> 70).
 //   channels and filters multiples of 64, on the tap kernel: from 512 pixels and 2.5e8 products on (64 -> 64 at 56 x 56, N=1: 13
-//     -> 17 us; 512 -> 512 at 3 x 3, N=32: 32 -> 34, at 7 x 7: 90 -> 65; 128 -> 256, 3 x 3 / 2 at 28 x 28: N=4 equal, N=32 52 -> 47).
+//     -> 17 us; 512 -> 512 at 3 x 3, N=32: 32 -> 34, at 7 x 7: 90 -> 65; 128 -> 256, 3 x 3 / 2 at 28 x 28: N=4 equal, N=32 47 -> 45;
+//     64 -> 128, 3 x 3 / 2 at 56 x 56, N=32: 43 -> 47, at half of the error).
 //   everything else: yes (32 -> 16, 7 x 7 at 109 x 109, N=5: 179 -> 53 us; 314 -> 32, 3 x 3 / 2 at 95 x 95, N=18: 288 -> 86).  Below
 //     3e6 products equal in the mean (81 layers, up to a third slower: 288 -> 15, 7 x 7 / 2 at 4 x 2, N=7: 9.2 -> 12.2) at half of the
 //     fp32 kernels' error.
