@@ -309,6 +309,8 @@ def test_conv_async_weight_gradients_of_a_sweep_share_the_second_stream(gpu):
     (5, 64, 7, 8, 64, 15, 15, 1, 1, 7, True, True),
     (1, 64, 7, 8, 64, 15, 15, 1, 1, 7, False, False),      # 5e7
     (5, 64, 7, 8, 64, 9, 9, 1, 1, 4, False, False),        # 5184 for a sum
+    (6, 90, 16, 30, 200, 7, 7, 2, 2, 3, False, True),      # 46 tiles, 9800 for a sum
+    (5, 200, 13, 13, 1000, 3, 3, 1, 1, 1, False, False),   # nine taps
     (29, 15, 25, 25, 160, 15, 15, 2, 2, 0, True, False),   # bf16, 142 tiles with 10240 for a sum
     (5, 9, 55, 55, 128, 15, 15, 1, 1, 0, True, False),     # the same with 2.2e9 products
 ])

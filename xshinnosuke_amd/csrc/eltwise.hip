@@ -141,10 +141,12 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     //     several of them land on a unit and stay there, for a time beside which the weight gradient's is short (9 -> 128, 15 x 15 at
     //     55 x 55, N=5: 1280 -> 883; 15 -> 160, 15 x 15 / 2 at 25 x 25, N=29: 506 -> 351).  Of 82 other bf16 layers beside costs 0.90 of in
     //     order in the mean; five lose 10 % or more;
-    //   a data gradient of either precision with at most 16 such tiles and 9000 or more products for a sum, from 1e8 products on: a
-    //     few workgroups with a long chain each (float32, beside -> in order: 256 -> 64, 15 x 15 / 3 at 2 x 5, N=22: 101 -> 134; 64 ->
-    //     410, 5 x 5 at 4 x 4, N=28: 55 -> 63; 384 -> 200, 7 x 7 at 8 x 8, N=1: 75 -> 82; of 56 layers in both precisions 0.93 in the
-    //     mean and 1.02 at the worst; below 1e8 products 2 of 78 lose 12 %);
+    //   a data gradient of either precision with at most 48 such tiles and filters of 25 taps or more that make 9000 or more products
+    //     for a sum, from 1e8 products on: a few workgroups with a long chain each (float32, beside -> in order: 256 -> 64, 15 x 15 / 3
+    //     at 2 x 5, N=22: 101 -> 134; 64 -> 410, 5 x 5 at 4 x 4, N=28: 55 -> 63; 90 -> 200, 7 x 7 / 2 at 16 x 30, N=6: 62 -> 76; 256 ->
+    //     300, 7 x 7 at 14 x 14, N=3: 116 -> 127.  Of 118 layers in both precisions 0.94 in the mean, two lose more than 2 %: 16 -> 96,
+    //     15 x 15 / 2 at 40 x 40, N=2: 67 -> 60.  Below 1e8 products and with smaller filters more lose: 200 -> 1000, 3 x 3 at 13 x 13,
+    //     N=5: 98 -> 87);
     //   layers of 2e9 products or more of a sweep that goes on, in float32 too: the passes between the convolutions find room
     //     (ResNet-18 steps: 224 x 224, N=32, 3.7e9 products a layer: 3.72 -> 4.01 ms; 192 x 192, 2.7e9: 3.13 -> 3.45; 224 x 224, N=16,
     //     1.85e9: 3.00 -> 2.76; 56 x 56, N=32: 3.01 -> 2.56).  A layer by itself is faster in order (64 -> 64 at 56 x 56, N=32, 3.7e9,
@@ -155,7 +157,7 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     const long long tiles = xsmi::data_gradient_tiles(N, C, H, W);
     const bool few_tiles = kflags && xsmi::tap_path_ok(K) && tiles <= xsmi::cu_count();
     const bool piles_up = few_tiles && tiles > 64 && (double)K * xsmi::ceil_div(R, sh) * xsmi::ceil_div(S, sw) >= 9500;
-    const bool long_chain = tiles <= 16 && (double)K * R * S >= 9000;
+    const bool long_chain = tiles <= 48 && R * S >= 25 && (double)K * R * S >= 9000;
     const bool pays = (few_tiles && products >= 4e8) || (long_chain && products >= 1e8) || (async && products >= 2e9);
     const bool beside = (pays && !piles_up) || (async && xsmi::side_pending());
     int rc = beside ? xsmi::side_begin() : xsmi::side_join();    // in main-stream order: after any earlier async work
