@@ -214,7 +214,7 @@ def test_weight_gradient_rounds_to_both_sides(gpu, w, pad, relu):
 
 @pytest.mark.parametrize("n,h,w,r,stride,pad,products", [      # at most, for an element of the gradient
     (1, 1, 1, 3, 1, 1, 1), (1, 2, 2, 7, 2, 3, 1), (1, 7, 7, 7, 1, 0, 1), (1, 1, 2, 5, 1, 2, 2), (2, 1, 1, 3, 2, 1, 2), (1, 1, 3, 5, 1, 2, 3),
-    (1, 2, 2, 3, 1, 1, 4), (1, 3, 3, 7, 2, 3, 4),              # the last of the fp32 kernels'
+    (1, 2, 2, 3, 1, 1, 4), (1, 3, 3, 7, 2, 3, 4),              # the last that are formed in float64
     (3, 1, 1, 3, 1, 1, 3), (2, 1, 2, 3, 1, 1, 4), (1, 3, 3, 3, 1, 1, 9), (1, 1, 8, 5, 1, 2, 8)])
 def test_weight_gradient_of_a_few_products(gpu, n, h, w, r, stride, pad, products):
     """One product is rounded once, to nearest; a few are no further from 64 bits than the fp32 kernels' sums."""

@@ -54,6 +54,7 @@ struct WgParams {
     int NS, subs, units;                              // slots of an octet in the LDS, sub-images of a tile, their units
     int kt, jt, splits, stages, per, rem;
     int KT, PX, P, NJ;
+    int few;                                          // sums of a few products: formed in float64
     uint32_t rOW, rOHW, rWx, rOH;                     // 2^23 over them, rounded up (small_div)
     xsmi::FastDiv dOW, dOH, dNS, dR;
 };
@@ -425,7 +426,7 @@ __global__ void __launch_bounds__(THREADS, 2) split_wgrad_kernel(WgParams p) {
         if (again) s_again = 1;
     }
     __syncthreads();
-    if (s_again) {
+    if (s_again || p.few) {
         xsmi::wait_vmcnt<0>();                        // what is overwritten now has been written
         __syncthreads();
         const int m1 = s1 * PX < p.M ? s1 * PX : p.M;
@@ -579,6 +580,13 @@ bool wg_plan(WgParams &p, int N, int C, int H, int W, int K, int R, int S, int s
     }
     if (best < 0 || (double)p.splits * p.kt * p.jt * 4096 * p.P * 4 >= 4e9) return false;
     p.per = p.stages / p.splits; p.rem = p.stages % p.splits;
+    // Sums of one to a few products: what the bf16 MFMA rounds downwards has no other half of the waves to cancel against, and one
+    // fp32 product is rounded to nearest.  `most` products for an element of dw, N for a corner's: error against 64 bits, of that of
+    // the fp32 kernels, 1.30 to 1.45 for one product, 1.05 to 1.27 for N = 1 and most = 2 to 4 or N = 2 and most = 2; 0.75 to 1.00
+    // for all larger ones (11 filters, 9 maps, N = 1 to 16).  Those few are formed in float64: 480 ->
+    // 416, 7 x 7 / 2 at 1 x 1, N=1: 67 -> 83 us (fp32 kernels 95); 452 -> 328, 3 x 3 / 2 at 5 x 2, N=1: 16.6 -> 19.7 (19.2).
+    const double most = (double)N * (OH < xsmi::ceil_div(H, sh) ? OH : xsmi::ceil_div(H, sh)) * (OW < xsmi::ceil_div(W, sw) ? OW : xsmi::ceil_div(W, sw));
+    p.few = N * most <= 4 ? 1 : 0;
     p.x_bytes = (uint32_t)((size_t)N * C * H * W * 4); p.dy_bytes = (uint32_t)((size_t)N * K * OH * OW * 4);
     auto last = [](uint32_t bytes, int plane) { const uint32_t e = (bytes / 4u - 1u) / (uint32_t)plane; return (int)(e < 7u ? e : 7u); };
     p.x_last = last(p.x_bytes, p.plane); p.dy_last = last(p.dy_bytes, p.OHW);
@@ -635,12 +643,6 @@ static bool split_wgrad_serves(WgParams &p, int N, int C, int H, int W, int K, i
     const long opt = option(OPT_CONV_SPLIT);
     const int OH = (H + 2 * pad - R) / sh + 1, OW = (W + 2 * pad - S) / sw + 1;
     if (opt == 0 || (opt < 2 && !split_wgrad_pays(C, K, R, S, (double)N * OH * OW))) return false;
-    // Sums of one to a few products: what the bf16 MFMA rounds downwards has no other half to cancel against, and one fp32 product
-    // is rounded to nearest.  `most` products for an element of dw, N for a corner's: error against 64 bits, of that of the fp32
-    // kernels, 1.30 to 1.45 for one product, 1.05 to 1.27 for N = 1 and most = 2 to 4 or N = 2 and most = 2; 0.75 to 1.00 for all
-    // larger ones (11 filters, 9 maps, N = 1 to 16).
-    const double most = (double)N * (OH < ceil_div(H, sh) ? OH : ceil_div(H, sh)) * (OW < ceil_div(W, sw) ? OW : ceil_div(W, sw));
-    if (opt < 2 && N * most <= 4) return false;
     // A workgroup here fills a compute unit's LDS and registers.  A bf16 data gradient of few tiles, which is started beside the
     // weight gradient (xsmi_conv2d_bwd), then waits and lands on the first units that come free, several of its workgroups on
     // one: the fp32 tap kernel lets it in (both gradients, 512 -> 512 at 7 x 7, N=32: 241 -> 170 us; 256 -> 512, 3 x 3 / 2 at 14 x
