@@ -72,13 +72,13 @@ def test_split_convolution_against_the_oracle(gpu, n, c, h, w, k, r, s, sh, sw, 
 
 @pytest.mark.parametrize("n,c,h,w,k,pad", [
     (1, 3, 3, 3, 2, 0),                      # one output pixel
-    (2, 65, 7, 8, 63, 1),                    # rows of one octet; a channel past its tile, a filter short of it
-    (3, 16, 5, 9, 64, 1),                    # the first width of two octets; odd rows
-    (2, 64, 6, 7, 64, 0),                    # no padding: the columns of dy begin two early
-    (3, 20, 11, 17, 70, 0),                  # two column blocks, the second with one column
+    (2, 65, 7, 8, 63, 1),                    # a channel past an octet, a filter short of a tile
+    (3, 16, 5, 9, 64, 1),                    # 45 pixels: two images end inside a stage
+    (2, 64, 6, 7, 64, 0),                    # no padding
+    (3, 20, 11, 17, 70, 0),                  # no padding, few filters past two tiles of 32
     (9, 64, 14, 14, 128, 1),                 # uneven splits
-    (2, 130, 56, 56, 64, 1),                 # many splits: a wave for every eighth
-    (40, 96, 14, 15, 200, 1),                # eight to thirty-one splits
+    (2, 130, 56, 56, 64, 1),                 # twenty splits: four waves share them
+    (40, 96, 14, 15, 200, 1),                # nine splits
 ])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_split_weight_gradient_against_the_oracle(gpu, n, c, h, w, k, pad, accumulate):
@@ -106,8 +106,8 @@ def test_split_weight_gradient_against_the_oracle(gpu, n, c, h, w, k, pad, accum
     (2, 24, 1, 70, 16, 1, 7, 1, 1, 3),       # one row, padding above and below it only
     (3, 96, 9, 9, 8, 3, 3, 1, 1, 2),         # more padding than the filter needs
     (9, 64, 14, 14, 128, 3, 3, 1, 1, 1),     # uneven splits
-    (40, 96, 14, 15, 200, 3, 3, 2, 2, 1),    # eight to thirty-one splits
-    (2, 12, 60, 60, 24, 5, 5, 1, 1, 2),      # many splits
+    (40, 96, 14, 15, 200, 3, 3, 2, 2, 1),    # nine splits: four waves share them
+    (2, 12, 60, 60, 24, 5, 5, 1, 1, 2),      # 113 splits: sixteen waves
     (1, 8, 3, 2700, 8, 1, 3, 1, 1, 0),       # rows that 24-bit division does not hold: the fp32 kernels
 ])
 def test_split_weight_gradient_of_any_filter(gpu, n, c, h, w, k, r, s, sh, sw, pad):
@@ -185,7 +185,7 @@ def test_split_weight_gradient_of_every_tile(gpu, tile, dims):
         gpu.set_option("wgrad_tile", 0)
 
 
-@pytest.mark.parametrize("w,pad", [(56, 1), (7, 1)])       # stages of two rows and of four
+@pytest.mark.parametrize("w,pad", [(56, 1), (7, 1)])       # a stage is 64 pixels: little more than a row, nine rows
 @pytest.mark.parametrize("relu", [False, True])
 def test_weight_gradient_rounds_to_both_sides(gpu, w, pad, relu):
     """The bf16 MFMA drops what small products have below an accumulator's last bits, always downwards; over the two halves of a
@@ -350,7 +350,7 @@ def test_weight_gradient_of_values_that_do_not_split(gpu):
     assert calm.any() and rel_l2(got[calm], ref[calm]) <= TOL
 
 
-@pytest.mark.parametrize("w,pad", [(13, 1), (16, 1), (7, 1), (32, 1), (16, 0)])      # the last block of columns ragged or full
+@pytest.mark.parametrize("w,pad", [(13, 1), (16, 1), (7, 1), (32, 1), (16, 0)])      # rows that end with a stage and inside one
 @pytest.mark.parametrize("column", [0, -1])
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 def test_weight_gradient_of_a_border_column_that_is_not_finite(gpu, w, pad, column, value):
