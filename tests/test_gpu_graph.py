@@ -23,6 +23,7 @@ def _fresh_state(gpu):
     xs.GLOBAL.INPUTS = None
     xs.GLOBAL.USE_CUDA = False
     xs.GLOBAL.TRAINING = True
+    be.release_cached_memory()
 
 
 def _batches(count, n, size, classes, seed):

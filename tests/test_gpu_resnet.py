@@ -19,6 +19,7 @@ def _fresh_state(gpu):
     yield
     xs.GLOBAL.INPUTS = None
     xs.GLOBAL.USE_CUDA = False
+    gpu.release_cached_memory()
 
 
 def test_resnet18_device_path_matches_host_path():
