@@ -305,11 +305,12 @@ def test_conv_async_weight_gradients_of_a_sweep_share_the_second_stream(gpu):
     (12, 64, 38, 38, 192, 3, 3, 1, 1, 1, True, True),      # 1.9e9 products, 136 tiles of a bf16 data gradient
     (12, 64, 38, 38, 194, 3, 3, 1, 1, 1, True, False),     # no bf16 kernel for 194 filters: the data gradient fills the chip
     (2, 64, 38, 38, 192, 3, 3, 1, 1, 1, True, False),      # 3.2e8 products
-    (5, 64, 7, 8, 64, 15, 15, 1, 1, 7, False, True),       # a few workgroups with a long chain: 2.6e8, 3 tiles, 14400 for a sum
-    (5, 64, 7, 8, 64, 15, 15, 1, 1, 7, True, True),
-    (1, 64, 7, 8, 64, 15, 15, 1, 1, 7, False, False),      # 5e7
-    (5, 64, 7, 8, 64, 9, 9, 1, 1, 4, False, False),        # 5184 for a sum
-    (6, 90, 16, 30, 200, 7, 7, 2, 2, 3, False, True),      # 46 tiles, 9800 for a sum
+    (13, 86, 11, 11, 224, 7, 7, 1, 1, 3, False, True),     # a few workgroups with a long chain: 1.5e9, 26 tiles, 10976 for a sum
+    (13, 86, 11, 11, 230, 7, 7, 1, 1, 3, True, True),      # the same without a bf16 kernel
+    (6, 86, 11, 11, 230, 7, 7, 1, 1, 3, True, True),       # 7.0e8, enough under the flag
+    (6, 86, 11, 11, 224, 7, 7, 1, 1, 3, False, False),
+    (13, 100, 11, 11, 180, 7, 7, 1, 1, 3, False, False),   # 8820 for a sum
+    (45, 100, 11, 11, 200, 7, 7, 2, 2, 3, False, False),   # 86 tiles
     (5, 200, 13, 13, 1000, 3, 3, 1, 1, 1, False, False),   # nine taps
     (29, 15, 25, 25, 160, 15, 15, 2, 2, 0, True, False),   # bf16, 142 tiles with 10240 for a sum
     (5, 9, 55, 55, 128, 15, 15, 1, 1, 0, True, False),     # the same with 2.2e9 products

@@ -142,11 +142,13 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     //     55 x 55, N=5: 1280 -> 883; 15 -> 160, 15 x 15 / 2 at 25 x 25, N=29: 506 -> 351).  Of 82 other bf16 layers beside costs 0.90 of in
     //     order in the mean; five lose 10 % or more;
     //   a data gradient of either precision with at most 48 such tiles and filters of 25 taps or more that make 9000 or more products
-    //     for a sum, from 1e8 products on: a few workgroups with a long chain each (float32, beside -> in order: 256 -> 64, 15 x 15 / 3
-    //     at 2 x 5, N=22: 101 -> 134; 64 -> 410, 5 x 5 at 4 x 4, N=28: 55 -> 63; 90 -> 200, 7 x 7 / 2 at 16 x 30, N=6: 62 -> 76; 256 ->
-    //     300, 7 x 7 at 14 x 14, N=3: 116 -> 127.  Of 118 layers in both precisions 0.94 in the mean, two lose more than 2 %: 16 -> 96,
-    //     15 x 15 / 2 at 40 x 40, N=2: 67 -> 60.  Below 1e8 products and with smaller filters more lose: 200 -> 1000, 3 x 3 at 13 x 13,
-    //     N=5: 98 -> 87);
+    //     for a sum, from 1e9 products on: a few workgroups with a long chain each (float32 layers forward and backward, beside -> in
+    //     order: 86 -> 224, 7 x 7 at 11 x 11, N=13: 147 -> 154; 256 -> 256, 7 x 7 at 20 x 20, N=2: 182 -> 198; 160 -> 352, 15 x 15 at 5
+    //     x 5, N=9: 485 -> 520; of 46 in both precisions 0.98 in the mean, 1.03 at the worst.  Below, the two gradients alone still
+    //     gain, 90 -> 200, 7 x 7 / 2 at 16 x 30, N=6: 62 -> 75, but a layer has no room for what the host pays: forward and backward of
+    //     48 -> 190, 7 x 7 at 7 x 7, N=5: 104 -> 88 us, inside a network 135 -> 93.  Under the bf16 flag, whose other passes are
+    //     longer, from 4e8 on: 44 -> 80, 15 x 15 / 2 at 68 x 68, N=1: 132 -> 149; 90 -> 200 as above 103 -> 117.  With smaller filters more lose: 200 -> 1000, 3 x 3
+    //     at 13 x 13, N=5, both gradients 98 -> 87);
     //   layers of 2e9 products or more of a sweep that goes on, in float32 too: the passes between the convolutions find room
     //     (ResNet-18 steps: 224 x 224, N=32, 3.7e9 products a layer: 3.72 -> 4.01 ms; 192 x 192, 2.7e9: 3.13 -> 3.45; 224 x 224, N=16,
     //     1.85e9: 3.00 -> 2.76; 56 x 56, N=32: 3.01 -> 2.56).  A layer by itself is faster in order (64 -> 64 at 56 x 56, N=32, 3.7e9,
@@ -158,7 +160,7 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     const bool few_tiles = kflags && xsmi::tap_path_ok(K) && tiles <= xsmi::cu_count();
     const bool piles_up = few_tiles && tiles > 64 && (double)K * xsmi::ceil_div(R, sh) * xsmi::ceil_div(S, sw) >= 9500;
     const bool long_chain = tiles <= 48 && R * S >= 25 && (double)K * R * S >= 9000;
-    const bool pays = (few_tiles && products >= 4e8) || (long_chain && products >= 1e8) || (async && products >= 2e9);
+    const bool pays = (few_tiles && products >= 4e8) || (long_chain && products >= (kflags ? 4e8 : 1e9)) || (async && products >= 2e9);
     const bool beside = (pays && !piles_up) || (async && xsmi::side_pending());
     int rc = beside ? xsmi::side_begin() : xsmi::side_join();    // in main-stream order: after any earlier async work
     if (rc) return rc;
