@@ -583,8 +583,8 @@ bool wg_plan(WgParams &p, int N, int C, int H, int W, int K, int R, int S, int s
     // Sums of one to a few products: what the bf16 MFMA rounds downwards has no other half of the waves to cancel against, and one
     // fp32 product is rounded to nearest.  `most` products for an element of dw, N for a corner's: error against 64 bits, of that of
     // the fp32 kernels, 1.30 to 1.45 for one product, 1.05 to 1.27 for N = 1 and most = 2 to 4 or N = 2 and most = 2; 0.75 to 1.00
-    // for all larger ones (11 filters, 9 maps, N = 1 to 16).  Those few are formed in float64: 480 ->
-    // 416, 7 x 7 / 2 at 1 x 1, N=1: 67 -> 83 us (fp32 kernels 95); 452 -> 328, 3 x 3 / 2 at 5 x 2, N=1: 16.6 -> 19.7 (19.2).
+    // for all larger ones (11 filters, 9 maps, N = 1 to 16).  Those few are formed in float64: 480 -> 416, 7 x 7 / 2 at 1 x 1, N=1: 67
+    // -> 83 us (fp32 kernels 95); 452 -> 328, 3 x 3 / 2 at 5 x 2, N=1: 16.6 -> 19.7 (19.2).
     const double most = (double)N * (OH < xsmi::ceil_div(H, sh) ? OH : xsmi::ceil_div(H, sh)) * (OW < xsmi::ceil_div(W, sw) ? OW : xsmi::ceil_div(W, sw));
     p.few = N * most <= 4 ? 1 : 0;
     p.x_bytes = (uint32_t)((size_t)N * C * H * W * 4); p.dy_bytes = (uint32_t)((size_t)N * K * OH * OW * 4);

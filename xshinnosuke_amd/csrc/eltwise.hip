@@ -147,8 +147,8 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     //     x 5, N=9: 485 -> 520; of 46 in both precisions 0.98 in the mean, 1.03 at the worst.  Below, the two gradients alone still
     //     gain, 90 -> 200, 7 x 7 / 2 at 16 x 30, N=6: 62 -> 75, but a layer has no room for what the host pays: forward and backward of
     //     48 -> 190, 7 x 7 at 7 x 7, N=5: 104 -> 88 us, inside a network 135 -> 93.  Under the bf16 flag, whose other passes are
-    //     longer, from 4e8 on: 44 -> 80, 15 x 15 / 2 at 68 x 68, N=1: 132 -> 149; 90 -> 200 as above 103 -> 117.  With smaller filters more lose: 200 -> 1000, 3 x 3
-    //     at 13 x 13, N=5, both gradients 98 -> 87);
+    //     longer, from 4e8 on: 44 -> 80, 15 x 15 / 2 at 68 x 68, N=1: 132 -> 149; 90 -> 200 as above 103 -> 117.  With smaller filters
+    //     more lose: 200 -> 1000, 3 x 3 at 13 x 13, N=5, both gradients 98 -> 87);
     //   layers of 2e9 products or more of a sweep that goes on, in float32 too: the passes between the convolutions find room
     //     (ResNet-18 steps: 224 x 224, N=32, 3.7e9 products a layer: 3.72 -> 4.01 ms; 192 x 192, 2.7e9: 3.13 -> 3.45; 224 x 224, N=16,
     //     1.85e9: 3.00 -> 2.76; 56 x 56, N=32: 3.01 -> 2.56).  A layer by itself is faster in order (64 -> 64 at 56 x 56, N=32, 3.7e9,
