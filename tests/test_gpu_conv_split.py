@@ -51,6 +51,10 @@ def _data(n, c, h, w, k, r, s, sh, sw, pad, gpu):
     (17, 31, 56, 56, 1, 5, 5, 1, 1, 2),      # the same with two images for five filter rows, one row
     (11, 17, 61, 70, 33, 7, 7, 1, 1, 3),     # a row past them: 64 x 256, images of 3, 3 and 1 filter rows
     (24, 33, 56, 57, 20, 5, 5, 2, 2, 2),     # few rows, strided: 28 x 29 outputs, backward-data of four classes
+    (17, 98, 57, 57, 97, 3, 3, 2, 2, 1),     # strided, 128 x 128: seven groups, the last of one or two channels
+    (34, 200, 29, 28, 96, 3, 3, 2, 2, 0),    # two row tiles backward, the second of 72 rows; images of 6, 4, 4 and 2 groups
+    (9, 80, 112, 113, 200, 3, 3, 2, 2, 1),   # rows of 57 pixels: three of the four phases in one image
+    (7, 96, 56, 130, 128, 2, 4, 2, 3, 1),    # filter sides and strides that differ
 ])
 def test_split_convolution_against_the_oracle(gpu, n, c, h, w, k, r, s, sh, sw, pad):
     K = gpu.kernels
@@ -248,6 +252,7 @@ FORMED_AGAIN = [   # what the kernel that forms sums again walks differently
     (1, 512, 7, 7, 512, 3, 3, 1, 1, 1),      # segments that begin and end anywhere in a tile
     (17, 31, 56, 56, 31, 5, 5, 1, 1, 2),     # tiles of 32 x 512 in both passes, two images for five filter rows
     (24, 33, 56, 57, 20, 5, 5, 2, 2, 2),     # 32 x 512 forward and strided
+    (17, 98, 57, 57, 97, 3, 3, 2, 2, 1),     # 128 x 128: images of several phases or channel groups
 ]
 
 

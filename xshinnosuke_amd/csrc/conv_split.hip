@@ -18,7 +18,7 @@
 // 64 x 64 halve the conversion and the LDS reads for a product, but their accumulators and fragments spill (128 -> 128 at 28 x
 // 28, N=256: 305 -> 342 us; the loop runs 1.22 PFLOP/s of bf16 products there, a large library product 1.30).  The reduction is a list of steps (phase, 16 input channels, tap).
 // A PHASE is a set of taps that read one sub-lattice of the input (stride 1: all taps; stride 2: the taps of one row and
-// column parity; or, where the input rows of all taps together would not fit the LDS, those of as many filter rows as do: 216 -> 2,
+// column parity, and in the 128 x 128 tiling an image holds several phases and channel groups (SpKind); or, where the input rows of all taps together would not fit the LDS, those of as many filter rows as do: 216 -> 2,
 // 5 x 5 at 32 x 32, N=52, in images of 3 and 2 rows instead of five of one: 202 -> 162 us).  In the phase's
 // own coordinates the walk has stride 1, so a tile needs one run of positions ("slots") of a grid of pitch Wp = OX + taps
 // across - 1, and a tap is nothing but an offset into the run.  The run is staged once per 16 channels for all taps of the
@@ -49,14 +49,15 @@ typedef uint32_t uint32x2 __attribute__((ext_vector_type(2)));
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 constexpr int SP_ROWS = 64;                          // rows of a filter block
-// Tilings: WR x WC waves of 32 rows x 64 pixels, slots of an LDS image, most workgroups of a launch.
+// Tilings: WR x WC waves of 32 rows x 64 pixels, slots of an LDS image, most workgroups of a launch, whether an image has parts.
 struct SpTiling {
     int wr, wc, slots, max_grid;
+    bool parts;
     constexpr int rows() const { return 32 * wr; }
     constexpr int pixels() const { return 64 * wc; }
     constexpr int threads() const { return 64 * wr * wc; }
 };
-constexpr SpTiling SP_TILINGS[] = {{2, 2, 384, 512}, {2, 4, 512, 256}, {1, 8, 768, 256}};
+constexpr SpTiling SP_TILINGS[] = {{2, 2, 384, 512, false}, {2, 4, 512, 256, false}, {1, 8, 768, 256, false}, {4, 2, 768, 256, true}};
 constexpr int SP_BLOCK = 3 * 2 * SP_ROWS * 16;       // bytes of a step's filter block
 constexpr int SP_MAX_CLASSES = 4, SP_MAX_PHASES = 16;
 constexpr bool sp_scratch_holds() {
@@ -70,14 +71,24 @@ struct SpPhase {
     int iy0, ix0;          // input place of slot (row v, column u): (v * sy + iy0, u * sx + ix0)
     int Tx, T;             // taps across, taps in all
     int tap0, step0;       // first tap of the class, first step of the tile
+    int stride, span;      // steps between channel groups; slots past the last pixel's own that the taps reach
     int r0, rs, s0, ss;    // filter place of tap (a, b): (r0 + rs a, s0 + ss b)
 };
+// What one image of the LDS serves: the taps of a phase for one group of channels, or (tilings with parts) those of several phases
+// and groups, part g nphase + i being phase i of the image's group g.
+struct SpKind {
+    int phase0, nphase, T, step0;                    // phases; their taps, first step of the tile
+    int groups, inv_nphase;                          // channel groups of an image; 256 / nphase + 1
+    uint64_t off_lo, off_hi;                         // slot that tap i reads for slot 0, ten bits each, six in off_lo
+};
+constexpr int SP_MAX_TAPS = 12;                      // of an image with parts: what off_lo and off_hi hold
 struct SpClass {
     int M, rows, OY, OX, os_y, os_x;
     long long os_n, os_k, o_base;
     xsmi::FastDiv dOX, dOY, dWp, dHp, dIT, dTM;      // dIT: steps per tile, dTM: pixel tiles
     int Wp, Hp, sy, sx;
-    int phase0, nphase, taps, span;                  // span: slots past the last pixel's own that its taps reach
+    int phase0, nphase, kind0, nkind, taps, blocks;  // blocks: of SP_ROWS rows
+    int part_chunks, inv_part_chunks;                // 64-slot chunks of an image's part; 256 / that + 1
     uint32_t iters, first_unit, end_unit, apk_off;
 };
 struct SpTapPlace { uint32_t off, iters, step, T; };  // block of (row tile, group): off + rt iters + step + group T
@@ -95,6 +106,7 @@ struct SpParams {
     int ncls, relu, accumulate, tiling;
     SpClass cls[SP_MAX_CLASSES];
     SpPhase ph[SP_MAX_PHASES];
+    SpKind kd[SP_MAX_PHASES];
     SpTapPlace tap[9];     // of a 3 x 3 filter's taps
 };
 
@@ -136,7 +148,7 @@ __device__ __forceinline__ double unsplit(uint32_t p0, uint32_t p1, uint32_t p2)
 // value (split8_any), so the filter itself is not read here either; a tap outside the input multiplies a zero, as the
 // reference's padding does.  Every workgroup does this for its own steps.  All of 64 -> 64 at 56 x 56, N=8, not finite:
 // 93 us (one product at a time, by the workgroups that store the outputs: 2490), 256 -> 256 at 14 x 14: 110 (10100).
-struct SpSteps { int rt, s_first, n, f, grp, tap; };
+struct SpSteps { int block, s_first, n, f, grp, tap; };   // filter block, steps of the tile, image kind and first group, tap of the image
 __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const SpClass &c, const SpSteps &sg, int row0, int m0, int lane,
                                            __amdgpu_buffer_rsrc_t rin, __amdgpu_buffer_rsrc_t rapk) {
     const int l15 = lane & 15, quarter = lane >> 4;
@@ -152,12 +164,17 @@ __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const
 #pragma unroll
     for (int j = 0; j < 4; ++j) d[j >> 1][j & 1] = doublex4{0.0, 0.0, 0.0, 0.0};
     const int a_lane = ((quarter >> 1) * SP_ROWS + row0 + l15) * 16 + (quarter & 1) * 8;
-    uint32_t block = c.apk_off + ((uint32_t)sg.rt * c.iters + (uint32_t)sg.s_first) * (uint32_t)SP_BLOCK;
+    uint32_t block = c.apk_off + ((uint32_t)sg.block * c.iters + (uint32_t)sg.s_first) * (uint32_t)SP_BLOCK;
     int f = sg.f, grp = sg.grp, tap = sg.tap;
 #pragma unroll 1
     for (int s = 0; s < sg.n; ++s, block += SP_BLOCK) {
-        const SpPhase &ph = p.ph[f];
-        const int ta = tap / ph.Tx, tb = tap - ta * ph.Tx, ch0 = grp * 16 + 4 * quarter;
+        const SpKind &kd = p.kd[f];
+        const int g = tap / kd.T;
+        int i = kd.phase0, ta = tap - g * kd.T;
+        while (ta >= p.ph[i].T) ta -= p.ph[i++].T;
+        const SpPhase &ph = p.ph[i];
+        const int tb = ta % ph.Tx, ch0 = (grp + g) * 16 + 4 * quarter;
+        ta /= ph.Tx;
         double a[2][4], b[2][4];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -181,7 +198,12 @@ __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 d[j >> 1][j & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j >> 1][i], b[j & 1][i], d[j >> 1][j & 1], 0, 0, 0);
-        if (++tap == ph.T) { tap = 0; if (++grp == p.groups) { grp = 0; ++f; } }
+        const int left = p.groups - grp;
+        if (++tap == kd.T * (left < kd.groups ? left : kd.groups)) {
+            tap = 0;
+            grp += kd.groups;
+            if (grp >= p.groups) { grp = 0; ++f; }
+        }
     }
     // to the 32 x 32 block's order: register v of lane l is row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32
 #pragma unroll
@@ -207,7 +229,7 @@ __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const
 constexpr int SP_DECIDED = 4;
 template <int BATCH>
 __device__ __forceinline__ void decide_signs(floatx16 &r, const floatx16 &sum, const SpParams &p, const SpClass &c, const float *bias,
-                                             int rt, int row0, int m0, int lane, __amdgpu_buffer_rsrc_t rin, __amdgpu_buffer_rsrc_t rapk) {
+                                             int rb, int row0, int m0, int lane, __amdgpu_buffer_rsrc_t rin, __amdgpu_buffer_rsrc_t rapk) {
     float largest = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; ++v) largest = __builtin_fmaxf(largest, __builtin_fabsf(sum[v]));
@@ -237,10 +259,10 @@ __device__ __forceinline__ void decide_signs(floatx16 &r, const floatx16 &sum, c
         const int oy = q - n * c.OY, ox = m - q * c.OX, image = n * p.in_n;
         // sixteen lanes for the channels of a step, four steps at a time, BATCH of those in flight
         double total = 0.0;
-        uint32_t block = c.apk_off + (uint32_t)rt * c.iters * (uint32_t)SP_BLOCK + (uint32_t)(a_lane + row * 16);
 #pragma unroll 1
         for (int f = c.phase0; f < c.phase0 + c.nphase; ++f) {
             const SpPhase &ph = p.ph[f];
+            const uint32_t block = c.apk_off + ((uint32_t)rb * c.iters + (uint32_t)ph.step0) * (uint32_t)SP_BLOCK + (uint32_t)(a_lane + row * 16);
             const uint32_t T = (uint32_t)ph.T, Tx = (uint32_t)ph.Tx, steps = T * (uint32_t)p.groups;
             const uint32_t on = 4 / T, by = 4 - on * T, inv = 65536u / Tx + 1;      // x inv >> 16 = x / Tx, at most 961 taps of 31 across
             uint32_t grp = ((uint32_t)lane >> 4) / T, tap = ((uint32_t)lane >> 4) - grp * T;
@@ -258,7 +280,7 @@ __device__ __forceinline__ void decide_signs(floatx16 &r, const floatx16 &sum, c
 #pragma unroll
                     for (int i = 0; i < 3; ++i)
                         piece[k][i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(
-                            rapk, (int)(step < steps ? block + step * (uint32_t)SP_BLOCK + (uint32_t)(i * 2 * SP_ROWS * 16) : 0x80000000u), 0, 0);
+                            rapk, (int)(step < steps ? block + (grp * (uint32_t)ph.stride + tap) * (uint32_t)SP_BLOCK + (uint32_t)(i * 2 * SP_ROWS * 16) : 0x80000000u), 0, 0);
                     grp += on; tap += by;
                     if (tap >= T) { tap -= T; ++grp; }
                 }
@@ -266,7 +288,6 @@ __device__ __forceinline__ void decide_signs(floatx16 &r, const floatx16 &sum, c
                 for (int k = 0; k < BATCH; ++k)
                     total += unsplit(piece[k][0], piece[k][1], piece[k][2]) * (double)__builtin_bit_cast(float, bits[k]);
             }
-            block += steps * (uint32_t)SP_BLOCK;
         }
 #pragma unroll
         for (int i = 1; i < 64; i *= 2) total += __shfl_xor(total, i);
@@ -282,6 +303,7 @@ template <int TILING, bool SIGNS>
 __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_kernel(SpParams p) {
     constexpr SpTiling TL = SP_TILINGS[TILING];
     constexpr int WC = TL.wc, ROWS = TL.rows(), SP_PIX = TL.pixels(), THREADS = TL.threads();
+    constexpr bool PARTS = TL.parts;
     constexpr int CHUNKS = THREADS / 128, NJ = TL.slots / 64 / CHUNKS;    // 64-slot chunks staged at a time, and how often
     constexpr int SP_PLANE = TL.slots * 16;              // bytes of one (piece, octet) plane
     constexpr int SP_IMAGE = 6 * SP_PLANE;
@@ -302,11 +324,12 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
     const __amdgpu_buffer_rsrc_t rapk = __builtin_amdgcn_make_buffer_rsrc((void *)p.apk, 0, (int)p.apk_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rpart =
         __builtin_amdgcn_make_buffer_rsrc((void *)p.part, 0, (int)(TL.max_grid * PART_BYTES), 0x00020000);
-    const int a_voff = (h * SP_ROWS + wr * 32 + l31) * 16;
+    const int row0 = (wr & 1) * 32;                    // in the filter block: a tile of 128 rows has two
+    const int a_voff = (h * SP_ROWS + row0 + l31) * 16;
     const int octet = wave & 1, chunk0 = wave >> 1;    // this wave stages slots 64 (chunk0 + CHUNKS j) .. + 63 of one octet
     const uint32_t plane4 = (uint32_t)p.plane * 4u;
 
-    // A segment: steps [s_first, s_first + n) of one tile, beginning with tap `tap` of channel group `grp` of phase f.
+    // A segment: steps [s_first, s_first + n) of one tile, beginning with tap `tap` of an image of kind f from channel group `grp` on.
     struct Segment {
         int ci, s_first, n, rt, m0, slot0, nslots, f, grp, tap;
     };
@@ -328,13 +351,19 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         sg.m0 = (int)(tile - rt * c.dTM.d) * SP_PIX;
         sg.slot0 = slot_of(c, sg.m0);
         const int m_last = sg.m0 + SP_PIX - 1 < c.M ? sg.m0 + SP_PIX - 1 : c.M - 1;
-        sg.nslots = slot_of(c, m_last) - sg.slot0 + 1 + c.span;
-        sg.f = c.phase0;
-        while (sg.f + 1 < c.phase0 + c.nphase && sg.s_first >= p.ph[sg.f + 1].step0) ++sg.f;
-        const int k = sg.s_first - p.ph[sg.f].step0, T = p.ph[sg.f].T;
-        sg.grp = k / T;
-        sg.tap = k - sg.grp * T;
+        sg.nslots = slot_of(c, m_last) - sg.slot0 + 1;
+        sg.f = c.kind0;
+        while (sg.f + 1 < c.kind0 + c.nkind && sg.s_first >= p.kd[sg.f + 1].step0) ++sg.f;
+        const SpKind &kd = p.kd[sg.f];
+        const int k = sg.s_first - kd.step0, T = PARTS ? kd.T * kd.groups : kd.T, image = k / T;
+        sg.grp = PARTS ? image * kd.groups : image;
+        sg.tap = k - image * T;
         return sg;
+    };
+    auto block_row = [&](const SpClass &c, int rt) {   // a last tile of 65 rows has one filter block: the other half multiplies it too
+        if constexpr (ROWS <= SP_ROWS) return rt;
+        const int b = rt * (ROWS / SP_ROWS) + (wr >> 1);
+        return b < c.blocks ? b : c.blocks - 1;
     };
     auto block_of = [&](uint32_t v) {                  // byte offset of unit v's filter block (any place past the range)
         if (v >= u1) return 0u;
@@ -342,42 +371,61 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         while (ci + 1 < p.ncls && v >= p.cls[ci].end_unit) ++ci;
         const SpClass &c = p.cls[ci];
         const uint32_t ul = v - c.first_unit, tile = xsmi::fdiv(ul, c.dIT);
-        return c.apk_off + (xsmi::fdiv(tile, c.dTM) * c.iters + (ul - tile * c.iters)) * (uint32_t)SP_BLOCK;
+        return c.apk_off + ((uint32_t)block_row(c, (int)xsmi::fdiv(tile, c.dTM)) * c.iters + (ul - tile * c.iters)) * (uint32_t)SP_BLOCK;
     };
     uint32_t voff[NJ];
+    int group_of[NJ];                                  // of an image with parts: group of each chunk, counted from the image's first
     auto place = [&](const Segment &sg, int f) {       // byte offsets of this lane's slots in channel 0
         const SpClass &c = p.cls[sg.ci];
-        const SpPhase &ph = p.ph[f];
+        const SpKind &kd = p.kd[f];
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            const int sl = 64 * (chunk0 + CHUNKS * j) + lane;
+            int chunk = chunk0 + CHUNKS * j, i = 0;
+            if constexpr (PARTS) {
+                const int part = chunk * c.inv_part_chunks >> 8;
+                group_of[j] = part * kd.inv_nphase >> 8;
+                i = part - group_of[j] * kd.nphase;
+                chunk -= part * c.part_chunks;
+            }
+            const SpPhase &ph = p.ph[kd.phase0 + i];
+            const int sl = 64 * chunk + lane;
             const uint32_t P = (uint32_t)(sg.slot0 + sl);
             const int q = (int)xsmi::fdiv(P, c.dWp), n_ = (int)xsmi::fdiv((uint32_t)q, c.dHp);
             const int iy = (q - n_ * c.Hp) * c.sy + ph.iy0, ix = ((int)P - q * c.Wp) * c.sx + ph.ix0;
-            const bool ok = sl < sg.nslots && n_ < p.N && iy >= 0 && iy < p.IH && ix >= 0 && ix < p.IW;
+            const bool ok = sl < sg.nslots + ph.span && n_ < p.N && iy >= 0 && iy < p.IH && ix >= 0 && ix < p.IW;
             voff[j] = ok ? (uint32_t)(n_ * p.in_n + iy * p.IW + ix) * 4u : 0x80000000u;
         }
     };
     float pre[NJ][8];
     // always the same number of loads (slots past the run fetch out of range): the waits below count them
     auto load_image = [&](int grp_) {
+        auto whole = [&](int j, int ch0) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                rin, (int)voff[j], (int)((uint32_t)(ch0 + e) * plane4), 0));
+        };
+        auto ragged = [&](int j, int ch0) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool there = ch0 + e < p.CH;
+                pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                rin, (int)(there ? voff[j] : 0x80000000u), (int)(there ? (uint32_t)(ch0 + e) * plane4 : 0u), 0));
+            }
+        };
         const int ch0 = grp_ * 16 + octet * 8;
-        if (ch0 + 8 <= p.CH) {
+        if constexpr (PARTS) {
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
+            for (int j = 0; j < NJ; ++j) {
+                const int ch = ch0 + 16 * group_of[j];
+                if (ch + 8 <= p.CH) whole(j, ch); else ragged(j, ch);
+            }
+        } else if (ch0 + 8 <= p.CH) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                    rin, (int)voff[j], (int)((uint32_t)(ch0 + e) * plane4), 0));
+            for (int j = 0; j < NJ; ++j) whole(j, ch0);
         } else {
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const bool there = ch0 + e < p.CH;
-                    pre[j][e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                    rin, (int)(there ? voff[j] : 0x80000000u), (int)(there ? (uint32_t)(ch0 + e) * plane4 : 0u), 0));
-                }
+            for (int j = 0; j < NJ; ++j) ragged(j, ch0);
         }
     };
     // the fetched values into an LDS image: a pair of channels at a time, then the three 16-byte pieces
@@ -417,7 +465,14 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
             fb[j][q] = *reinterpret_cast<const bf16x8 *>(s_img + b_rd[j] + off + (int)q * 2 * SP_PLANE);
     };
     int t_left = 0, tb = 0, off = 0, Tx = 1, row_end = 0;
+    uint64_t off_lo = 0, off_hi = 0;
     auto next_off = [&]() {                            // past the last tap: back to a place inside the image
+        if constexpr (PARTS) {
+            off_lo = off_lo >> 10 | (off_hi & 1023) << 50;
+            off_hi >>= 10;
+            off = (int)(off_lo & 1023) * 16;
+            return;
+        }
         off += ++tb == Tx ? row_end : 16;
         tb = tb == Tx ? 0 : tb;
         off = --t_left == 0 ? 0 : off;
@@ -550,18 +605,27 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
                     fa[2][q] = turn == 1 ? x : y;
                 }
             }
-            const int T = p.ph[f].T;
+            const SpKind &kd = p.kd[f];
+            const int there = PARTS ? p.groups - grp < kd.groups ? p.groups - grp : kd.groups : 1, T = kd.T * there;
             const int taps = left < T - tap ? left : T - tap;
             left -= taps;
-            Tx = p.ph[f].Tx;
-            t_left = T - tap;
-            tb = tap % Tx;
-            off = (tap / Tx * Wp + tb) * 16;
-            row_end = (Wp - Tx + 1) * 16;
+            if constexpr (PARTS) {
+                off_lo = kd.off_lo;
+                off_hi = kd.off_hi;
+                off = (int)(off_lo & 1023) * 16;
+                for (int i = 0; i < tap; ++i) next_off();
+            } else {
+                Tx = p.ph[kd.phase0].Tx;
+                t_left = T - tap;
+                tb = tap % Tx;
+                off = (tap / Tx * Wp + tb) * 16;
+                row_end = (Wp - Tx + 1) * 16;
+            }
             tap = 0;
             // the next image, requested while this one is multiplied
             if (left > 0) {
-                if (++grp == p.groups) { grp = 0; ++f; place(sg, f); }
+                grp += there;
+                if (grp == p.groups) { grp = 0; ++f; place(sg, f); }
             } else if (more) {
                 grp = nx.grp;
                 place(nx, nx.f);
@@ -585,7 +649,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
 #pragma unroll
             for (int v = 0; v < 16; ++v) test.add(acc[j][v]);
             if (__builtin_amdgcn_ballot_w64(!test.all()) != 0)
-                form_again(acc[j], p, c, SpSteps{rt, sg.s_first, sg.n, sg.f, sg.grp, sg.tap}, wr * 32, m0 + wc * 64 + 32 * j, lane, rin, rapk);
+                form_again(acc[j], p, c, SpSteps{block_row(c, rt), sg.s_first, sg.n, sg.f, sg.grp, sg.tap}, row0, m0 + wc * 64 + 32 * j, lane, rin, rapk);
         }
         if (!head) {
 #pragma unroll
@@ -656,7 +720,8 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
                     floatx16 r = acc[j];
 #pragma unroll
                     for (int v = 0; v < 16; ++v) r[v] += bias ? bias[wr * 32 + 4 * h + 8 * (v >> 2) + (v & 3)] : 0.f;
-                    decide_signs<TILING != 0 ? 8 : 4>(r, acc[j], p, c, bias, rt, wr * 32, m0 + wc * 64 + 32 * j, lane, rin, rapk);
+                    decide_signs<TILING != 0 ? 8 : 4>(r, acc[j], p, c, bias ? bias + (wr >> 1) * SP_ROWS : nullptr, block_row(c, rt), row0,
+                                                                 m0 + wc * 64 + 32 * j, lane, rin, rapk);
                     acc[j] = r;
                     bias = nullptr;
                 }
@@ -735,7 +800,7 @@ __global__ void __launch_bounds__(256) split_pack_kernel(SpParams p, char *apk) 
             }
             uint32x4 q0, q1, q2;
             split8_any(v, q0, q1, q2);
-            const uint32_t step = (row / SP_ROWS) * c.iters + (uint32_t)ph.step0 + (o >> 1) * (uint32_t)ph.T + (uint32_t)tl;
+            const uint32_t step = (row / SP_ROWS) * c.iters + (uint32_t)ph.step0 + (o >> 1) * (uint32_t)ph.stride + (uint32_t)tl;
             char *dst = apk + c.apk_off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + row % SP_ROWS) * 16;
             *reinterpret_cast<uint32x4 *>(dst) = q0;
             *reinterpret_cast<uint32x4 *>(dst + 2 * SP_ROWS * 16) = q1;
@@ -754,7 +819,7 @@ long sp_slots(int pix, int OY, int OX, int ty, int tx) {
 // Adds a class whose taps are r = r0 + rs a (a < R), s = s0 + ss b (b < S), reading input place (y sy + iy(r), ...), split
 // into phases of sub-lattice taps; false if the tables or the LDS image do not hold it.
 struct SpTaps { int R, S, r0, rs, s0, ss, iy0, ix0; };            // tap (a, b) reads (y sy + iy0 + a, x sx + ix0 + b)
-bool sp_add_class(SpParams &p, int &nph, uint32_t &steps_bytes, const SpTaps &k, int M, int rows, int OY, int OX, int sy, int sx) {
+bool sp_add_class(SpParams &p, int &nph, int &nkd, uint32_t &steps_bytes, const SpTaps &k, int M, int rows, int OY, int OX, int sy, int sx) {
     if (p.ncls == SP_MAX_CLASSES || k.R < 1 || k.S < 1) return false;
     SpClass &c = p.cls[p.ncls];
     const int ny = sy < k.R ? sy : k.R, nx = sx < k.S ? sx : k.S;
@@ -764,8 +829,8 @@ bool sp_add_class(SpParams &p, int &nph, uint32_t &steps_bytes, const SpTaps &k,
     if (tl.rows() < SP_ROWS && rows > tl.rows()) return false;
     const int pix = tl.pixels();
     int ty = ty_max;
-    while (ty > 1 && sp_slots(pix, OY, OX, ty, tx_max) > tl.slots) --ty;
-    if (sp_slots(pix, OY, OX, ty, tx_max) > tl.slots) return false;
+    while (ty > 1 && (sp_slots(pix, OY, OX, ty, tx_max) > tl.slots || (tl.parts && ty * tx_max > SP_MAX_TAPS))) --ty;
+    if (sp_slots(pix, OY, OX, ty, tx_max) > tl.slots || (tl.parts && tx_max > SP_MAX_TAPS)) return false;
     // no more rows than the images need: seven in threes are 3 + 3 + 1, in images of 3 + 2 + 2 no fewer, but shorter ones
     const int images = (ty_max + ty - 1) / ty;
     ty = (ty_max + images - 1) / images;
@@ -776,8 +841,7 @@ bool sp_add_class(SpParams &p, int &nph, uint32_t &steps_bytes, const SpTaps &k,
     c.phase0 = nph; c.nphase = nphase; c.taps = k.R * k.S;
     c.M = M; c.rows = rows; c.OY = OY; c.OX = OX; c.sy = sy; c.sx = sx;
     c.Wp = OX + tx_max - 1; c.Hp = OY + ty - 1;
-    c.span = (ty - 1) * c.Wp + tx_max - 1;
-    int step = 0, tap = 0;
+    int tap = 0;
     for (int i = 0; i < ny; ++i)
         for (int first = i; first < k.R; first += ny * ty)        // filter rows first, first + ny, ...: at most ty
             for (int j = 0; j < nx; ++j) {
@@ -785,12 +849,38 @@ bool sp_add_class(SpParams &p, int &nph, uint32_t &steps_bytes, const SpTaps &k,
                 const int left = (k.R - first + ny - 1) / ny, na = left < ty ? left : ty, nb = (k.S - j + nx - 1) / nx;
                 f.iy0 = k.iy0 + first; f.ix0 = k.ix0 + j;
                 f.Tx = nb; f.T = na * nb;
-                f.tap0 = tap; f.step0 = step;
+                f.tap0 = tap; f.span = (na - 1) * c.Wp + nb - 1;
                 f.r0 = k.r0 + k.rs * first; f.rs = k.rs * ny; f.s0 = k.s0 + k.ss * j; f.ss = k.ss * nx;
-                tap += f.T; step += f.T * p.groups;
+                tap += f.T;
             }
+    // images: a phase and a group of channels each, or as many of both as make up to nine taps
+    const int chunks = xsmi::ceil_div((int)sp_slots(pix, OY, OX, ty, tx_max), 64), parts = tl.parts ? tl.slots / 64 / chunks : 1;
+    c.part_chunks = chunks; c.inv_part_chunks = 256 / chunks + 1;
+    c.kind0 = nkd;
+    int step = 0;
+    for (int f = c.phase0; f < nph;) {
+        SpKind &kd = p.kd[nkd++];
+        kd.phase0 = f; kd.nphase = 0; kd.T = 0; kd.step0 = step;
+        do {
+            kd.T += p.ph[f].T; ++kd.nphase; ++f;
+        } while (f < nph && kd.nphase < parts && kd.T + p.ph[f].T <= 9);
+        kd.groups = parts / kd.nphase;
+        if (kd.groups > 9 / kd.T) kd.groups = 9 / kd.T;
+        if (kd.groups < 1) kd.groups = 1;
+        kd.inv_nphase = 256 / kd.nphase + 1;
+        int within = 0, n = 0;
+        for (int i = kd.phase0; i < f; ++i) { p.ph[i].step0 = step + within; p.ph[i].stride = kd.T; within += p.ph[i].T; }
+        for (int part = 0; tl.parts && part < kd.groups * kd.nphase; ++part) {
+            const SpPhase &ph = p.ph[kd.phase0 + part % kd.nphase];
+            for (int t = 0; t < ph.T; ++t, ++n)
+                (n < 6 ? kd.off_lo : kd.off_hi) |= (uint64_t)(part * chunks * 64 + t / ph.Tx * c.Wp + t % ph.Tx) << 10 * (n % 6);
+        }
+        step += kd.T * p.groups;
+    }
+    c.nkind = nkd - c.kind0;
     c.iters = (uint32_t)step;
     const int tiles_m = xsmi::ceil_div(M, pix), tiles_r = xsmi::ceil_div(rows, tl.rows()), blocks_r = xsmi::ceil_div(rows, SP_ROWS);
+    c.blocks = blocks_r;
     c.dOX = xsmi::make_fastdiv(OX); c.dOY = xsmi::make_fastdiv(OY); c.dWp = xsmi::make_fastdiv(c.Wp); c.dHp = xsmi::make_fastdiv(c.Hp);
     c.dIT = xsmi::make_fastdiv(c.iters); c.dTM = xsmi::make_fastdiv(tiles_m);
     c.apk_off = steps_bytes;
@@ -814,19 +904,30 @@ uint32_t sp_least(const SpParams &p) {
     return least;
 }
 
+// Steps from which a strided pass takes the 128 x 128 tiling: below, its quarter as many workgroups bound the launch.
+constexpr uint32_t SP_STRIDED_UNITS = 3300;
+
+bool sp_parts(int CH, int R, int S, int sh, int sw) { return (sh > 1 || sw > 1) && R * S <= 9 && CH >= 64; }
+
 // The tiling of a pass of m pixels (of its largest class), and its plan.
 //   256-pixel tiles stage 2.0 values for each pixel of a 3 x 3 layer's tile where 128-pixel tiles stage 3.0; passes below 1024
 //   pixels keep the smaller tile, whose last one is emptier by less.
 //   At most 32 rows leave half of a 64-row tile's matrix work to zeros: tiles of 32 x 512 instead, where 64 x 256 would fill the
 //   chip (44 x 64 -> 16, 83 x 83: 139 -> 87 us; 10 x 448 -> 5, 5 x 5 at 66 x 66: 278 -> 161).  Below that the number of
 //   workgroups bounds the launch, of which there are then half as many (8 x 160 -> 17 at 12 x 59: 25.7 us, 29.5 in wide tiles).
+//   Strided passes of at most nine taps and four groups of channels or more, whose row tiles are three quarters full: 128 x 128.  The sub-lattices that the taps of a 3 x 3 / 2 filter read are disjoint, so
+//   an image of all of them stages no value twice and serves nine taps, where an image a sub-lattice serves one to four; half as
+//   many pixels, so that the four parts fit, for twice as many rows.  Backward-data reads one lattice, with one to four taps a
+//   class: there the parts are channel groups.  128 -> 256 at 28 x 28, N=32: forward 58 -> 41 us, backward-data 70 -> 47 (fp32
+//   kernels 48 and 49); at N=128 147 -> 98 and 215 -> 124 (153, 154).
 template <typename Plan>
-bool sp_plan_tiled(SpParams &p, long m, int rows, const Plan &plan) {
+bool sp_plan_tiled(SpParams &p, long m, int rows, bool parts, const Plan &plan) {
     auto as = [&](int tiling) {
         memset(&p, 0, sizeof(p));
         p.tiling = tiling;
         return plan(p);
     };
+    if (parts && 4 * rows >= 3 * xsmi::ceil_div(rows, SP_TILINGS[3].rows()) * SP_TILINGS[3].rows() && as(3) && p.units >= SP_STRIDED_UNITS) return true;
     if (m < 1024) return as(0);
     if (!as(1)) return false;
     if (rows > SP_TILINGS[2].rows() || p.units < 256u * sp_least(p)) return true;
@@ -834,12 +935,12 @@ bool sp_plan_tiled(SpParams &p, long m, int rows, const Plan &plan) {
 }
 
 bool sp_plan_fwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
-    return sp_plan_tiled(p, (long)N * OH * OW, K, [&](SpParams &p) {
+    return sp_plan_tiled(p, (long)N * OH * OW, K, sp_parts(C, R, S, sh, sw), [&](SpParams &p) {
         p.N = N; p.CH = C; p.groups = xsmi::ceil_div(C, 16); p.IH = H; p.IW = W; p.in_n = C * H * W; p.plane = H * W;
         p.w_row = C * R * S; p.w_ch = R * S; p.FS = S;
-        int nph = 0;
+        int nph = 0, nkd = 0;
         const SpTaps k = {R, S, 0, 1, 0, 1, -pad, -pad};
-        if (!sp_add_class(p, nph, p.apk_bytes, k, N * OH * OW, K, OH, OW, sh, sw)) return false;
+        if (!sp_add_class(p, nph, nkd, p.apk_bytes, k, N * OH * OW, K, OH, OW, sh, sw)) return false;
         SpClass &c = p.cls[0];
         c.os_n = (long long)K * OH * OW; c.os_k = (long long)OH * OW; c.o_base = 0; c.os_y = OW; c.os_x = 1;
         p.in_bytes = (uint32_t)((size_t)N * C * H * W * 4); p.out_bytes = (uint32_t)((size_t)N * K * OH * OW * 4);
@@ -849,17 +950,17 @@ bool sp_plan_fwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, i
 
 // backward-data: a class per residue (h mod sh, w mod sw); taps in ascending order of the dy row they read
 bool sp_plan_bwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
-    return sp_plan_tiled(p, (long)N * H * W / (sh * sw), C, [&](SpParams &p) {
+    return sp_plan_tiled(p, (long)N * H * W / (sh * sw), C, sp_parts(K, R, S, sh, sw), [&](SpParams &p) {
         p.N = N; p.CH = K; p.groups = xsmi::ceil_div(K, 16); p.IH = OH; p.IW = OW; p.in_n = K * OH * OW; p.plane = OH * OW;
         p.w_row = R * S; p.w_ch = C * R * S; p.FS = S;
-        int nph = 0;
+        int nph = 0, nkd = 0;
         for (int ph = 0; ph < sh && ph < H; ++ph) {
             const int r0 = (ph + pad) % sh, T = r0 < R ? xsmi::ceil_div(R - r0, sh) : 0, cy = (ph + pad - r0) / sh;
             for (int pw = 0; pw < sw && pw < W; ++pw) {
                 const int s0 = (pw + pad) % sw, U = s0 < S ? xsmi::ceil_div(S - s0, sw) : 0, cx = (pw + pad - s0) / sw;
                 const int OYc = xsmi::ceil_div(H - ph, sh), OXc = xsmi::ceil_div(W - pw, sw);
                 const SpTaps k = {T, U, r0 + sh * (T - 1), -sh, s0 + sw * (U - 1), -sw, cy - (T - 1), cx - (U - 1)};
-                if (!sp_add_class(p, nph, p.apk_bytes, k, N * OYc * OXc, C, OYc, OXc, 1, 1)) return false;
+                if (!sp_add_class(p, nph, nkd, p.apk_bytes, k, N * OYc * OXc, C, OYc, OXc, 1, 1)) return false;
                 SpClass &c = p.cls[p.ncls - 1];
                 c.os_n = (long long)C * H * W; c.os_k = (long long)H * W; c.o_base = (long long)ph * W + pw;
                 c.os_y = sh * W; c.os_x = sw;
@@ -883,7 +984,7 @@ int sp_run(SpParams &p, int opts, void *workspace) {
                     for (int t = 0; t < p.ph[f].T; ++t) {
                         const SpPhase &ph = p.ph[f];
                         const int r = ph.r0 + ph.rs * (t / ph.Tx), q = ph.s0 + ph.ss * (t % ph.Tx);
-                        p.tap[3 * r + q] = SpTapPlace{p.cls[i].apk_off, p.cls[i].iters, (uint32_t)(ph.step0 + t), (uint32_t)ph.T};
+                        p.tap[3 * r + q] = SpTapPlace{p.cls[i].apk_off, p.cls[i].iters, (uint32_t)(ph.step0 + t), (uint32_t)ph.stride};
                     }
             hipLaunchKernelGGL(split_pack9_kernel, dim3(row_tiles * octets), dim3(64), 0, st, p, (char *)workspace, p.cls[0].rows);
         } else {
@@ -899,7 +1000,9 @@ int sp_run(SpParams &p, int opts, void *workspace) {
     const SpTiling &tl = SP_TILINGS[p.tiling];
     const int which = p.mask ? TILINGS + p.tiling : p.tiling, threads = tl.threads();
     void (*const kernels[2 * TILINGS])(SpParams) = {split_conv_kernel<0, false>, split_conv_kernel<1, false>, split_conv_kernel<2, false>,
-                                                    split_conv_kernel<0, true>, split_conv_kernel<1, true>, split_conv_kernel<2, true>};
+                                                    split_conv_kernel<3, false>,
+                                                    split_conv_kernel<0, true>, split_conv_kernel<1, true>, split_conv_kernel<2, true>,
+                                                    split_conv_kernel<3, true>};
     int &res = resident[which];
     if (res == 0) {
         int per_cu = 0;
@@ -935,29 +1038,37 @@ namespace xsmi {
 //   1 x 1 to 3 taps: no.  An image then serves one tap, and its staging costs more than the fp32 kernels' loads (64 -> 128
 //     at 28 x 28, N=32: 12.1 -> 19.2 us).
 //   fewer than 16 channels: no.  A step multiplies 16, the rest zeros (4 -> 120, 3 x 3 at 102 x 102, N=53: 109 -> 226 us).
-//   strided with whole chunks of 32 channels: only where one pixel tile holds all pixels.  The phases of a 3 x 3 / 2
-//     filter have 1, 2, 2 and 4 taps (128 -> 256 at 28 x 28, N=32: 43 -> 55 us); with one image the fp32 kernels have a few
+//   strided with whole chunks of 32 channels: in the 128 x 128 tiling (sp_plan_tiled), not with emptier row tiles (160 rows,
+//     224 -> 160 at 42 x 42, N=17: 73 -> 92 us) or fewer channels (32 -> 296 at 21 x 70, N=35: 37 -> 45); backward-data, whose
+//     images have one to four taps of a few groups, from twice as many steps on (128 -> 256 at 29 x 29, N=14, 3280: 34 -> 36;
+//     at 28 x 28, N=32, 7056: 49 -> 47).  And where one pixel tile holds all pixels: the fp32 kernels then have a few
 //     workgroups with a long chain each (256 -> 512 at 14 x 14, N=1: 59 -> 42 us).
 //   everything else: yes (64 -> 64 at 56 x 56, N=32: 67 -> 52 us; 369 -> 37, 5 x 5 at 76 x 76, N=2, which had only the
 //     table-driven kernel: 801 -> 93 us; equal at the smallest sizes, 64 -> 64 at 56 x 56, N=1: 20.2 -> 21.1 us).
 static bool split_pays(int CH, int R, int S, int sh, int sw, long pixels) {
     if (option(OPT_CONV_SPLIT) >= 2) return true;        // wherever it applies, for tests and measurements
     if (R * S < 4 || CH < 16) return false;
-    return (sh == 1 && sw == 1) || CH % 32 != 0 || pixels <= 256;
+    return (sh == 1 && sw == 1) || CH % 32 != 0 || pixels <= 256 || sp_parts(CH, R, S, sh, sw);
+}
+// ... and whether this plan does.
+static bool split_plan_pays(const SpParams &p, int sh, int sw, long pixels, bool backward) {
+    if (option(OPT_CONV_SPLIT) >= 2 || (sh == 1 && sw == 1) || p.CH % 32 != 0 || pixels <= 256) return true;
+    return SP_TILINGS[p.tiling].parts && (!backward || p.units >= 2 * SP_STRIDED_UNITS);
 }
 
 // Workspace bytes of the split form, 0 where it does not serve the geometry or does not pay.
 size_t split_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
     SpParams p;
     if (option(OPT_CONV_SPLIT) == 0 || !split_pays(C, R, S, sh, sw, (long)N * OH * OW)) return 0;
-    if (!sp_plan_fwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW)) return 0;
+    if (!sp_plan_fwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW) || !split_plan_pays(p, sh, sw, (long)N * OH * OW, false)) return 0;
     return align_up(p.apk_bytes, 256);
 }
 size_t split_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
     SpParams p;
     if (option(OPT_CONV_SPLIT) == 0 || sh > R || sw > S) return 0;
-    if (!split_pays(K, R, S, sh, sw, (long)N * ceil_div(H, sh) * ceil_div(W, sw))) return 0;
-    if (!sp_plan_bwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW)) return 0;
+    const long pixels = (long)N * ceil_div(H, sh) * ceil_div(W, sw);
+    if (!split_pays(K, R, S, sh, sw, pixels)) return 0;
+    if (!sp_plan_bwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW) || !split_plan_pays(p, sh, sw, pixels, true)) return 0;
     return align_up(p.apk_bytes, 256);
 }
 
