@@ -55,6 +55,9 @@ def _data(n, c, h, w, k, r, s, sh, sw, pad, gpu):
     (34, 200, 29, 28, 96, 3, 3, 2, 2, 0),    # two row tiles backward, the second of 72 rows; images of 6, 4, 4 and 2 groups
     (9, 80, 112, 113, 200, 3, 3, 2, 2, 1),   # rows of 57 pixels: three of the four phases in one image
     (7, 96, 56, 130, 128, 2, 4, 2, 3, 1),    # filter sides and strides that differ
+    (1, 40, 28, 37, 130, 3, 3, 1, 1, 1),     # tiles with workgroups of their own: 1036 pixels, two rows past two tiles
+    (2, 100, 9, 9, 24, 5, 5, 2, 2, 2),       # ... in classes of 9, 6, 6 and 4 taps, shared by different numbers of them
+    (8, 16, 40, 40, 10, 3, 3, 1, 1, 1),      # ... one for each
 ])
 def test_split_convolution_against_the_oracle(gpu, n, c, h, w, k, r, s, sh, sw, pad):
     K = gpu.kernels

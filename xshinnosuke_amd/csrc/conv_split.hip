@@ -29,7 +29,7 @@
 // each wave fetches its fragments straight into registers three steps ahead (the waves of a workgroup read the same block at
 // about the same time: L1), so the loop has no barrier except around the image of a channel group.
 //
-// Scheduling is the even split of conv_tap_sk.hip: the steps of all tiles in a row are dealt over the resident workgroups; a
+// Scheduling is the even split of conv_tap_sk.hip (small launches deal tiles instead, sp_deal_tiles): the steps of all tiles in a row are dealt over the resident workgroups; a
 // workgroup whose range starts inside a tile hands its accumulators to the one that holds the tile's first step, which adds
 // them in ascending order (bounded wait, deterministic sums).  Row tiles vary slowest, so that an XCD's workgroups read few
 // filter blocks.
@@ -90,6 +90,8 @@ struct SpClass {
     int phase0, nphase, kind0, nkind, taps, blocks;  // blocks: of SP_ROWS rows
     int part_chunks, inv_part_chunks;                // 64-slot chunks of an image's part; 256 / that + 1
     uint32_t iters, first_unit, end_unit, apk_off;
+    xsmi::FastDiv dSH;                               // of a launch that deals tiles: workgroups that share one,
+    uint32_t end_group;                              // end of the class's workgroups
 };
 struct SpTapPlace { uint32_t off, iters, step, T; };  // block of (row tile, group): off + rt iters + step + group T
 struct SpParams {
@@ -299,7 +301,9 @@ __device__ __forceinline__ void decide_signs(floatx16 &r, const floatx16 &sum, c
 }
 
 // SIGNS: a sign mask is kept (a kernel of its own: the others would pay for the registers of decide_signs, half a microsecond)
-template <int TILING, bool SIGNS>
+// TILES: every tile has workgroups of its own, which divide its steps and then its output (sp_deal_tiles); otherwise the steps of
+// all tiles are dealt evenly.
+template <int TILING, bool SIGNS, bool TILES>
 __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_kernel(SpParams p) {
     constexpr SpTiling TL = SP_TILINGS[TILING];
     constexpr int WC = TL.wc, ROWS = TL.rows(), SP_PIX = TL.pixels(), THREADS = TL.threads();
@@ -316,8 +320,22 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
     const int wr = wave / WC, wc = wave % WC, h = lane >> 5, l31 = lane & 31;
     const uint32_t G = gridDim.x, g = xsmi::xcd_contiguous_id(blockIdx.x, G);
     auto range_start = [&](uint32_t j) { return j * p.upg + (j < p.urem ? j : p.urem); };
-    const uint32_t u1 = range_start(g + 1);
-    uint32_t u = range_start(g);
+    uint32_t u = 0, u1 = 0;
+    uint32_t share = 0, sharers = 1;                   // this workgroup among those of its tile
+    if constexpr (TILES) {
+        uint32_t ci = 0;
+        while (g >= p.cls[ci].end_group) ++ci;
+        const SpClass &c = p.cls[ci];
+        const uint32_t first = ci == 0 ? 0u : p.cls[ci - 1].end_group, tile = xsmi::fdiv(g - first, c.dSH);
+        sharers = c.dSH.d;
+        share = g - first - tile * sharers;
+        const uint32_t n = xsmi::fdiv(c.iters, c.dSH), rest = c.iters - n * sharers;
+        u = c.first_unit + tile * c.iters + share * n + (share < rest ? share : rest);
+        u1 = u + n + (share < rest ? 1u : 0u);
+    } else {
+        u = range_start(g);
+        u1 = range_start(g + 1);
+    }
     if (t == 0) s_fail = 0;
 
     const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc((void *)p.in, 0, (int)p.in_bytes, 0x00020000);
@@ -360,7 +378,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         sg.tap = k - image * T;
         return sg;
     };
-    auto block_row = [&](const SpClass &c, int rt) {   // a last tile of 65 rows has one filter block: the other half multiplies it too
+    auto block_row = [&](const SpClass &c, int rt, int wr) {   // a last tile of 65 rows has one filter block: the other half multiplies it too
         if constexpr (ROWS <= SP_ROWS) return rt;
         const int b = rt * (ROWS / SP_ROWS) + (wr >> 1);
         return b < c.blocks ? b : c.blocks - 1;
@@ -371,7 +389,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         while (ci + 1 < p.ncls && v >= p.cls[ci].end_unit) ++ci;
         const SpClass &c = p.cls[ci];
         const uint32_t ul = v - c.first_unit, tile = xsmi::fdiv(ul, c.dIT);
-        return c.apk_off + ((uint32_t)block_row(c, (int)xsmi::fdiv(tile, c.dTM)) * c.iters + (ul - tile * c.iters)) * (uint32_t)SP_BLOCK;
+        return c.apk_off + ((uint32_t)block_row(c, (int)xsmi::fdiv(tile, c.dTM), wr) * c.iters + (ul - tile * c.iters)) * (uint32_t)SP_BLOCK;
     };
     uint32_t voff[NJ];
     int group_of[NJ];                                  // of an image with parts: group of each chunk, counted from the image's first
@@ -477,7 +495,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         tb = tb == Tx ? 0 : tb;
         off = --t_left == 0 ? 0 : off;
     };
-    floatx16 hi[2], lo[2];
+    floatx16 hi[2], lo[2], images[2];                  // images (TILES): large products of the images before this one
     auto mm = [&](auto par, floatx16 (&acc)[2], int qa, int qb) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -579,7 +597,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         const bool head = sg.s_first == 0, complete = sg.s_first + sg.n == (int)c.iters;
         const uint32_t tile_end = u + (c.iters - (uint32_t)sg.s_first), u_next = u + (uint32_t)sg.n;
         const int m0 = sg.m0, rt = sg.rt, Wp = c.Wp;
-        const bool more = u_next < u1;
+        const bool more = !TILES && u_next < u1;
         if (more) nx = segment_at(u_next);
         a_next[0] = block_of(u_next);
 #pragma unroll
@@ -591,9 +609,10 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
             b_rd[j] = h * SP_PLANE + (slot_of(c, m < c.M ? m : c.M - 1) - sg.slot0) * 16;
 #pragma unroll
             for (int v = 0; v < 16; ++v) { hi[j][v] = 0.f; lo[j][v] = 0.f; }
+            if constexpr (TILES) images[j] = hi[j];
         }
         bias_buf ^= 1;                                 // the other waves may still be reading the one before
-        if (p.bias && head && t < ROWS) s_bias[bias_buf][t] = rt * ROWS + t < c.rows ? p.bias[rt * ROWS + t] : 0.f;
+        if (p.bias && (TILES || head) && t < ROWS) s_bias[bias_buf][t] = rt * ROWS + t < c.rows ? p.bias[rt * ROWS + t] : 0.f;
         int left = sg.n, f = sg.f, grp = sg.grp, tap = sg.tap;
         while (left > 0) {
             if (turn) {
@@ -636,6 +655,17 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
             xsmi::wait_lgkmcnt0();
             xsmi::block_barrier();                     // this image is complete, and nobody reads the other one any more
             run(taps);
+            // The MFMA drops what lies below its accumulator's last bits, so the large products of an image add up from zero
+            // and enter the sum in one rounding to nearest: error against 64 bits 0.8 of the even deal's.
+            if constexpr (TILES)
+                if (left > 0) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        images[j] += hi[j];
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) hi[j][v] = 0.f;
+                    }
+                }
             turn = taps % 3;
             image = SP_IMAGE - image;
         }
@@ -645,13 +675,27 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             acc[j] = hi[j] + lo[j];
+            if constexpr (TILES) acc[j] += images[j];
             xsmi::CarriedTest test;
 #pragma unroll
             for (int v = 0; v < 16; ++v) test.add(acc[j][v]);
             if (__builtin_amdgcn_ballot_w64(!test.all()) != 0)
-                form_again(acc[j], p, c, SpSteps{block_row(c, rt), sg.s_first, sg.n, sg.f, sg.grp, sg.tap}, row0, m0 + wc * 64 + 32 * j, lane, rin, rapk);
+                form_again(acc[j], p, c, SpSteps{block_row(c, rt, wr), sg.s_first, sg.n, sg.f, sg.grp, sg.tap}, row0, m0 + wc * 64 + 32 * j, lane, rin, rapk);
         }
-        if (!head) {
+        auto finish = [&](floatx16 &r, int wr, int m) {   // a 32 x 32 block of the output
+            const float *bias = p.bias ? s_bias[bias_buf] : nullptr;
+            if constexpr (SIGNS) {
+                const floatx16 sum = r;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) r[v] += bias ? bias[wr * 32 + 4 * h + 8 * (v >> 2) + (v & 3)] : 0.f;
+                decide_signs<TILING != 0 ? 8 : 4>(r, sum, p, c, bias ? bias + (wr >> 1) * SP_ROWS : nullptr, block_row(c, rt, wr),
+                                                  (wr & 1) * 32, m, lane, rin, rapk);
+                bias = nullptr;
+            }
+            xsmi::store_block_32x32(r, c, p.out, p.out_bytes, SIGNS ? p.mask : nullptr, bias, p.relu, p.accumulate, rt * ROWS, ROWS,
+                                    wr * 32, m, lane);
+        };
+        if (TILES ? sharers > 1 : !head) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 uint32x4 q;
@@ -661,7 +705,75 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
             }
             xsmi::wait_vmcnt<0>();                     // written through, this thread's ...
             __syncthreads();                           // ... and everybody else's
-            if (t == 0) __hip_atomic_store(p.flags + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!TILES && t == 0) __hip_atomic_store(p.flags + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if constexpr (TILES) {
+            if (sharers == 1) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) finish(acc[j], wr, m0 + wc * 64 + 32 * j);
+                return;
+            }
+            // Every part is in the scratch memory; the tile's 32 x 32 blocks are dealt over the waves of its workgroups, each of
+            // which adds a block's parts in ascending order, all of them at once.  The first workgroup's flag counts who has
+            // arrived, then who has read; the last one clears it.
+            uint32_t *count = p.flags + (g - share);
+            if (t == 0) {
+                __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                uint32_t spins = 0;
+                bool there = false;
+                while (p.spin_limit != 0u &&
+                       !(there = __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= sharers) && ++spins < p.spin_limit)
+                    __builtin_amdgcn_s_sleep(1);
+                if (!there) {                          // give up, as below
+                    s_fail = 1u;
+                    __hip_atomic_store(p.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
+            }
+            __syncthreads();
+            if (s_fail) return;
+            const uint32_t block = share + sharers * (uint32_t)wave;
+            const bool mine = block < 2u * (THREADS / 64);
+            const int bw = (int)(block >> 1), bj = (int)(block & 1);
+            double sum[16];                            // in float32 a dozen parts would cost up to half as much error again
+            if (mine) {
+                constexpr uint32_t DEPTH = 4;          // parts in flight
+                uint32x4 part[DEPTH][4];
+                auto fetch = [&](auto d, uint32_t i) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        part[d][k] = __builtin_amdgcn_raw_buffer_load_b128(
+                            rpart, (bw * 64 + lane) * 16, (int)((g - share + i) * PART_BYTES + (uint32_t)(bj * 4 + k) * (THREADS * 16u)), AGENT);
+                };
+                auto add = [&](auto d) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const uint32_t bits = part[d][v >> 2][v & 3];
+                        sum[v] += (double)__builtin_bit_cast(float, bits);
+                    }
+                };
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sum[v] = -0.0;   // the sum of negative zeros is one
+                for (uint32_t i = 0; i < sharers; i += DEPTH) {
+                    fetch(IC<0>{}, i);
+                    if (i + 1 < sharers) fetch(IC<1>{}, i + 1);
+                    if (i + 2 < sharers) fetch(IC<2>{}, i + 2);
+                    if (i + 3 < sharers) fetch(IC<3>{}, i + 3);
+                    add(IC<0>{});
+                    if (i + 1 < sharers) add(IC<1>{});
+                    if (i + 2 < sharers) add(IC<2>{});
+                    if (i + 3 < sharers) add(IC<3>{});
+                }
+            }
+            __syncthreads();
+            if (t == 0 && __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 2 * sharers - 1)
+                __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (mine) {
+                floatx16 r;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) r[v] = (float)sum[v];
+                finish(r, bw / WC, m0 + bw % WC * 64 + 32 * bj);
+            }
+            return;
         }
         if (head && !complete) {
             // the rest of the tile was multiplied by the workgroups that follow: a lane waits for each of them, then their
@@ -714,20 +826,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         }
         if (head) {
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const float *bias = p.bias ? s_bias[bias_buf] : nullptr;
-                if constexpr (SIGNS) {
-                    floatx16 r = acc[j];
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) r[v] += bias ? bias[wr * 32 + 4 * h + 8 * (v >> 2) + (v & 3)] : 0.f;
-                    decide_signs<TILING != 0 ? 8 : 4>(r, acc[j], p, c, bias ? bias + (wr >> 1) * SP_ROWS : nullptr, block_row(c, rt), row0,
-                                                                 m0 + wc * 64 + 32 * j, lane, rin, rapk);
-                    acc[j] = r;
-                    bias = nullptr;
-                }
-                xsmi::store_block_32x32(acc[j], c, p.out, p.out_bytes, SIGNS ? p.mask : nullptr, bias, p.relu, p.accumulate,
-                                        rt * ROWS, ROWS, wr * 32, m0 + wc * 64 + 32 * j, lane);
-            }
+            for (int j = 0; j < 2; ++j) finish(acc[j], wr, m0 + wc * 64 + 32 * j);
         }
         if (!more) break;
         sg = nx;
@@ -971,6 +1070,70 @@ bool sp_plan_bwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, i
     });
 }
 
+// Small launches: every tile has workgroups of its own, n steps each, and all of them add the tile's parts, a block of 32 x 32 a
+// wave.  Dealt evenly, the workgroup with a tile's first step adds the others' parts alone, 1.8 us each (64 KB by one compute
+// unit): 512 -> 512 at 7 x 7, N=1 22.1 -> 15.1 us, 64 -> 64 at 56 x 56, N=1 16.4 -> 13.6, 448 -> 407, 3 x 3 / 2 at 15 x 15, N=2
+// 48 -> 26; 180 layers, both passes, 0.79 of the time.  The stamps of a launch of nine steps a workgroup: parameters 1.6
+// us, image 1.5, steps 4.4, parts written 2.1, the others waited for 1.0, parts added 1.5, output 0.4.
+// The grid, 0 where the even deal is estimated to be faster.  Times in twentieths of a microsecond beside what both have, fitted to
+// those layers (the rule's choice is within 4 % of the best n): a step 8, an image begun 20, parts 20, 4 for each sharer and 80 for
+// 256 workgroups; the even deal 200 and 10 a step.  n is tried at the smallest that the resident
+// workgroups hold, at whole images and at even parts of one.
+uint32_t sp_deal_tiles(SpParams &p, uint32_t res, uint32_t even_grid) {
+    uint32_t tiles[SP_MAX_CLASSES], taps[SP_MAX_CLASSES], total = 0, longest = 0, steps = 1;
+    bool equal[SP_MAX_CLASSES];                        // images of one length
+    for (int i = 0; i < p.ncls; ++i) {
+        const SpClass &c = p.cls[i];
+        uint32_t images = 0;
+        for (int k = c.kind0; k < c.kind0 + c.nkind; ++k) images += (uint32_t)xsmi::ceil_div(p.groups, p.kd[k].groups);
+        equal[i] = images * (uint32_t)p.kd[c.kind0].T * (uint32_t)p.kd[c.kind0].groups == c.iters;
+        tiles[i] = (c.end_unit - c.first_unit) / c.iters;
+        taps[i] = (c.iters + images - 1) / images;
+        total += tiles[i];
+        if (c.iters > longest) { longest = c.iters; steps = taps[i]; }
+    }
+    if (res > 256) res = 256;                          // 512 small workgroups write twice the parts (8 x 512 -> 512 at 7 x 7: 26.8 us, 22.5)
+    if (total > res) return 0;
+    auto grid_of = [&](uint32_t n) {
+        uint32_t groups = 0;
+        for (int i = 0; i < p.ncls; ++i) groups += tiles[i] * ((p.cls[i].iters + n - 1) / n);
+        return groups;
+    };
+    uint32_t best = 0, best_time = 200 + 10 * ((p.units + even_grid - 1) / even_grid);
+    auto attempt = [&](uint32_t n) {
+        const uint32_t groups = grid_of(n);
+        if (groups > res) return;
+        uint32_t time = 0;
+        for (int i = 0; i < p.ncls; ++i) {
+            const uint32_t iters = p.cls[i].iters, sharers = (iters + n - 1) / n, most = (iters + sharers - 1) / sharers, T = taps[i];
+            const bool whole = equal[i] && iters % sharers == 0 && (most % T == 0 || T % most == 0);
+            uint32_t images = most / T + (whole ? most < T : most == 1 ? 1 : 2);
+            if (images > (iters + T - 1) / T) images = (iters + T - 1) / T;
+            const uint32_t cost = 8 * most + 20 * images + (sharers > 1 ? 20 + 4 * sharers + 80 * groups / 256 : 0);
+            if (cost > time) time = cost;
+        }
+        if (time < best_time) { best_time = time; best = n; }
+    };
+    uint32_t n = (p.units + res - 1) / res;
+    if (n < 2) n = 2;
+    while (grid_of(n) > res) ++n;
+    attempt(n);
+    for (uint32_t k = 1; k <= 4; ++k)
+        if (steps % k == 0 && steps / k > n) attempt(steps / k);
+    for (uint32_t k = (n + steps - 1) / steps, end = k + 3; k < end; ++k) attempt(k * steps);
+    attempt(longest);
+    if (best == 0) return 0;
+    uint32_t groups = 0;
+    for (int i = 0; i < p.ncls; ++i) {
+        SpClass &c = p.cls[i];
+        const uint32_t sharers = (c.iters + best - 1) / best;
+        groups += tiles[i] * sharers;
+        c.dSH = xsmi::make_fastdiv(sharers);
+        c.end_group = groups;
+    }
+    return groups;
+}
+
 int sp_run(SpParams &p, int opts, void *workspace) {
     hipStream_t st = xsmi::stream();
     p.apk = (const char *)workspace;
@@ -996,26 +1159,36 @@ int sp_run(SpParams &p, int opts, void *workspace) {
     }
     if (opts & 4) return XSMI_OK;
     constexpr int TILINGS = sizeof(SP_TILINGS) / sizeof(SP_TILINGS[0]);
-    static int resident[2 * TILINGS] = {};
+    static int resident[4 * TILINGS] = {};
     const SpTiling &tl = SP_TILINGS[p.tiling];
-    const int which = p.mask ? TILINGS + p.tiling : p.tiling, threads = tl.threads();
-    void (*const kernels[2 * TILINGS])(SpParams) = {split_conv_kernel<0, false>, split_conv_kernel<1, false>, split_conv_kernel<2, false>,
-                                                    split_conv_kernel<3, false>,
-                                                    split_conv_kernel<0, true>, split_conv_kernel<1, true>, split_conv_kernel<2, true>,
-                                                    split_conv_kernel<3, true>};
-    int &res = resident[which];
-    if (res == 0) {
-        int per_cu = 0;
-        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernels[which], threads, 0);
-        if (e != hipSuccess || per_cu < 1) per_cu = 1;
-        const int all = per_cu * xsmi::cu_count(), cap = tl.max_grid;
-        res = (all > cap ? cap : all < 8 ? 8 : all) & ~7;
-    }
-    uint32_t grid = (uint32_t)res;
+    const int threads = tl.threads();
+    void (*const kernels[4 * TILINGS])(SpParams) = {
+        split_conv_kernel<0, false, false>, split_conv_kernel<1, false, false>, split_conv_kernel<2, false, false>, split_conv_kernel<3, false, false>,
+        split_conv_kernel<0, true, false>, split_conv_kernel<1, true, false>, split_conv_kernel<2, true, false>, split_conv_kernel<3, true, false>,
+        split_conv_kernel<0, false, true>, split_conv_kernel<1, false, true>, split_conv_kernel<2, false, true>, split_conv_kernel<3, false, true>,
+        split_conv_kernel<0, true, true>, split_conv_kernel<1, true, true>, split_conv_kernel<2, true, true>, split_conv_kernel<3, true, true>};
+    auto resident_groups = [&](int which) {
+        int &res = resident[which];
+        if (res == 0) {
+            int per_cu = 0;
+            const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernels[which], threads, 0);
+            if (e != hipSuccess || per_cu < 1) per_cu = 1;
+            const int all = per_cu * xsmi::cu_count(), cap = tl.max_grid;
+            res = (all > cap ? cap : all < 8 ? 8 : all) & ~7;
+        }
+        return (uint32_t)res;
+    };
+    int which = p.mask ? TILINGS + p.tiling : p.tiling;
     const uint32_t least = sp_least(p);
+    uint32_t grid = resident_groups(which);
     if (grid > p.units / least) grid = p.units / least;
     if (grid == 0) grid = 1;
-    p.upg = p.units / grid; p.urem = p.units % grid;
+    if (const uint32_t groups = sp_deal_tiles(p, resident_groups(which + 2 * TILINGS), grid)) {
+        which += 2 * TILINGS;
+        grid = groups;
+    } else {
+        p.upg = p.units / grid; p.urem = p.units % grid;
+    }
     const int rc = xsmi::check_device_error("split convolution");
     if (rc) return rc;
     const xsmi::SkScratch scr = xsmi::sk_scratch();
