@@ -247,6 +247,25 @@ def test_dense_gemm_all_transposes(gpu):
         assert rel_l2(K.gemm(da, dg, trans_a=True).numpy(), a.T.astype(np.float64) @ g) <= 1e-5
 
 
+# edges of the 16 x 16 and 32 x 32 tiles, of a lane group's four k, of a wave's steps and rounds, one to sixteen waves, k split
+# over workgroups with a last one that is shorter
+@pytest.mark.parametrize("m,n,k", [(1, 1, 3), (17, 15, 4), (16, 16, 33), (33, 31, 63), (15, 17, 65), (40, 10, 511), (9, 100, 999),
+                                   (352, 513, 7), (385, 353, 100), (513, 289, 261), (31, 5, 5003), (2050, 1030, 9)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_dense_gemm_edges(gpu, m, n, k, ta, tb):
+    K = gpu.kernels
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k)).astype(np.float32); b = rng.standard_normal((k, n)).astype(np.float32)
+    da = gpu.to_device(np.ascontiguousarray(a.T) if ta else a)
+    db_ = gpu.to_device(np.ascontiguousarray(b.T) if tb else b)
+    bias = rng.standard_normal(n).astype(np.float32)
+    got = K.gemm(da, db_, bias=gpu.to_device(bias), trans_a=ta, trans_b=tb).numpy()
+    ref = a.astype(np.float64) @ b + bias
+    # a result passes through at most 128 sums of its wave, 4 + 6 + 5 of accumulators, waves and splits, and the bias
+    bound = 150 * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b) + np.abs(bias))
+    assert (np.abs(got - ref) <= bound).all()
+
+
 @pytest.mark.parametrize("m,n", [(37, 100), (32, 1000), (3, 2500)])
 def test_softmax_cross_entropy(gpu, m, n):
     """xs/nn/functional.py:984-1010 and xs/nn/grad_fn.py:604-620; rows longer than what a workgroup keeps in

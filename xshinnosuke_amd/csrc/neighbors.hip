@@ -918,73 +918,144 @@ __global__ void __launch_bounds__(256) avgpool_bwd_strided_kernel(const float *_
 }
 
 // ---- small GEMM (dense layer) ----------------------------------------------------
-// 32x32 output tile per 256 threads, K in chunks of 128 through LDS: the dense layer's matrices are skinny (a
-// batch of 32 rows), so few workgroups run and each must keep many loads in flight; a chunk is 32 independent
-// loads per thread.  Lanes always run along the contiguous axis of the operand in memory, whichever way it is
-// transposed.  Each of the four waves multiplies a quarter of the chunk (32 values of k: sixteen
-// v_mfma_f32_32x32x2_f32) into its own 32x32 accumulator; the four are added in wave order at the end.
-constexpr int GEMM_KC = 128;
-typedef float gemm_f16v __attribute__((ext_vector_type(16)));
-__global__ void __launch_bounds__(256) gemm_kernel(const float *__restrict__ A, const float *__restrict__ B,
-                                                    const float *__restrict__ bias, float *__restrict__ C, int M, int N,
-                                                    int K, int ta, int tb, int chunks_per_split) {
-    __shared__ float As[32][GEMM_KC + 1], Bs[GEMM_KC][33];
-    static_assert(sizeof(As) >= 4 * 1024 * sizeof(float), "the accumulators of four waves are exchanged through As");
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, l31 = lane & 31, half = lane >> 5;
-    const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
-    gemm_f16v acc = {0};
-    // split z multiplies K range [kbeg, kend) and writes its own M x N slab of C (C is then the partial buffer)
-    const int kbeg = blockIdx.z * chunks_per_split * GEMM_KC;
-    const int kend = min(K, kbeg + chunks_per_split * GEMM_KC);
+// Skinny products (a batch of 32 rows, ten classes): bound by latency, so the waves of a workgroup share the k of one tile of
+// T x T results, each with its loads straight into the operand registers of the MFMA, up to 32 of them in flight, no LDS
+// and no barrier before the waves' sums are added, in a fixed order.  Both operands of an MFMA take any assignment of k to
+// lanes as long as it is the same: a lane group takes four consecutive k, which is one 16-byte load of an operand that
+// is contiguous along k.  The steps of a wave go to several accumulators in turn, which keeps the chains of sums short.
+// Against chunks of 128 k staged through the LDS and a second launch for their sums: 32 x 1000 x 512 (M x N x K) 10.3 -> 4.7 us,
+// 256 x 10 x 1352 11.6 -> 5.9, 1352 x 10 x 256 transposed 9.1 -> 4.8, 256 x 1000 x 512 19.6 -> 6.9, 1024 x 1024 x 1024 139 -> 42,
+// 7 x 3 x 5 5.3 -> 5.5, of which about 4.5 are the launch; error against 64 bits 0.6 to 0.95 of before from K = 32 on.
+template <int T> struct GemmTile;
+template <> struct GemmTile<16> {
+    typedef float acc_t __attribute__((ext_vector_type(4)));
+    static constexpr int ACCS = 4;
+    static __device__ acc_t mfma(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+    static __device__ int row(int v, int lane) { return 4 * (lane >> 4) + v; }
+};
+template <> struct GemmTile<32> {
+    typedef float acc_t __attribute__((ext_vector_type(16)));
+    static constexpr int ACCS = 2;
+    static __device__ acc_t mfma(float a, float b, acc_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+    static __device__ int row(int v, int lane) { return 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3); }
+};
+// Four consecutive k of one row (column): with ALONG they are neighbours in memory (one 16-byte load, which needs no more
+// than the alignment of a float), else `stride` elements apart.
+template <bool ALONG>
+__device__ __forceinline__ void gemm_load4(float (&v)[4], const float *row, size_t stride, int k) {
+    if (ALONG) {
+        __builtin_memcpy(v, row + k, sizeof(v));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = row[(size_t)(k + e) * stride];
+    }
+}
+// The same where k reaches kend: from there on zeros, and the address stays inside the matrix.
+template <bool ALONG>
+__device__ __forceinline__ void gemm_load4_end(float (&v)[4], const float *row, size_t stride, int k, int kend) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const size_t kk = k + e < kend ? k + e : 0;
+        v[e] = row[ALONG ? kk : kk * stride];
+        v[e] = k + e < kend ? v[e] : 0.f;
+    }
+}
+
+template <int T, bool TA, bool TB>
+__global__ void __launch_bounds__(1024) gemm_kernel(const float *__restrict__ A, const float *__restrict__ B,
+                                                     const float *__restrict__ bias, float *__restrict__ C, int M, int N, int K,
+                                                     int k_split, int k_wave) {
+    typedef GemmTile<T> Tile;
+    constexpr int STEP = 4 * (64 / T), U = 4, VREGS = T * T / 64;
+    extern __shared__ float gemm_red[];                     // [waves][T * T]
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, waves = blockDim.x >> 6, lr = lane % T, lg = lane / T;
+    const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+    const int m = min(m0 + lr, M - 1), n = min(n0 + lr, N - 1);   // rows and columns past the end repeat the last one
+    const float *arow = TA ? A + m : A + (size_t)m * K;
+    const float *brow = TB ? B + (size_t)n * K : B + n;
+    // split z multiplies k_split values of k and writes its own M x N slab of C (C is then the partial buffer); each of its
+    // waves takes k_wave of them
+    const int kbeg = blockIdx.z * k_split + wv * k_wave;
+    const int kend = min(min(K, ((int)blockIdx.z + 1) * k_split), kbeg + k_wave);
     C += (size_t)blockIdx.z * M * N;
-    for (int k0 = kbeg; k0 < kend; k0 += GEMM_KC) {
-        // all loads of the chunk first (independent, so their latencies overlap), then the LDS stores
-        float ra[GEMM_KC / 8], rb[GEMM_KC / 8];
+    typename Tile::acc_t acc[Tile::ACCS] = {};
+    for (int k0 = kbeg; k0 < kend; k0 += U * STEP) {
+        float a[U][4], b[U][4];
 #pragma unroll
-        for (int u = 0; u < GEMM_KC / 8; ++u) {
-            const int i = threadIdx.x + 256 * u;
-            if (ta) {                                   // A stored (K, M): lanes along m
-                const int kk = i >> 5, r = i & 31;
-                ra[u] = (m0 + r < M && k0 + kk < kend) ? A[(size_t)(k0 + kk) * M + m0 + r] : 0.f;
-            } else {                                    // A stored (M, K): lanes along k
-                const int r = i / GEMM_KC, kk = i % GEMM_KC;
-                ra[u] = (m0 + r < M && k0 + kk < kend) ? A[(size_t)(m0 + r) * K + k0 + kk] : 0.f;
-            }
-            if (tb) {                                   // B stored (N, K): lanes along k
-                const int c = i / GEMM_KC, kk = i % GEMM_KC;
-                rb[u] = (n0 + c < N && k0 + kk < kend) ? B[(size_t)(n0 + c) * K + k0 + kk] : 0.f;
-            } else {                                    // B stored (K, N): lanes along n
-                const int kk = i >> 5, c = i & 31;
-                rb[u] = (n0 + c < N && k0 + kk < kend) ? B[(size_t)(k0 + kk) * N + n0 + c] : 0.f;
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u * STEP + 4 * lg;
+            if (k0 + (u + 1) * STEP <= kend) {
+                gemm_load4<!TA>(a[u], arow, (size_t)M, k);
+                gemm_load4<TB>(b[u], brow, (size_t)N, k);
+            } else if (k0 + u * STEP < kend) {
+                gemm_load4_end<!TA>(a[u], arow, (size_t)M, k, kend);
+                gemm_load4_end<TB>(b[u], brow, (size_t)N, k, kend);
             }
         }
 #pragma unroll
-        for (int u = 0; u < GEMM_KC / 8; ++u) {
-            const int i = threadIdx.x + 256 * u;
-            if (ta) As[i & 31][i >> 5] = ra[u]; else As[i / GEMM_KC][i % GEMM_KC] = ra[u];
-            if (tb) Bs[i % GEMM_KC][i / GEMM_KC] = rb[u]; else Bs[i >> 5][i & 31] = rb[u];
-        }
-        __syncthreads();
-        // operand lane l of an MFMA holds row (column) l % 32 at k = l / 32
+        for (int u = 0; u < U; ++u) {
+            if (k0 + u * STEP >= kend) break;
 #pragma unroll
-        for (int s = 0; s < GEMM_KC / 8; ++s) {
-            const int kk = wv * (GEMM_KC / 4) + 2 * s + half;
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[l31][kk], Bs[kk][l31], acc, 0, 0, 0);
+            for (int e = 0; e < 4; ++e) acc[u % Tile::ACCS] = Tile::mfma(a[u][e], b[u][e], acc[u % Tile::ACCS]);
         }
-        __syncthreads();
     }
-    // register v of lane l holds row 8 * (v / 4) + 4 * (l / 32) + v % 4, column l % 32 of the tile
-    float *red = &As[0][0];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) red[wv * 1024 + v * 64 + lane] = acc[v];
+    for (int d = Tile::ACCS / 2; d; d /= 2)
+#pragma unroll
+        for (int i = 0; i < d; ++i) acc[i] += acc[i + d];
+#pragma unroll
+    for (int v = 0; v < VREGS; ++v) gemm_red[(wv * VREGS + v) * 64 + lane] = acc[0][v];
     __syncthreads();
+    for (int e = threadIdx.x; e < T * T; e += blockDim.x) {
+        float part[4] = {};                                 // short chains of sums here too
+        for (int w = 0; w < waves; w += 4)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int e = (int)threadIdx.x + 256 * i, v = e >> 6, l = e & 63;
-        const float sum = ((red[e] + red[1024 + e]) + red[2048 + e]) + red[3072 + e];
-        const int m = m0 + 8 * (v >> 2) + 4 * (l >> 5) + (v & 3), n = n0 + (l & 31);
-        if (m < M && n < N) C[(size_t)m * N + n] = sum + (bias ? bias[n] : 0.f);
+            for (int i = 0; i < 4; ++i) part[i] += w + i < waves ? gemm_red[(w + i) * T * T + e] : 0.f;
+        const float sum = (part[0] + part[1]) + (part[2] + part[3]);
+        const int l = e & 63, mm = m0 + Tile::row(e >> 6, l), nn = n0 + l % T;
+        if (mm < M && nn < N) C[(size_t)mm * N + nn] = sum + (bias ? bias[nn] : 0.f);
     }
+}
+
+struct GemmPlan { int tile, waves, k_wave, splits, k_split; };
+
+// Tiles of 32 x 32 from half a workgroup a CU on, of 16 x 16 below, which spreads the loads of a few rows over four times as
+// many CUs; waves of at least 32 k (one round of loads).  k is split over workgroups as well, with a second launch for the
+// sums (4 us), only where sixteen waves would have more than 128 of it each and there are few tiles: 32 x 10 x 25088 11 us, in
+// one launch of two tiles over 40.
+GemmPlan gemm_plan(int M, int N, int K, size_t ws_bytes) {
+    GemmPlan g;
+    const long long tiles32 = (long long)((M + 31) / 32) * ((N + 31) / 32);
+    g.tile = tiles32 >= xsmi::cu_count() / 2 ? 32 : 16;
+    const long long tiles = g.tile == 32 ? tiles32 : (long long)((M + 15) / 16) * ((N + 15) / 16);
+    const int step = g.tile == 32 ? 8 : 16, most = tiles >= 16LL * xsmi::cu_count() ? 4 : 16;
+    g.splits = 1;
+    const long long room = 4LL * xsmi::cu_count() / tiles;
+    const size_t fit = ws_bytes / ((size_t)M * N * sizeof(float));
+    int want = (K + 16 * 128 - 1) / (16 * 128);
+    if (want > room) want = (int)room;
+    if ((size_t)want > fit) want = (int)fit;
+    if (want > 1) g.splits = want;
+    g.k_split = (K + g.splits - 1) / g.splits;
+    g.k_split = (g.k_split + step - 1) / step * step;
+    g.splits = (K + g.k_split - 1) / g.k_split;
+    const int waves = g.k_split <= 32 ? 1 : (g.k_split + 31) / 32 < most ? (g.k_split + 31) / 32 : most;
+    g.k_wave = ((g.k_split + waves - 1) / waves + step - 1) / step * step;
+    g.waves = (g.k_split + g.k_wave - 1) / g.k_wave;
+    return g;
+}
+
+template <int T, bool TA, bool TB>
+void gemm_launch(const GemmPlan &g, const float *A, const float *B, const float *bias, float *C, int M, int N, int K) {
+    hipLaunchKernelGGL((gemm_kernel<T, TA, TB>), dim3((N + T - 1) / T, (M + T - 1) / T, g.splits), dim3(64 * g.waves),
+                       (size_t)g.waves * T * T * sizeof(float), xsmi::stream(), A, B, bias, C, M, N, K, g.k_split, g.k_wave);
+}
+template <int T>
+void gemm_launch(bool ta, bool tb, const GemmPlan &g, const float *A, const float *B, const float *bias, float *C, int M, int N, int K) {
+    if (ta && tb) gemm_launch<T, true, true>(g, A, B, bias, C, M, N, K);
+    else if (ta) gemm_launch<T, true, false>(g, A, B, bias, C, M, N, K);
+    else if (tb) gemm_launch<T, false, true>(g, A, B, bias, C, M, N, K);
+    else gemm_launch<T, false, false>(g, A, B, bias, C, M, N, K);
 }
 // C = bias + the K-split partial products, added in ascending split order
 __global__ void __launch_bounds__(256) gemm_reduce_kernel(const float *__restrict__ part, const float *__restrict__ bias,
@@ -1398,35 +1469,18 @@ int xsmi_gemm(const float *A, const float *B, const float *bias, float *C, int M
     XSMI_CHECK_ARG(M > 0 && N > 0 && K > 0, "xsmi_gemm: empty matrix");
     XSMI_CHECK_ARG(A && B && C, "xsmi_gemm: null pointer");
     XSMI_CHECK_ARG((double)M * N < 2147483648.0, "xsmi_gemm: outputs of 2^31 elements or more are not supported");
-    // A skinny product (a batch of 32 rows) has few 32 x 32 output tiles and a long K: with a workspace, K is
-    // split over enough workgroups to occupy the chip and the partial products are added in a second pass.  A
-    // workgroup spends most of a chunk waiting for its loads, so "occupy" means about four workgroups per CU
-    // (256 x 1000 x 512, the ResNet-18 classifier at N=256: one workgroup per CU 56 us, four 21 us).
-    const int tiles = ((N + 31) / 32) * ((M + 31) / 32), chunks = (K + GEMM_KC - 1) / GEMM_KC;
-    const int want = 4 * xsmi::cu_count();
-    int splits = 1;
-    if (ws && chunks > 1 && tiles < want) {
-        splits = (want + tiles - 1) / tiles;
-        if (splits > chunks) splits = chunks;
-        const size_t fit = ws_bytes / ((size_t)M * N * sizeof(float));
-        if ((size_t)splits > fit) splits = (int)fit;
-        if (splits < 1) splits = 1;
-    }
-    const int cps = (chunks + splits - 1) / splits;
-    splits = (chunks + cps - 1) / cps;
-    hipStream_t st = xsmi::stream();
-    if (splits == 1) {
-        hipLaunchKernelGGL(gemm_kernel, dim3((N + 31) / 32, (M + 31) / 32, 1), dim3(256), 0, st, A, B, bias, C, M, N, K,
-                           trans_a, trans_b, chunks);
-        XSMI_LAUNCH_CHECK("gemm_kernel");
-        return XSMI_OK;
-    }
-    hipLaunchKernelGGL(gemm_kernel, dim3((N + 31) / 32, (M + 31) / 32, splits), dim3(256), 0, st, A, B,
-                       (const float *)nullptr, (float *)ws, M, N, K, trans_a, trans_b, cps);
+    const GemmPlan g = gemm_plan(M, N, K, ws ? ws_bytes : 0);
+    float *const out = g.splits > 1 ? (float *)ws : C;
+    const float *const b = g.splits > 1 ? nullptr : bias;
+    if (g.tile == 32) gemm_launch<32>(trans_a != 0, trans_b != 0, g, A, B, b, out, M, N, K);
+    else gemm_launch<16>(trans_a != 0, trans_b != 0, g, A, B, b, out, M, N, K);
     XSMI_LAUNCH_CHECK("gemm_kernel");
-    const uint32_t MN = (uint32_t)((size_t)M * N);
-    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((MN + 255) / 256), dim3(256), 0, st, (const float *)ws, bias, C, MN, N, splits);
-    XSMI_LAUNCH_CHECK("gemm_reduce_kernel");
+    if (g.splits > 1) {
+        const uint32_t MN = (uint32_t)((size_t)M * N);
+        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((MN + 255) / 256), dim3(256), 0, xsmi::stream(), (const float *)ws, bias, C, MN, N,
+                           g.splits);
+        XSMI_LAUNCH_CHECK("gemm_reduce_kernel");
+    }
     return XSMI_OK;
 }
 
