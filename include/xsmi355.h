@@ -111,7 +111,8 @@ int xsmi_sync(void);
  * apply; 1: 16-byte loads tap by tap; 0: one-dword loads everywhere), "pool_bwd" (workgroups per compute unit of the 3x3/2 max-pool gradient kernel whose workgroups walk
  * several pieces; 0: one piece per workgroup), "pack_lanes" (1 to 4: streams over which xsmi_conv2d_pack deals its
  * layout launches), "wgrad_tile" (the split-operand weight gradient's tile, as the digits of filters, pixels of a stage, pairs
- * of units for a wave and rounds of staging, for instance 646453; 0: the one of the least estimated time), "tap_stages",
+ * of units for a wave and rounds of staging, for instance 646453; 0: the one of the least estimated time), "conv_thin" (forward
+ * and weight gradient of at most 32 products a result by the vector units: 1: where that pays, 0: never, 2: wherever it applies), "tap_stages",
  * "tap_persist", "cl_halo", "cl_stem".  Each starts from the environment variable XSMI_<NAME IN CAPITALS> when that is set.
  * A caller that changes one must drop every workspace content it counted on (XSMI_CONV_WS_PACKED) and ask for
  * workspace sizes again.  No counterpart in the reference. */

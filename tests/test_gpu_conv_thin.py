@@ -1,0 +1,51 @@
+"""Forward and weight gradient of few products a result (csrc/conv_thin.hip) against the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_conv_variants import options
+from util import he_normal
+
+pytestmark = pytest.mark.gpu
+
+# n c h w k r s sh sw pad: every width of the gathered row (4, 8, 16, 32 products) at its edges, filters around the groups of 2, 4,
+# 8 and 32, pixels around 256 and 512 and over several images, borders wider than the image's inside, strides, one pixel
+GEOMETRIES = [
+    (1, 1, 1, 1, 1, 1, 1, 1, 1, 0), (2, 1, 28, 28, 8, 2, 2, 1, 1, 0), (3, 4, 16, 32, 9, 1, 1, 1, 1, 0), (7, 1, 19, 27, 33, 2, 2, 1, 2, 1),
+    (2, 5, 16, 16, 7, 1, 1, 1, 1, 0), (3, 2, 13, 11, 32, 2, 2, 2, 1, 2), (5, 1, 12, 9, 31, 3, 3, 1, 1, 1), (2, 8, 17, 15, 130, 1, 1, 1, 1, 0),
+    (4, 1, 9, 40, 5, 1, 11, 1, 2, 5), (2, 16, 8, 33, 6, 1, 1, 1, 1, 0), (1, 1, 23, 23, 3, 4, 4, 3, 3, 3), (2, 17, 9, 9, 3, 1, 1, 1, 1, 0),
+    (3, 3, 14, 18, 65, 3, 3, 1, 1, 1), (2, 1, 12, 12, 2, 5, 5, 2, 2, 4), (2, 32, 7, 11, 5, 1, 1, 1, 1, 0), (300, 1, 21, 20, 4, 2, 2, 1, 1, 0),
+]
+
+
+@pytest.mark.parametrize("geom", GEOMETRIES)
+def test_few_products_against_the_oracle(gpu, geom):
+    n, c, h, w, k, r, s, sh, sw, pad = geom
+    K = gpu.kernels
+    rng = np.random.default_rng(sum(geom))
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt = he_normal(rng, (k, c, r, s))
+    b = rng.standard_normal((k,)).astype(np.float32)
+    oh, ow = K.conv_out_hw(h, w, r, s, (sh, sw), pad)
+    dy = rng.standard_normal((n, k, oh, ow)).astype(np.float32)
+    y_ref, col = oracle.conv2d_fwd(x, wt, b, (sh, sw), pad)
+    dw0 = rng.standard_normal(wt.shape).astype(np.float32); db0 = rng.standard_normal((k,)).astype(np.float32)
+    _, dw_ref, db_ref = oracle.conv2d_bwd(dy, x.shape, wt, col, (sh, sw), pad, np.zeros_like(x), dw0.copy(), db0.copy())
+    _, dw_abs, db_abs = oracle.conv2d_bwd(np.abs(dy), x.shape, wt, np.abs(col), (sh, sw), pad, np.zeros_like(x), np.abs(dw0), np.abs(db0))
+    y_abs, _ = oracle.conv2d_fwd(np.abs(x), np.abs(wt), np.abs(b), (sh, sw), pad)
+    dx_, dw_, db_, ddy = (gpu.to_device(a) for a in (x, wt, b, dy))
+    u = 2.0 ** -24
+    with options(gpu, conv_thin=2, conv_split=0):
+        y = K.conv2d_fwd(dx_, dw_, db_, (sh, sw), pad).numpy()
+        assert (np.abs(y - y_ref) <= (c * r * s + 3) * u * y_abs).all()      # one chain of products, the bias, the oracle's rounding
+        mask = gpu.empty(y.shape, np.uint8)
+        act = K.conv2d_fwd(dx_, dw_, db_, (sh, sw), pad, relu=True, neg_mask=mask).numpy()
+        np.testing.assert_array_equal(act, np.maximum(y, 0.0))
+        np.testing.assert_array_equal(mask.numpy(), (y < 0).astype(np.uint8))
+        gw, gb = gpu.to_device(dw0), gpu.to_device(db0)
+        K.conv2d_bwd_weight(ddy, dx_, wt.shape, (sh, sw), pad, dw=gw, db=gb, accumulate=True)
+        # at most 4 pixels of a thread here, 6 + 2 sums over the wave and the workgroup, two roundings of the result
+        assert (np.abs(gw.numpy() - dw_ref) <= 14 * u * dw_abs).all()
+        assert (np.abs(gb.numpy() - db_ref) <= 3 * u * db_abs).all()
+        only, _ = K.conv2d_bwd_weight(ddy, dx_, wt.shape, (sh, sw), pad)
+    assert (np.abs(only.numpy() + dw0.astype(np.float64) - dw_ref) <= 14 * u * dw_abs).all()

@@ -327,7 +327,7 @@ size_t conv_bwd_data_ws_bytes(int C, int K, int R, int S, int sh, int sw) {
 
 // Which forward / backward-data kernel family serves a geometry with the given flags and workspace size: one place,
 // so that xsmi_conv2d_pack lays a filter out for exactly the kernel that the later call will pick.
-enum class FwdPath { ChannelsLast, FirstLayer, Split, EvenSplit, Tap, Generic };
+enum class FwdPath { ChannelsLast, Thin, FirstLayer, Split, EvenSplit, Tap, Generic };
 enum class BwdDataPath { Split, EvenSplit, Tap, Generic };
 
 static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW, unsigned flags,
@@ -335,13 +335,14 @@ static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh,
     const bool bf16 = (flags & XSMI_CONV_BF16) != 0;
     if (bf16 && xsmi::nhwc_fwd_ok(N, C, H, W, K, R, S, pad) && workspace_bytes >= xsmi::nhwc_fwd_ws_bytes(N, C, H, W, K, R, S, pad))
         return FwdPath::ChannelsLast;
-    if (!bf16 && xsmi::stem_fwd_ok(N, C, H, W, K, R, S, sh, sw, pad) &&
-        workspace_bytes >= xsmi::stem_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad))
-        return FwdPath::FirstLayer;
-    if (xsmi::split_may_serve(C, bf16) && !(flags & XSMI_CONV_WS_ONLY) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
+    const bool first = !bf16 && xsmi::stem_fwd_ok(N, C, H, W, K, R, S, sh, sw, pad) &&
+                       workspace_bytes >= xsmi::stem_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad);
+    if (!first && xsmi::split_may_serve(C, bf16) && !(flags & XSMI_CONV_WS_ONLY) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
         const size_t need = xsmi::split_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
         if (need && workspace_bytes >= need) return FwdPath::Split;
     }
+    if (!bf16 && xsmi::thin_fwd_ok(C, K, R, S, pad)) return FwdPath::Thin;
+    if (first) return FwdPath::FirstLayer;
     if (!bf16 && !(flags & XSMI_CONV_WS_ONLY) && xsmi::sk_path_ok(C, K) && xsmi::sk_fwd_pays(N * OH * OW, K, R, S, sh, sw) &&
         workspace_bytes >= xsmi::sk_fwd_ws_bytes(C, K, R, S))
         return FwdPath::EvenSplit;
@@ -384,6 +385,9 @@ int xsmi_conv2d_fwd(const float *x, const float *w, const float *bias, float *y,
     case FwdPath::ChannelsLast:
         return xsmi::nhwc_conv_fwd(x, nullptr, 0, w, bias, y, nullptr, 0, neg_mask, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW,
                                    relu, opts, workspace);
+    case FwdPath::Thin:
+        if (flags & XSMI_CONV_PACK_ONLY) return XSMI_OK;
+        return xsmi::thin_conv_fwd(x, w, bias, y, neg_mask, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, relu);
     case FwdPath::FirstLayer:
         return xsmi::stem_conv_fwd(x, w, bias, y, neg_mask, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, relu, opts, workspace);
     case FwdPath::Split:

@@ -303,6 +303,8 @@ int xsmi_conv2d_bwd_weight(const float *dy, const float *x, float *dw, float *db
     const int rs = xsmi::split_conv_bwd_weight(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, (flags & XSMI_CONV_BF16) != 0,
                                                beta == 1.f ? 1 : 0, workspace, workspace_bytes, served);
     if (served) return rs;
+    if (xsmi::thin_wgrad_ok(C, K, R, S, pad))
+        return xsmi::thin_conv_bwd_weight(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, OH, OW, beta == 1.f ? 1 : 0, workspace, need);
     if (xsmi::wgrad_tap_ok(dy, x, C, K, OH, OW))
         return xsmi::wgrad_tap(dy, x, dw, db, N, C, H, W, K, R, S, sh, sw, pad, OH, OW, beta == 1.f ? 1 : 0, workspace);
 

@@ -42,6 +42,7 @@ OptionRow g_options[xsmi::OPT_COUNT] = {
     {"pack_lanes", "XSMI_PACK_LANES", 2, false},
     {"conv_split", "XSMI_CONV_SPLIT", 1, false},
     {"wgrad_tile", "XSMI_WGRAD_TILE", 0, false},
+    {"conv_thin", "XSMI_CONV_THIN", 1, false},
 };
 
 // Streams beside the second one for runs of short independent launches (filter layouts), see side_lane().

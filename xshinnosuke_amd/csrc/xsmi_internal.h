@@ -30,7 +30,7 @@ bool capturing();            // a step graph is being recorded: nothing runs, no
 bool ready();
 int cu_count();
 // Tuning switches (xsmi_set_option / environment variable / default); the order is that of the table in runtime.hip.
-enum Option { OPT_TAP_SK, OPT_SK_SPIN_LIMIT, OPT_TAP_STAGES, OPT_TAP_PERSIST, OPT_CL_HALO, OPT_CL_STEM, OPT_SK_WIDE, OPT_POOL_BWD, OPT_PACK_LANES, OPT_CONV_SPLIT, OPT_WGRAD_TILE, OPT_COUNT };
+enum Option { OPT_TAP_SK, OPT_SK_SPIN_LIMIT, OPT_TAP_STAGES, OPT_TAP_PERSIST, OPT_CL_HALO, OPT_CL_STEM, OPT_SK_WIDE, OPT_POOL_BWD, OPT_PACK_LANES, OPT_CONV_SPLIT, OPT_WGRAD_TILE, OPT_CONV_THIN, OPT_COUNT };
 long option(Option o);
 // Partial tiles and flags of the convolution kernels that share tiles between workgroups, for the stream that stream() hands out; allocated
 // by xsmi_init, the flags are zero between launches.
@@ -176,6 +176,15 @@ bool stem_fwd_ok(int N, int C, int H, int W, int K, int R, int S, int sh, int sw
 size_t stem_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad);
 int stem_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
                   int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace);
+
+// forward and weight gradient of few products a result on the vector units (conv_thin.hip), fp32; the forward needs no workspace,
+// the weight gradient at most what conv_bwd_weight_ws_bytes says, which is what it is to be told
+bool thin_fwd_ok(int C, int K, int R, int S, int pad);
+bool thin_wgrad_ok(int C, int K, int R, int S, int pad);
+int thin_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W, int K, int R,
+                  int S, int sh, int sw, int pad, int OH, int OW, int relu);
+int thin_conv_bwd_weight(const float *dy, const float *x, float *dw, float *db, int N, int C, int H, int W, int K, int R, int S, int sh,
+                         int sw, int pad, int OH, int OW, int accumulate, void *workspace, size_t workspace_bytes);
 
 // bf16 forward on a channels-last bf16 copy of the activations (conv_tap.hip): channels a multiple of 32, or
 // at most 8 (a stem); the workspace holds the packed filter followed by the copy
