@@ -341,6 +341,43 @@ def test_a_filter_whose_layout_is_in_place_is_not_read(gpu, pass_):
     assert calm.any() and rel_l2(got[calm], plain[calm]) <= TOL
 
 
+@pytest.mark.parametrize("count", [1, 20, 21, 43])
+def test_layouts_made_in_one_call(gpu, count):
+    """A launch takes the layouts of 20 filters: bit-identical to the layout that a call makes for itself, also where a filter
+    of another size has a launch of its own in between."""
+    import ctypes
+    from xshinnosuke_amd.backend import capi
+    K = gpu.kernels
+    geometries = [(2, 17, 9, 9, 65, 3, 3, 1, 1, 1), (1, 40, 12, 11, 64, 3, 3, 2, 2, 1), (1, 20, 8, 8, 18, 5, 5, 1, 1, 2),
+                  (1, 130, 7, 7, 24, 3, 3, 1, 1, 1)]
+    calls, jobs = [], (capi.PackJob * count)()
+    with split_everywhere(gpu):
+        for i in range(count):
+            dims, pass_ = geometries[i % 4], (i // 4) % 2
+            n, c, h, w, k, r, s, sh, sw, pad = dims
+            rng = np.random.default_rng(i)
+            wt = gpu.to_device(he_normal(rng, (k, c, r, s)))
+            oh, ow = K.conv_out_hw(h, w, r, s, (sh, sw), pad)
+            x = gpu.to_device(rng.standard_normal((n, k, oh, ow) if pass_ else (n, c, h, w)).astype(np.float32))
+            ref = (K.conv2d_bwd_data(x, wt, (n, c, h, w), (sh, sw), pad) if pass_ else K.conv2d_fwd(x, wt, None, (sh, sw), pad)).numpy()
+            size = capi.lib.raw("xsmi_conv2d_pass_workspace_bytes")(*dims, pass_, 0)
+            ws = gpu.empty(((size + 3) // 4,))
+            jobs[i].w, jobs[i].workspace, jobs[i].workspace_bytes = wt.ptr, ws.ptr, size
+            for field, v in zip(("N", "C", "H", "W", "K", "R", "S", "sh", "sw", "pad", "pass_"), dims + (pass_,)):
+                setattr(jobs[i], field, v)
+            calls.append((dims, pass_, wt, x, ws, size, ref))
+        capi.lib.call("xsmi_conv2d_pack", count, ctypes.cast(jobs, ctypes.c_void_p))
+        capi.lib.call("xsmi_conv2d_bwd_join")
+        for i, (dims, pass_, wt, x, ws, size, ref) in enumerate(calls):
+            assert jobs[i].packed == 1
+            y = gpu.empty(ref.shape)
+            if pass_:
+                capi.lib.call("xsmi_conv2d_bwd_data", x.ptr, wt.ptr, y.ptr, *dims, 0.0, capi.CONV_WS_PACKED, ws.ptr, size)
+            else:
+                capi.lib.call("xsmi_conv2d_fwd", x.ptr, wt.ptr, None, y.ptr, None, *dims, capi.CONV_WS_PACKED, ws.ptr, size)
+            assert y.numpy().tobytes() == ref.tobytes()
+
+
 def test_weight_gradient_of_values_that_do_not_split(gpu):
     K = gpu.kernels
     x, wt, b, dy, _ = _data(2, 20, 12, 13, 70, 3, 3, 1, 1, 1, gpu)

@@ -561,6 +561,7 @@ int xsmi_conv2d_pack(int count, xsmi_pack_job_t *jobs) {
     int rc = XSMI_OK, lanes = 0;
     const long opt_lanes = xsmi::option(xsmi::OPT_PACK_LANES);
     const int nlanes = opt_lanes < 1 ? 1 : opt_lanes > xsmi::SIDE_LANES ? xsmi::SIDE_LANES : (int)opt_lanes;
+    xsmi::split_pack_collect();
     for (int i = 0; i < count && rc == XSMI_OK; ++i) {
         xsmi_pack_job_t &j = jobs[i];
         j.packed = 0;
@@ -599,10 +600,16 @@ int xsmi_conv2d_pack(int count, xsmi_pack_job_t *jobs) {
         if (rc == XSMI_OK) j.packed = 1;
     }
     if (forked) {
+        const int rp = xsmi::split_pack_launch(rc == XSMI_OK);
+        if (rc == XSMI_OK) rc = rp;
         const int rl = xsmi::side_lanes_end();
         xsmi::side_end();
         if (rc == XSMI_OK) rc = rl;
+    } else {
+        xsmi::split_pack_launch(false);
     }
+    if (rc != XSMI_OK)
+        for (int i = 0; i < count; ++i) jobs[i].packed = 0;
     return rc;
 }
 

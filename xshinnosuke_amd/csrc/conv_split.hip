@@ -109,8 +109,24 @@ struct SpParams {
     SpClass cls[SP_MAX_CLASSES];
     SpPhase ph[SP_MAX_PHASES];
     SpKind kd[SP_MAX_PHASES];
-    SpTapPlace tap[9];     // of a 3 x 3 filter's taps
 };
+// The layout of one 3 x 3 filter, and as many as a launch takes in its arguments (4 KB).
+struct SpPackJob {
+    const float *w;
+    char *apk;
+    uint32_t end_block, row_tiles;                   // end of its workgroups in the launch
+    int rows, CH, w_row, w_ch;
+    SpTapPlace tap[9];
+};
+constexpr int SP_PACK_JOBS = 20;
+template <int JOBS>
+struct SpPackArgs {
+    SpPackJob job[JOBS];
+    int count;
+};
+typedef SpPackArgs<SP_PACK_JOBS> SpPackJobs;
+static_assert(sizeof(SpPackJobs) <= 4096, "arguments of one launch");
+thread_local SpPackJobs *g_pack_jobs = nullptr;      // where layouts are collected instead of launched (split_pack_collect)
 
 constexpr int AGENT = 16;                            // sc1: past the caches that are not coherent across XCDs
 
@@ -836,10 +852,17 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
 // The filter in its steps' blocks.  A thread owns a row and an octet of channels; lanes are consecutive rows, so a
 // wavefront writes whole kilobytes.
 // 3 x 3: all nine taps of the octet in registers (each filter line is fetched once; 512 -> 512: 16 -> 6 us against a
-// thread per tap, whose 16-byte writes were scattered); every place a tap goes to is in the table `tap`.
-__global__ void __launch_bounds__(64) split_pack9_kernel(SpParams p, char *apk, int rows) {
-    const uint32_t padded = (uint32_t)((rows + SP_ROWS - 1) / SP_ROWS * SP_ROWS);
-    const uint32_t o = blockIdx.x / (padded / SP_ROWS), rt = blockIdx.x - o * (padded / SP_ROWS), row = rt * SP_ROWS + threadIdx.x;
+// thread per tap, whose 16-byte writes were scattered); every place a tap goes to is in the table `tap`.  A launch of its own
+// is 5 to 10 us of fetching its first instructions and lines, whatever the layer's size, so the layouts that are made ahead
+// of a step share launches (ResNet-18 step, 33 layouts in two launches: 56 x 56 images 2776 -> 2713 us, 224 x 224 3707 -> 3611).
+template <int JOBS>
+__global__ void __launch_bounds__(64) split_pack9_kernel(SpPackArgs<JOBS> jobs) {
+    int ji = 0;
+    while (JOBS > 1 && ji + 1 < jobs.count && blockIdx.x >= jobs.job[ji].end_block) ++ji;
+    const SpPackJob &p = jobs.job[ji];
+    const uint32_t block = blockIdx.x - (ji ? jobs.job[ji - 1].end_block : 0u);
+    const uint32_t o = block / p.row_tiles, rt = block - o * p.row_tiles, row = rt * SP_ROWS + threadIdx.x;
+    const int rows = p.rows;
     float v[9][8];
     xsmi::SplitTest test;
 #pragma unroll
@@ -853,7 +876,7 @@ __global__ void __launch_bounds__(64) split_pack9_kernel(SpParams p, char *apk, 
     auto put = [&](int t, const uint32x4 &q0, const uint32x4 &q1, const uint32x4 &q2) {
         const SpTapPlace &w = p.tap[t];
         const uint32_t step = rt * w.iters + w.step + (o >> 1) * w.T;
-        char *dst = apk + w.off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + threadIdx.x) * 16;
+        char *dst = p.apk + w.off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + threadIdx.x) * 16;
         *reinterpret_cast<uint32x4 *>(dst) = q0;
         *reinterpret_cast<uint32x4 *>(dst + 2 * SP_ROWS * 16) = q1;
         *reinterpret_cast<uint32x4 *>(dst + 4 * SP_ROWS * 16) = q2;
@@ -1134,6 +1157,19 @@ uint32_t sp_deal_tiles(SpParams &p, uint32_t res, uint32_t even_grid) {
     return groups;
 }
 
+int sp_launch_pack(SpPackJobs &jobs) {
+    if (jobs.count == 0) return XSMI_OK;
+    const dim3 grid(jobs.job[jobs.count - 1].end_block);
+    if (jobs.count == 1) {                             // 4 KB of arguments cost a launch by itself 2 us
+        hipLaunchKernelGGL(split_pack9_kernel<1>, grid, dim3(64), 0, xsmi::stream(), SpPackArgs<1>{{jobs.job[0]}, 1});
+    } else {
+        hipLaunchKernelGGL(split_pack9_kernel<SP_PACK_JOBS>, grid, dim3(64), 0, xsmi::stream(), jobs);
+    }
+    jobs.count = 0;
+    XSMI_LAUNCH_CHECK("split_pack9_kernel");
+    return XSMI_OK;
+}
+
 int sp_run(SpParams &p, int opts, void *workspace) {
     hipStream_t st = xsmi::stream();
     p.apk = (const char *)workspace;
@@ -1142,20 +1178,31 @@ int sp_run(SpParams &p, int opts, void *workspace) {
         for (int i = 0; i < p.ncls; ++i) taps += p.cls[i].taps;
         const uint32_t row_tiles = (uint32_t)xsmi::ceil_div(p.cls[0].rows, SP_ROWS), octets = 2u * (uint32_t)p.groups;
         if (taps == 9 && p.FS == 3) {
+            SpPackJobs own;
+            own.count = 0;
+            SpPackJobs &jobs = g_pack_jobs ? *g_pack_jobs : own;
+            if (jobs.count == SP_PACK_JOBS)
+                if (const int rc = sp_launch_pack(jobs)) return rc;
+            SpPackJob &job = jobs.job[jobs.count];
+            job.w = p.w; job.apk = (char *)workspace; job.row_tiles = row_tiles;
+            job.end_block = row_tiles * octets + (jobs.count ? jobs.job[jobs.count - 1].end_block : 0u);
+            job.rows = p.cls[0].rows; job.CH = p.CH; job.w_row = p.w_row; job.w_ch = p.w_ch;
             for (int i = 0; i < p.ncls; ++i)
                 for (int f = p.cls[i].phase0; f < p.cls[i].phase0 + p.cls[i].nphase; ++f)
                     for (int t = 0; t < p.ph[f].T; ++t) {
                         const SpPhase &ph = p.ph[f];
                         const int r = ph.r0 + ph.rs * (t / ph.Tx), q = ph.s0 + ph.ss * (t % ph.Tx);
-                        p.tap[3 * r + q] = SpTapPlace{p.cls[i].apk_off, p.cls[i].iters, (uint32_t)(ph.step0 + t), (uint32_t)ph.stride};
+                        job.tap[3 * r + q] = SpTapPlace{p.cls[i].apk_off, p.cls[i].iters, (uint32_t)(ph.step0 + t), (uint32_t)ph.stride};
                     }
-            hipLaunchKernelGGL(split_pack9_kernel, dim3(row_tiles * octets), dim3(64), 0, st, p, (char *)workspace, p.cls[0].rows);
+            ++jobs.count;
+            if (!g_pack_jobs)
+                if (const int rc = sp_launch_pack(jobs)) return rc;
         } else {
             uint32_t blocks = row_tiles * octets * (uint32_t)p.cls[0].taps / 4 + 1;
             if (blocks > 4096) blocks = 4096;
             hipLaunchKernelGGL(split_pack_kernel, dim3(blocks), dim3(256), 0, st, p, (char *)workspace);
+            XSMI_LAUNCH_CHECK("split_pack_kernel");
         }
-        XSMI_LAUNCH_CHECK("split_pack_kernel");
     }
     if (opts & 4) return XSMI_OK;
     constexpr int TILINGS = sizeof(SP_TILINGS) / sizeof(SP_TILINGS[0]);
@@ -1243,6 +1290,19 @@ size_t split_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, 
     if (!split_pays(K, R, S, sh, sw, pixels)) return 0;
     if (!sp_plan_bwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW) || !split_plan_pays(p, sh, sw, pixels, true)) return 0;
     return align_up(p.apk_bytes, 256);
+}
+
+// Between the two, layouts of 3 x 3 filters (XSMI_CONV_PACK_ONLY) share launches, on the stream that is current when one is full
+// and, for the rest, at the end.
+void split_pack_collect() {
+    static thread_local SpPackJobs jobs;
+    jobs.count = 0;
+    g_pack_jobs = &jobs;
+}
+int split_pack_launch(bool launch) {
+    SpPackJobs *jobs = g_pack_jobs;
+    g_pack_jobs = nullptr;
+    return launch && jobs ? sp_launch_pack(*jobs) : XSMI_OK;
 }
 
 int split_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,

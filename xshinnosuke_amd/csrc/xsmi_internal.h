@@ -159,6 +159,8 @@ inline bool split_may_serve(int reduce_channels, bool bf16) { return !bf16 || !t
 // workspace queries return 0 for geometries the kernel does not serve
 size_t split_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW);
 size_t split_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW);
+void split_pack_collect();
+int split_pack_launch(bool launch);
 int split_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
                    int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace);
 int split_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, int H, int W, int K, int R, int S, int sh,
