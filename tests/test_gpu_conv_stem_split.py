@@ -1,0 +1,69 @@
+"""First layers (1 or 3 channels, stride 2) on split operands: against the oracle at the edges of tiles, rows and images.
+
+Bound: as for the other split kernels, at most 2^-24 of each term is dropped and sums of at most 147 terms are float32:
+1e-6 in relative L2 norm is far above rounding and far below any misplaced term."""
+import numpy as np
+import pytest
+
+import oracle
+from util import he_normal, rel_l2
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-6
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,pad", [
+    (1, 3, 64, 64, 64, 7, 3),        # one wide tile across, four down
+    (2, 3, 63, 65, 32, 7, 3),        # a pixel past the tile, half of the filters
+    (3, 3, 32, 32, 65, 7, 3),        # square tiles; a filter past the row tile
+    (1, 3, 7, 200, 64, 7, 0),        # one row of outputs, 97 across
+    (5, 3, 224, 31, 40, 7, 2),       # narrow images
+    (40, 3, 64, 48, 128, 7, 3),      # more tiles than workgroups, two row tiles
+    (9, 3, 97, 113, 33, 5, 2),
+    (2, 3, 50, 34, 64, 5, 0),
+    (4, 3, 65, 33, 96, 3, 1),
+    (3, 3, 33, 32, 64, 3, 5),        # a border wider than the filter
+    (3, 1, 61, 97, 48, 7, 3),        # one channel: the last filter row by itself
+    (2, 1, 29, 30, 64, 5, 1),
+    (300, 1, 28, 28, 32, 3, 1),
+])
+def test_first_layer_against_the_oracle(gpu, n, c, h, w, k, r, pad):
+    K = gpu.kernels
+    rng = np.random.default_rng(n + 5 * h + k)
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt, b = he_normal(rng, (k, c, r, r)), rng.standard_normal((k,)).astype(np.float32)
+    y_ref, _ = oracle.conv2d_fwd(x, wt, b, (2, 2), pad)
+    dx, dw, db = (gpu.to_device(a) for a in (x, wt, b))
+    y = K.conv2d_fwd(dx, dw, db, (2, 2), pad).numpy()
+    assert rel_l2(y, y_ref) <= TOL
+    mask = gpu.empty(y.shape, np.uint8)
+    act = K.conv2d_fwd(dx, dw, db, (2, 2), pad, relu=True, neg_mask=mask).numpy()
+    np.testing.assert_array_equal(act, np.maximum(y, 0.0))
+    np.testing.assert_array_equal(mask.numpy(), (y < 0).astype(np.uint8))
+
+
+@pytest.mark.parametrize("c,h,w,r,pad", [(3, 40, 44, 7, 3), (1, 33, 66, 5, 2)])
+def test_values_that_do_not_split(gpu, c, h, w, r, pad):
+    """Infinities, NaN, the largest floats and values near the smallest: sums are what the fp32 kernels give, and no value
+    reaches a sum whose window it is not in."""
+    K = gpu.kernels
+    rng = np.random.default_rng(c)
+    x = (rng.standard_normal((3, c, h, w)) * 0.1).astype(np.float32)
+    wt = he_normal(rng, (40, c, r, r))
+    x[0, 0, 5, 9], x[1, c - 1, h - 1, w - 1], x[1, 0, 0, 0] = np.inf, np.nan, np.float32(3.4e38)
+    wt[3, 0, 0, 1], wt[7, c - 1, r - 1, r - 1] = -np.inf, np.nan
+    x[2] *= np.float32(2.0 ** -120)
+    dx, dw = gpu.to_device(x), gpu.to_device(wt)
+    got = K.conv2d_fwd(dx, dw, None, (2, 2), pad).numpy()
+    old = gpu.set_option("conv_split", 0)
+    try:
+        plain = K.conv2d_fwd(dx, dw, None, (2, 2), pad).numpy()
+    finally:
+        gpu.set_option("conv_split", old)
+    for test in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(test(got), test(plain))
+    calm = np.isfinite(plain[:2])
+    assert calm.any() and not calm.all() and rel_l2(got[:2][calm], plain[:2][calm]) <= TOL
+    good = [i for i in range(40) if i not in (3, 7)]
+    y_ref, _ = oracle.conv2d_fwd(x[2:].astype(np.float64) * 2.0 ** 120, wt[good], np.zeros(len(good), np.float32), (2, 2), pad)
+    assert rel_l2(got[2:, good].astype(np.float64) * 2.0 ** 120, y_ref) <= 1e-5      # sums near the smallest normal float

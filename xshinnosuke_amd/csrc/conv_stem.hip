@@ -441,6 +441,7 @@ size_t stem_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh
 
 int stem_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
                   int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace) {
+    if (stem_split_pays(C, R, K, sh, sw, OH, OW)) return stem_split_fwd(x, w, bias, y, mask, N, C, H, W, K, R, pad, OH, OW, relu);
     hipStream_t st = stream();
     const int rowtiles = ceil_div(K, 64);
     const int Hp = H + 2 * pad, Wp = stem_Wp(W, S, sw, pad, OW);

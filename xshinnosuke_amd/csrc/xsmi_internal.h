@@ -207,6 +207,9 @@ int halo_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk, co
 
 // first layer (at most 4 channels, 7-row filter, stride 2) with channels-last bf16 output (conv_cl_halo.hip); called by
 // nhwc_conv_fwd after it has made the bordered 4-channel copy
+bool stem_split_pays(int C, int R, int K, int sh, int sw, int OH, int OW);
+int stem_split_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W, int K, int R,
+                   int pad, int OH, int OW, int relu);
 bool stem_cl_ok(int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OW, int y_border);
 size_t stem_cl_apk_bytes();
 int stem_cl_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk, const float *bias, void *y_cl, int N, int C,
