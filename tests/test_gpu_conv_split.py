@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import oracle
-from util import he_normal, rel_l2
+from util import he_normal, rel_l2, round_bf16
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-6
@@ -339,6 +339,48 @@ def test_a_filter_whose_layout_is_in_place_is_not_read(gpu, pass_):
         np.testing.assert_array_equal(test(got), test(plain))
     calm = np.isfinite(plain)
     assert calm.any() and rel_l2(got[calm], plain[calm]) <= TOL
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad", [
+    (1, 64, 1, 255, 32, 1, 3, 1, 1, 1),      # one pixel short of two 128-pixel tiles
+    (1, 65, 16, 16, 64, 3, 3, 1, 1, 1),      # a row past the tile
+    (3, 17, 32, 32, 96, 3, 3, 1, 1, 0),      # wide tiles
+    (2, 40, 45, 61, 32, 5, 5, 1, 1, 2),      # an image does not hold all rows' taps
+    (1, 512, 7, 7, 512, 3, 3, 1, 1, 1),      # every tile shared by many workgroups
+    (20, 64, 56, 56, 32, 3, 3, 1, 1, 1),     # more tiles than workgroups
+    (20, 16, 45, 57, 64, 3, 3, 1, 1, 1),     # few rows: tiles of 32 x 512
+    (34, 96, 29, 28, 224, 3, 3, 2, 2, 0),    # strided, 128 x 128
+    (2, 24, 19, 23, 64, 7, 7, 2, 2, 3),      # four classes
+    (2, 18, 12, 12, 32, 3, 3, 3, 3, 0),      # nine of one tap
+    (2, 30, 15, 17, 64, 1, 1, 1, 1, 0),
+    (13, 98, 57, 57, 64, 2, 2, 1, 1, 1),
+])
+def test_bf16_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad):
+    """On operands rounded to bf16 only the float32 sums differ from the oracle's: 1e-5, as for the other bf16 kernels.  What
+    is not finite is so where it is with the kernel that gathers dy tap by tap."""
+    K = gpu.kernels
+    x, wt, b, dy, dx0 = _data(n, c, h, w, k, r, s, sh, sw, pad, gpu)
+    _, col = oracle.conv2d_fwd(x, round_bf16(wt), b, (sh, sw), pad)
+    ref, _, _ = oracle.conv2d_bwd(round_bf16(dy), x.shape, round_bf16(wt), col, (sh, sw), pad, dx0.copy(), np.zeros_like(wt), np.zeros_like(b))
+    dw_, ddy, gx = gpu.to_device(wt), gpu.to_device(dy), gpu.to_device(dx0)
+    with split_everywhere(gpu):
+        K.conv2d_bwd_data(ddy, dw_, x.shape, (sh, sw), pad, dx=gx, accumulate=True, bf16=True)
+    assert rel_l2(gx.numpy(), ref) <= 1e-5
+    dy[0, 1, 0, 0], dy[-1, -1, -1, -1], dy[0, 0, -1, -1] = np.inf, np.nan, np.float32(3.4e38)
+    wt[0, -1, 0, 0] = -np.inf
+    dw_, ddy = gpu.to_device(wt), gpu.to_device(dy)
+    run = lambda: K.conv2d_bwd_data(ddy, dw_, x.shape, (sh, sw), pad, bf16=True).numpy()  # noqa: E731
+    with split_everywhere(gpu):
+        got = run()
+    old = gpu.set_option("conv_split", 0)
+    try:
+        plain = run()
+    finally:
+        gpu.set_option("conv_split", old)
+    for test in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(test(got), test(plain))
+    calm = np.isfinite(plain)
+    assert not calm.all() and rel_l2(got[calm], plain[calm]) <= 1e-5
 
 
 @pytest.mark.parametrize("count", [1, 20, 21, 43])

@@ -328,7 +328,7 @@ size_t conv_bwd_data_ws_bytes(int C, int K, int R, int S, int sh, int sw) {
 // Which forward / backward-data kernel family serves a geometry with the given flags and workspace size: one place,
 // so that xsmi_conv2d_pack lays a filter out for exactly the kernel that the later call will pick.
 enum class FwdPath { ChannelsLast, Thin, FirstLayer, Split, EvenSplit, Tap, Generic };
-enum class BwdDataPath { Split, EvenSplit, Tap, Generic };
+enum class BwdDataPath { SplitBf16, Split, EvenSplit, Tap, Generic };
 
 static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW, unsigned flags,
                         size_t workspace_bytes) {
@@ -352,6 +352,10 @@ static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh,
 
 static BwdDataPath bwd_data_path(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW,
                                  unsigned flags, size_t workspace_bytes) {
+    if ((flags & XSMI_CONV_BF16) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
+        const size_t need = xsmi::split_bf16_bwd_data_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
+        if (need && workspace_bytes >= need) return BwdDataPath::SplitBf16;
+    }
     if (xsmi::split_may_serve(K, (flags & XSMI_CONV_BF16) != 0) && xsmi::option(xsmi::OPT_TAP_SK) == 1) {
         const size_t need = xsmi::split_bwd_data_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
         if (need && workspace_bytes >= need) return BwdDataPath::Split;
@@ -481,9 +485,12 @@ int xsmi_conv2d_bwd_data(const float *dy, const float *w, float *dx, int N, int 
     XSMI_CHECK_ARG(workspace && workspace_bytes >= need, "xsmi_conv2d_bwd_data: workspace of %zu bytes needed, %zu given",
                    need, workspace_bytes);
     const int opts = ((flags & XSMI_CONV_WS_PACKED) ? 2 : 0) | ((flags & XSMI_CONV_PACK_ONLY) ? 4 : 0);
-    switch (bwd_data_path(N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, flags, workspace_bytes)) {
+    const BwdDataPath path = bwd_data_path(N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, flags, workspace_bytes);
+    switch (path) {
     case BwdDataPath::Split:
-        return xsmi::split_conv_bwd_data(dy, w, dx, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, beta == 1.f ? 1 : 0, opts, workspace);
+    case BwdDataPath::SplitBf16:
+        return xsmi::split_conv_bwd_data(dy, w, dx, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, beta == 1.f ? 1 : 0, opts, workspace,
+                                         path == BwdDataPath::SplitBf16 ? 1 : 3);
     case BwdDataPath::EvenSplit:
         return xsmi::sk_conv_bwd_data(dy, w, dx, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, beta == 1.f ? 1 : 0, opts, workspace);
     case BwdDataPath::Tap:

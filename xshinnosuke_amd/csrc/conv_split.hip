@@ -58,7 +58,8 @@ struct SpTiling {
     constexpr int threads() const { return 64 * wr * wc; }
 };
 constexpr SpTiling SP_TILINGS[] = {{2, 2, 384, 512, false}, {2, 4, 512, 256, false}, {1, 8, 768, 256, false}, {4, 2, 768, 256, true}};
-constexpr int SP_BLOCK = 3 * 2 * SP_ROWS * 16;       // bytes of a step's filter block
+constexpr int sp_block(int pieces) { return pieces * 2 * SP_ROWS * 16; }   // bytes of a step's filter block
+constexpr int SP_BLOCK = sp_block(3);
 constexpr int SP_MAX_CLASSES = 4, SP_MAX_PHASES = 16;
 constexpr bool sp_scratch_holds() {
     for (const SpTiling &k : SP_TILINGS)
@@ -106,6 +107,7 @@ struct SpParams {
     int N, CH, groups, IH, IW, in_n, plane;          // input channels, their groups of 16, floats per image / plane
     int w_row, w_ch, FS;                             // of the layout launches: floats between rows / channels of the filter, filter width
     int ncls, relu, accumulate, tiling;
+    int pieces;                                      // 3, or 1: operands rounded to bf16
     SpClass cls[SP_MAX_CLASSES];
     SpPhase ph[SP_MAX_PHASES];
     SpKind kd[SP_MAX_PHASES];
@@ -116,6 +118,7 @@ struct SpPackJob {
     char *apk;
     uint32_t end_block, row_tiles;                   // end of its workgroups in the launch
     int rows, CH, w_row, w_ch;
+    int pieces;
     SpTapPlace tap[9];
 };
 constexpr int SP_PACK_JOBS = 20;
@@ -319,14 +322,14 @@ __device__ __forceinline__ void decide_signs(floatx16 &r, const floatx16 &sum, c
 // SIGNS: a sign mask is kept (a kernel of its own: the others would pay for the registers of decide_signs, half a microsecond)
 // TILES: every tile has workgroups of its own, which divide its steps and then its output (sp_deal_tiles); otherwise the steps of
 // all tiles are dealt evenly.
-template <int TILING, bool SIGNS, bool TILES>
+template <int TILING, bool SIGNS, bool TILES, int PIECES>
 __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_kernel(SpParams p) {
     constexpr SpTiling TL = SP_TILINGS[TILING];
     constexpr int WC = TL.wc, ROWS = TL.rows(), SP_PIX = TL.pixels(), THREADS = TL.threads();
     constexpr bool PARTS = TL.parts;
     constexpr int CHUNKS = THREADS / 128, NJ = TL.slots / 64 / CHUNKS;    // 64-slot chunks staged at a time, and how often
     constexpr int SP_PLANE = TL.slots * 16;              // bytes of one (piece, octet) plane
-    constexpr int SP_IMAGE = 6 * SP_PLANE;
+    constexpr int SP_IMAGE = 2 * PIECES * SP_PLANE, SP_BLOCK = sp_block(PIECES);
     constexpr uint32_t PART_BYTES = 32 * THREADS * 4;    // a workgroup's partial tile
     __shared__ __attribute__((aligned(16))) unsigned char s_img[2 * SP_IMAGE];
     __shared__ __attribute__((aligned(16))) float s_bias[2][ROWS];
@@ -463,21 +466,27 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         }
     };
     // the fetched values into an LDS image: a pair of channels at a time, then the three 16-byte pieces
-    uint32x4 piece[3];
+    uint32x4 piece[PIECES];
     xsmi::SmallTest small;
     auto split_one = [&](auto jt, auto it) {
         constexpr int j = decltype(jt)::value, i = decltype(it)::value;
-        uint32_t a, b, c;
-        if constexpr (i == 0) small = xsmi::SmallTest{};
-        small.add(pre[j][2 * i], pre[j][2 * i + 1]);
-        xsmi::split_pair3(pre[j][2 * i], pre[j][2 * i + 1], a, b, c);
-        piece[0][i] = a; piece[1][i] = b; piece[2][i] = c;
+        if constexpr (PIECES == 1) {
+            const xsmi::bf16x2 two = {(__bf16)pre[j][2 * i], (__bf16)pre[j][2 * i + 1]};
+            piece[0][i] = __builtin_bit_cast(uint32_t, two);
+            return;
+        } else {
+            uint32_t a, b, c;
+            if constexpr (i == 0) small = xsmi::SmallTest{};
+            small.add(pre[j][2 * i], pre[j][2 * i + 1]);
+            xsmi::split_pair3(pre[j][2 * i], pre[j][2 * i + 1], a, b, c);
+            piece[0][i] = a; piece[1][i] = b; piece[2][i] = c;
+        }
     };
     auto put = [&](auto j, int to) {
         unsigned char *dst = s_img + to + octet * SP_PLANE + (64 * (chunk0 + CHUNKS * j) + lane) * 16;
-        piece[0][0] = small.found() ? xsmi::NAN_PAIR : piece[0][0];
+        if constexpr (PIECES == 3) piece[0][0] = small.found() ? xsmi::NAN_PAIR : piece[0][0];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32x4 *>(dst + 2 * q * SP_PLANE) = piece[q];
+        for (int q = 0; q < PIECES; ++q) *reinterpret_cast<uint32x4 *>(dst + 2 * q * SP_PLANE) = piece[q];
     };
     auto stage = [&](auto j, int to) {
         split_one(j, IC<0>{}); split_one(j, IC<1>{}); split_one(j, IC<2>{}); split_one(j, IC<3>{});
@@ -488,15 +497,21 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
     // Three steps of filter fragments and one of pixel fragments in registers.  A step's filter loads are issued while the
     // step three before it multiplies: vector loads return in order, so they also wait for the image's loads in front of
     // them, which come from memory.
-    bf16x8 fa[3][3], fb[2][3];                         // [step % 3][piece], [pixel block][piece]
+    // (With one piece a step is a single product: its pixel fragments are read while the step before multiplies.)
+    constexpr int SETS = PIECES == 1 ? 3 : 1;
+    bf16x8 fa[3][PIECES], fb[SETS][2][PIECES];         // [step % 3][piece], [step % SETS][pixel block][piece]
     auto load_a = [&](auto par, auto q) {
         fa[par][q] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
                          rapk, a_voff + (int)q * 2 * SP_ROWS * 16, (int)a_off, 0));
     };
-    auto read_b = [&](auto q, int off) {
+    auto load_step = [&](auto par) {
+        if constexpr (PIECES == 3) { load_a(par, IC<2>{}); load_a(par, IC<1>{}); }
+        load_a(par, IC<0>{});
+    };
+    auto read_b = [&](auto set, auto q, int off) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            fb[j][q] = *reinterpret_cast<const bf16x8 *>(s_img + b_rd[j] + off + (int)q * 2 * SP_PLANE);
+            fb[set][j][q] = *reinterpret_cast<const bf16x8 *>(s_img + b_rd[j] + off + (int)q * 2 * SP_PLANE);
     };
     int t_left = 0, tb = 0, off = 0, Tx = 1, row_end = 0;
     uint64_t off_lo = 0, off_hi = 0;
@@ -515,7 +530,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
     auto mm = [&](auto par, floatx16 (&acc)[2], int qa, int qb) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[par][qa], fb[j][qb], acc[j], 0, 0, 0);
+            acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[par][qa], fb[par % SETS][j][qb], acc[j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
     // One step.  A piece's registers take the next tap's fragments (past a group's last tap: places that are not used), or
@@ -529,35 +544,47 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         next_off();
         a_off = a_left > 3 ? a_off + (uint32_t)SP_BLOCK : a_left == 3 ? a_next[0] : a_left == 2 ? a_next[1] : a_next[2];
         --a_left;
-        mm(par, lo, 2, 0);
-        load_a(par, IC<2>{});
-        if constexpr (J >= 0) split_one(jt, IC<0>{});
-        __builtin_amdgcn_sched_barrier(0);
-        mm(par, lo, 1, 0);
-        if constexpr (J >= 0) split_one(jt, IC<1>{});
-        __builtin_amdgcn_sched_barrier(0);
-        mm(par, hi, 0, 0);
-        read_b(IC<0>{}, image + off);
-        if constexpr (J >= 0) split_one(jt, IC<2>{});
-        __builtin_amdgcn_sched_barrier(0);
-        mm(par, lo, 1, 1);
-        load_a(par, IC<1>{});
-        if constexpr (J >= 0) split_one(jt, IC<3>{});
-        __builtin_amdgcn_sched_barrier(0);
-        mm(par, lo, 0, 1);
-        read_b(IC<1>{}, image + off);
-        if constexpr (J >= 0) put(jt, SP_IMAGE - image);
-        __builtin_amdgcn_sched_barrier(0);
-        mm(par, lo, 0, 2);
-        load_a(par, IC<0>{});
-        read_b(IC<2>{}, image + off);
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (PIECES == 1) {
+            read_b(IC<(par + 1) % 3>{}, IC<0>{}, image + off);
+            mm(par, hi, 0, 0);
+            load_a(par, IC<0>{});
+            if constexpr (J >= 0) {
+                split_one(jt, IC<0>{}); split_one(jt, IC<1>{}); split_one(jt, IC<2>{}); split_one(jt, IC<3>{});
+                put(jt, SP_IMAGE - image);
+            }
+            return;
+        } else {
+            mm(par, lo, 2, 0);
+            load_a(par, IC<2>{});
+            if constexpr (J >= 0) split_one(jt, IC<0>{});
+            __builtin_amdgcn_sched_barrier(0);
+            mm(par, lo, 1, 0);
+            if constexpr (J >= 0) split_one(jt, IC<1>{});
+            __builtin_amdgcn_sched_barrier(0);
+            mm(par, hi, 0, 0);
+            read_b(IC<0>{}, IC<0>{}, image + off);
+            if constexpr (J >= 0) split_one(jt, IC<2>{});
+            __builtin_amdgcn_sched_barrier(0);
+            mm(par, lo, 1, 1);
+            load_a(par, IC<1>{});
+            if constexpr (J >= 0) split_one(jt, IC<3>{});
+            __builtin_amdgcn_sched_barrier(0);
+            mm(par, lo, 0, 1);
+            read_b(IC<0>{}, IC<1>{}, image + off);
+            if constexpr (J >= 0) put(jt, SP_IMAGE - image);
+            __builtin_amdgcn_sched_barrier(0);
+            mm(par, lo, 0, 2);
+            load_a(par, IC<0>{});
+            read_b(IC<0>{}, IC<2>{}, image + off);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     // The taps of one image.  Written out up to nine: the waits of each step and the places where the next image is
     // staged are then compile-time facts.
     const auto none = IC<-1>{};
     auto run = [&](int taps) {
-        read_b(IC<0>{}, image + off); read_b(IC<1>{}, image + off); read_b(IC<2>{}, image + off);
+        read_b(IC<0>{}, IC<0>{}, image + off);
+        if constexpr (PIECES == 3) { read_b(IC<0>{}, IC<1>{}, image + off); read_b(IC<0>{}, IC<2>{}, image + off); }
         int staged = 0;
         const auto third = IC<NJ == 3 ? 2 : -1>{};
         do {
@@ -599,11 +626,11 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
     place(sg, sg.f);
     load_image(sg.grp);
     a_off = block_of(u);
-    load_a(IC<0>{}, IC<2>{}); load_a(IC<0>{}, IC<1>{}); load_a(IC<0>{}, IC<0>{});
+    load_step(IC<0>{});
     a_off = sg.n > 1 ? a_off + (uint32_t)SP_BLOCK : block_of(u + 1);
-    load_a(IC<1>{}, IC<2>{}); load_a(IC<1>{}, IC<1>{}); load_a(IC<1>{}, IC<0>{});
+    load_step(IC<1>{});
     a_off = sg.n > 2 ? a_off + (uint32_t)SP_BLOCK : block_of(u + 2);
-    load_a(IC<2>{}, IC<2>{}); load_a(IC<2>{}, IC<1>{}); load_a(IC<2>{}, IC<0>{});
+    load_step(IC<2>{});
     stage(IC<0>{}, 0); stage(IC<1>{}, 0);
     if constexpr (NJ == 3) stage(IC<2>{}, 0);
     int turn = 0;                                      // the set that the next step's filter block is in
@@ -624,7 +651,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
             const int m = m0 + wc * 64 + 32 * j + l31;
             b_rd[j] = h * SP_PLANE + (slot_of(c, m < c.M ? m : c.M - 1) - sg.slot0) * 16;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) { hi[j][v] = 0.f; lo[j][v] = 0.f; }
+            for (int v = 0; v < 16; ++v) { hi[j][v] = 0.f; lo[j][v] = 0.f; }   // (lo: not used with one piece)
             if constexpr (TILES) images[j] = hi[j];
         }
         bias_buf ^= 1;                                 // the other waves may still be reading the one before
@@ -633,7 +660,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         while (left > 0) {
             if (turn) {
 #pragma unroll
-                for (int q = 0; q < 3; ++q) {
+                for (int q = 0; q < PIECES; ++q) {
                     const bf16x8 x = fa[0][q], y = fa[1][q], z = fa[2][q];
                     fa[0][q] = turn == 1 ? y : z;
                     fa[1][q] = turn == 1 ? z : x;
@@ -690,13 +717,15 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
         floatx16 acc[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            acc[j] = hi[j] + lo[j];
+            acc[j] = PIECES == 3 ? hi[j] + lo[j] : hi[j];
             if constexpr (TILES) acc[j] += images[j];
-            xsmi::CarriedTest test;
+            if constexpr (PIECES == 3) {
+                xsmi::CarriedTest test;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) test.add(acc[j][v]);
-            if (__builtin_amdgcn_ballot_w64(!test.all()) != 0)
-                form_again(acc[j], p, c, SpSteps{block_row(c, rt, wr), sg.s_first, sg.n, sg.f, sg.grp, sg.tap}, row0, m0 + wc * 64 + 32 * j, lane, rin, rapk);
+                for (int v = 0; v < 16; ++v) test.add(acc[j][v]);
+                if (__builtin_amdgcn_ballot_w64(!test.all()) != 0)
+                    form_again(acc[j], p, c, SpSteps{block_row(c, rt, wr), sg.s_first, sg.n, sg.f, sg.grp, sg.tap}, row0, m0 + wc * 64 + 32 * j, lane, rin, rapk);
+            }
         }
         auto finish = [&](floatx16 &r, int wr, int m) {   // a 32 x 32 block of the output
             const float *bias = p.bias ? s_bias[bias_buf] : nullptr;
@@ -708,7 +737,7 @@ __global__ void __launch_bounds__(SP_TILINGS[TILING].threads(), 2) split_conv_ke
                                                   (wr & 1) * 32, m, lane, rin, rapk);
                 bias = nullptr;
             }
-            xsmi::store_block_32x32(r, c, p.out, p.out_bytes, SIGNS ? p.mask : nullptr, bias, p.relu, p.accumulate, rt * ROWS, ROWS,
+            xsmi::store_block_32x32(r, c, p.out, p.out_bytes, SIGNS || PIECES == 1 ? p.mask : nullptr, bias, p.relu, p.accumulate, rt * ROWS, ROWS,
                                     wr * 32, m, lane);
         };
         if (TILES ? sharers > 1 : !head) {
@@ -876,13 +905,14 @@ __global__ void __launch_bounds__(64) split_pack9_kernel(SpPackArgs<JOBS> jobs) 
     auto put = [&](int t, const uint32x4 &q0, const uint32x4 &q1, const uint32x4 &q2) {
         const SpTapPlace &w = p.tap[t];
         const uint32_t step = rt * w.iters + w.step + (o >> 1) * w.T;
-        char *dst = p.apk + w.off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + threadIdx.x) * 16;
+        char *dst = p.apk + w.off + (size_t)step * sp_block(p.pieces) + ((o & 1) * SP_ROWS + threadIdx.x) * 16;
         *reinterpret_cast<uint32x4 *>(dst) = q0;
+        if (p.pieces == 1) return;
         *reinterpret_cast<uint32x4 *>(dst + 2 * SP_ROWS * 16) = q1;
         *reinterpret_cast<uint32x4 *>(dst + 4 * SP_ROWS * 16) = q2;
     };
     uint32x4 q0, q1, q2;
-    if (__builtin_amdgcn_ballot_w64(!test.all()) == 0) {
+    if (p.pieces == 1 || __builtin_amdgcn_ballot_w64(!test.all()) == 0) {
 #pragma unroll
         for (int t = 0; t < 9; ++t) { split8(v[t], q0, q1, q2); put(t, q0, q1, q2); }
         return;
@@ -921,10 +951,11 @@ __global__ void __launch_bounds__(256) split_pack_kernel(SpParams p, char *apk) 
                 v[e] = (int)row < c.rows && ch < p.CH ? src[(size_t)row * p.w_row + (size_t)ch * p.w_ch] : 0.f;
             }
             uint32x4 q0, q1, q2;
-            split8_any(v, q0, q1, q2);
+            if (p.pieces == 1) split8(v, q0, q1, q2); else split8_any(v, q0, q1, q2);
             const uint32_t step = (row / SP_ROWS) * c.iters + (uint32_t)ph.step0 + (o >> 1) * (uint32_t)ph.stride + (uint32_t)tl;
-            char *dst = apk + c.apk_off + (size_t)step * SP_BLOCK + ((o & 1) * SP_ROWS + row % SP_ROWS) * 16;
+            char *dst = apk + c.apk_off + (size_t)step * sp_block(p.pieces) + ((o & 1) * SP_ROWS + row % SP_ROWS) * 16;
             *reinterpret_cast<uint32x4 *>(dst) = q0;
+            if (p.pieces == 1) continue;
             *reinterpret_cast<uint32x4 *>(dst + 2 * SP_ROWS * 16) = q1;
             *reinterpret_cast<uint32x4 *>(dst + 4 * SP_ROWS * 16) = q2;
         }
@@ -1006,9 +1037,9 @@ bool sp_add_class(SpParams &p, int &nph, int &nkd, uint32_t &steps_bytes, const 
     c.dOX = xsmi::make_fastdiv(OX); c.dOY = xsmi::make_fastdiv(OY); c.dWp = xsmi::make_fastdiv(c.Wp); c.dHp = xsmi::make_fastdiv(c.Hp);
     c.dIT = xsmi::make_fastdiv(c.iters); c.dTM = xsmi::make_fastdiv(tiles_m);
     c.apk_off = steps_bytes;
-    const double bytes = (double)steps_bytes + (double)blocks_r * c.iters * SP_BLOCK, units = (double)p.units + (double)tiles_m * tiles_r * c.iters;
+    const double bytes = (double)steps_bytes + (double)blocks_r * c.iters * sp_block(p.pieces), units = (double)p.units + (double)tiles_m * tiles_r * c.iters;
     if (bytes >= 2e9 || units >= 1e9 || (double)c.Wp * c.Hp * p.N >= 1e9) return false;
-    steps_bytes += (uint32_t)blocks_r * c.iters * (uint32_t)SP_BLOCK;
+    steps_bytes += (uint32_t)blocks_r * c.iters * (uint32_t)sp_block(p.pieces);
     c.first_unit = p.units;
     p.units += (uint32_t)tiles_m * (uint32_t)tiles_r * c.iters;
     c.end_unit = p.units;
@@ -1031,6 +1062,8 @@ constexpr uint32_t SP_STRIDED_UNITS = 3300;
 
 bool sp_parts(int CH, int R, int S, int sh, int sw) { return (sh > 1 || sw > 1) && R * S <= 9 && CH >= 64; }
 
+bool sp_fills_rows(int rows, const SpTiling &k) { return 4 * rows >= 3 * xsmi::ceil_div(rows, k.rows()) * k.rows(); }   // three quarters
+
 // The tiling of a pass of m pixels (of its largest class), and its plan.
 //   256-pixel tiles stage 2.0 values for each pixel of a 3 x 3 layer's tile where 128-pixel tiles stage 3.0; passes below 1024
 //   pixels keep the smaller tile, whose last one is emptier by less.
@@ -1043,13 +1076,14 @@ bool sp_parts(int CH, int R, int S, int sh, int sw) { return (sh > 1 || sw > 1) 
 //   class: there the parts are channel groups.  128 -> 256 at 28 x 28, N=32: forward 58 -> 41 us, backward-data 70 -> 47 (fp32
 //   kernels 48 and 49); at N=128 147 -> 98 and 215 -> 124 (153, 154).
 template <typename Plan>
-bool sp_plan_tiled(SpParams &p, long m, int rows, bool parts, const Plan &plan) {
+bool sp_plan_tiled(SpParams &p, int pieces, long m, int rows, bool parts, const Plan &plan) {
     auto as = [&](int tiling) {
         memset(&p, 0, sizeof(p));
         p.tiling = tiling;
+        p.pieces = pieces;
         return plan(p);
     };
-    if (parts && 4 * rows >= 3 * xsmi::ceil_div(rows, SP_TILINGS[3].rows()) * SP_TILINGS[3].rows() && as(3) && p.units >= SP_STRIDED_UNITS) return true;
+    if (parts && sp_fills_rows(rows, SP_TILINGS[3]) && as(3) && p.units >= SP_STRIDED_UNITS) return true;
     if (m < 1024) return as(0);
     if (!as(1)) return false;
     if (rows > SP_TILINGS[2].rows() || p.units < 256u * sp_least(p)) return true;
@@ -1057,7 +1091,7 @@ bool sp_plan_tiled(SpParams &p, long m, int rows, bool parts, const Plan &plan) 
 }
 
 bool sp_plan_fwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
-    return sp_plan_tiled(p, (long)N * OH * OW, K, sp_parts(C, R, S, sh, sw), [&](SpParams &p) {
+    return sp_plan_tiled(p, 3, (long)N * OH * OW, K, sp_parts(C, R, S, sh, sw), [&](SpParams &p) {
         p.N = N; p.CH = C; p.groups = xsmi::ceil_div(C, 16); p.IH = H; p.IW = W; p.in_n = C * H * W; p.plane = H * W;
         p.w_row = C * R * S; p.w_ch = R * S; p.FS = S;
         int nph = 0, nkd = 0;
@@ -1071,8 +1105,8 @@ bool sp_plan_fwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, i
 }
 
 // backward-data: a class per residue (h mod sh, w mod sw); taps in ascending order of the dy row they read
-bool sp_plan_bwd(SpParams &p, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
-    return sp_plan_tiled(p, (long)N * H * W / (sh * sw), C, sp_parts(K, R, S, sh, sw), [&](SpParams &p) {
+bool sp_plan_bwd(SpParams &p, int pieces, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
+    return sp_plan_tiled(p, pieces, (long)N * H * W / (sh * sw), C, sp_parts(K, R, S, sh, sw), [&](SpParams &p) {
         p.N = N; p.CH = K; p.groups = xsmi::ceil_div(K, 16); p.IH = OH; p.IW = OW; p.in_n = K * OH * OW; p.plane = OH * OW;
         p.w_row = R * S; p.w_ch = C * R * S; p.FS = S;
         int nph = 0, nkd = 0;
@@ -1186,7 +1220,7 @@ int sp_run(SpParams &p, int opts, void *workspace) {
             SpPackJob &job = jobs.job[jobs.count];
             job.w = p.w; job.apk = (char *)workspace; job.row_tiles = row_tiles;
             job.end_block = row_tiles * octets + (jobs.count ? jobs.job[jobs.count - 1].end_block : 0u);
-            job.rows = p.cls[0].rows; job.CH = p.CH; job.w_row = p.w_row; job.w_ch = p.w_ch;
+            job.rows = p.cls[0].rows; job.CH = p.CH; job.w_row = p.w_row; job.w_ch = p.w_ch; job.pieces = p.pieces;
             for (int i = 0; i < p.ncls; ++i)
                 for (int f = p.cls[i].phase0; f < p.cls[i].phase0 + p.cls[i].nphase; ++f)
                     for (int t = 0; t < p.ph[f].T; ++t) {
@@ -1206,14 +1240,16 @@ int sp_run(SpParams &p, int opts, void *workspace) {
     }
     if (opts & 4) return XSMI_OK;
     constexpr int TILINGS = sizeof(SP_TILINGS) / sizeof(SP_TILINGS[0]);
-    static int resident[4 * TILINGS] = {};
+    static int resident[6 * TILINGS] = {};
     const SpTiling &tl = SP_TILINGS[p.tiling];
     const int threads = tl.threads();
-    void (*const kernels[4 * TILINGS])(SpParams) = {
-        split_conv_kernel<0, false, false>, split_conv_kernel<1, false, false>, split_conv_kernel<2, false, false>, split_conv_kernel<3, false, false>,
-        split_conv_kernel<0, true, false>, split_conv_kernel<1, true, false>, split_conv_kernel<2, true, false>, split_conv_kernel<3, true, false>,
-        split_conv_kernel<0, false, true>, split_conv_kernel<1, false, true>, split_conv_kernel<2, false, true>, split_conv_kernel<3, false, true>,
-        split_conv_kernel<0, true, true>, split_conv_kernel<1, true, true>, split_conv_kernel<2, true, true>, split_conv_kernel<3, true, true>};
+#define XSMI_SP_KERNELS(SIGNS, TILES, PIECES)                                                                                      \
+    split_conv_kernel<0, SIGNS, TILES, PIECES>, split_conv_kernel<1, SIGNS, TILES, PIECES>, split_conv_kernel<2, SIGNS, TILES, PIECES>, \
+        split_conv_kernel<3, SIGNS, TILES, PIECES>
+    void (*const kernels[6 * TILINGS])(SpParams) = {                  // the tilings of a form; a form's tiles are two forms on
+        XSMI_SP_KERNELS(false, false, 3), XSMI_SP_KERNELS(true, false, 3), XSMI_SP_KERNELS(false, true, 3), XSMI_SP_KERNELS(true, true, 3),
+        XSMI_SP_KERNELS(false, false, 1), XSMI_SP_KERNELS(false, true, 1)};
+#undef XSMI_SP_KERNELS
     auto resident_groups = [&](int which) {
         int &res = resident[which];
         if (res == 0) {
@@ -1225,13 +1261,14 @@ int sp_run(SpParams &p, int opts, void *workspace) {
         }
         return (uint32_t)res;
     };
-    int which = p.mask ? TILINGS + p.tiling : p.tiling;
+    int which = (p.pieces == 1 ? 4 * TILINGS : p.mask ? TILINGS : 0) + p.tiling;
+    const int tiles_form = which + (p.pieces == 1 ? TILINGS : 2 * TILINGS);
     const uint32_t least = sp_least(p);
     uint32_t grid = resident_groups(which);
     if (grid > p.units / least) grid = p.units / least;
     if (grid == 0) grid = 1;
-    if (const uint32_t groups = sp_deal_tiles(p, resident_groups(which + 2 * TILINGS), grid)) {
-        which += 2 * TILINGS;
+    if (const uint32_t groups = sp_deal_tiles(p, resident_groups(tiles_form), grid)) {
+        which = tiles_form;
         grid = groups;
     } else {
         p.upg = p.units / grid; p.urem = p.units % grid;
@@ -1288,7 +1325,7 @@ size_t split_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, 
     if (option(OPT_CONV_SPLIT) == 0 || sh > R || sw > S) return 0;
     const long pixels = (long)N * ceil_div(H, sh) * ceil_div(W, sw);
     if (!split_pays(K, R, S, sh, sw, pixels)) return 0;
-    if (!sp_plan_bwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW) || !split_plan_pays(p, sh, sw, pixels, true)) return 0;
+    if (!sp_plan_bwd(p, 3, N, C, H, W, K, R, S, sh, sw, pad, OH, OW) || !split_plan_pays(p, sh, sw, pixels, true)) return 0;
     return align_up(p.apk_bytes, 256);
 }
 
@@ -1305,6 +1342,22 @@ int split_pack_launch(bool launch) {
     return launch && jobs ? sp_launch_pack(*jobs) : XSMI_OK;
 }
 
+// Backward-data with operands rounded to bf16: the same kernel with one piece, so one product for six, which reads dy as it
+// is and shares small launches' tiles.  Kept against the tap-major bf16 kernel, which gathers dy for every tap:
+//   from 4 taps on (1 x 1, 128 -> 128 at 56 x 56, N=32: 34 -> 45 us);
+//   strided in the 128 x 128 tiling, as in fp32 (128 -> 256 at 28 x 28, N=32: 40 -> 29 us; 64 -> 128 at 56 x 56, which has 64
+//     rows: 46 -> 54), or where one pixel tile holds a class.
+// 25 layers with stride 1: 0.08 to 0.84 of the time (128 -> 128 at 28 x 28, N=32 38 -> 27 us; 512 -> 512 at 7 x 7 131 -> 33, N=1 110
+// -> 17; 64 -> 64 at 56 x 56, N=256 220 -> 160).  The forward stays with the channels-last kernels: its sums have one order,
+// whatever the batch and the form of the result.
+size_t split_bf16_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
+    SpParams p;
+    if (option(OPT_CONV_SPLIT) == 0 || !tap_path_ok(K) || sh > R || sw > S || (R * S < 4 && option(OPT_CONV_SPLIT) < 2)) return 0;
+    if (!sp_plan_bwd(p, 1, N, C, H, W, K, R, S, sh, sw, pad, OH, OW)) return 0;
+    if (option(OPT_CONV_SPLIT) < 2 && (sh > 1 || sw > 1) && !SP_TILINGS[p.tiling].parts && (long)N * H * W > 256L * sh * sw) return 0;
+    return align_up(p.apk_bytes, 256);
+}
+
 int split_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
                    int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace) {
     SpParams p;
@@ -1315,9 +1368,9 @@ int split_conv_fwd(const float *x, const float *w, const float *bias, float *y, 
 }
 
 int split_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, int H, int W, int K, int R, int S, int sh,
-                        int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace) {
+                        int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace, int pieces) {
     SpParams p;
-    if (!sp_plan_bwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW))
+    if (!sp_plan_bwd(p, pieces, N, C, H, W, K, R, S, sh, sw, pad, OH, OW))
         return set_error("split convolution: geometry not served"), XSMI_ERR_INVALID;
     p.in = dy; p.w = w; p.out = dx; p.accumulate = accumulate;
     return sp_run(p, opts, workspace);

@@ -161,10 +161,12 @@ size_t split_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int s
 size_t split_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW);
 void split_pack_collect();
 int split_pack_launch(bool launch);
+// pieces: 3, or 1 for operands rounded to bf16 (the bf16 query says where that pays)
+size_t split_bf16_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW);
 int split_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
                    int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace);
 int split_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, int H, int W, int K, int R, int S, int sh,
-                        int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace);
+                        int sw, int pad, int OH, int OW, int accumulate, int opts, void *workspace, int pieces);
 
 // weight gradient, likewise (conv_split_wgrad.hip): filters up to 16 x 16, any stride; `served` is false, and nothing done, for a
 // geometry or a workspace that it does not serve
