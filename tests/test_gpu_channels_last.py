@@ -56,6 +56,24 @@ def test_channels_last_output_is_the_plain_result_rounded_to_bf16(gpu, n, c, h, 
     np.testing.assert_array_equal(y.numpy(), got)              # and the float32 memory now holds it
 
 
+@pytest.mark.parametrize("n,c,h,k", [
+    (64, 32, 30, 128),                       # 256 tiles of 128 rows: 64 rows
+    (65, 32, 30, 128),                       # 260: 128 rows
+    (65, 64, 30, 72),                        # ... a partial one
+    (65, 32, 30, 192),                       # three times 64 rows: 64
+])
+def test_rows_of_a_tile_do_not_change_a_bit(gpu, n, c, h, k):
+    """The float32 result comes from tiles of 64 rows, the channels-last one from 64 or 128, by the size of the launch."""
+    K = gpu.kernels
+    x, w, b = _inputs(np.random.default_rng(n + k), n, c, h, k, 3)
+    dx, dw, db = gpu.to_device(x), gpu.to_device(w), gpu.to_device(b)
+    plain = K.conv2d_fwd(dx, dw, db, (1, 1), 1, bf16=True).numpy()
+    ws = K.Workspace()
+    for packed in (False, True):
+        y = K.conv2d_fwd(dx, dw, db, (1, 1), 1, bf16=True, channels_last=True, workspace=ws, packed=packed)
+        np.testing.assert_array_equal(y.numpy(), bf16_round(plain))
+
+
 @pytest.mark.parametrize("stride2,r2,pad2", [(1, 3, 1), (2, 3, 1), (2, 1, 0), (1, 1, 0)])
 def test_channels_last_chain_equals_the_plain_path(gpu, stride2, r2, pad2):
     """conv -> conv with the activation never leaving channels-last form; the second conv also covers a border wider

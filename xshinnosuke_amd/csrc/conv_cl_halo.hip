@@ -553,17 +553,32 @@ int stem_cl_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk,
     return XSMI_OK;
 }
 
+// Rows of a tile.  128 rows stage the input half as often and stream the filter through twice the MFMAs; 64 give the launch
+// twice the workgroups.  64 where they multiply fewer zero rows (96 -> 192 at 30 x 30, N=256: 110 -> 102 us), where tiles of 128
+// rows leave compute units idle (128 -> 128 at 28 x 28, N=32, 113 of them: 23.2 -> 15.8; 225: 28.0 -> 25.1; 338: 39.8 and 38.9;
+// 450: 44.9 and 46.3; 512 -> 384 at 14 x 14, N=96, 288: 100 and 106), and where every result is float32, whose stores are what
+// the fewer waves wait for (128 -> 128 at 28 x 28 with the copy of the input, N=32 43.0 -> 32.5, N=256 136 -> 127; 512 -> 384 at
+// 14 x 14, N=96 125 -> 131).  The filter's layout follows, so neither the form of this call's result nor of its input decides:
+// `f32_only` is a fact of the entry point.  The order of the sums is the same.
+static int halo_rows(int K, uint32_t tiles, bool f32_only) {
+    if (K <= 64 || f32_only || ceil_div(K, 64) % 2 != 0) return 64;
+    return tiles * (uint32_t)ceil_div(K, 128) <= (uint32_t)cu_count() ? 64 : 128;
+}
+
 size_t halo_apk_bytes(int C, int K) {
-    const int ROWS = K <= 64 ? 64 : 128;
+    const int ROWS = K <= 64 ? 64 : 128;               // the larger of the two
     return align_up((size_t)ceil_div(K, ROWS) * (C / 32) * 9 * ROWS * 64, 256);
 }
 
 // xp: the bordered channels-last input (border 1); apk: workspace for the packed filter (halo_apk_bytes);
 // y (fp32 NCHW) or y_cl (bordered channels-last bf16, border 1) receives the result.
 int halo_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk, const float *bias, float *y, void *y_cl,
-                  uint8_t *mask, int N, int C, int H, int W, int K, int relu, bool packed) {
+                  uint8_t *mask, int N, int C, int H, int W, int K, int relu, bool packed, bool f32_only) {
     hipStream_t st = stream();
-    const int ROWS = K <= 64 ? 64 : 128;
+    const uint32_t pixels = (uint32_t)N * (uint32_t)(H + 2) * (uint32_t)(W + 2), skipped = 2u * (uint32_t)(W + 3);
+    // local position i of tile t is position t * PIX + i + Wp + 1: the first Wp + 1 positions (border) are skipped
+    const uint32_t tiles = pixels > skipped ? (pixels - skipped + HALO_PIX - 1) / HALO_PIX : 0u;
+    const int ROWS = halo_rows(K, tiles, f32_only);
     const int rowtiles = ceil_div(K, ROWS), NG = C / 32;
     const size_t apk_elems = (size_t)rowtiles * NG * 9 * ROWS * 32;
     if (!packed) {
@@ -576,10 +591,8 @@ int halo_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk, co
     p.xp = (const __bf16 *)xp; p.apk = (const __bf16 *)apk; p.bias = bias; p.out = y; p.out_cl = (__bf16 *)y_cl; p.mask = (relu && !y_cl) ? mask : nullptr;
     p.xp_bytes = (uint32_t)xp_bytes; p.apk_bytes = (uint32_t)(apk_elems * 2);
     p.Hp = H + 2; p.Wp = W + 2; p.H = H; p.W = W;
-    p.pixels = (uint32_t)N * (uint32_t)p.Hp * (uint32_t)p.Wp;
-    // local position i of tile t is position t * PIX + i + Wp + 1: the first Wp + 1 positions (border) are skipped
-    const uint32_t positions = p.pixels > 2u * (uint32_t)(p.Wp + 1) ? p.pixels - 2u * (uint32_t)(p.Wp + 1) : 0u;
-    p.tiles = (positions + HALO_PIX - 1) / HALO_PIX;
+    p.pixels = pixels;
+    p.tiles = tiles;
     p.rowtiles = rowtiles; p.groups = NG; p.rows = K; p.C = C;
     p.dWp = make_fastdiv(p.Wp); p.dHp = make_fastdiv(p.Hp);
     p.relu = relu;

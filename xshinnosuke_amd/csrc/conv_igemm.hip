@@ -388,7 +388,7 @@ int xsmi_conv2d_fwd(const float *x, const float *w, const float *bias, float *y,
     switch (fwd_path(N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, flags, workspace_bytes)) {
     case FwdPath::ChannelsLast:
         return xsmi::nhwc_conv_fwd(x, nullptr, 0, w, bias, y, nullptr, 0, neg_mask, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW,
-                                   relu, opts, workspace);
+                                   relu, opts | 8, workspace);
     case FwdPath::Thin:
         if (flags & XSMI_CONV_PACK_ONLY) return XSMI_OK;
         return xsmi::thin_conv_fwd(x, w, bias, y, neg_mask, N, C, H, W, K, R, S, sh, sw, pad, g.OH, g.OW, relu);

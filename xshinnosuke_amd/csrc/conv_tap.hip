@@ -1455,7 +1455,7 @@ size_t nhwc_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int pa
 
 // x_cl: the input as a channels-last bf16 tensor [N][H + 2 xb][W + 2 xb][C] with a zero border xb >= pad (C a multiple
 // of 32), instead of x: no copy is made.  y_cl: the output goes to a channels-last bf16 tensor with border yb
-// (K a multiple of 8; only its interior is written) instead of y.
+// (K a multiple of 8; only its interior is written) instead of y.  opts & 8: the caller's entry point has no y_cl.
 int nhwc_conv_fwd(const float *x, const void *x_cl, int xb, const float *w, const float *bias, float *y, void *y_cl, int yb,
                   uint8_t *mask, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW,
                   int relu, int opts, void *workspace) {
@@ -1508,7 +1508,7 @@ int nhwc_conv_fwd(const float *x, const void *x_cl, int xb, const float *w, cons
         return stem_cl_conv_fwd(xp, ((size_t)N * Hp * Wp + 1) * CP * 2, w, apk, bias, y_cl, N, C, H, W, K, R, S, pad, OH, OW, relu,
                                 (opts & 2) != 0);
     if (halo) {
-        return halo_conv_fwd(xp, (size_t)N * Hp * Wp * CP * 2, w, apk, bias, y, y_cl, mask, N, C, H, W, K, relu, (opts & 2) != 0);
+        return halo_conv_fwd(xp, (size_t)N * Hp * Wp * CP * 2, w, apk, bias, y, y_cl, mask, N, C, H, W, K, relu, (opts & 2) != 0, (opts & 8) != 0);
     }
     NhwcParams p;
     p.xp = xp; p.apk = (const float *)apk; p.bias = bias; p.out = y; p.mask = relu ? mask : nullptr;

@@ -205,7 +205,7 @@ int nhwc_conv_fwd(const float *x, const void *x_cl, int xb, const float *w, cons
 bool halo_fwd_ok(int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int border);
 size_t halo_apk_bytes(int C, int K);
 int halo_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk, const float *bias, float *y, void *y_cl,
-                  uint8_t *mask, int N, int C, int H, int W, int K, int relu, bool packed);
+                  uint8_t *mask, int N, int C, int H, int W, int K, int relu, bool packed, bool f32_only);
 
 // first layer (at most 4 channels, 7-row filter, stride 2) with channels-last bf16 output (conv_cl_halo.hip); called by
 // nhwc_conv_fwd after it has made the bordered 4-channel copy
