@@ -214,6 +214,8 @@ int xsmi_cl_add(const void *a, const void *b, void *out, size_t count, int relu)
  * the max; writes the interior of y_cl (border y_border).  No argmax: inference only. */
 int xsmi_cl_maxpool2d(const void *x_cl, int x_border, void *y_cl, int y_border,
                       int N, int C, int H, int W, int k, int sh, int sw, int pad);
+/* avg_pool2d (xs/nn/functional.py:539-583) over whole planes of a channels-last tensor: y (fp32, N,C,1,1). */
+int xsmi_cl_avgpool(const void *x_cl, int border, float *y, int N, int C, int H, int W);
 /* y (fp32, N,C,H,W) = the interior of a channels-last tensor: for every consumer that
  * reads float32 NCHW. */
 int xsmi_cl_to_nchw(const void *x_cl, int border, float *y, int N, int C, int H, int W);

@@ -755,6 +755,10 @@ def avgpool_fwd(x, k, stride=None):
     if k > h or k > w or sh < 1 or sw < 1:
         raise ValueError("avg_pool2d: window %d does not fit the input %dx%d" % (k, h, w))
     y = empty((n, c, (h - k) // sh + 1, (w - k) // sw + 1))
+    xcl = x.channels_last() if k == h == w else None
+    if xcl is not None:                           # whole planes of an input that lives in channels-last form
+        lib.call("xsmi_cl_avgpool", xcl.buf.ptr, xcl.border, y.ptr, n, c, h, w)
+        return y
     lib.call("xsmi_avgpool_fwd", x.ptr, y.ptr, n, c, h, w, int(k), sh, sw)
     return y
 

@@ -7,6 +7,7 @@
 //   cl_add_relu   out = max(0, a + b) (or a + b) over whole buffers, borders included (0 + 0 = 0 keeps them zero)
 //   cl_maxpool    k x k / stride max pooling; the zero border of the input IS the reference's zero-valued padding
 //                 that takes part in the max (xs/nn/functional.py:445-491), so no bounds tests in the window loop
+//   cl_avgpool    the mean over each whole plane, fp32: the end of a network without its map as fp32 NCHW in between
 //   cl_to_nchw    the fp32 NCHW form of a channels-last tensor, for every consumer that does not read channels-last
 #include "xsmi_internal.h"
 
@@ -75,6 +76,40 @@ __global__ void __launch_bounds__(256) cl_maxpool_kernel(const bf16x8 *__restric
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = (__bf16)m[e];
     y[(((size_t)n * Hpo + oy + ob) * Wpo + ox + ob) * C8 + c8] = o;
+}
+
+// A workgroup takes 64 octets of channels (consecutive lanes: whole kilobytes of a pixel's record) and deals the plane's pixels
+// over its eight waves.  Sums in float64, as over fp32 planes; of bf16 values they are exact in any order.  Bound by the latency
+// of a wave's few loads: 256 x 512 x 7 x 7 5 us, against 40 for the conversion to fp32 and the mean over that.
+__global__ void __launch_bounds__(512) cl_avgpool_kernel(const bf16x8 *__restrict__ x, float *__restrict__ y, int C8, int H, int W, int b,
+                                                          uint32_t octets, xsmi::FastDiv dC8, xsmi::FastDiv dW) {
+    __shared__ double part[8][64 * 8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t i = blockIdx.x * 64u + (uint32_t)lane;
+    double s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = 0.0;
+    if (i < octets) {
+        const uint32_t n = xsmi::fdiv(i, dC8), o = i - n * (uint32_t)C8;
+        const int Wp = W + 2 * b;
+        const bf16x8 *src = x + (((size_t)n * (H + 2 * b) + b) * Wp + b) * C8 + o;
+#pragma unroll 4
+        for (int p = wave; p < H * W; p += 8) {
+            const int h = (int)xsmi::fdiv((uint32_t)p, dW);
+            const bf16x8 v = src[((size_t)h * Wp + (p - h * W)) * C8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s[e] += (double)(float)v[e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) part[wave][lane * 8 + e] = s[e];
+    __syncthreads();
+    const uint32_t out = blockIdx.x * 512u + threadIdx.x;
+    if (out >= octets * 8u) return;
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) sum += part[w][threadIdx.x];
+    y[out] = (float)(sum / (double)(H * W));
 }
 
 // A workgroup converts one segment (at most 255 pixels) of an image row for 64 channels through an LDS tile
@@ -153,6 +188,20 @@ int xsmi_cl_maxpool2d(const void *x_cl, int x_border, void *y_cl, int y_border, 
     else XSMI_CL_POOL(0);
 #undef XSMI_CL_POOL
     XSMI_LAUNCH_CHECK("cl_maxpool_kernel");
+    return XSMI_OK;
+}
+
+int xsmi_cl_avgpool(const void *x_cl, int border, float *y, int N, int C, int H, int W) {
+    XSMI_REQUIRE_INIT();
+    XSMI_CHECK_ARG(x_cl && y, "xsmi_cl_avgpool: null pointer");
+    XSMI_CHECK_ARG(N > 0 && C > 0 && C % 8 == 0 && H > 0 && W > 0 && border >= 0,
+                   "xsmi_cl_avgpool: needs C %% 8 == 0 (N=%d C=%d H=%d W=%d border=%d)", N, C, H, W, border);
+    XSMI_CHECK_ARG(((uintptr_t)x_cl & 15) == 0, "xsmi_cl_avgpool: x_cl must be 16-byte aligned");
+    const size_t octets = (size_t)N * (C / 8);
+    XSMI_CHECK_ARG(octets < ((size_t)1 << 28) && (size_t)H * W < ((size_t)1 << 31), "xsmi_cl_avgpool: too many planes or pixels");
+    hipLaunchKernelGGL(cl_avgpool_kernel, dim3((unsigned)((octets + 63) / 64)), dim3(512), 0, xsmi::stream(), (const bf16x8 *)x_cl, y,
+                       C / 8, H, W, border, (uint32_t)octets, xsmi::make_fastdiv(C / 8), xsmi::make_fastdiv(W));
+    XSMI_LAUNCH_CHECK("cl_avgpool_kernel");
     return XSMI_OK;
 }
 
