@@ -737,7 +737,7 @@ def main():
         "over_fp32_mfma_peak": value / FP32_MFMA_PEAK_TFLOPS,
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": SPLIT_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / SPLIT_MFMA_PEAK_TFLOPS, "traffic": tap_sk_traffic_bytes(),
-                     "kernel": "split_conv_kernel<1, false>", "flop_per_launch": flops_pass, "avg_launch_ms": igemm_ms},
+                     "kernel": "split_conv_kernel<1, false, false, 3>", "flop_per_launch": flops_pass, "avg_launch_ms": igemm_ms},
         "ops_ms": {"conv_fwd": per["fwd"], "conv_bwd_data": per["bwd_data"], "conv_bwd_weight": per["bwd_weight"]},
         "kernels_ms": {"fwd": per["fwd_kernel"], "bwd_data": per["bwd_data_kernel"]},
         "ops_tflops": {k: flops_pass / (per[k] * 1e-3) / 1e12 for k in ("fwd", "bwd_data", "bwd_weight")},

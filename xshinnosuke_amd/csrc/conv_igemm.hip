@@ -595,8 +595,8 @@ int xsmi_conv2d_pack(int count, xsmi_pack_job_t *jobs) {
             if (rc) break;
             forked = true;
         }
-        // the layouts are short independent launches (3-8 us each, mostly dispatch latency): they are dealt over
-        // four streams that all start behind the fork, so a ResNet's ~40 of them take a quarter of the time in a row
+        // layouts of 3 x 3 filters for the split kernel share launches; the others are short independent launches (3-8 us
+        // each, mostly dispatch latency), dealt over up to four streams that all start behind the fork
         rc = xsmi::side_lane(lanes++ % nlanes);
         if (rc) break;
         float *unused = const_cast<float *>(j.w);        // activations are not touched by a layout-only call
