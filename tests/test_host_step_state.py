@@ -128,6 +128,41 @@ def test_a_filter_layout_is_current_exactly_until_the_filter_address_is_handed_o
     assert other is not entry and not current
 
 
+@pytest.mark.parametrize("call", ("forward", "backward-data", "both gradients"))
+def test_a_recording_keeps_a_filter_whose_layout_is_in_place(recorder, call):
+    x, w, dw = dev.empty((2, 3, 32, 32)), dev.empty((64, 3, 7, 7)), dev.empty((64, 3, 7, 7))
+    y, dx = dev.empty((2, 64, 16, 16)), dev.empty((2, 3, 32, 32))
+    run = {"forward": lambda: K.conv2d_fwd(x, w, None, (2, 2), 3, out=y, keep_layout=True),
+           "backward-data": lambda: K.conv2d_bwd_data(y, w, x.shape, (2, 2), 3, dx=dx, keep_layout=True),
+           "both gradients": lambda: K.conv2d_bwd(y, x, w, dx, dw, None, (2, 2), 3, keep_layout=True)}[call]
+    run()                                             # the filter is laid out, if its kernel has a layout at all
+    state = w.state()
+    graph = StepGraph()
+    with graph.capture():
+        run()                                         # first-layer and table-driven kernels read the filter all the same
+    assert w.state() == state
+    assert id(w._block) in graph._refs and id(y._block) in graph._refs
+    address = w.address()
+    del w, run
+    gc.collect()
+    assert address not in _pooled()                   # nobody else is handed the memory that replays read
+    graph.close()
+    gc.collect()
+    assert address in _pooled()
+
+
+def test_a_read_address_carries_out_what_is_pending_and_does_not_count_as_handed_out(recorder):
+    w = dev.empty((8, 8, 3, 3))
+    state = w.state()
+    assert w.read_ptr == w.address() and w.state() == state
+    w.fill_zero(lazy=True)
+    w.read_ptr
+    assert recorder.calls[-1] == "xsmi_memset" and not w.is_fresh()
+    w.never_written("fused")
+    with pytest.raises(capi.XsmiError):
+        w.read_ptr
+
+
 def test_operands_are_kept_only_for_a_weight_gradient_that_the_library_left_on_its_second_stream(recorder):
     x, dy, w, dx, dw = (dev.empty(s) for s in ((2, 8, 6, 6), (2, 8, 6, 6), (8, 8, 3, 3), (2, 8, 6, 6), (8, 8, 3, 3)))
     run = lambda **kw: K.conv2d_bwd(dy, x, w, dx, dw, None, (1, 1), 1, **kw)  # noqa: E731

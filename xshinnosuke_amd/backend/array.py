@@ -175,6 +175,18 @@ class DeviceArray:
             lib.call("xsmi_cl_to_nchw", cl.buf.cptr, cl.border, ctypes.c_void_p(blk.ptr), cl.n, cl.c, cl.h, cl.w)
         return blk.ptr + self._offset
 
+    @property
+    def read_ptr(self):
+        """``ptr`` for a kernel that only reads: an open capture keeps the memory alive and a pending clear or conversion
+        is carried out as there, but contents that are in place do not count as handed out (``state`` stays)."""
+        blk = self._block
+        if blk.unwritten is not None or blk.lazy_zero or (blk.cl is not None and blk.cl.valid):
+            return self.ptr
+        graph = _CAPTURE[0]
+        if graph is not None and blk.owner is not graph:
+            graph._refs[id(blk)] = blk
+        return blk.ptr + self._offset
+
     def state(self):
         """(allocation, version): equal to an earlier value exactly when the address has not been handed out (to a
         kernel, a copy, the host) and no clear was scheduled since, i.e. the contents cannot have changed.  Lets
@@ -183,7 +195,7 @@ class DeviceArray:
 
     def address(self):
         """The device address as an integer; unlike ``ptr`` it leaves a pending clear pending (for alignment and
-        aliasing checks)."""
+        aliasing checks).  Never for a kernel: an open capture does not learn of the memory."""
         return self._block.ptr + self._offset
 
     def channels_last(self):

@@ -235,8 +235,9 @@ def conv2d_fwd(x, w, bias=None, stride=(1, 1), pad=0, relu=False, out=None, neg_
                      flags & ~CONV_BF16, ws, ws_bytes)
             return out
     out._overwritten()
-    # a filter whose layout is in place is not read: its address goes along without counting as handed out
-    wptr = ctypes.c_void_p(w.address()) if layout is not None and packed else w.ptr
+    # a filter whose layout is in place does not count as handed out: the kernel reads the layout, or, where none of it is
+    # made ahead (first layers, few products, the table-driven kernel), the filter itself, and writes neither
+    wptr = w.read_ptr if layout is not None and packed else w.ptr
     lib.call("xsmi_conv2d_fwd", x.ptr, wptr, bias.ptr if bias is not None else None, out.ptr,
              neg_mask.ptr if neg_mask is not None else None, *dims, flags, ws, ws_bytes)
     if layout is not None and not packed:
@@ -274,7 +275,7 @@ def conv2d_bwd_data(dy, w, x_shape, stride=(1, 1), pad=0, dx=None, accumulate=Fa
         layout, packed = _layout_for(w, 1, dims)
     ws, ws_bytes = _workspace(dims) if layout is None else layout.ws.get(_need_pass(dims, 1))
     beta = _beta(accumulate, dx)
-    wptr = ctypes.c_void_p(w.address()) if layout is not None and packed else w.ptr
+    wptr = w.read_ptr if layout is not None and packed else w.ptr
     lib.call("xsmi_conv2d_bwd_data", dy.ptr, wptr, dx.ptr, *dims, beta,
              (CONV_BF16 if bf16 else 0) | (CONV_WS_PACKED if packed else 0), ws, ws_bytes)
     if layout is not None and not packed:
@@ -334,7 +335,7 @@ def conv2d_bwd(dy, x, w, dx, dw, db=None, stride=(1, 1), pad=0, accumulate=False
     beta_dw = _beta(accumulate, dw, db)
     beta_dx = _beta(accumulate, dx)
     flags = (CONV_BF16 if bf16 else 0) | (CONV_DW_ASYNC if async_dw else 0) | (CONV_WS_PACKED if packed else 0)
-    wptr = ctypes.c_void_p(w.address()) if layout is not None and packed else w.ptr
+    wptr = w.read_ptr if layout is not None and packed else w.ptr
     lib.call("xsmi_conv2d_bwd", dy.ptr, x.ptr, wptr, dx.ptr, dw.ptr, db.ptr if db is not None else None, *dims,
              beta_dx, beta_dw, flags, ws, ws_bytes, ws_dw, ws_dw_bytes)
     if layout is not None and not packed:
