@@ -383,6 +383,30 @@ def test_bf16_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad):
     assert not calm.all() and rel_l2(got[calm], plain[calm]) <= 1e-5
 
 
+@pytest.mark.parametrize("n,c,h,w,k,r,s,st,pad,bf16,split", [
+    (32, 128, 28, 28, 256, 3, 3, 2, 1, False, True),     # strided: a compute unit for every tile
+    (59, 448, 18, 18, 128, 3, 3, 2, 0, False, False),    # more tiles, few steps each
+    (13, 192, 51, 51, 128, 3, 3, 2, 1, False, False),    # the second row tile half empty
+    (45, 128, 32, 31, 320, 3, 3, 2, 1, False, True),     # 15000 steps and more
+    (38, 256, 34, 32, 64, 3, 3, 2, 1, False, False),     # fewer than 128 filters
+])
+def test_which_kernel_a_data_gradient_takes(gpu, n, c, h, w, k, r, s, st, pad, bf16, split):
+    """By the rule on either side of its lines: the split kernel's sums have another order than the others'."""
+    K = gpu.kernels
+    _, wt, _, dy, _ = _data(n, c, h, w, k, r, s, st, st, pad, gpu)
+    dw_, ddy = gpu.to_device(wt), gpu.to_device(dy)
+    run = lambda: K.conv2d_bwd_data(ddy, dw_, (n, c, h, w), (st, st), pad, bf16=bf16).numpy()  # noqa: E731
+    got = run()
+    old = gpu.set_option("conv_split", 0)
+    try:
+        plain = run()
+    finally:
+        gpu.set_option("conv_split", old)
+    assert rel_l2(got, plain) <= TOL
+    other_bits = got.tobytes() != plain.tobytes()
+    assert other_bits == split
+
+
 @pytest.mark.parametrize("count", [1, 20, 21, 43])
 def test_layouts_made_in_one_call(gpu, count):
     """A launch takes the layouts of 20 filters: bit-identical to the layout that a call makes for itself, also where a filter

@@ -1297,9 +1297,8 @@ namespace xsmi {
 //   fewer than 16 channels: no.  A step multiplies 16, the rest zeros (4 -> 120, 3 x 3 at 102 x 102, N=53: 109 -> 226 us).
 //   strided with whole chunks of 32 channels: in the 128 x 128 tiling (sp_plan_tiled), not with emptier row tiles (160 rows,
 //     224 -> 160 at 42 x 42, N=17: 73 -> 92 us) or fewer channels (32 -> 296 at 21 x 70, N=35: 37 -> 45); backward-data, whose
-//     images have one to four taps of a few groups, from twice as many steps on (128 -> 256 at 29 x 29, N=14, 3280: 34 -> 36;
-//     at 28 x 28, N=32, 7056: 49 -> 47).  And where one pixel tile holds all pixels: the fp32 kernels then have a few
-//     workgroups with a long chain each (256 -> 512 at 14 x 14, N=1: 59 -> 42 us).
+//     images have one to four taps of a few groups, by split_plan_pays.  And where one pixel tile holds all pixels: the fp32
+//     kernels then have a few workgroups with a long chain each (256 -> 512 at 14 x 14, N=1: 59 -> 42 us).
 //   everything else: yes (64 -> 64 at 56 x 56, N=32: 67 -> 52 us; 369 -> 37, 5 x 5 at 76 x 76, N=2, which had only the
 //     table-driven kernel: 801 -> 93 us; equal at the smallest sizes, 64 -> 64 at 56 x 56, N=1: 20.2 -> 21.1 us).
 static bool split_pays(int CH, int R, int S, int sh, int sw, long pixels) {
@@ -1307,10 +1306,28 @@ static bool split_pays(int CH, int R, int S, int sh, int sw, long pixels) {
     if (R * S < 4 || CH < 16) return false;
     return (sh == 1 && sw == 1) || CH % 32 != 0 || pixels <= 256 || sp_parts(CH, R, S, sh, sw);
 }
-// ... and whether this plan does.
+// ... and whether this plan does.  Strided backward-data (fp32 kernels -> split, of 190 layers): a tile's steps must pay for its
+// start and its stores, and its second 64 rows must not be zeros, of which the fp32 kernels' 64-row tiles have none.
+//   From twice the forward's steps on where every tile has a compute unit (384 -> 512 at 46 x 31, N=3: 50 -> 45 us; 128 -> 256 at 28
+//     x 28, N=32: 47 -> 44; below, 256 -> 320 at 35 x 35, N=6, 5520 steps: 40 -> 41), from 15000 on where workgroups go from tile to
+//     tile (128 -> 320 at 32 x 31, N=45, 15600: 82 -> 75; 448 -> 128 at 18 x 18, N=59, 10944: 68 -> 85);
+//   an even number of 64-row blocks (192 -> 128 at 51 x 51, N=13: 51 -> 77; 192 -> 256 at 32 x 32, N=69: 154 -> 192), or seven and
+//     more, from 50000 on (448 -> 512 at 45 x 62, N=8: 226 -> 212; 416 -> 224 at 69 x 69, N=8, 37464: 174 -> 179);
+//   from 128 filters on (512 -> 64 at 32 x 51, N=55: 192 -> 208), 256 where the last tile is not whole (352 -> 480 at 40 x 40, N=56:
+//     667 -> 501; 352 -> 128 at 28 x 49, N=64: 220 -> 246).
+static uint32_t sp_tiles(const SpParams &p) {
+    uint32_t tiles = 0;
+    for (int i = 0; i < p.ncls; ++i) tiles += (p.cls[i].end_unit - p.cls[i].first_unit) / p.cls[i].iters;
+    return tiles;
+}
 static bool split_plan_pays(const SpParams &p, int sh, int sw, long pixels, bool backward) {
     if (option(OPT_CONV_SPLIT) >= 2 || (sh == 1 && sw == 1) || p.CH % 32 != 0 || pixels <= 256) return true;
-    return SP_TILINGS[p.tiling].parts && (!backward || p.units >= 2 * SP_STRIDED_UNITS);
+    if (!SP_TILINGS[p.tiling].parts) return false;
+    if (!backward) return true;
+    const int rows = p.cls[0].rows, blocks = p.cls[0].blocks;
+    if (p.CH < (rows % SP_TILINGS[3].rows() == 0 ? 128 : 256)) return false;
+    if (blocks % 2 != 0) return blocks >= 7 && p.units >= 50000;
+    return p.units >= (sp_tiles(p) <= (uint32_t)cu_count() ? 2 * SP_STRIDED_UNITS : 15000u);
 }
 
 // Workspace bytes of the split form, 0 where it does not serve the geometry or does not pay.
