@@ -389,6 +389,14 @@ def test_bf16_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad):
     (13, 192, 51, 51, 128, 3, 3, 2, 1, False, False),    # the second row tile half empty
     (45, 128, 32, 31, 320, 3, 3, 2, 1, False, True),     # 15000 steps and more
     (38, 256, 34, 32, 64, 3, 3, 2, 1, False, False),     # fewer than 128 filters
+    (32, 128, 28, 28, 256, 3, 3, 2, 1, True, True),
+    (22, 224, 54, 54, 128, 3, 3, 2, 1, True, False),     # more tiles than units, more channels than filters
+    (1, 512, 32, 32, 352, 2, 2, 2, 0, True, False),      # one tap a class
+    (1, 512, 7, 7, 512, 3, 3, 1, 1, True, True),
+    (14, 23, 48, 48, 32, 4, 2, 1, 0, True, False),       # 32 channels to at most 32 rows
+    (44, 160, 47, 45, 64, 2, 2, 1, 1, True, False),      # more tiles than units: four taps an image,
+    (40, 64, 54, 54, 64, 3, 3, 1, 1, True, True),        # nine,
+    (20, 128, 64, 64, 64, 3, 3, 1, 0, True, False),      # six and three
 ])
 def test_which_kernel_a_data_gradient_takes(gpu, n, c, h, w, k, r, s, st, pad, bf16, split):
     """By the rule on either side of its lines: the split kernel's sums have another order than the others'."""

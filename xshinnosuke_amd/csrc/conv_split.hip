@@ -1360,18 +1360,44 @@ int split_pack_launch(bool launch) {
 }
 
 // Backward-data with operands rounded to bf16: the same kernel with one piece, so one product for six, which reads dy as it
-// is and shares small launches' tiles.  Kept against the tap-major bf16 kernel, which gathers dy for every tap:
-//   from 4 taps on (1 x 1, 128 -> 128 at 56 x 56, N=32: 34 -> 45 us);
-//   strided in the 128 x 128 tiling, as in fp32 (128 -> 256 at 28 x 28, N=32: 40 -> 29 us; 64 -> 128 at 56 x 56, which has 64
-//     rows: 46 -> 54), or where one pixel tile holds a class.
-// 25 layers with stride 1: 0.08 to 0.84 of the time (128 -> 128 at 28 x 28, N=32 38 -> 27 us; 512 -> 512 at 7 x 7 131 -> 33, N=1 110
-// -> 17; 64 -> 64 at 56 x 56, N=256 220 -> 160).  The forward stays with the channels-last kernels: its sums have one order,
-// whatever the batch and the form of the result.
+// is and shares small launches' tiles.  Against the tap-major bf16 kernel, which gathers dy for every tap (tap-major -> this one,
+// of 500 layers):
+//   from 4 taps on (1 x 1, 128 -> 128 at 56 x 56, N=32: 34 -> 45 us).
+//   Stride 1, launches of at most a tile a compute unit, whose idle units are what the tap-major kernel loses: yes, 0.14 to 0.95 of
+//     the time (512 -> 512 at 7 x 7: N=32 131 -> 33, N=1 110 -> 17; 128 -> 192, 2 x 2 at 29 x 29, N=35: 32 -> 28), but for 32 channels
+//     to at most 32 rows (23 -> 32, 4 x 2 at 48 x 48, N=14: 16 -> 18).
+//   Stride 1, larger launches: from 64 reduced channels on (506 -> 32 at 32 x 32, N=125: 125 -> 158) where an image serves nine taps
+//     or more in row tiles three quarters full (128 -> 128 at 28 x 28, N=128: 94 -> 71; 64 -> 64 at 56 x 56, N=256: 220 -> 160;
+//     512 -> 128, 2 x 2 at 42 x 42, N=84: 231 -> 323; 310 -> 160, 1 x 7 at 68 x 46, N=36: 177 -> 202; 249 -> 288 at 50 x 67 without
+//     padding, N=15, whose rows make two images: 150 -> 185; 86 -> 64 at 59 x 59, N=36: 54 -> 58), or for at most 32 rows (16 -> 480,
+//     2 x 3 at 35 x 59, N=59: 209 -> 72).
+//   Strided, in the 128 x 128 tiling as in fp32 (64 -> 128 at 56 x 56, N=32, which has 64 rows: 46 -> 54), with more than two taps a
+//     class (193 -> 512, 2 x 2 / 2 at 10 x 62, N=100: 62 -> 100): up to a tile a compute unit (128 -> 256 at 28 x 28, N=32: 40 -> 29;
+//     192 -> 384 at 27 x 27, N=12: 55 -> 33), to one and a quarter with filters for three quarters of the channels (256 -> 352 at 63 x
+//     63, N=5, 312 tiles: 53 -> 49; 476 -> 224 at 68 x 68, N=2, 304: 42 -> 48; 320 -> 320 at 59 x 67, N=4, 384: 51 -> 57), beyond with
+//     twice as many filters as channels and whole row tiles (128 -> 256 at 28 x 28, N=128: 100 -> 89; 113 -> 256 at 36 x 36, N=41:
+//     51 -> 62; 224 -> 128 at 54 x 54, N=22: 58 -> 108; 384 -> 128 at 48 x 29, N=126: 230 -> 324).
+//   Strided, where one pixel tile holds a class of more than one tap (512 -> 352, 2 x 2 / 2 at 32 x 32, N=1: 24 -> 27).
+// The forward stays with the channels-last kernels: its sums have one order, whatever the batch and the form of the result.
+static bool split_bf16_plan_pays(const SpParams &p, int sh, int sw, long pixels) {
+    const uint32_t tiles = sp_tiles(p), cus = (uint32_t)cu_count();
+    const int rows = p.cls[0].rows;
+    if (sh > 1 || sw > 1) {
+        int taps = 0;
+        for (int i = 0; i < p.ncls; ++i) taps += p.cls[i].taps;
+        if (pixels <= 256L * sh * sw) return taps > sh * sw;
+        if (!SP_TILINGS[p.tiling].parts || taps <= 2 * sh * sw) return false;
+        return tiles <= cus || (4 * tiles <= 5 * cus && 4 * p.CH >= 3 * rows) || (p.CH >= 2 * rows && rows % SP_TILINGS[3].rows() == 0);
+    }
+    if (tiles <= cus) return p.CH >= 64 || rows > SP_TILINGS[2].rows();
+    return p.CH >= 64 && (rows <= SP_TILINGS[2].rows() ||
+                          (p.cls[0].taps >= 9 * p.cls[0].nphase && (rows <= SP_ROWS || sp_fills_rows(rows, SP_TILINGS[1]))));
+}
 size_t split_bf16_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
     SpParams p;
     if (option(OPT_CONV_SPLIT) == 0 || !tap_path_ok(K) || sh > R || sw > S || (R * S < 4 && option(OPT_CONV_SPLIT) < 2)) return 0;
     if (!sp_plan_bwd(p, 1, N, C, H, W, K, R, S, sh, sw, pad, OH, OW)) return 0;
-    if (option(OPT_CONV_SPLIT) < 2 && (sh > 1 || sw > 1) && !SP_TILINGS[p.tiling].parts && (long)N * H * W > 256L * sh * sw) return 0;
+    if (option(OPT_CONV_SPLIT) < 2 && !split_bf16_plan_pays(p, sh, sw, (long)N * H * W)) return 0;
     return align_up(p.apk_bytes, 256);
 }
 
