@@ -302,7 +302,8 @@ def test_conv_async_weight_gradients_of_a_sweep_share_the_second_stream(gpu):
 
 
 @pytest.mark.parametrize("n,c,h,w,k,r,s,sh,sw,pad,bf16,beside", [
-    (12, 64, 38, 38, 192, 3, 3, 1, 1, 1, True, True),      # 1.9e9 products, 136 tiles of a bf16 data gradient
+    (8, 64, 56, 56, 128, 3, 3, 2, 2, 1, True, True),       # 4.6e8 products, 196 tiles of a bf16 data gradient by taps
+    (12, 64, 38, 38, 192, 3, 3, 1, 1, 1, True, False),     # 1.9e9 products, 136 tiles, of the split kernel: it fills the chip
     (12, 64, 38, 38, 194, 3, 3, 1, 1, 1, True, False),     # no bf16 kernel for 194 filters: the data gradient fills the chip
     (2, 64, 38, 38, 192, 3, 3, 1, 1, 1, True, False),      # 3.2e8 products
     (13, 86, 11, 11, 224, 7, 7, 1, 1, 3, False, True),     # a few workgroups with a long chain: 1.5e9, 26 tiles, 10976 for a sum
@@ -312,8 +313,13 @@ def test_conv_async_weight_gradients_of_a_sweep_share_the_second_stream(gpu):
     (13, 100, 11, 11, 180, 7, 7, 1, 1, 3, False, False),   # 8820 for a sum
     (45, 100, 11, 11, 200, 7, 7, 2, 2, 3, False, False),   # 86 tiles
     (5, 200, 13, 13, 1000, 3, 3, 1, 1, 1, False, False),   # nine taps
+    (16, 31, 19, 19, 477, 5, 5, 2, 2, 2, False, False),    # strided, 25 taps: 6.0e8 products, not enough in float32
+    (16, 31, 19, 19, 477, 5, 5, 2, 2, 2, True, True),
+    (2, 116, 20, 32, 415, 5, 5, 1, 1, 2, False, False),    # 25 taps with stride 1
+    (3, 45, 32, 20, 435, 7, 7, 1, 1, 3, False, False),     # 45 channels with stride 1
     (29, 15, 25, 25, 160, 15, 15, 2, 2, 0, True, False),   # bf16, 142 tiles with 10240 for a sum
-    (5, 9, 55, 55, 128, 15, 15, 1, 1, 0, True, False),     # the same with 2.2e9 products
+    (32, 15, 25, 25, 160, 15, 15, 2, 2, 4, True, False),   # the same with 2.1e9 products
+    (5, 9, 55, 55, 128, 15, 15, 1, 1, 0, True, True),      # 2.2e9, of the split kernel
 ])
 def test_conv_weight_gradient_beside_a_small_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad, bf16, beside):
     """The second stream below 2e9 products: beside a data gradient that leaves compute units idle."""

@@ -133,22 +133,22 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     // The two kernels share only their inputs.  On the second stream (XSMI_CONV_DW_ASYNC: until xsmi_conv2d_bwd_join, otherwise
     // joined at once) the weight gradient runs beside what follows, but the fork and the join cost the host 18 us each, and the
     // split-operand kernels fill the chip alone.  In order on the main stream therefore, but for
-    //   a bf16 data gradient whose grid (128-pixel x 64-channel tiles) leaves compute units idle, from 4e8 products on (both
-    //     gradients, beside -> in order: 512 -> 512 at 7 x 7, N=32: 168 -> 212 us; 256 -> 224 at 14 x 14, N=8: 78 -> 90; below, 48 -> 64
-    //     at 28 x 28, N=16: 56 -> 51).  Under the flag, filters that no bf16 kernel takes have a split data gradient like float32
-    //     (96 -> 200 at 44 x 44, N=6: 107 -> 94; 160 -> 40, 5 x 5 at 51 x 51, N=3: 86 -> 74).  Not where more
-    //     than 64 tiles have 9500 or more products for a sum of one residue class: started behind the weight gradient's workgroups,
-    //     several of them land on a unit and stay there, for a time beside which the weight gradient's is short (9 -> 128, 15 x 15 at
-    //     55 x 55, N=5: 1280 -> 883; 15 -> 160, 15 x 15 / 2 at 25 x 25, N=29: 506 -> 351).  Of 82 other bf16 layers beside costs 0.90 of in
-    //     order in the mean; five lose 10 % or more;
-    //   a data gradient of either precision with at most 48 such tiles and filters of 25 taps or more that make 9000 or more products
-    //     for a sum, from 1e9 products on: a few workgroups with a long chain each (float32 layers forward and backward, beside -> in
-    //     order: 86 -> 224, 7 x 7 at 11 x 11, N=13: 147 -> 154; 256 -> 256, 7 x 7 at 20 x 20, N=2: 182 -> 198; 160 -> 352, 15 x 15 at 5
-    //     x 5, N=9: 485 -> 520; of 46 in both precisions 0.98 in the mean, 1.03 at the worst.  Below, the two gradients alone still
-    //     gain, 90 -> 200, 7 x 7 / 2 at 16 x 30, N=6: 62 -> 75, but a layer has no room for what the host pays: forward and backward of
-    //     48 -> 190, 7 x 7 at 7 x 7, N=5: 104 -> 88 us, inside a network 135 -> 93.  Under the bf16 flag, whose other passes are
-    //     longer, from 4e8 on: 44 -> 80, 15 x 15 / 2 at 68 x 68, N=1: 132 -> 149; 90 -> 200 as above 103 -> 117.  With smaller filters
-    //     more lose: 200 -> 1000, 3 x 3 at 13 x 13, N=5, both gradients 98 -> 87);
+    //   a data gradient by the tap-major bf16 kernel whose grid (128-pixel x 64-channel tiles) leaves compute units idle, from 4e8
+    //     products on (both gradients, in order -> beside: 64 -> 192, 7 x 7 / 2 at 32 x 56, N=8: 152 -> 134 us; 256 -> 512, 3 x 3 / 2 at 14 x
+    //     14, N=8: 92 -> 81; 64 -> 128, 3 x 3 / 2 at 56 x 56, N=8: 52 -> 48; 21 layers 0.79 to 1.06 of in order, 0.90 in the mean;
+    //     below, 64 -> 128 at 56 x 56, N=4: 44 -> 45).  Not where more than 64 tiles have 9500 or more products for a sum of one
+    //     residue class: started behind the weight gradient's workgroups, several of them land on a unit and stay there, for a time
+    //     beside which the weight gradient's is short (15 -> 160, 15 x 15 / 2 at 25 x 25, N=29: 417 -> 587).  Beside the one-piece split
+    //     kernel, which deals a small launch over all units, nothing is gained (512 -> 512 at 7 x 7, N=32: 101 -> 116; 128 -> 128 at 28 x
+    //     28, N=8: 45 -> 58; 190 layers of up to 256 tiles 1.01 to 1.5 of in order);
+    //   a data gradient of either precision with at most 48 such tiles and large filters that make 9000 or more products for a sum, a
+    //     few workgroups with a long chain each, from 1e9 products on; 4e8 under the bf16 flag, whose other passes are longer.  Strided,
+    //     from 25 taps on, below 7e9 products (in order -> beside, 100 -> 364, 7 x 7 / 2 at 18 x 36, N=4: 101 -> 85; 31 -> 477, 5 x 5 / 2 at
+    //     19 x 19, N=16: 65 -> 63; 30 layers 0.77 to 1.00); with stride 1 from 49 taps and more than 48 channels on, below 3e9 products (98
+    //     -> 160, 15 x 15 at 4 x 22, N=6: 139 -> 120; 115 -> 189, 7 x 7 at 39 x 39: 80 -> 78; 40 layers 0.87 to 1.0).  Beyond these lines
+    //     the workgroups that wait for one another's parts may hold units that the weight gradient could use (116 -> 415, 5 x 5 at 20 x
+    //     32, N=2: 85 -> 129; 25 -> 229, 7 x 7 at 34 x 8, N=21: 98 -> 126; 84 -> 118, 15 x 15 at 30 x 16, N=4, 4.3e9: 166 -> 184; 45 -> 435, 15 x 15
+    //     at 32 x 20, N=3, 8.4e9: 296 -> 369);
     //   layers of 2e9 products or more of a sweep that goes on, in float32 too: the passes between the convolutions find room
     //     (ResNet-18 steps: 224 x 224, N=32, 3.7e9 products a layer: 3.72 -> 4.01 ms; 192 x 192, 2.7e9: 3.13 -> 3.45; 224 x 224, N=16,
     //     1.85e9: 3.00 -> 2.76; 56 x 56, N=32: 3.01 -> 2.56).  A layer by itself is faster in order (64 -> 64 at 56 x 56, N=32, 3.7e9,
@@ -157,10 +157,12 @@ int xsmi_conv2d_bwd(const float *dy, const float *x, const float *w, float *dx, 
     const bool async = (flags & XSMI_CONV_DW_ASYNC) != 0;
     const double products = (double)N * OH * OW * C * K * R * S;
     const long long tiles = xsmi::data_gradient_tiles(N, C, H, W);
-    const bool few_tiles = kflags && xsmi::tap_path_ok(K) && tiles <= xsmi::cu_count();
+    const bool few_tiles = kflags && products >= 4e8 && tiles <= xsmi::cu_count() &&
+                           xsmi::bf16_data_gradient_by_taps(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
     const bool piles_up = few_tiles && tiles > 64 && (double)K * xsmi::ceil_div(R, sh) * xsmi::ceil_div(S, sw) >= 9500;
-    const bool long_chain = tiles <= 48 && R * S >= 25 && (double)K * R * S >= 9000;
-    const bool pays = (few_tiles && products >= 4e8) || (long_chain && products >= (kflags ? 4e8 : 1e9)) || (async && products >= 2e9);
+    const bool long_chain = tiles <= 48 && (double)K * R * S >= 9000 && products >= (kflags ? 4e8 : 1e9) &&
+                            (sh * sw > 1 ? R * S >= 25 && products < 7e9 : R * S >= 49 && C > 48 && products < 3e9);
+    const bool pays = few_tiles || long_chain || (async && products >= 2e9);
     const bool beside = (pays && !piles_up) || (async && xsmi::side_pending());
     int rc = beside ? xsmi::side_begin() : xsmi::side_join();    // in main-stream order: after any earlier async work
     if (rc) return rc;

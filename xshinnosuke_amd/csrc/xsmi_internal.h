@@ -163,6 +163,10 @@ void split_pack_collect();
 int split_pack_launch(bool launch);
 // pieces: 3, or 1 for operands rounded to bf16 (the bf16 query says where that pays)
 size_t split_bf16_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW);
+// whether a bf16 data gradient runs on the tap-major kernel
+inline bool bf16_data_gradient_by_taps(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
+    return tap_path_ok(K) && (option(OPT_TAP_SK) != 1 || !split_bf16_bwd_data_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW));
+}
 int split_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
                    int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace);
 int split_conv_bwd_data(const float *dy, const float *w, float *dx, int N, int C, int H, int W, int K, int R, int S, int sh,
@@ -325,7 +329,8 @@ __device__ __forceinline__ void block_barrier() {
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
-// 128-pixel x 64-channel tiles of a data gradient: up to cu_count() of them leave compute units to a weight gradient beside it
+// 128-pixel x 64-channel tiles of a data gradient: on the tap-major kernel up to cu_count() of them leave compute units to a weight
+// gradient beside it
 inline long long data_gradient_tiles(int N, int C, int H, int W) {
     return (((long long)N * H * W + 127) / 128) * ceil_div(C, 64);
 }
