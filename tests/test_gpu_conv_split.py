@@ -259,26 +259,30 @@ FORMED_AGAIN = [   # what the kernel that forms sums again walks differently
 ]
 
 
-@pytest.mark.parametrize("n,c,h,k,split", [
-    (32, 512, 7, 512, False),                # 104 tiles of the data gradient
-    (41, 256, 14, 128, False),               # 252: the most that leave a compute unit
-    (42, 256, 14, 128, True),                # 260: the data gradient fills the chip
-    (4, 64, 56, 256, True),                  # four times as many filters as channels
-    (5, 64, 56, 255, True),                  # no bf16 kernel for 255 filters, so no bf16 data gradient to let in
+@pytest.mark.parametrize("n,c,h,k,st,split", [
+    (32, 64, 32, 128, 2, False),             # 256 tiles of a data gradient by taps: the most that leave a compute unit
+    (33, 64, 32, 128, 2, True),              # 264: the data gradient fills the chip
+    (20, 64, 28, 256, 2, True),              # four times as many filters as channels
+    (8, 128, 28, 128, 1, False),             # a split data gradient of few tiles: in order, 9.2e8 products
+    (16, 128, 28, 128, 1, True),             # 1.8e9
+    (32, 512, 7, 512, 1, True),
+    (42, 256, 14, 128, 1, True),             # 260 tiles
+    (5, 64, 56, 255, 1, True),               # no bf16 kernel for 255 filters, so no bf16 data gradient to let in
 ])
-def test_weight_gradient_beside_a_bf16_data_gradient(gpu, n, c, h, k, split):
-    """A bf16 data gradient that leaves compute units idle runs beside the weight gradient, whose split form would keep it
-    out of them.  One call for both gradients and one for each give the same bits."""
+def test_weight_gradient_beside_a_bf16_data_gradient(gpu, n, c, h, k, st, split):
+    """A bf16 data gradient by taps that leaves compute units idle runs beside the weight gradient, whose split form would keep
+    it out of them; before a split one few products run on the tap kernel.  One call for both gradients and one for each give
+    the same bits."""
     K = gpu.kernels
     rng = np.random.default_rng(h)
-    x, w, dy = (gpu.to_device(rng.standard_normal(s).astype(np.float32)) for s in ((n, c, h, h), (k, c, 3, 3), (n, k, h, h)))
-    own = K.conv2d_bwd_weight(dy, x, w.shape, (1, 1), 1, bf16=True)[0].numpy()
+    x, w, dy = (gpu.to_device(rng.standard_normal(s).astype(np.float32)) for s in ((n, c, h, h), (k, c, 3, 3), (n, k, h // st, h // st)))
+    own = K.conv2d_bwd_weight(dy, x, w.shape, (st, st), 1, bf16=True)[0].numpy()
     dw = gpu.empty(w.shape)
-    K.conv2d_bwd(dy, x, w, gpu.empty(x.shape), dw, None, (1, 1), 1, bf16=True)
+    K.conv2d_bwd(dy, x, w, gpu.empty(x.shape), dw, None, (st, st), 1, bf16=True)
     np.testing.assert_array_equal(dw.numpy(), own)
     old = gpu.set_option("conv_split", 0)
     try:
-        fp32 = K.conv2d_bwd_weight(dy, x, w.shape, (1, 1), 1)[0].numpy()
+        fp32 = K.conv2d_bwd_weight(dy, x, w.shape, (st, st), 1)[0].numpy()
     finally:
         gpu.set_option("conv_split", old)
     assert np.array_equal(own, fp32) is not split

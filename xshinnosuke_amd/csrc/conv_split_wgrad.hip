@@ -643,15 +643,19 @@ static bool split_wgrad_serves(WgParams &p, int N, int C, int H, int W, int K, i
     const long opt = option(OPT_CONV_SPLIT);
     const int OH = (H + 2 * pad - R) / sh + 1, OW = (W + 2 * pad - S) / sw + 1;
     if (opt == 0 || (opt < 2 && !split_wgrad_pays(C, K, R, S, (double)N * OH * OW))) return false;
-    // A workgroup here fills a compute unit's LDS and registers.  A bf16 data gradient of few tiles, which is started beside the
-    // weight gradient (xsmi_conv2d_bwd), then waits and lands on the first units that come free, several of its workgroups on
-    // one: the fp32 tap kernel lets it in (both gradients, 512 -> 512 at 7 x 7, N=32: 241 -> 170 us; 256 -> 512, 3 x 3 / 2 at 14 x
-    // 14: 144 -> 103; 256 -> 256 at 14 x 14: 139 -> 118; 128 -> 128 at 28 x 28, N=8: 64 -> 59).  With four times as many filters as
-    // channels this kernel stays ahead (64 -> 512 at 56 x 56, N=4: 153 us, tap 185), beside a float32 data gradient (512 -> 512, N=32:
-    // 146, tap 163) or one that fills the chip by itself as well (N=128: 310, tap 453).  The table-driven fp32 kernel is too slow
-    // for that (64 -> 224 at 56 x 56, N=5: 99 us, table-driven 141; 96 -> 160, 5 x 5 at 40 x 40, N=4: 113, 158).  The rule looks at
-    // the flag, so that both ways to ask for a weight gradient give the same bits.
-    if (opt < 2 && bf16 && K < 4 * C && C % 64 == 0 && K % 64 == 0 && data_gradient_tiles(N, C, H, W) <= cu_count()) return false;
+    // Under the bf16 flag, at most a tile of the data gradient a compute unit, channels and filters multiples of 64.  A workgroup here
+    // fills a unit's LDS and registers: a data gradient on the tap-major kernel, which is started beside the weight gradient
+    // (xsmi_conv2d_bwd), waits and lands on the first units that come free, several of its workgroups on one, where the fp32 tap kernel
+    // lets it in (both gradients, split -> tap: 192 -> 384, 5 x 5 / 2 at 38 x 38, N=3: 184 -> 139 us; 256 -> 448, 3 x 3 / 2 at 18 x 18, N=9: 96
+    // -> 77; 64 -> 128 at 56 x 56, N=8: 60 -> 48; 64 -> 192, 7 x 7 / 2 at 32 x 56, N=8: 121 -> 134).  With four times as many filters as
+    // channels this kernel stays ahead (64 -> 512 at 56 x 56, N=4: 90 us, tap 99).  In order, before a split data gradient, the tap
+    // kernel is ahead below 1e9 products at 64 channels (64 -> 64 at 56 x 56: N=4 41 -> 36, N=8 49 -> 47; 128 -> 128 at 28 x 28, N=8: 45 -> 50), behind
+    // from there on (128 -> 128 at 28 x 28, N=16: 60 and 67; 256 -> 256 at 14 x 14, N=32: 90 and 102; 512 -> 512 at 7 x 7, N=32: 101 and 115).
+    // The table-driven fp32 kernel is too slow for either (64 -> 224 at 56 x 56, N=5: 67 us, table-driven 125).  The rule looks at the
+    // flag, so that both ways to ask for a weight gradient give the same bits.
+    if (opt < 2 && bf16 && K < 4 * C && C % 64 == 0 && K % 64 == 0 && data_gradient_tiles(N, C, H, W) <= cu_count() &&
+        ((double)N * OH * OW * C * K * R * S < 1e9 || bf16_data_gradient_by_taps(N, C, H, W, K, R, S, sh, sw, pad, OH, OW)))
+        return false;
     return wg_plan(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
 }
 static size_t wg_ws_bytes(const WgParams &p) { return wg_part_bytes(p) + align_up((size_t)p.splits * p.K * sizeof(float), 256); }
