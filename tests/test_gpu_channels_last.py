@@ -61,13 +61,17 @@ def test_channels_last_output_is_the_plain_result_rounded_to_bf16(gpu, n, c, h, 
     (65, 32, 30, 128),                       # 260: 128 rows
     (65, 64, 30, 72),                        # ... a partial one
     (65, 32, 30, 192),                       # three times 64 rows: 64
+    (129, 384, 14, 256),                     # 258 tiles of many channels: 128 rows for the float32 result too
+    (90, 384, 14, 376),                      # 270, the last row tile not whole
+    (260, 384, 14, 256),                     # 520: 64
 ])
 def test_rows_of_a_tile_do_not_change_a_bit(gpu, n, c, h, k):
-    """The float32 result comes from tiles of 64 rows, the channels-last one from 64 or 128, by the size of the launch."""
+    """Either result comes from tiles of 64 or of 128 rows, by the size of the launch; one image always from 64."""
     K = gpu.kernels
     x, w, b = _inputs(np.random.default_rng(n + k), n, c, h, k, 3)
     dx, dw, db = gpu.to_device(x), gpu.to_device(w), gpu.to_device(b)
     plain = K.conv2d_fwd(dx, dw, db, (1, 1), 1, bf16=True).numpy()
+    np.testing.assert_array_equal(K.conv2d_fwd(dx[n - 1:n], dw, db, (1, 1), 1, bf16=True).numpy(), plain[n - 1:])
     ws = K.Workspace()
     for packed in (False, True):
         y = K.conv2d_fwd(dx, dw, db, (1, 1), 1, bf16=True, channels_last=True, workspace=ws, packed=packed)

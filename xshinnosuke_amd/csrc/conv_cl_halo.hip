@@ -554,15 +554,19 @@ int stem_cl_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk,
 }
 
 // Rows of a tile.  128 rows stage the input half as often and stream the filter through twice the MFMAs; 64 give the launch
-// twice the workgroups.  64 where they multiply fewer zero rows (96 -> 192 at 30 x 30, N=256: 110 -> 102 us), where tiles of 128
+// twice the workgroups.  64 where they multiply fewer zero rows (96 -> 192 at 30 x 30, N=256: 110 -> 102 us) and where tiles of 128
 // rows leave compute units idle (128 -> 128 at 28 x 28, N=32, 113 of them: 23.2 -> 15.8; 225: 28.0 -> 25.1; 338: 39.8 and 38.9;
-// 450: 44.9 and 46.3; 512 -> 384 at 14 x 14, N=96, 288: 100 and 106), and where every result is float32, whose stores are what
-// the fewer waves wait for (128 -> 128 at 28 x 28 with the copy of the input, N=32 43.0 -> 32.5, N=256 136 -> 127; 512 -> 384 at
-// 14 x 14, N=96 125 -> 131).  The filter's layout follows, so neither the form of this call's result nor of its input decides:
-// `f32_only` is a fact of the entry point.  The order of the sums is the same.
-static int halo_rows(int K, uint32_t tiles, bool f32_only) {
-    if (K <= 64 || f32_only || ceil_div(K, 64) % 2 != 0) return 64;
-    return tiles * (uint32_t)ceil_div(K, 128) <= (uint32_t)cu_count() ? 64 : 128;
+// 450: 44.9 and 46.3; 512 -> 384 at 14 x 14, N=96, 288: 100 and 106).  Where every result is float32 the stores are what the fewer
+// waves wait for: 64 (with the copy of the input, 128 -> 128 at 28 x 28, N=32 43.0 -> 32.5, N=256 136 -> 127; 384 -> 512 at 14 x 14, N=96
+// 110 -> 106; 384 -> 256 at 40 x 40, N=38, 524 tiles: 196 -> 189), but for 384 channels and more in one to two tiles of 128 rows a
+// compute unit, two or three of them over the filters: there the shorter of two rounds is the smaller loss (of 43 such layers 64
+// rows take 0.98 to 1.07 of the time, 1.03 in the mean: 512 -> 384 at 14 x 14, N=96, 288 tiles: 133 and 137; 448 -> 384 at 40 x 40, N=19, 393:
+// 139 and 149).  The filter's layout follows, so neither the form of this call's result nor of its input decides: `f32_only` is
+// a fact of the entry point.  The order of the sums is the same.
+static int halo_rows(int C, int K, uint32_t tiles, bool f32_only) {
+    const uint32_t over = (uint32_t)ceil_div(K, 128), all = tiles * over, cus = (uint32_t)cu_count();
+    if (K <= 64 || ceil_div(K, 64) % 2 != 0 || all <= cus) return 64;
+    return !f32_only || (C >= 384 && all <= 2 * cus && (over == 2 || over == 3)) ? 128 : 64;
 }
 
 size_t halo_apk_bytes(int C, int K) {
@@ -578,7 +582,7 @@ int halo_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk, co
     const uint32_t pixels = (uint32_t)N * (uint32_t)(H + 2) * (uint32_t)(W + 2), skipped = 2u * (uint32_t)(W + 3);
     // local position i of tile t is position t * PIX + i + Wp + 1: the first Wp + 1 positions (border) are skipped
     const uint32_t tiles = pixels > skipped ? (pixels - skipped + HALO_PIX - 1) / HALO_PIX : 0u;
-    const int ROWS = halo_rows(K, tiles, f32_only);
+    const int ROWS = halo_rows(C, K, tiles, f32_only);
     const int rowtiles = ceil_div(K, ROWS), NG = C / 32;
     const size_t apk_elems = (size_t)rowtiles * NG * 9 * ROWS * 32;
     if (!packed) {
