@@ -16,6 +16,7 @@ TOL = 1e-6
     (1, 3, 64, 64, 64, 7, 3),        # one wide tile across, four down
     (2, 3, 63, 65, 32, 7, 3),        # a pixel past the tile, half of the filters
     (3, 3, 32, 32, 65, 7, 3),        # square tiles; a filter past the row tile
+    (2, 3, 40, 41, 36, 7, 3),        # the last rows in one half of the lanes only
     (1, 3, 7, 200, 64, 7, 0),        # one row of outputs, 97 across
     (5, 3, 224, 31, 40, 7, 2),       # narrow images
     (40, 3, 64, 48, 128, 7, 3),      # more tiles than workgroups, two row tiles

@@ -137,10 +137,10 @@ __global__ void __launch_bounds__(SS_THREADS) stem_split_kernel(StemSplitParams 
         for (int k = 0; k < S::TURNS; ++k) {
             const int ix = ix0 + (place[k] >> 16);
             const bool row = at[k] >= 0 && (unsigned)(iy0 + (place[k] & 0xffff)) < (unsigned)p.H;
-            const int off = (first + from[k]) * 4;
+            const uint32_t off = (uint32_t)(first + from[k]) * 4u;
 #pragma unroll
             for (int e = 0; e < 2; ++e)
-                raw[k][e] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rin, row && (unsigned)(ix + e) < (unsigned)p.W ? off + 4 * e : (int)0x80000000u, 0, 0);
+                raw[k][e] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rin, row && (unsigned)(ix + e) < (unsigned)p.W ? (int)(off + 4u * e) : (int)0x80000000u, 0, 0);
         }
     };
     auto stage = [&](uint32_t *img) {
@@ -271,25 +271,30 @@ __global__ void __launch_bounds__(SS_THREADS) stem_split_kernel(StemSplitParams 
         const __amdgpu_buffer_rsrc_t rmask = __builtin_amdgcn_make_buffer_rsrc((void *)(p.mask + (p.mask ? image : 0)), 0, p.mask ? p.os_n : 0, 0x00020000);
         int os_k = p.os_k;
         asm("" : "+s"(os_k));                          // 64 offsets formed ahead of the loop do not fit the scalar registers
-        const int lane_off = mine ? y * p.OX + x + 4 * h * os_k : (int)0x20000000u;
-        const int rows_left = p.rows - tile_row0 - 4 * h;
+        // 0x20000000 is past every image (fewer than 2^29 outputs), four times that past its bytes; rows past the last one have
+        // the last one's scalar offset, which the range check takes off the length
+        const uint32_t lane_off = mine ? (uint32_t)(y * p.OX + x + 4 * h * os_k) : 0x20000000u;
+        const int rows_here = p.rows - tile_row0;
         // MODE 0: bias only; 1: bias + relu; 2: bias + relu + sign mask
         auto emit = [&](auto mode, auto guard) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 2; ++i) {
+                if (guard && 32 * i >= rows_here) break;
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const float4 bias = *reinterpret_cast<const float4 *>(&s_bias[4 * h + 32 * i + 8 * g]);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const int ro = 32 * i + 8 * g + e, row_off = (tile_row0 + ro) * os_k;
-                        const int off = !guard || ro < rows_left ? lane_off : (int)0x20000000u;
+                        const int ro = 32 * i + 8 * g + e;
+                        const uint32_t row_off = (uint32_t)(tile_row0 + (!guard || ro < rows_here ? ro : rows_here - 1)) * (uint32_t)os_k;
+                        const uint32_t off = !guard || ro + 4 * h < rows_here ? lane_off : 0x20000000u;
                         float v = large[i][4 * g + e] + (e == 0 ? bias.x : e == 1 ? bias.y : e == 2 ? bias.z : bias.w);
-                        if (mode == 2) __builtin_amdgcn_raw_buffer_store_b8((unsigned char)(v < 0.f ? 1 : 0), rmask, off, row_off, 0);
+                        if (mode == 2) __builtin_amdgcn_raw_buffer_store_b8((unsigned char)(v < 0.f ? 1 : 0), rmask, (int)off, (int)row_off, 0);
                         if (mode >= 1) v = v > 0.f ? v : 0.f;
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rout, off * 4, row_off * 4, 0);
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rout, (int)(off * 4u), (int)(row_off * 4u), 0);
                     }
                 }
+            }
         };
         auto emit_mode = [&](auto guard) {
             if (!p.relu) emit(xsmi::IC<0>{}, guard);
