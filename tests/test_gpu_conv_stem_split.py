@@ -68,3 +68,22 @@ def test_values_that_do_not_split(gpu, c, h, w, r, pad):
     good = [i for i in range(40) if i not in (3, 7)]
     y_ref, _ = oracle.conv2d_fwd(x[2:].astype(np.float64) * 2.0 ** 120, wt[good], np.zeros(len(good), np.float32), (2, 2), pad)
     assert rel_l2(got[2:, good].astype(np.float64) * 2.0 ** 120, y_ref) <= 1e-5      # sums near the smallest normal float
+
+
+def test_a_workspace_without_room_for_a_copy(gpu):
+    """The kernel reads image and filter themselves: the size that the library asks for has no copy of the input (20 MB here), and
+    that size, or the static buffer of the forward that takes none, gives the same bits."""
+    from xshinnosuke_amd.backend import capi
+    K = gpu.kernels
+    rng = np.random.default_rng(3)
+    dims = (32, 3, 224, 224, 64, 7, 7, 2, 2, 3)
+    x, w = gpu.to_device(rng.standard_normal(dims[:4]).astype(np.float32)), gpu.to_device(he_normal(rng, (64, 3, 7, 7)))
+    want = K.conv2d_fwd(x, w, None, (2, 2), 3).numpy()
+    size = capi.lib.raw("xsmi_conv2d_pass_workspace_bytes")(*dims, 0, 0)
+    assert size < 1 << 20
+    ws, y = gpu.empty(((size + 3) // 4,)), gpu.empty(want.shape)
+    capi.lib.call("xsmi_conv2d_fwd", x.ptr, w.ptr, None, y.ptr, None, *dims, 0, ws.ptr, size)
+    np.testing.assert_array_equal(y.numpy(), want)
+    z = gpu.empty(want.shape)
+    capi.lib.call("xsmi_conv2d_fwd_noalloc", x.ptr, w.ptr, None, z.ptr, None, *dims, 0)
+    np.testing.assert_array_equal(z.numpy(), want)

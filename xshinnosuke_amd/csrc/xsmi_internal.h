@@ -179,11 +179,15 @@ int split_conv_bwd_weight(const float *dy, const float *x, float *dw, float *db,
                           int sw, int pad, bool bf16, int accumulate, void *workspace, size_t workspace_bytes, bool &served);
 
 // forward for very few input channels (conv_stem.hip): 1 or 3 channels, square filter of 3, 5 or 7, horizontal stride 2;
-// the workspace holds the packed filter followed by a zero-bordered copy of the input
+// the workspace holds the packed filter followed by a zero-bordered copy of the input.  Where stem_split_pays it runs on split
+// operands (conv_stem_split.hip), which read the filter and the input themselves, on every call, and need no workspace
 bool stem_fwd_ok(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad);
 size_t stem_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad);
 int stem_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
                   int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace);
+bool stem_split_pays(int C, int R, int K, int sh, int sw, int OH, int OW);
+int stem_split_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W, int K, int R,
+                   int pad, int OH, int OW, int relu);
 
 // forward and weight gradient of few products a result on the vector units (conv_thin.hip), fp32; the forward needs no workspace,
 // the weight gradient at most what conv_bwd_weight_ws_bytes says, which is what it is to be told
@@ -213,9 +217,6 @@ int halo_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk, co
 
 // first layer (at most 4 channels, 7-row filter, stride 2) with channels-last bf16 output (conv_cl_halo.hip); called by
 // nhwc_conv_fwd after it has made the bordered 4-channel copy
-bool stem_split_pays(int C, int R, int K, int sh, int sw, int OH, int OW);
-int stem_split_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W, int K, int R,
-                   int pad, int OH, int OW, int relu);
 bool stem_cl_ok(int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OW, int y_border);
 size_t stem_cl_apk_bytes();
 int stem_cl_conv_fwd(const void *xp, size_t xp_bytes, const float *w, void *apk, const float *bias, void *y_cl, int N, int C,
