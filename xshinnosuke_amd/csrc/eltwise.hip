@@ -89,6 +89,7 @@ size_t xsmi_conv2d_pass_workspace_bytes(int N, int C, int H, int W, int K, int R
         m = xsmi::conv_bwd_data_ws_bytes(C, K, R, S, sh, sw);
         if (!bf16 && xsmi::sk_bwd_data_ok(C, K, R, S, sh, sw)) m = larger(m, xsmi::sk_bwd_data_ws_bytes(C, K, R, S, sh, sw));
         if (xsmi::split_may_serve(K, bf16)) m = larger(m, xsmi::split_bwd_data_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW));
+        if (bf16) m = larger(m, xsmi::split_bf16_bwd_data_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW));
     } else if (pass == 2) {
         m = xsmi::conv_bwd_weight_ws_bytes(N, C, K, R, S, OH, OW);
         if (!bf16 && xsmi::stem_wgrad_ok(N, C, H, W, K, R, S, sh, sw, pad))
