@@ -80,7 +80,7 @@ def test_rows_of_a_tile_do_not_change_a_bit(gpu, n, c, h, k):
 
 @pytest.mark.parametrize("n,c,h", [(1, 8, 1), (3, 24, 5), (2, 512, 7), (5, 72, 13), (40, 128, 3)])
 def test_channels_last_average_over_planes(gpu, n, c, h):
-    """Bit for bit the mean over the float32 planes (float64 sums of bf16 values are exact); the input stays as it is."""
+    """Bit for bit the mean over the float32 planes (float64 sums of values this close together are exact); the input stays as it is."""
     K = gpu.kernels
     x, w, b = _inputs(np.random.default_rng(n + c + h), n, 32, h, c, 1)
     y = K.conv2d_fwd(gpu.to_device(x), gpu.to_device(w), gpu.to_device(b), (1, 1), 0, bf16=True, channels_last=True)

@@ -355,7 +355,8 @@ def test_a_filter_whose_layout_is_in_place_is_not_read(gpu, pass_):
     (20, 16, 45, 57, 64, 3, 3, 1, 1, 1),     # few rows: tiles of 32 x 512
     (34, 96, 29, 28, 224, 3, 3, 2, 2, 0),    # strided, 128 x 128
     (2, 24, 19, 23, 64, 7, 7, 2, 2, 3),      # four classes
-    (2, 18, 12, 12, 32, 3, 3, 3, 3, 0),      # nine of one tap
+    (2, 18, 13, 12, 32, 2, 2, 2, 2, 0),      # four of one tap
+    (3, 18, 12, 14, 32, 4, 3, 2, 1, 1),      # two
     (2, 30, 15, 17, 64, 1, 1, 1, 1, 0),
     (13, 98, 57, 57, 64, 2, 2, 1, 1, 1),
 ])
@@ -385,6 +386,7 @@ def test_bf16_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad):
         np.testing.assert_array_equal(test(got), test(plain))
     calm = np.isfinite(plain)
     assert not calm.all() and rel_l2(got[calm], plain[calm]) <= 1e-5
+    assert (got[calm] != plain[calm]).any()              # the sums of two kernels
 
 
 @pytest.mark.parametrize("n,c,h,w,k,r,s,st,pad,bf16,split", [

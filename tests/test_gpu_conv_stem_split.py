@@ -12,6 +12,15 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-6
 
 
+def _fp32_kernel(gpu, x, w, b, pad):
+    """The same by the kernel on the fp32 matrix instructions, whose sums have another order."""
+    old = gpu.set_option("conv_split", 0)
+    try:
+        return gpu.kernels.conv2d_fwd(x, w, b, (2, 2), pad).numpy()
+    finally:
+        gpu.set_option("conv_split", old)
+
+
 @pytest.mark.parametrize("n,c,h,w,k,r,pad", [
     (1, 3, 64, 64, 64, 7, 3),        # one wide tile across, four down
     (2, 3, 63, 65, 32, 7, 3),        # a pixel past the tile, half of the filters
@@ -25,8 +34,8 @@ TOL = 1e-6
     (4, 3, 65, 33, 96, 3, 1),
     (3, 3, 33, 32, 64, 3, 5),        # a border wider than the filter
     (3, 1, 61, 97, 48, 7, 3),        # one channel: the last filter row by itself
-    (2, 1, 29, 30, 64, 5, 1),
-    (300, 1, 28, 28, 32, 3, 1),
+    (5, 1, 30, 29, 65, 7, 0),
+    (130, 1, 28, 28, 32, 7, 3),      # ... more tiles than workgroups
 ])
 def test_first_layer_against_the_oracle(gpu, n, c, h, w, k, r, pad):
     K = gpu.kernels
@@ -37,13 +46,14 @@ def test_first_layer_against_the_oracle(gpu, n, c, h, w, k, r, pad):
     dx, dw, db = (gpu.to_device(a) for a in (x, wt, b))
     y = K.conv2d_fwd(dx, dw, db, (2, 2), pad).numpy()
     assert rel_l2(y, y_ref) <= TOL
+    assert (y != _fp32_kernel(gpu, dx, dw, db, pad)).any()
     mask = gpu.empty(y.shape, np.uint8)
     act = K.conv2d_fwd(dx, dw, db, (2, 2), pad, relu=True, neg_mask=mask).numpy()
     np.testing.assert_array_equal(act, np.maximum(y, 0.0))
     np.testing.assert_array_equal(mask.numpy(), (y < 0).astype(np.uint8))
 
 
-@pytest.mark.parametrize("c,h,w,r,pad", [(3, 40, 44, 7, 3), (1, 33, 66, 5, 2)])
+@pytest.mark.parametrize("c,h,w,r,pad", [(3, 40, 44, 7, 3), (1, 33, 66, 7, 2), (3, 31, 70, 5, 2), (3, 45, 33, 3, 1)])
 def test_values_that_do_not_split(gpu, c, h, w, r, pad):
     """Infinities, NaN, the largest floats and values near the smallest: sums are what the fp32 kernels give, and no value
     reaches a sum whose window it is not in."""
@@ -56,15 +66,12 @@ def test_values_that_do_not_split(gpu, c, h, w, r, pad):
     x[2] *= np.float32(2.0 ** -120)
     dx, dw = gpu.to_device(x), gpu.to_device(wt)
     got = K.conv2d_fwd(dx, dw, None, (2, 2), pad).numpy()
-    old = gpu.set_option("conv_split", 0)
-    try:
-        plain = K.conv2d_fwd(dx, dw, None, (2, 2), pad).numpy()
-    finally:
-        gpu.set_option("conv_split", old)
+    plain = _fp32_kernel(gpu, dx, dw, None, pad)
     for test in (np.isnan, np.isposinf, np.isneginf):
         np.testing.assert_array_equal(test(got), test(plain))
     calm = np.isfinite(plain[:2])
     assert calm.any() and not calm.all() and rel_l2(got[:2][calm], plain[:2][calm]) <= TOL
+    assert (got[:2][calm] != plain[:2][calm]).any()
     good = [i for i in range(40) if i not in (3, 7)]
     y_ref, _ = oracle.conv2d_fwd(x[2:].astype(np.float64) * 2.0 ** 120, wt[good], np.zeros(len(good), np.float32), (2, 2), pad)
     assert rel_l2(got[2:, good].astype(np.float64) * 2.0 ** 120, y_ref) <= 1e-5      # sums near the smallest normal float

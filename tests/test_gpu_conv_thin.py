@@ -9,12 +9,14 @@ from util import he_normal
 pytestmark = pytest.mark.gpu
 
 # n c h w k r s sh sw pad: every width of the gathered row (4, 8, 16, 32 products) at its edges, filters around the groups of 2, 4,
-# 8 and 32, pixels around 256 and 512 and over several images, borders wider than the image's inside, strides, one pixel
+# 8 and 32, pixels around 256 and 512 and over several images, borders wider than the image's inside, strides, one pixel; then many
+# filters, which leave few splits of the weight gradient: 2 to 8 pixels a thread, the last split ragged, for 4, 8, 16 and 32 products
 GEOMETRIES = [
     (1, 1, 1, 1, 1, 1, 1, 1, 1, 0), (2, 1, 28, 28, 8, 2, 2, 1, 1, 0), (3, 4, 16, 32, 9, 1, 1, 1, 1, 0), (7, 1, 19, 27, 33, 2, 2, 1, 2, 1),
     (2, 5, 16, 16, 7, 1, 1, 1, 1, 0), (3, 2, 13, 11, 32, 2, 2, 2, 1, 2), (5, 1, 12, 9, 31, 3, 3, 1, 1, 1), (2, 8, 17, 15, 130, 1, 1, 1, 1, 0),
     (4, 1, 9, 40, 5, 1, 11, 1, 2, 5), (2, 16, 8, 33, 6, 1, 1, 1, 1, 0), (1, 1, 23, 23, 3, 4, 4, 3, 3, 3), (2, 17, 9, 9, 3, 1, 1, 1, 1, 0),
     (3, 3, 14, 18, 65, 3, 3, 1, 1, 1), (2, 1, 12, 12, 2, 5, 5, 2, 2, 4), (2, 32, 7, 11, 5, 1, 1, 1, 1, 0), (300, 1, 21, 20, 4, 2, 2, 1, 1, 0),
+    (9, 1, 41, 40, 301, 2, 2, 1, 1, 0), (9, 2, 30, 31, 300, 2, 2, 1, 1, 0), (12, 1, 33, 35, 257, 4, 4, 1, 1, 1), (5, 3, 40, 41, 130, 3, 3, 1, 1, 0),
 ]
 
 
@@ -44,8 +46,21 @@ def test_few_products_against_the_oracle(gpu, geom):
         np.testing.assert_array_equal(mask.numpy(), (y < 0).astype(np.uint8))
         gw, gb = gpu.to_device(dw0), gpu.to_device(db0)
         K.conv2d_bwd_weight(ddy, dx_, wt.shape, (sh, sw), pad, dw=gw, db=gb, accumulate=True)
-        # at most 4 pixels of a thread here, 6 + 2 sums over the wave and the workgroup, two roundings of the result
-        assert (np.abs(gw.numpy() - dw_ref) <= 14 * u * dw_abs).all()
+        # pixels of a thread (the last geometries are planned with 2 to 8; a small workspace halves the splits), 6 + 2 sums over the wave
+        # and the workgroup, two roundings of the result
+        bound = (16 if k >= 130 and n * h * w > 8000 else 1) + 10
+        assert (np.abs(gw.numpy() - dw_ref) <= bound * u * dw_abs).all()
         assert (np.abs(gb.numpy() - db_ref) <= 3 * u * db_abs).all()
         only, _ = K.conv2d_bwd_weight(ddy, dx_, wt.shape, (sh, sw), pad)
-    assert (np.abs(only.numpy() + dw0.astype(np.float64) - dw_ref) <= 14 * u * dw_abs).all()
+    assert (np.abs(only.numpy() + dw0.astype(np.float64) - dw_ref) <= bound * u * dw_abs).all()
+
+
+def test_groups_of_filters_in_a_large_forward(gpu):
+    """536 workgroups of pixels, each with the filters in groups of 32: two groups, the second of eight."""
+    K = gpu.kernels
+    rng = np.random.default_rng(5)
+    x, wt, b = rng.standard_normal((67, 1, 63, 63)).astype(np.float32), he_normal(rng, (40, 1, 2, 2)), rng.standard_normal((40,)).astype(np.float32)
+    y_ref, _ = oracle.conv2d_fwd(x, wt, b, (1, 1), 1)
+    y_abs, _ = oracle.conv2d_fwd(np.abs(x), np.abs(wt), np.abs(b), (1, 1), 1)
+    y = K.conv2d_fwd(gpu.to_device(x), gpu.to_device(wt), gpu.to_device(b), (1, 1), 1).numpy()
+    assert (np.abs(y - y_ref) <= 7 * 2.0 ** -24 * y_abs).all()
