@@ -645,3 +645,52 @@ def test_bf16_calls_without_a_bf16_kernel_have_float32_precision(gpu, n, c, h, w
         assert rel_l2(y, np.maximum(y_ref, 0)) <= TOL
     dx = K.conv2d_bwd_data(ddy, dw_, x.shape, (stride, stride), pad, bf16=True).numpy()
     assert rel_l2(dx, dx_ref) <= TOL
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,stride,pad,most", [
+    (32, 128, 28, 28, 256, 3, 2, 1, 2.5),    # strided tiles of 128 x 128: measured 1.3 (before the sums that have settled: 4.5)
+    (32, 64, 56, 56, 64, 3, 1, 1, 3.0),      # the even deal: 1.8 (4.7)
+    (32, 3, 224, 224, 64, 7, 2, 3, 3.0),     # a first layer: 1.5 (5.2)
+    (1, 512, 7, 7, 512, 3, 1, 1, 2.5),       # tiles with workgroups of their own: 1.8 (3.0)
+])
+def test_nan_throughout_costs_its_first_terms(gpu, n, c, h, w, k, r, stride, pad, most):
+    """A sum that has become a NaN is not followed to its end; sums beside it, finite and infinite, are."""
+    K = gpu.kernels
+    rng = np.random.default_rng(k + h)
+    x, wt = rng.standard_normal((n, c, h, w)).astype(np.float32), he_normal(rng, (k, c, r, r))
+    dw = gpu.to_device(wt)
+
+    def forward(host):
+        dx, best = gpu.to_device(host), np.inf
+        y = K.conv2d_fwd(dx, dw, None, (stride, stride), pad).numpy()
+        gpu.profiling(True)
+        try:
+            for _ in range(12):
+                K.conv2d_fwd(dx, dw, None, (stride, stride), pad)
+                best = min(best, gpu.last_kernel_ms())
+        finally:
+            gpu.profiling(False)
+        return y, best
+
+    y, ordinary = forward(x)
+    none, slow = forward(np.full_like(x, np.nan))
+    assert np.isnan(none).all()
+    assert slow <= most * ordinary, (slow, ordinary)
+    mixed = x.copy()
+    mixed[0, 0] = np.nan                               # settles with the first channel ...
+    mixed[-1, c - 1, h - 1, :3] = np.inf               # ... does not until the last one, in the same tile where n = 1
+    got, _ = forward(mixed)
+    plain = _plain(gpu, mixed, dw, stride, pad)
+    for test in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(test(got), test(plain))
+    same = np.isfinite(got[1:])
+    np.testing.assert_array_equal(got[1:][same], y[1:][same])
+
+
+def _plain(gpu, x, dw, stride, pad):
+    """The same on the fp32 matrix instructions."""
+    old = gpu.set_option("conv_split", 0)
+    try:
+        return gpu.kernels.conv2d_fwd(gpu.to_device(x), dw, None, (stride, stride), pad).numpy()
+    finally:
+        gpu.set_option("conv_split", old)

@@ -46,7 +46,6 @@ using xsmi::uint32x4;
 using xsmi::IC;
 using xsmi::carried;
 typedef uint32_t uint32x2 __attribute__((ext_vector_type(2)));
-typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 constexpr int SP_ROWS = 64;                          // rows of a filter block
 // Tilings: WR x WC waves of 32 rows x 64 pixels, slots of an LDS image, most workgroups of a launch, whether an image has parts.
@@ -163,12 +162,12 @@ __device__ __forceinline__ double unsplit(uint32_t p0, uint32_t p1, uint32_t p2)
     return (double)((p0 & 0x7fffu) > 0x7f80u ? wide(p1 << 16 | (p2 & 0xffffu)) : (wide(p0 << 16) + wide(p1 << 16)) + wide(p2 << 16));
 }
 
-// The sums of a segment that the split does not carry (split3.h) are formed again in float64, 16 x 16 blocks on the fp64 matrix
-// instructions (D: register v of lane l is row l / 16 + 4 v, column l % 16): a step's 16 channels are four products deep,
-// a lane has channels 4 (l / 16) .. + 3 of a row and of a pixel.  The filter comes out of its layout, whose pieces are the
-// value (split8_any), so the filter itself is not read here either; a tap outside the input multiplies a zero, as the
-// reference's padding does.  Every workgroup does this for its own steps.  All of 64 -> 64 at 56 x 56, N=8, not finite:
-// 93 us (one product at a time, by the workgroups that store the outputs: 2490), 256 -> 256 at 14 x 14: 110 (10100).
+// The sums of a segment that the split does not carry (split3.h) are formed again in float64: a step's 16 channels are four
+// products deep, a lane has channels 4 (l / 16) .. + 3 of a row and of a pixel.  The filter comes out of its layout, whose pieces are
+// the value (split8_any), so the filter itself is not read here either; a tap outside the input multiplies a zero, as the
+// reference's padding does.  Every workgroup does this for its own steps.  Forward, ordinary values, NaN throughout, one infinity (and
+// by the fp32 kernels), us: 32 x 128 x 28 x 28 -> 256, 3 x 3 / 2: 44, 58, 107 (49, 45, 49); 32 x 64 x 56 x 56 -> 64: 58, 102, 116
+// (67); without the test for settled sums 44, 200, 115 and 58, 270, 125.
 struct SpSteps { int block, s_first, n, f, grp, tap; };   // filter block, steps of the tile, image kind and first group, tap of the image
 __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const SpClass &c, const SpSteps &sg, int row0, int m0, int lane,
                                            __amdgpu_buffer_rsrc_t rin, __amdgpu_buffer_rsrc_t rapk) {
@@ -181,14 +180,13 @@ __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const
         there[j] = m < c.M;
         ox[j] = m - q * c.OX; oy[j] = q - n * c.OY; image[j] = n * p.in_n;
     }
-    doublex4 d[2][2];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) d[j >> 1][j & 1] = doublex4{0.0, 0.0, 0.0, 0.0};
+    xsmi::FormAgain again(r, m0 + (lane & 31) < c.M, lane);
     const int a_lane = ((quarter >> 1) * SP_ROWS + row0 + l15) * 16 + (quarter & 1) * 8;
     uint32_t block = c.apk_off + ((uint32_t)sg.block * c.iters + (uint32_t)sg.s_first) * (uint32_t)SP_BLOCK;
     int f = sg.f, grp = sg.grp, tap = sg.tap;
 #pragma unroll 1
     for (int s = 0; s < sg.n; ++s, block += SP_BLOCK) {
+        if ((s < 4 || (s & 3) == 0) && again.settled()) break;   // (the test is as long as a step)
         const SpKind &kd = p.kd[f];
         const int g = tap / kd.T;
         int i = kd.phase0, ta = tap - g * kd.T;
@@ -196,7 +194,7 @@ __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const
         const SpPhase &ph = p.ph[i];
         const int tb = ta % ph.Tx, ch0 = (grp + g) * 16 + 4 * quarter;
         ta /= ph.Tx;
-        double a[2][4], b[2][4];
+        double a[4][2], b[4][2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             uint32x2 piece[3];
@@ -209,16 +207,13 @@ __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const
             for (int i = 0; i < 4; ++i) {
                 const uint32_t place = ((uint32_t)image[j] + (uint32_t)(ch0 + i) * (uint32_t)p.plane + (uint32_t)(iy * p.IW + ix)) * 4u;
                 const int bits = __builtin_amdgcn_raw_buffer_load_b32(rin, in && ch0 + i < p.CH ? (int)place : (int)0x80000000u, 0, 0);
-                b[j][i] = (double)__builtin_bit_cast(float, bits);
+                b[i][j] = (double)__builtin_bit_cast(float, bits);
                 const int sh = 16 * (i & 1);
-                a[j][i] = unsplit(piece[0][i >> 1] >> sh, piece[1][i >> 1] >> sh, piece[2][i >> 1] >> sh);
+                a[i][j] = unsplit(piece[0][i >> 1] >> sh, piece[1][i >> 1] >> sh, piece[2][i >> 1] >> sh);
             }
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                d[j >> 1][j & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j >> 1][i], b[j & 1][i], d[j >> 1][j & 1], 0, 0, 0);
+        for (int i = 0; i < 4; ++i) again.add(a[i], b[i]);
         const int left = p.groups - grp;
         if (++tap == kd.T * (left < kd.groups ? left : kd.groups)) {
             tap = 0;
@@ -226,17 +221,7 @@ __device__ __forceinline__ void form_again(floatx16 &r, const SpParams &p, const
             if (grp >= p.groups) { grp = 0; ++f; }
         }
     }
-    // to the 32 x 32 block's order: register v of lane l is row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        float from[2][2];                              // [right half of the columns][upper half of the lanes]
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            from[k >> 1][k & 1] = __shfl((float)d[v >> 3][k >> 1][2 * ((v >> 2) & 1) + (k & 1)], 16 * (v & 3) + l15);
-        const float low = (lane & 16) ? from[1][0] : from[0][0], high = (lane & 16) ? from[1][1] : from[0][1];
-        const float again = (lane & 32) ? high : low;
-        r[v] = carried(r[v]) ? r[v] : again;
-    }
+    again.take(r, lane);
 }
 
 // Where a sign mask is kept, the sign of a pre-activation decides which gradients flow, and one within rounding of zero falls on

@@ -25,9 +25,7 @@ namespace {
 
 using xsmi::bf16x8;
 using xsmi::uint32x4;
-using xsmi::carried;
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef double doublex4 __attribute__((ext_vector_type(4)));
+using xsmi::floatx16;
 
 constexpr int SS_THREADS = 512;
 
@@ -54,49 +52,44 @@ struct StemShape {
 };
 
 // The sums of a 32 x 32 block that are not carried, formed in float64 from the image and the filter.  Rare: a wave meets it
-// only where a value of its sums has no split (8 x 3 x 224 x 224, NaN throughout: 100 us, fp32 kernel 39, ordinary values 20).
+// only where a value of its sums has no split.  8 x 3 x 224 x 224 -> 64, 7 x 7: ordinary values 22 us, NaN throughout 33, one infinity 46 (fp32
+// kernel 38); N=32: 61, 92, 89 (fp32 103).  Without the test for settled sums NaN took 95 and 316; the test inside the loop over the
+// terms costs 9 us.
 template <int R, int C>
 __device__ __forceinline__ void stem_form_again(floatx16 &r, const float *in, const float *w, uint32_t in_bytes, int rows, int H, int W,
-                                                          int row0, int image, int iy0, int ix0, int lane) {
+                                                int row0, int image, int iy0, int ix0, bool mine, int lane) {
+    constexpr int TERMS = C * R * R, STEPS = (TERMS + 3) / 4;
     const int l15 = lane & 15, quarter = lane >> 4;
-    int iy[2], ix[2], n[2];                          // of the lane's column in either half of the block
+    int iy[2], ix[2], n[2];                            // of the lane's column in either half of the block
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         iy[j] = __shfl(iy0, 16 * j + l15); ix[j] = __shfl(ix0, 16 * j + l15); n[j] = __shfl(image, 16 * j + l15);
     }
     const __amdgpu_buffer_rsrc_t rin = __builtin_amdgcn_make_buffer_rsrc((void *)in, 0, (int)in_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)w, 0, rows * C * R * R * 4, 0x00020000);
-    doublex4 d[2][2];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) d[j >> 1][j & 1] = doublex4{0.0, 0.0, 0.0, 0.0};
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)w, 0, rows * TERMS * 4, 0x00020000);
+    xsmi::FormAgain again(mine, lane);
+    // a NaN throughout shows in the first terms, at the image's border after those of the padding
 #pragma unroll 1
-    for (int k0 = 0; k0 < C * R * R; k0 += 4) {
-        const int k = k0 + quarter, c = k / (R * R), rs = k - c * (R * R), y = rs / R, s = rs - y * R;
-        double a[2], b[2];
+    for (int i = 0, end = 1;; end = i == 1 && STEPS > 8 ? 8 : STEPS) {
+#pragma unroll 1
+        for (; i < end; ++i) {
+            const int k = 4 * i + quarter, c = k / (R * R), rs = k - c * (R * R), y = rs / R, s = rs - y * R;
+            double a[2], b[2];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int row = row0 + 16 * j + l15;
-            const int wb = __builtin_amdgcn_raw_buffer_load_b32(rw, k < C * R * R && row < rows ? (row * (C * R * R) + k) * 4 : (int)0x80000000u, 0, 0);
-            const bool there = k < C * R * R && (unsigned)(iy[j] + y) < (unsigned)H && (unsigned)(ix[j] + s) < (unsigned)W;
-            const uint32_t place = (uint32_t)(((n[j] * C + c) * H + iy[j] + y) * W + ix[j] + s) * 4u;
-            const int xb = __builtin_amdgcn_raw_buffer_load_b32(rin, there ? (int)place : (int)0x80000000u, 0, 0);
-            a[j] = (double)__builtin_bit_cast(float, wb);
-            b[j] = (double)__builtin_bit_cast(float, xb);
+            for (int j = 0; j < 2; ++j) {
+                const int row = row0 + 16 * j + l15;
+                const int wb = __builtin_amdgcn_raw_buffer_load_b32(rw, k < TERMS && row < rows ? (row * TERMS + k) * 4 : (int)0x80000000u, 0, 0);
+                const bool there = k < TERMS && (unsigned)(iy[j] + y) < (unsigned)H && (unsigned)(ix[j] + s) < (unsigned)W;
+                const uint32_t place = (uint32_t)(((n[j] * C + c) * H + iy[j] + y) * W + ix[j] + s) * 4u;
+                const int xb = __builtin_amdgcn_raw_buffer_load_b32(rin, there ? (int)place : (int)0x80000000u, 0, 0);
+                a[j] = (double)__builtin_bit_cast(float, wb);
+                b[j] = (double)__builtin_bit_cast(float, xb);
+            }
+            again.add(a, b);
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) d[j >> 1][j & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[j >> 1], b[j & 1], d[j >> 1][j & 1], 0, 0, 0);
+        if (i == STEPS || again.settled()) break;
     }
-    // to the 32 x 32 block's order: register v of lane l is row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        float from[2][2];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            from[k >> 1][k & 1] = __shfl((float)d[v >> 3][k >> 1][2 * ((v >> 2) & 1) + (k & 1)], 16 * (v & 3) + l15);
-        const float low = (lane & 16) ? from[1][0] : from[0][0], high = (lane & 16) ? from[1][1] : from[0][1];
-        const float again = (lane & 32) ? high : low;
-        r[v] = carried(r[v]) ? r[v] : again;
-    }
+    again.take(r, lane);
 }
 
 template <int R, int C, int TX>
@@ -262,7 +255,7 @@ __global__ void __launch_bounds__(SS_THREADS) stem_split_kernel(StemSplitParams 
 #pragma unroll 1
             for (int i = 0; i < 2; ++i) {
                 floatx16 r = i ? large[1] : large[0];
-                stem_form_again<R, C>(r, p.in, p.w, p.in_bytes, p.rows, p.H, p.W, tile_row0 + 32 * i, here.n, 2 * y - p.pad, 2 * x - p.pad, lane);
+                stem_form_again<R, C>(r, p.in, p.w, p.in_bytes, p.rows, p.H, p.W, tile_row0 + 32 * i, here.n, 2 * y - p.pad, 2 * x - p.pad, mine, lane);
                 if (i) large[1] = r; else large[0] = r;
             }
         // an image's outputs from a resource of its own: a lane's offset, a row's in a scalar register

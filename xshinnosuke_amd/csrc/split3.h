@@ -82,4 +82,66 @@ struct CarriedTest {
 };
 static_assert(__builtin_bit_cast(float, 0x0d800000u) == 0x1p-100f, "the bits of 2^-100");
 
+// The sums of a 32 x 32 block (register v of lane l is row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32) that are not carried, formed
+// in float64: four 16 x 16 blocks on the fp64 matrix instruction (D: register k of lane l is row l / 16 + 4 k, column l % 16).
+// Blocks that have no such sum are left out, and a sum that has become a NaN stays one: once all of them have, the terms that
+// are left are not read.  A tensor that holds NaN throughout then costs its first terms instead of all.
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+struct FormAgain {
+    doublex4 d[2][2];                                  // [rows][columns]
+    uint32_t need;                                     // bit 8 i + 4 (k / 2) + 2 (k % 2) + j for register k of rows i, columns j
+    uint32_t use;                                      // bit 2 i + j: whether any lane needs the block
+    // every sum of the columns that are there, in short code: what a kernel rarely does it also fetches for the occasion
+    __device__ __forceinline__ FormAgain(bool column_there, int lane) : need(0), use(15) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            need |= __shfl((int)column_there, 16 * j + (lane & 15)) ? 0x5555u << j : 0u;
+            d[0][j] = d[1][j] = doublex4{0.0, 0.0, 0.0, 0.0};
+        }
+    }
+    // those that are not carried, for long sums
+    __device__ __forceinline__ FormAgain(const floatx16 &r, bool column_there, int lane) : need(0), use(0) {
+        uint32_t open = 0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) open |= (carried(r[v]) ? 0u : 1u) << v;
+        open = column_there ? open : 0u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            need |= (((uint32_t)__shfl((int)open, 32 * (i >> 1) + 16 * (i & 1) + (lane & 15)) >> (lane >> 4)) & 0x1111u) << i;
+            d[i >> 1][i & 1] = doublex4{0.0, 0.0, 0.0, 0.0};
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) use |= (__builtin_amdgcn_ballot_w64((need & (0x55u << (8 * (i >> 1) + (i & 1)))) != 0) != 0 ? 1u : 0u) << i;
+    }
+    __device__ __forceinline__ void add(const double (&a)[2], const double (&b)[2]) {   // four terms
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (use >> i & 1) d[i >> 1][i & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i >> 1], b[i & 1], d[i >> 1][i & 1], 0, 0, 0);
+    }
+    __device__ __forceinline__ bool settled() const {
+        uint32_t open = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const double v = d[i >> 1][i & 1][k];
+                open |= v == v ? need & (1u << (8 * (i >> 1) + 4 * (k >> 1) + 2 * (k & 1) + (i & 1))) : 0u;
+            }
+        return __builtin_amdgcn_ballot_w64(open != 0) == 0;
+    }
+    __device__ __forceinline__ void take(floatx16 &r, int lane) const {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            float from[2][2];                          // [right half of the columns][upper half of the lanes]
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                from[k >> 1][k & 1] = __shfl((float)d[v >> 3][k >> 1][2 * ((v >> 2) & 1) + (k & 1)], 16 * (v & 3) + (lane & 15));
+            const float low = (lane & 16) ? from[1][0] : from[0][0], high = (lane & 16) ? from[1][1] : from[0][1];
+            const float again = (lane & 32) ? high : low;
+            r[v] = carried(r[v]) ? r[v] : again;
+        }
+    }
+};
+
 }  // namespace xsmi
