@@ -64,3 +64,49 @@ def test_groups_of_filters_in_a_large_forward(gpu):
     y_abs, _ = oracle.conv2d_fwd(np.abs(x), np.abs(wt), np.abs(b), (1, 1), 1)
     y = K.conv2d_fwd(gpu.to_device(x), gpu.to_device(wt), gpu.to_device(b), (1, 1), 1).numpy()
     assert (np.abs(y - y_ref) <= 7 * 2.0 ** -24 * y_abs).all()
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,s,stride,thin", [
+    (45, 16, 190, 26, 74, 1, 1, 2, False),       # strided, 16 products: 4.1e6 results
+    (9, 16, 190, 26, 74, 1, 1, 2, True),         # 0.8e6
+    (45, 16, 190, 26, 32, 1, 1, 2, True),        # one group of filters
+    (37, 11, 70, 70, 125, 1, 1, 1, False),       # stride 1, 1 x 1: 2.3e7
+    (20, 11, 70, 70, 125, 1, 1, 1, True),
+    (170, 1, 44, 16, 440, 3, 3, 1, False),       # stride 1, 3 x 3: 4.4e7
+    (100, 1, 44, 16, 440, 3, 3, 1, True),
+])
+def test_large_forwards_of_many_filters_go_to_the_generic_kernel(gpu, n, c, h, w, k, r, s, stride, thin):
+    """It was up to 2.8 times as fast there.  The sums' order tells the kernels apart."""
+    K = gpu.kernels
+    rng = np.random.default_rng(k)
+    x, wt = gpu.to_device(rng.standard_normal((n, c, h, w)).astype(np.float32)), gpu.to_device(he_normal(rng, (k, c, r, s)))
+    b = gpu.to_device(rng.standard_normal((k,)).astype(np.float32))
+    got = K.conv2d_fwd(x, wt, b, (stride, stride), 0).numpy()
+    with options(gpu, conv_thin=0):
+        generic = K.conv2d_fwd(x, wt, b, (stride, stride), 0).numpy()
+    with options(gpu, conv_thin=2):
+        every = K.conv2d_fwd(x, wt, b, (stride, stride), 0).numpy()
+    assert (generic != every).any()
+    np.testing.assert_array_equal(got, every if thin else generic)
+
+
+def test_a_large_strided_forward_of_six_products(gpu):
+    """Too few products for the order to show: the time does (measured 36 us and, by the vector units, 57)."""
+    K = gpu.kernels
+    rng = np.random.default_rng(6)
+    x, wt = gpu.to_device(rng.standard_normal((354, 6, 50, 50)).astype(np.float32)), gpu.to_device(he_normal(rng, (122, 6, 1, 1)))
+
+    def best(mode):
+        with options(gpu, conv_thin=mode):
+            gpu.profiling(True)
+            try:
+                times = []
+                for _ in range(12):
+                    K.conv2d_fwd(x, wt, None, (2, 2), 0)
+                    times.append(gpu.last_kernel_ms())
+            finally:
+                gpu.profiling(False)
+        return min(times)
+
+    generic, every, rule = best(0), best(2), best(1)
+    assert rule < (generic + every) / 2 < every, (generic, every, rule)

@@ -341,7 +341,7 @@ static FwdPath fwd_path(int N, int C, int H, int W, int K, int R, int S, int sh,
         const size_t need = xsmi::split_fwd_ws_bytes(N, C, H, W, K, R, S, sh, sw, pad, OH, OW);
         if (need && workspace_bytes >= need) return FwdPath::Split;
     }
-    if (!bf16 && xsmi::thin_fwd_ok(C, K, R, S, pad)) return FwdPath::Thin;
+    if (!bf16 && xsmi::thin_fwd_ok(C, K, R, S, sh, sw, pad, (long)N * OH * OW)) return FwdPath::Thin;
     if (first) return FwdPath::FirstLayer;
     if (!bf16 && !(flags & XSMI_CONV_WS_ONLY) && xsmi::sk_path_ok(C, K) && xsmi::sk_fwd_pays(N * OH * OW, K, R, S, sh, sw) &&
         workspace_bytes >= xsmi::sk_fwd_ws_bytes(C, K, R, S))

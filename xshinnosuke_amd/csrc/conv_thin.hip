@@ -193,11 +193,23 @@ void launch_thin_fwd(const ThinParams &p) {
 
 namespace xsmi {
 
-// Up to 16 products the forward was faster at every size tried (from 32 filters on as well: 16 products, 256 filters, 110 MB 36 ->
-// 31 us); at 18 to 32 only while it is small (27 products, 3 MB 10.8 -> 8.5; 27 MB 17 -> 20).
-bool thin_fwd_ok(int C, int K, int R, int S, int pad) {
+// Up to 16 products the forward is the faster one up to 32 filters, which share a gather of x, and in launches that the generic kernel does
+// not fill; of 1350 layers it takes 0.71 of the time (18 to 32 products: only while it is small, 27 products, 3 MB 10.8 -> 8.5; 27 MB
+// 17 -> 20).  It gathers x again for every 32 (8) filters, though, and reads half of every line under a stride, while the generic
+// kernel's tile is free of zeros from 64 filters on.  Not, therefore (generic -> this one, us),
+//   strided, 9 products and more: from 3e6 results on (45 x 16 x 190 x 26 -> 74, 1 x 1 / 2: 14.0 -> 23.8; 285 x 15 x 50 x 50 -> 248: 62 -> 175;
+//     139 x 3 x 27 x 27 -> 316, 2 x 2 / 2, 8.6e6 results: 18.5 -> 16.9; 58 x 58 -> 120, 1 x 3 / 2, 1.6e7: 25 -> 31; below 0.72 in the mean);
+//   strided, 5 to 8 products for more than 96 filters: from 2.5e7 results on (354 x 6 x 50 x 50 -> 122, 1 x 1 / 2: 36 -> 57; at 2.2e7 0.95);
+//   stride 1, 9 products and more for more than 96 filters: from 1.4e7 results on at 1 x 1 (37 x 11 x 70 x 70 -> 125: 30 -> 36), where
+//     neighbouring taps share no lines, from 4e7 on otherwise (169 x 1 x 44 x 16 -> 440, 3 x 3: 47 -> 50).
+bool thin_fwd_ok(int C, int K, int R, int S, int sh, int sw, int pad, long pixels) {
     const long mode = option(OPT_CONV_THIN);
-    return mode && pad < 32768 && C * R * S <= (mode == 2 ? MAX_J : 16);
+    const int J = C * R * S;
+    if (!mode || pad >= 32768 || J > (mode == 2 ? MAX_J : 16)) return false;
+    if (mode == 2 || K <= 32) return true;
+    const double results = (double)pixels * K;
+    if (sh > 1 || sw > 1) return J > 8 ? results < 3e6 : J <= 4 || K <= 96 || results < 2.5e7;
+    return J <= 8 || K <= 96 || results < (R * S == 1 ? 1.4e7 : 4e7);
 }
 
 // The weight gradient gathers x again for every group of filters, while the generic kernel's tile of 64 filters is free of zeros

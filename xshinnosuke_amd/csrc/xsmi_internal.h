@@ -191,7 +191,7 @@ int stem_split_fwd(const float *x, const float *w, const float *bias, float *y, 
 
 // forward and weight gradient of few products a result on the vector units (conv_thin.hip), fp32; the forward needs no workspace,
 // the weight gradient at most what conv_bwd_weight_ws_bytes says, which is what it is to be told
-bool thin_fwd_ok(int C, int K, int R, int S, int pad);
+bool thin_fwd_ok(int C, int K, int R, int S, int sh, int sw, int pad, long pixels);
 bool thin_wgrad_ok(int C, int K, int R, int S, int pad);
 int thin_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W, int K, int R,
                   int S, int sh, int sw, int pad, int OH, int OW, int relu);
