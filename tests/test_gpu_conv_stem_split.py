@@ -94,3 +94,19 @@ def test_a_workspace_without_room_for_a_copy(gpu):
     z = gpu.empty(want.shape)
     capi.lib.call("xsmi_conv2d_fwd_noalloc", x.ptr, w.ptr, None, z.ptr, None, *dims, 0)
     np.testing.assert_array_equal(z.numpy(), want)
+
+
+@pytest.mark.parametrize("n,c,h,w,k,r,pad,split", [
+    (244, 1, 12, 12, 177, 7, 0, False),      # 9 outputs in a tile of 256, three row tiles
+    (210, 3, 14, 9, 186, 7, 0, False),
+    (77, 1, 56, 21, 240, 7, 3, False),       # 0.60 full
+    (28, 1, 12, 12, 177, 7, 0, True),        # the same in 84 tiles
+    (70, 3, 54, 54, 128, 7, 3, True),        # 27 x 27 outputs: 0.71 full
+])
+def test_images_that_leave_their_tiles_empty_go_to_the_fp32_kernel(gpu, n, c, h, w, k, r, pad, split):
+    """Where there are more tiles than compute units it was up to twice as fast there; the bits tell the kernels apart."""
+    rng = np.random.default_rng(k)
+    x, wt = gpu.to_device(rng.standard_normal((n, c, h, w)).astype(np.float32)), gpu.to_device(he_normal(rng, (k, c, r, r)))
+    got, plain = gpu.kernels.conv2d_fwd(x, wt, None, (2, 2), pad).numpy(), _fp32_kernel(gpu, x, wt, None, pad)
+    assert rel_l2(got, plain) <= TOL
+    assert (got != plain).any() == split

@@ -435,7 +435,7 @@ bool stem_fwd_ok(int N, int C, int H, int W, int K, int R, int S, int sh, int sw
 
 size_t stem_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad) {
     const int OH = (H + 2 * pad - R) / sh + 1, OW = (W + 2 * pad - S) / sw + 1;
-    if (stem_split_pays(C, R, K, sh, sw, OH, OW)) return 0;
+    if (stem_split_pays(N, C, R, K, sh, sw, OH, OW)) return 0;
     const size_t apk = align_up((size_t)ceil_div(K, 64) * R * C * 512 * sizeof(float), 256);
     const size_t xp = align_up((size_t)N * C * (H + 2 * pad) * stem_Wp(W, S, sw, pad, OW) * sizeof(float), 256);
     return apk + xp;
@@ -443,7 +443,7 @@ size_t stem_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh
 
 int stem_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
                   int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace) {
-    if (stem_split_pays(C, R, K, sh, sw, OH, OW)) return stem_split_fwd(x, w, bias, y, mask, N, C, H, W, K, R, pad, OH, OW, relu);
+    if (stem_split_pays(N, C, R, K, sh, sw, OH, OW)) return stem_split_fwd(x, w, bias, y, mask, N, C, H, W, K, R, pad, OH, OW, relu);
     hipStream_t st = stream();
     const int rowtiles = ceil_div(K, 64);
     const int Hp = H + 2 * pad, Wp = stem_Wp(W, S, sw, pad, OW);

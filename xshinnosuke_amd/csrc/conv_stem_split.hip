@@ -304,12 +304,20 @@ __global__ void __launch_bounds__(SS_THREADS) stem_split_kernel(StemSplitParams 
     }
 }
 
+// Tiles of 16 x 16 where they cover the image with fewer (112 x 112: 49 against 56); of 32 x 8, whose rows are whole cache
+// lines, otherwise.
+int stem_tile_width(int OY, int OX) {
+    const double wide = (double)xsmi::ceil_div(OX, 32) * xsmi::ceil_div(OY, 8), square = (double)xsmi::ceil_div(OX, 16) * xsmi::ceil_div(OY, 16);
+    return square < wide ? 16 : 32;
+}
+double stem_split_tiles(int OY, int OX) {
+    const int tx = stem_tile_width(OY, OX);
+    return (double)xsmi::ceil_div(OX, tx) * xsmi::ceil_div(OY, 256 / tx);
+}
+
 template <int R, int C>
 void stem_split_launch(StemSplitParams p, int N, int rowtiles) {
-    // tiles of 16 x 16 where they cover the image with fewer (112 x 112: 49 against 56); of 32 x 8, whose rows are whole cache
-    // lines, otherwise
-    const int wide = xsmi::ceil_div(p.OX, 32) * xsmi::ceil_div(p.OY, 8), square = xsmi::ceil_div(p.OX, 16) * xsmi::ceil_div(p.OY, 16);
-    const int tx = square < wide ? 16 : 32, across = xsmi::ceil_div(p.OX, tx), down = xsmi::ceil_div(p.OY, 256 / tx);
+    const int tx = stem_tile_width(p.OY, p.OX), across = xsmi::ceil_div(p.OX, tx), down = xsmi::ceil_div(p.OY, 256 / tx);
     p.tiles = (uint32_t)N * (uint32_t)(across * down);
     p.dTX = xsmi::make_fastdiv(across); p.dTY = xsmi::make_fastdiv(down);
     uint32_t groups = (uint32_t)xsmi::cu_count() & ~7u;              // one a compute unit: the filter fills half of its LDS
@@ -325,11 +333,17 @@ void stem_split_launch(StemSplitParams p, int N, int rowtiles) {
 
 namespace xsmi {
 
-// Of what stem_fwd_ok serves: stride 2 in both directions, images of fewer than 2^29 outputs (byte offsets), and 21 terms and
-// more: with one channel and 3 x 3 or 5 x 5 taps a step of 16 has too few (8 x 1 x 112 x 112 -> 320, 5 x 5: 15.1 -> 17.0 us).
-bool stem_split_pays(int C, int R, int K, int sh, int sw, int OH, int OW) {
-    return option(OPT_CONV_SPLIT) != 0 && option(OPT_TAP_SK) == 1 && sh == 2 && sw == 2 && (C == 3 || R == 7) &&
-           (size_t)K * OH * OW < ((size_t)1 << 29);
+// Of what stem_fwd_ok serves: stride 2 in both directions, images of fewer than 2^29 outputs (byte offsets), 21 terms and
+// more: with one channel and 3 x 3 or 5 x 5 taps a step of 16 has too few (8 x 1 x 112 x 112 -> 320, 5 x 5: 15.1 -> 17.0 us); and tiles
+// that the image fills to five eighths, unless every tile has a compute unit.  The fp32 kernel's tiles go on from image to image, these do not
+// (fp32 -> split: 244 x 1 x 12 x 12 -> 177, 7 x 7, 3 x 3 outputs in tiles of 256: 9.7 -> 17.8; 210 x 3 x 14 x 9 -> 186, 7 x 7: 16 -> 34; 89 x 3 x
+// 39 x 39 -> 163, 3 x 3, 0.47 full: 20 -> 27; 77 x 1 x 56 x 21 -> 240, 0.60: 17 -> 22).  705 layers: 0.76 of the fp32 kernel's time in the mean, at
+// most 1.04.
+bool stem_split_pays(int N, int C, int R, int K, int sh, int sw, int OH, int OW) {
+    if (option(OPT_CONV_SPLIT) == 0 || option(OPT_TAP_SK) != 1 || sh != 2 || sw != 2 || (C != 3 && R != 7) || (size_t)K * OH * OW >= ((size_t)1 << 29))
+        return false;
+    const double tiles = stem_split_tiles(OH, OW);
+    return (double)N * tiles * ceil_div(K, 64) <= (double)cu_count() || 8.0 * OH * OW >= 5.0 * 256.0 * tiles;
 }
 
 int stem_split_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W, int K, int R,

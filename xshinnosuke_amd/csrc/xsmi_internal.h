@@ -185,7 +185,7 @@ bool stem_fwd_ok(int N, int C, int H, int W, int K, int R, int S, int sh, int sw
 size_t stem_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad);
 int stem_conv_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W,
                   int K, int R, int S, int sh, int sw, int pad, int OH, int OW, int relu, int opts, void *workspace);
-bool stem_split_pays(int C, int R, int K, int sh, int sw, int OH, int OW);
+bool stem_split_pays(int N, int C, int R, int K, int sh, int sw, int OH, int OW);
 int stem_split_fwd(const float *x, const float *w, const float *bias, float *y, uint8_t *mask, int N, int C, int H, int W, int K, int R,
                    int pad, int OH, int OW, int relu);
 
