@@ -110,3 +110,39 @@ def test_a_large_strided_forward_of_six_products(gpu):
 
     generic, every, rule = best(0), best(2), best(1)
     assert rule < (generic + every) / 2 < every, (generic, every, rule)
+
+
+@pytest.mark.parametrize("geom", [(196, 5, 26, 26, 14, 1, 3, 2, 2, 0), (98, 16, 18, 18, 1, 1, 1, 1, 1, 0), (32, 1, 17, 17, 5, 3, 3, 1, 1, 1),
+                                  (33, 1, 17, 17, 5, 2, 2, 1, 1, 0)])
+def test_weight_gradient_of_some_thirty_to_a_hundred_splits(gpu, geom):
+    """120, 124, 37 and 33 splits: their sums were a chain of loads (16 us for the first two, 9 now, the table-driven kernel 14)."""
+    n, c, h, w, k, r, s, sh, sw, pad = geom
+    K = gpu.kernels
+    rng = np.random.default_rng(k + r)
+    x, wt = rng.standard_normal((n, c, h, w)).astype(np.float32), he_normal(rng, (k, c, r, s))
+    oh, ow = K.conv_out_hw(h, w, r, s, (sh, sw), pad)
+    dy = rng.standard_normal((n, k, oh, ow)).astype(np.float32)
+    _, col = oracle.conv2d_fwd(x, wt, np.zeros(k, np.float32), (sh, sw), pad)
+    zero = np.zeros_like(x)
+    _, dw_ref, db_ref = oracle.conv2d_bwd(dy, x.shape, wt, col, (sh, sw), pad, zero, np.zeros_like(wt), np.zeros(k, np.float32))
+    _, dw_abs, db_abs = oracle.conv2d_bwd(np.abs(dy), x.shape, wt, np.abs(col), (sh, sw), pad, zero, np.zeros_like(wt), np.zeros(k, np.float32))
+    dx_, ddy = gpu.to_device(x), gpu.to_device(dy)
+    dw, db = gpu.empty(wt.shape), gpu.empty((k,))
+    K.conv2d_bwd_weight(ddy, dx_, wt.shape, (sh, sw), pad, dw=dw, db=db)
+    u = 2.0 ** -24
+    assert (np.abs(dw.numpy() - dw_ref) <= 11 * u * dw_abs).all()      # one pixel a thread; 6 + 2 sums, two roundings
+    assert (np.abs(db.numpy() - db_ref) <= 3 * u * db_abs).all()
+
+    def best(mode):
+        with options(gpu, conv_thin=mode):
+            times = []
+            for _ in range(6):
+                events = [gpu.Event() for _ in range(2)]
+                events[0].record()
+                for _ in range(10):
+                    K.conv2d_bwd_weight(ddy, dx_, wt.shape, (sh, sw), pad, dw=dw, db=db)
+                events[1].record()
+                times.append(events[0].elapsed_ms(events[1]))
+        return min(times)
+
+    assert best(1) < best(0)

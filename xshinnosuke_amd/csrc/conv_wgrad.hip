@@ -219,11 +219,13 @@ __global__ void __launch_bounds__(THREADS) wgrad_reduce_kernel(const float *__re
 }
 
 // Many splits of few results (the first layer of the README network: 8 x 4 results, 972 splits) are a chain of loads: 64
-// threads for a result instead of 4, 33 -> 6 us.  Few splits keep 64 neighbouring results for a workgroup.
+// threads for a result instead of 4, 33 -> 6 us.  Few splits keep 64 neighbouring results for a workgroup.  Where all results are
+// few (`thin`) that is from 33 splits on, the first that four threads do not fetch at once (whole weight gradient, 196 x 5 x 26 x 26 -> 14,
+// 1 x 3 / 2, 120 splits: 16.3 -> 9.2 us; 98 x 16 x 18 x 18 -> 1, 1 x 1, 124: 15.7 -> 8.7).
 void launch_wgrad_reduce(const float *part, float *dw, const float *dbpart, float *db, int K, int J, int Kp, int Jp, int splits,
-                         int accumulate) {
+                         int accumulate, bool thin) {
     hipStream_t st = xsmi::stream();
-    const int cl = splits >= 128 ? 16 : 64;
+    const int cl = splits >= (thin ? 33 : 128) ? 16 : 64;
     const int dw_blocks = K * xsmi::ceil_div(J, cl), blocks = dw_blocks + (db ? xsmi::ceil_div(K, cl) : 0);
     if (cl == 16)
         hipLaunchKernelGGL((wgrad_reduce_kernel<16, 1024>), dim3(blocks), dim3(1024), 0, st, part, dw, dbpart, db, K, J, Kp, Jp, splits,
@@ -262,7 +264,7 @@ size_t conv_bwd_weight_ws_bytes(int N, int C, int K, int R, int S, int OH, int O
 
 int wgrad_reduce_partials(const float *part, float *dw, const float *dbpart, float *db, int K, int J, int Kp, int Jp, int splits,
                           int accumulate) {
-    launch_wgrad_reduce(part, dw, dbpart, db, K, J, Kp, Jp, splits, accumulate);
+    launch_wgrad_reduce(part, dw, dbpart, db, K, J, Kp, Jp, splits, accumulate, true);
     XSMI_LAUNCH_CHECK("wgrad_reduce_kernel");
     return XSMI_OK;
 }
@@ -332,7 +334,7 @@ int xsmi_conv2d_bwd_weight(const float *dy, const float *x, float *dw, float *db
     xsmi::prof_end();
     XSMI_LAUNCH_CHECK("wgrad_f32_kernel");
     const int acc = beta == 1.f ? 1 : 0;
-    launch_wgrad_reduce(p.part, dw, dbpart, db, K, p.J, p.Kp, p.Jp, splits, acc);
+    launch_wgrad_reduce(p.part, dw, dbpart, db, K, p.J, p.Kp, p.Jp, splits, acc, false);
     XSMI_LAUNCH_CHECK("wgrad_reduce_kernel");
     return XSMI_OK;
 }

@@ -228,8 +228,8 @@ bool stem_wgrad_ok(int N, int C, int H, int W, int K, int R, int S, int sh, int 
 size_t stem_wgrad_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad);
 int stem_conv_bwd_weight(const float *dy, const float *x, float *dw, float *db, int N, int C, int H, int W, int K, int R, int S,
                          int sh, int sw, int pad, int OH, int OW, int accumulate, void *workspace);
-// dw[k][j] = (accumulate ? dw : 0) + sum over splits of part[split][k][j] (float64, ascending), db likewise from
-// dbpart[split][k] when given (conv_wgrad.hip)
+// dw[k][j] = (accumulate ? dw : 0) + sum over splits of part[split][k][j] (float64, in a fixed order), db likewise from
+// dbpart[split][k] when given; for the few results of conv_thin.hip (conv_wgrad.hip)
 int wgrad_reduce_partials(const float *part, float *dw, const float *dbpart, float *db, int K, int J, int Kp, int Jp, int splits,
                           int accumulate);
 
