@@ -400,6 +400,10 @@ def test_bf16_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad):
     (1, 512, 32, 32, 352, 2, 2, 2, 0, True, False),      # one tap a class
     (1, 512, 7, 7, 512, 3, 3, 1, 1, True, True),
     (14, 23, 48, 48, 32, 4, 2, 1, 0, True, False),       # 32 channels to at most 32 rows
+    (3, 9, 12, 11, 32, 3, 3, 2, 1, True, False),         # the same strided
+    (6, 65, 10, 10, 32, 7, 7, 2, 3, True, True),         # more rows
+    (1, 83, 7, 7, 32, 7, 7, 2, 3, True, False),          # ... of few pixels
+    (3, 9, 12, 11, 64, 3, 3, 2, 1, True, True),          # more channels
     (44, 160, 47, 45, 64, 2, 2, 1, 1, True, False),      # more tiles than units: four taps an image,
     (40, 64, 54, 54, 64, 3, 3, 1, 1, True, True),        # nine,
     (20, 128, 64, 64, 64, 3, 3, 1, 0, True, False),      # six and three

@@ -1362,19 +1362,22 @@ int split_pack_launch(bool launch) {
 //     63, N=5, 312 tiles: 53 -> 49; 476 -> 224 at 68 x 68, N=2, 304: 42 -> 48; 320 -> 320 at 59 x 67, N=4, 384: 51 -> 57), beyond with
 //     twice as many filters as channels and whole row tiles (128 -> 256 at 28 x 28, N=128: 100 -> 89; 113 -> 256 at 36 x 36, N=41:
 //     51 -> 62; 224 -> 128 at 54 x 54, N=22: 58 -> 108; 384 -> 128 at 48 x 29, N=126: 230 -> 324).
-//   Strided, where one pixel tile holds a class of more than one tap (512 -> 352, 2 x 2 / 2 at 32 x 32, N=1: 24 -> 27).
+//   Strided, where one pixel tile holds a class of more than one tap (512 -> 352, 2 x 2 / 2 at 32 x 32, N=1: 24 -> 27), but for 32
+//     channels to at most 32 rows, as above, or of fewer than 256 pixels (9 -> 32, 3 x 3 / 2 at 12 x 11, N=3: 11.7 -> 14.4; 2 -> 32, 5 x 5 / 2
+//     at 10 x 10: 13.7 -> 17.8; 42 -> 32, 3 x 3 / 2 at 6 x 6, N=3: 12.1 -> 14.9; 70 -> 32, 7 x 7 / 2 at 18 x 18: 25.7 -> 21.0).
 // The forward stays with the channels-last kernels: its sums have one order, whatever the batch and the form of the result.
 static bool split_bf16_plan_pays(const SpParams &p, int sh, int sw, long pixels) {
     const uint32_t tiles = sp_tiles(p), cus = (uint32_t)cu_count();
     const int rows = p.cls[0].rows;
+    const bool few = p.CH < 64 && rows <= SP_TILINGS[2].rows();
     if (sh > 1 || sw > 1) {
         int taps = 0;
         for (int i = 0; i < p.ncls; ++i) taps += p.cls[i].taps;
-        if (pixels <= 256L * sh * sw) return taps > sh * sw;
+        if (pixels <= 256L * sh * sw) return taps > sh * sw && !few && (p.CH >= 64 || pixels >= 256);
         if (!SP_TILINGS[p.tiling].parts || taps <= 2 * sh * sw) return false;
         return tiles <= cus || (4 * tiles <= 5 * cus && 4 * p.CH >= 3 * rows) || (p.CH >= 2 * rows && rows % SP_TILINGS[3].rows() == 0);
     }
-    if (tiles <= cus) return p.CH >= 64 || rows > SP_TILINGS[2].rows();
+    if (tiles <= cus) return !few;
     return p.CH >= 64 && (rows <= SP_TILINGS[2].rows() ||
                           (p.cls[0].taps >= 9 * p.cls[0].nphase && (rows <= SP_ROWS || sp_fills_rows(rows, SP_TILINGS[1]))));
 }
