@@ -425,6 +425,33 @@ def test_which_kernel_a_data_gradient_takes(gpu, n, c, h, w, k, r, s, st, pad, b
     assert other_bits == split
 
 
+@pytest.mark.parametrize("n,c,h,w,k,r,s,pad,split", [
+    (11, 416, 54, 8, 320, 2, 2, 1, False),               # four taps over several row tiles
+    (21, 384, 65, 43, 118, 2, 2, 1, True),               # ... in one
+    (12, 288, 13, 51, 448, 5, 1, 0, False),              # a filter of one column: few steps,
+    (14, 64, 108, 48, 480, 5, 1, 0, False),              # few of them a tile,
+    (10, 448, 41, 41, 288, 1, 5, 0, True),               # 13440 steps
+    (8, 192, 23, 98, 192, 3, 3, 1, False),               # three blocks of 64 rows, 7992 steps
+    (45, 128, 33, 33, 192, 3, 3, 0, True),               # ... 12960
+    (5, 288, 23, 59, 288, 3, 3, 0, False),               # five, 6318
+    (5, 256, 46, 41, 320, 3, 3, 1, True),                # ... 8208
+    (32, 128, 28, 28, 256, 3, 3, 1, True),
+])
+def test_which_kernel_a_strided_forward_takes(gpu, n, c, h, w, k, r, s, pad, split):
+    """By the rule on either side of its lines, as above."""
+    K = gpu.kernels
+    x, wt, b, _, _ = _data(n, c, h, w, k, r, s, 2, 2, pad, gpu)
+    dx, dw, db = gpu.to_device(x), gpu.to_device(wt), gpu.to_device(b)
+    got = K.conv2d_fwd(dx, dw, db, (2, 2), pad).numpy()
+    old = gpu.set_option("conv_split", 0)
+    try:
+        plain = K.conv2d_fwd(dx, dw, db, (2, 2), pad).numpy()
+    finally:
+        gpu.set_option("conv_split", old)
+    assert rel_l2(got, plain) <= TOL
+    assert (got.tobytes() != plain.tobytes()) == split
+
+
 @pytest.mark.parametrize("count", [1, 20, 21, 43])
 def test_layouts_made_in_one_call(gpu, count):
     """A launch takes the layouts of 20 filters: bit-identical to the layout that a call makes for itself, also where a filter

@@ -1291,7 +1291,14 @@ static bool split_pays(int CH, int R, int S, int sh, int sw, long pixels) {
     if (R * S < 4 || CH < 16) return false;
     return (sh == 1 && sw == 1) || CH % 32 != 0 || pixels <= 256 || sp_parts(CH, R, S, sh, sw);
 }
-// ... and whether this plan does.  Strided backward-data (fp32 kernels -> split, of 190 layers): a tile's steps must pay for its
+// ... and whether this plan does.  Strided forward (fp32 kernels -> split, of 320 layers, 0.79 of the time in the mean, at most 1.09):
+//   not 4 taps over several row tiles, whose phases have a tap each (320 filters, 2 x 2 / 2, 416 x 54 x 8, N=11: 35 -> 46 us; 250, 64 x
+//     107 x 107, N=19: 85 -> 95; one row tile, 118, 384 x 65 x 43, N=21: 95 -> 74);
+//   filters of one row or column from 8000 steps of 32 and more a tile on (288 -> 448, 5 x 1 / 2 at 13 x 51, N=12, 4680: 39 -> 46; 64 -> 480 at
+//     108 x 48, N=14, 20 a tile: 71 -> 77; 448 -> 288, 1 x 5 / 2 at 41 x 41, N=10, 13440: 125 -> 77);
+//   with an odd number of 64-row blocks from 38000 block-steps on (192 -> 192 at 23 x 98, N=8, 7992 steps: 46 -> 54; 512 -> 192 at 20 x 73, N=5,
+//     8640: 51 -> 64; 128 -> 192 at 33 x 33, N=45, 12960: 84 -> 61; 288 -> 288 at 23 x 59, N=5, 6318: 44 -> 47; 320 -> 416 at 23 x 23: 46 -> 45).
+// Strided backward-data (of 190 layers): a tile's steps must pay for its
 // start and its stores, and its second 64 rows must not be zeros, of which the fp32 kernels' 64-row tiles have none.
 //   From twice the forward's steps on where every tile has a compute unit (384 -> 512 at 46 x 31, N=3: 50 -> 45 us; 128 -> 256 at 28
 //     x 28, N=32: 47 -> 44; below, 256 -> 320 at 35 x 35, N=6, 5520 steps: 40 -> 41), from 15000 on where workgroups go from tile to
@@ -1305,11 +1312,15 @@ static uint32_t sp_tiles(const SpParams &p) {
     for (int i = 0; i < p.ncls; ++i) tiles += (p.cls[i].end_unit - p.cls[i].first_unit) / p.cls[i].iters;
     return tiles;
 }
-static bool split_plan_pays(const SpParams &p, int sh, int sw, long pixels, bool backward) {
+static bool split_plan_pays(const SpParams &p, int R, int S, int sh, int sw, long pixels, bool backward) {
     if (option(OPT_CONV_SPLIT) >= 2 || (sh == 1 && sw == 1) || p.CH % 32 != 0 || pixels <= 256) return true;
     if (!SP_TILINGS[p.tiling].parts) return false;
-    if (!backward) return true;
     const int rows = p.cls[0].rows, blocks = p.cls[0].blocks;
+    if (!backward) {
+        if (R * S == 4 && rows > SP_TILINGS[3].rows()) return false;
+        if ((R == 1 || S == 1) && (p.units < 8000 || p.cls[0].iters < 32)) return false;
+        return blocks % 2 == 0 || (double)p.units * blocks >= 38000.0;
+    }
     if (p.CH < (rows % SP_TILINGS[3].rows() == 0 ? 128 : 256)) return false;
     if (blocks % 2 != 0) return blocks >= 7 && p.units >= 50000;
     return p.units >= (sp_tiles(p) <= (uint32_t)cu_count() ? 2 * SP_STRIDED_UNITS : 15000u);
@@ -1319,7 +1330,7 @@ static bool split_plan_pays(const SpParams &p, int sh, int sw, long pixels, bool
 size_t split_fwd_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
     SpParams p;
     if (option(OPT_CONV_SPLIT) == 0 || !split_pays(C, R, S, sh, sw, (long)N * OH * OW)) return 0;
-    if (!sp_plan_fwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW) || !split_plan_pays(p, sh, sw, (long)N * OH * OW, false)) return 0;
+    if (!sp_plan_fwd(p, N, C, H, W, K, R, S, sh, sw, pad, OH, OW) || !split_plan_pays(p, R, S, sh, sw, (long)N * OH * OW, false)) return 0;
     return align_up(p.apk_bytes, 256);
 }
 size_t split_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
@@ -1327,7 +1338,7 @@ size_t split_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, 
     if (option(OPT_CONV_SPLIT) == 0 || sh > R || sw > S) return 0;
     const long pixels = (long)N * ceil_div(H, sh) * ceil_div(W, sw);
     if (!split_pays(K, R, S, sh, sw, pixels)) return 0;
-    if (!sp_plan_bwd(p, 3, N, C, H, W, K, R, S, sh, sw, pad, OH, OW) || !split_plan_pays(p, sh, sw, pixels, true)) return 0;
+    if (!sp_plan_bwd(p, 3, N, C, H, W, K, R, S, sh, sw, pad, OH, OW) || !split_plan_pays(p, R, S, sh, sw, pixels, true)) return 0;
     return align_up(p.apk_bytes, 256);
 }
 
