@@ -1360,13 +1360,16 @@ int split_pack_launch(bool launch) {
 // of 500 layers):
 //   from 4 taps on (1 x 1, 128 -> 128 at 56 x 56, N=32: 34 -> 45 us).
 //   Stride 1, launches of at most a tile a compute unit, whose idle units are what the tap-major kernel loses: yes, 0.14 to 0.95 of
-//     the time (512 -> 512 at 7 x 7: N=32 131 -> 33, N=1 110 -> 17; 128 -> 192, 2 x 2 at 29 x 29, N=35: 32 -> 28), but for 32 channels
-//     to at most 32 rows (23 -> 32, 4 x 2 at 48 x 48, N=14: 16 -> 18).
+//     the time (512 -> 512 at 7 x 7: N=32 131 -> 33, N=1 110 -> 17; 128 -> 192, 2 x 2 at 29 x 29, N=35: 32 -> 28), but for at most 32 rows
+//     of 32 channels (23 -> 32, 4 x 2 at 48 x 48, N=14: 16 -> 18) or of few products: channels times taps of an image from 384 on, from
+//     512 in more than 48 tiles (13 -> 96, 4 x 1 at 99 x 199, N=2, two images of two taps: 19 -> 28; 10 -> 64, 4 x 1 at 12 x 87, N=53, 256,
+//     109 tiles: 15 -> 21; 4 -> 64, 2 x 2 at 30 x 30, N=68: 15 -> 19; 7 -> 96, 4 x 1 at 22 x 80, N=45, 384, 155 tiles: 24 -> 27; 6 -> 64, 3 x 2 at
+//     30 x 30, N=11, 384, 20 tiles: 18 -> 15; 9 -> 128, 2 x 2 at 42 x 35, N=36: 22.4 -> 21.8).
 //   Stride 1, larger launches: from 64 reduced channels on (506 -> 32 at 32 x 32, N=125: 125 -> 158) where an image serves nine taps
 //     or more in row tiles three quarters full (128 -> 128 at 28 x 28, N=128: 94 -> 71; 64 -> 64 at 56 x 56, N=256: 220 -> 160;
 //     512 -> 128, 2 x 2 at 42 x 42, N=84: 231 -> 323; 310 -> 160, 1 x 7 at 68 x 46, N=36: 177 -> 202; 249 -> 288 at 50 x 67 without
 //     padding, N=15, whose rows make two images: 150 -> 185; 86 -> 64 at 59 x 59, N=36: 54 -> 58), or for at most 32 rows (16 -> 480,
-//     2 x 3 at 35 x 59, N=59: 209 -> 72).
+//     2 x 3 at 35 x 59, N=59: 209 -> 72), 256 products of an image and more (18 -> 64, 4 x 1 at 39 x 157, N=28, two images: 31 -> 49).
 //   Strided, in the 128 x 128 tiling as in fp32 (64 -> 128 at 56 x 56, N=32, which has 64 rows: 46 -> 54), with more than two taps a
 //     class (193 -> 512, 2 x 2 / 2 at 10 x 62, N=100: 62 -> 100): up to a tile a compute unit (128 -> 256 at 28 x 28, N=32: 40 -> 29;
 //     192 -> 384 at 27 x 27, N=12: 55 -> 33), to one and a quarter with filters for three quarters of the channels (256 -> 352 at 63 x
@@ -1388,8 +1391,9 @@ static bool split_bf16_plan_pays(const SpParams &p, int sh, int sw, long pixels)
         if (!SP_TILINGS[p.tiling].parts || taps <= 2 * sh * sw) return false;
         return tiles <= cus || (4 * tiles <= 5 * cus && 4 * p.CH >= 3 * rows) || (p.CH >= 2 * rows && rows % SP_TILINGS[3].rows() == 0);
     }
-    if (tiles <= cus) return !few;
-    return p.CH >= 64 && (rows <= SP_TILINGS[2].rows() ||
+    if (tiles <= cus)
+        return !few && (rows > SP_TILINGS[2].rows() || p.CH * p.cls[0].taps >= (tiles > 48 ? 512 : 384) * p.cls[0].nphase);
+    return p.CH >= 64 && ((rows <= SP_TILINGS[2].rows() && p.CH * p.cls[0].taps >= 256 * p.cls[0].nphase) ||
                           (p.cls[0].taps >= 9 * p.cls[0].nphase && (rows <= SP_ROWS || sp_fills_rows(rows, SP_TILINGS[1]))));
 }
 size_t split_bf16_bwd_data_ws_bytes(int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int pad, int OH, int OW) {
