@@ -73,7 +73,7 @@ def test_groups_of_filters_in_a_large_forward(gpu):
     (37, 11, 70, 70, 125, 1, 1, 1, False),       # stride 1, 1 x 1: 2.3e7
     (20, 11, 70, 70, 125, 1, 1, 1, True),
     (170, 1, 44, 16, 440, 3, 3, 1, False),       # stride 1, 3 x 3: 4.4e7
-    (100, 1, 44, 16, 440, 3, 3, 1, True),
+    (70, 1, 44, 16, 440, 3, 3, 1, True),
 ])
 def test_large_forwards_of_many_filters_go_to_the_generic_kernel(gpu, n, c, h, w, k, r, s, stride, thin):
     """It was up to 2.8 times as fast there.  The sums' order tells the kernels apart."""

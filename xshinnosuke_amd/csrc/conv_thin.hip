@@ -201,7 +201,8 @@ namespace xsmi {
 //     139 x 3 x 27 x 27 -> 316, 2 x 2 / 2, 8.6e6 results: 18.5 -> 16.9; 58 x 58 -> 120, 1 x 3 / 2, 1.6e7: 25 -> 31; below 0.72 in the mean);
 //   strided, 5 to 8 products for more than 96 filters: from 2.5e7 results on (354 x 6 x 50 x 50 -> 122, 1 x 1 / 2: 36 -> 57; at 2.2e7 0.95);
 //   stride 1, 9 products and more for more than 96 filters: from 1.4e7 results on at 1 x 1 (37 x 11 x 70 x 70 -> 125: 30 -> 36), where
-//     neighbouring taps share no lines, from 4e7 on otherwise (169 x 1 x 44 x 16 -> 440, 3 x 3: 47 -> 50).
+//     neighbouring taps share no lines, from 2e7 on otherwise (169 x 1 x 44 x 16 -> 440, 3 x 3: 47 -> 50; 147 x 2 x 56 x 10 -> 416, 1 x 5,
+//     2.1e7: 26 -> 29; 56 x 3 x 42 x 42 -> 184, 2 x 2, 1.9e7: 27 -> 25).
 bool thin_fwd_ok(int C, int K, int R, int S, int sh, int sw, int pad, long pixels) {
     const long mode = option(OPT_CONV_THIN);
     const int J = C * R * S;
@@ -209,7 +210,7 @@ bool thin_fwd_ok(int C, int K, int R, int S, int sh, int sw, int pad, long pixel
     if (mode == 2 || K <= 32) return true;
     const double results = (double)pixels * K;
     if (sh > 1 || sw > 1) return J > 8 ? results < 3e6 : J <= 4 || K <= 96 || results < 2.5e7;
-    return J <= 8 || K <= 96 || results < (R * S == 1 ? 1.4e7 : 4e7);
+    return J <= 8 || K <= 96 || results < (R * S == 1 ? 1.4e7 : 2e7);
 }
 
 // The weight gradient gathers x again for every group of filters, while the generic kernel's tile of 64 filters is free of zeros
