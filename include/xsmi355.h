@@ -81,9 +81,8 @@ int xsmi_is_initialized(void);
 const char *xsmi_last_error(void);
 int xsmi_device_info(xsmi_device_info_t *info);
 /* Device memory the library itself holds on a GPU once initialised there: the exchange
- * buffers of the fp32 convolution kernels that share tiles between workgroups (one per stream
- * of the library) and
- * the static array of xsmi_conv2d_fwd_noalloc.  Everything else is the caller's
+ * buffers of the convolution kernels that share tiles between workgroups, in float32 and in the bf16
+ * data gradient (one per stream of the library), and the static array of xsmi_conv2d_fwd_noalloc.  Everything else is the caller's
  * (tensors, workspaces).  No counterpart in the reference. */
 size_t xsmi_scratch_bytes(void);
 int xsmi_malloc(void **ptr, size_t bytes);
@@ -101,15 +100,16 @@ int xsmi_memcpy_d2d(void *dst, const void *src, size_t bytes);   /* async on the
 int xsmi_memset(void *dst, int byte_value, size_t bytes);        /* async on the stream (a fill kernel) */
 int xsmi_sync(void);
 /* Tuning switches of the kernel selection, by name: "conv_split" (fp32 convolutions on the bf16 matrix instructions,
- * operands split into three bf16 values: 1: where that pays, 0: never, all products on the fp32 matrix instructions,
- * 2: wherever it applies), "tap_sk" (of the fp32 forward and data gradient; 1: the split-operand kernel where
- * conv_split says so, otherwise an even split of the chunks where that pays; 0: one tile per workgroup only, 3: even
- * split of the chunks wherever it applies, both without the split-operand kernel), "sk_spin_limit" (polls before a
+ * operands split into three bf16 values, and the data gradient under XSMI_CONV_BF16 by the same kernel with one: 1: where that
+ * pays, 0: never, all fp32 products on the fp32 matrix instructions, bf16 data gradients tap by tap, 2: wherever it applies),
+ * "tap_sk" (of the forward and data gradient; 1: the split-operand kernel where
+ * conv_split says so, otherwise, in fp32, an even split of the chunks where that pays; 0: one tile per workgroup only, 3: even
+ * split of the chunks wherever it applies, both without the split-operand kernel, also in the bf16 data gradient), "sk_spin_limit" (polls before a
  * workgroup that shares a tile gives up waiting for another's part of it; the calls that wait for the device then fail
  * with XSMI_ERR_RUNTIME), "sk_wide" (the even-split kernel's activation loads: 2: input rows staged once for the three taps of
  * a filter row where that form pays, 16-byte loads tap by tap where only those apply; 3: staged rows wherever they
- * apply; 1: 16-byte loads tap by tap; 0: one-dword loads everywhere), "pool_bwd" (workgroups per compute unit of the 3x3/2 max-pool gradient kernel whose workgroups walk
- * several pieces; 0: one piece per workgroup), "pack_lanes" (1 to 4: streams over which xsmi_conv2d_pack deals its
+ * apply; 1: 16-byte loads tap by tap; 0: one-dword loads everywhere), "pool_bwd" (workgroups per compute unit of the 3x3/2
+ * max-pool gradient kernel whose workgroups walk several pieces; 0: one piece per workgroup), "pack_lanes" (1 to 4: streams over which xsmi_conv2d_pack deals its
  * layout launches), "wgrad_tile" (the split-operand weight gradient's tile, as the digits of filters, pixels of a stage, pairs
  * of units for a wave and rounds of staging, for instance 646453; 0: the one of the least estimated time), "conv_thin" (forward
  * and weight gradient of at most 32 products a result by the vector units: 1: where that pays, 0: never, 2: wherever it applies), "tap_stages",

@@ -16,10 +16,11 @@
 // Work layout.  Rows = output channels (64 per tile), columns = output pixels in NCHW order (256 per tile, 128 in small
 // launches), 2 x 4 (2 x 2) waves of 32 rows x 64 pixels; passes of at most 32 rows 1 x 8 such waves (sp_plan_tiled).  Waves of
 // 64 x 64 halve the conversion and the LDS reads for a product, but their accumulators and fragments spill (128 -> 128 at 28 x
-// 28, N=256: 305 -> 342 us; the loop runs 1.22 PFLOP/s of bf16 products there, a large library product 1.30).  The reduction is a list of steps (phase, 16 input channels, tap).
-// A PHASE is a set of taps that read one sub-lattice of the input (stride 1: all taps; stride 2: the taps of one row and
-// column parity, and in the 128 x 128 tiling an image holds several phases and channel groups (SpKind); or, where the input rows of all taps together would not fit the LDS, those of as many filter rows as do: 216 -> 2,
-// 5 x 5 at 32 x 32, N=52, in images of 3 and 2 rows instead of five of one: 202 -> 162 us).  In the phase's
+// 28, N=256: 305 -> 342 us; the loop runs 1.22 PFLOP/s of bf16 products there, a large library product 1.30).  The reduction is
+// a list of steps (phase, 16 input channels, tap).  A PHASE is a set of taps that read one sub-lattice of the input.  Stride 1:
+// all taps; stride 2: the taps of one row and column parity; or, where the input rows of all taps together would not fit the
+// LDS, those of as many filter rows as do (216 -> 2, 5 x 5 at 32 x 32, N=52, in images of 3 and 2 rows instead of five of one:
+// 202 -> 162 us).  An LDS image holds a phase, in the 128 x 128 tiling several phases and channel groups (SpKind).  In the phase's
 // own coordinates the walk has stride 1, so a tile needs one run of positions ("slots") of a grid of pitch Wp = OX + taps
 // across - 1, and a tap is nothing but an offset into the run.  The run is staged once per 16 channels for all taps of the
 // phase: float32 values are fetched through registers (lanes = slots, eight channels per lane), split there, and written to
@@ -29,10 +30,10 @@
 // each wave fetches its fragments straight into registers three steps ahead (the waves of a workgroup read the same block at
 // about the same time: L1), so the loop has no barrier except around the image of a channel group.
 //
-// Scheduling is the even split of conv_tap_sk.hip (small launches deal tiles instead, sp_deal_tiles): the steps of all tiles in a row are dealt over the resident workgroups; a
-// workgroup whose range starts inside a tile hands its accumulators to the one that holds the tile's first step, which adds
-// them in ascending order (bounded wait, deterministic sums).  Row tiles vary slowest, so that an XCD's workgroups read few
-// filter blocks.
+// Scheduling is the even split of conv_tap_sk.hip (small launches deal tiles instead, sp_deal_tiles): the steps of all tiles in
+// a row are dealt over the resident workgroups; a workgroup whose range starts inside a tile hands its accumulators to the one
+// that holds the tile's first step, which adds them in ascending order (bounded wait, deterministic sums).  Row tiles vary
+// slowest, so that an XCD's workgroups read few filter blocks.
 #include "conv_store.h"
 #include "split3.h"
 
@@ -1055,9 +1056,10 @@ bool sp_fills_rows(int rows, const SpTiling &k) { return 4 * rows >= 3 * xsmi::c
 //   At most 32 rows leave half of a 64-row tile's matrix work to zeros: tiles of 32 x 512 instead, where 64 x 256 would fill the
 //   chip (44 x 64 -> 16, 83 x 83: 139 -> 87 us; 10 x 448 -> 5, 5 x 5 at 66 x 66: 278 -> 161).  Below that the number of
 //   workgroups bounds the launch, of which there are then half as many (8 x 160 -> 17 at 12 x 59: 25.7 us, 29.5 in wide tiles).
-//   Strided passes of at most nine taps and four groups of channels or more, whose row tiles are three quarters full: 128 x 128.  The sub-lattices that the taps of a 3 x 3 / 2 filter read are disjoint, so
-//   an image of all of them stages no value twice and serves nine taps, where an image a sub-lattice serves one to four; half as
-//   many pixels, so that the four parts fit, for twice as many rows.  Backward-data reads one lattice, with one to four taps a
+//   Strided passes of at most nine taps and four groups of channels or more, whose row tiles are three quarters full: 128 x 128.
+//   The sub-lattices that the taps of a 3 x 3 / 2 filter read are disjoint, so an image of all of them stages no value twice and
+//   serves nine taps, where an image a sub-lattice serves one to four; half as many pixels, so that the four parts fit, for twice
+//   as many rows.  Backward-data reads one lattice, with one to four taps a
 //   class: there the parts are channel groups.  128 -> 256 at 28 x 28, N=32: forward 58 -> 41 us, backward-data 70 -> 47 (fp32
 //   kernels 48 and 49); at N=128 147 -> 98 and 215 -> 124 (153, 154).
 template <typename Plan>

@@ -1,6 +1,7 @@
 // Forward convolution for layers with very few input channels (a network's first layer: 3 -> 64, 7x7, stride 2),
 // fp32 MFMA.  Stride 2 in both directions with three channels or 7 x 7 runs on split operands instead (conv_stem_split.hip: 3 -> 64,
-// 7 x 7 at 224 x 224, N=256 727 -> 412 us); this kernel serves the rest, and what the options keep on the fp32 pipe.
+// 7 x 7 at 224 x 224, N=256 727 -> 412 us); this kernel serves the rest, many images that fill those tiles badly among them, and
+// what the options keep on the fp32 pipe.
 //
 // With three input channels the tap-major kernels have nothing to chunk (they reduce 32 channels per tap) and the
 // table-driven gather kernel spends its time on addresses.  Here the reduction index is (filter row r, channel c,
