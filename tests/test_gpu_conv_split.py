@@ -404,6 +404,7 @@ def test_bf16_data_gradient(gpu, n, c, h, w, k, r, s, sh, sw, pad):
     (45, 7, 22, 80, 96, 4, 1, 1, 0, True, False),        # 384 in 155 tiles,
     (2, 13, 99, 199, 96, 4, 1, 1, 0, True, False),       # in two images of a tile,
     (28, 18, 39, 157, 64, 4, 1, 1, 0, True, False),      # also in more tiles than units,
+    (32, 37, 12, 156, 128, 2, 2, 1, 1, True, False),     # and for more rows,
     (11, 6, 30, 30, 64, 3, 2, 1, 1, True, True),         # in one, 20 tiles
     (3, 9, 12, 11, 32, 3, 3, 2, 1, True, False),         # 32 channels to at most 32 rows, strided
     (6, 65, 10, 10, 32, 7, 7, 2, 3, True, True),         # more rows

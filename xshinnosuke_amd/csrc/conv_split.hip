@@ -1367,6 +1367,8 @@ int split_pack_launch(bool launch) {
 //     512 in more than 48 tiles (13 -> 96, 4 x 1 at 99 x 199, N=2, two images of two taps: 19 -> 28; 10 -> 64, 4 x 1 at 12 x 87, N=53, 256,
 //     109 tiles: 15 -> 21; 4 -> 64, 2 x 2 at 30 x 30, N=68: 15 -> 19; 7 -> 96, 4 x 1 at 22 x 80, N=45, 384, 155 tiles: 24 -> 27; 6 -> 64, 3 x 2 at
 //     30 x 30, N=11, 384, 20 tiles: 18 -> 15; 9 -> 128, 2 x 2 at 42 x 35, N=36: 22.4 -> 21.8).
+//   Stride 1, not where rows are so long that an image has two or three taps of fewer than 1024 products (37 -> 128, 2 x 2 at 12 x 156,
+//     N=32: 27 -> 36; 40 -> 128, 4 x 1 at 14 x 158, N=15: 25 -> 35; 125 -> 288, 2 x 3 at 12 x 127, N=18: 53 -> 60).
 //   Stride 1, larger launches: from 64 reduced channels on (506 -> 32 at 32 x 32, N=125: 125 -> 158) where an image serves nine taps
 //     or more in row tiles three quarters full (128 -> 128 at 28 x 28, N=128: 94 -> 71; 64 -> 64 at 56 x 56, N=256: 220 -> 160;
 //     512 -> 128, 2 x 2 at 42 x 42, N=84: 231 -> 323; 310 -> 160, 1 x 7 at 68 x 46, N=36: 177 -> 202; 249 -> 288 at 50 x 67 without
@@ -1393,6 +1395,7 @@ static bool split_bf16_plan_pays(const SpParams &p, int sh, int sw, long pixels)
         if (!SP_TILINGS[p.tiling].parts || taps <= 2 * sh * sw) return false;
         return tiles <= cus || (4 * tiles <= 5 * cus && 4 * p.CH >= 3 * rows) || (p.CH >= 2 * rows && rows % SP_TILINGS[3].rows() == 0);
     }
+    if (p.cls[0].nphase > 1 && p.cls[0].taps <= 3 * p.cls[0].nphase && p.CH * p.cls[0].taps < 1024 * p.cls[0].nphase) return false;
     if (tiles <= cus)
         return !few && (rows > SP_TILINGS[2].rows() || p.CH * p.cls[0].taps >= (tiles > 48 ? 512 : 384) * p.cls[0].nphase);
     return p.CH >= 64 && ((rows <= SP_TILINGS[2].rows() && p.CH * p.cls[0].taps >= 256 * p.cls[0].nphase) ||
