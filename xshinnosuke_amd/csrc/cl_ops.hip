@@ -79,8 +79,9 @@ __global__ void __launch_bounds__(256) cl_maxpool_kernel(const bf16x8 *__restric
 }
 
 // A workgroup takes 64 octets of channels (consecutive lanes: whole kilobytes of a pixel's record) and deals the plane's pixels
-// over its eight waves.  Sums in float64, as over fp32 planes; of bf16 values (8 bits) they are exact, in any order, while the exponents
-// of a plane span less than 45 less the bits of H W (53 of a double less 8; 39 for 7 x 7).  Bound by the latency of a wave's few loads: 256 x 512 x 7 x 7 5 us, against 40 for the conversion to fp32 and the mean over that.
+// over its eight waves.  Sums in float64, as over fp32 planes; of bf16 values (8 bits) they are exact, in any order, while the
+// exponents of a plane span less than 45 less the bits of H W (53 of a double less 8; 39 for 7 x 7).  Bound by the latency of a
+// wave's few loads: 256 x 512 x 7 x 7 5 us, against 40 for the conversion to fp32 and the mean over that.
 __global__ void __launch_bounds__(512) cl_avgpool_kernel(const bf16x8 *__restrict__ x, float *__restrict__ y, int C8, int H, int W, int b,
                                                           uint32_t octets, xsmi::FastDiv dC8, xsmi::FastDiv dW) {
     __shared__ double part[8][64 * 8];
